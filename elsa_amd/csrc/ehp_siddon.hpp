@@ -222,6 +222,221 @@ namespace ehp
         }
     }
 
+    // ---------------------------------------------------------------------------------
+    // The forward kernel's traversal: plane by plane of the driving axis A, without a loop over the crossings. On a
+    // plane the ray crosses each transverse axis at most once (the driving axis has the largest
+    // |d|), so its crossings there are the sorted values of at most two parameters below the plane's
+    // exit T_A, and three segments (2D: two) cover them. The same parameters, segments and order as
+    // siddon_traverse, so the same crossings bit for bit.
+
+    // State of a ray between two planes: the exit parameter of the last plane, the parameter at
+    // which the ray leaves the volume, per axis the steps taken (as a float: exact below 2^24) and
+    // the next crossing, and the byte offset of the current voxel in a plane of the view with its
+    // changes per step along b1 and b2.
+    struct SidSpan {
+        float t, tend;
+        float ka, kb, kc;
+        float Tb, Tc;
+        uint32_t off;
+        uint32_t db, dc;
+    };
+
+    // The parameter of the crossing by which axis i leaves [0, n): its step number n - cur0 upwards,
+    // cur0 + 1 downwards (T_i rises with the step number)
+    EHP_HD inline float sid_exit_T(const SidRec& r, int i, int n)
+    {
+        const int st = sid_step(r, i);
+        return st == 0 ? kSidMax : sid_T(r, i, st > 0 ? n - 1 - (int) r.cur0[i] : (int) r.cur0[i]);
+    }
+
+    // V: the plane-major view of driving axis A (bytes per row RS4, elements of 2^lg bytes); FB2: its
+    // fastest axis is b2 (else b1).
+    template <int D, int A, bool FB2>
+    EHP_HD inline SidSpan sid_span_init(const SidRec& r, const int* vol, uint32_t RS4, uint32_t lg)
+    {
+        constexpr int b1 = TileAxes<D, A>::b1, b2 = TileAxes<D, A>::b2;
+        SidSpan s;
+        s.t = 0.0f;
+        s.tend = fminf(sid_exit_T(r, 0, vol[0]), sid_exit_T(r, 1, vol[1]));
+        if (D == 3)
+            s.tend = fminf(s.tend, sid_exit_T(r, D - 1, vol[D - 1]));
+        s.ka = s.kb = s.kc = 0.0f;
+        s.Tb = r.T0[b1];
+        s.Tc = D == 3 ? r.T0[b2] : kSidMax;
+        const uint32_t e = 1u << lg;
+        if (D == 3) {
+            const int m = FB2 ? b1 : b2, f = FB2 ? b2 : b1;
+            s.off = mul24((uint32_t) (r.cur0[m] + 2), RS4) + ((uint32_t) (r.cur0[f] + 2) << lg);
+            s.db = (uint32_t) sid_step(r, b1) * (FB2 ? RS4 : e);
+            s.dc = (uint32_t) sid_step(r, b2) * (FB2 ? e : RS4);
+        } else {
+            s.off = (uint32_t) (r.cur0[b1] + 2) << lg;
+            s.db = (uint32_t) sid_step(r, b1) * e;
+            s.dc = 0;
+        }
+        return s;
+    }
+
+    // Smallest and middle of three crossing parameters and the smaller of two, one instruction each
+    // (crossing parameters are never NaN: fminf would first quiet one)
+    EHP_HD inline float sid_min3(float a, float b, float c)
+    {
+#if defined(__HIP_DEVICE_COMPILE__)
+        float r;
+        asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+        return r;
+#else
+        return fminf(fminf(a, b), c);
+#endif
+    }
+    EHP_HD inline float sid_min(float a, float b)
+    {
+#if defined(__HIP_DEVICE_COMPILE__)
+        float r;
+        asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+        return r;
+#else
+        return fminf(a, b);
+#endif
+    }
+    EHP_HD inline float sid_med3(float a, float b, float c)
+    {
+#if defined(__HIP_DEVICE_COMPILE__)
+        float r;
+        asm("v_med3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+        return r;
+#else
+        return fmaxf(fminf(a, b), fminf(fmaxf(a, b), c));
+#endif
+    }
+
+    // Whether the ray may cross a transverse axis twice on one plane of its driving axis A: the
+    // crossings of an axis lie dt apart up to the roundings of two parameters, a plane is dt[A] long up
+    // to the same, and no parameter inside the volume passes tend.
+    template <int D, int A>
+    EHP_HD inline bool sid_may_cross_twice(const SidRec& r, float tend)
+    {
+        constexpr int b1 = TileAxes<D, A>::b1, b2 = TileAxes<D, A>::b2;
+        const float least = D == 3 ? fminf(r.dt[b1], r.dt[b2]) : r.dt[b1];
+        return !(least > r.dt[A] + 4.0f * 1.1920929e-7f * (tend + 2.0f * r.dt[A]));
+    }
+
+    // The values and lengths of the segments of one plane, in ray order (2D: two)
+    template <class T>
+    struct SidSegments {
+        T v1, v2, v3;
+        float w1, w2, w3;
+    };
+
+    template <int D, class T>
+    EHP_HD inline T sid_segments_add(const SidSegments<T>& g, T acc)
+    {
+        acc += g.v1 * (T) g.w1;
+        acc += g.v2 * (T) g.w2;
+        if (D == 3)
+            acc += g.v3 * (T) g.w3;
+        return acc;
+    }
+
+    // The next plane of a ray that crosses each transverse axis at most once on it (ta: its exit;
+    // kb, kc, Tb, Tc: the state after it): its segments (ld(off): the view's element at byte offset off
+    // of the plane), and the ray's state moved past it. Off-path elements are never read: a segment
+    // that is not there reads offset 0, a zero of the padding.
+    template <int D, class T, class Ld>
+    EHP_HD inline SidSegments<T> sid_plane_once(SidSpan& s, float ta, float kb, float kc, float Tb, float Tc, Ld ld)
+    {
+        SidSegments<T> g;
+        const bool sb = s.Tb <= ta, sc = D == 3 && s.Tc <= ta;
+        if (D == 3) {
+            const float first = sid_min3(s.Tb, s.Tc, ta);
+            const float second = sid_min(sid_med3(s.Tb, s.Tc, ta), ta);
+            const uint32_t o2 = s.off + (s.Tb <= s.Tc ? s.db : s.dc), o3 = s.off + (s.db + s.dc);
+            g.v1 = ld(s.off);
+            g.v2 = ld(first < second ? o2 : 0u);
+            g.v3 = ld(second < ta ? o3 : 0u);
+            g.w1 = first - s.t;
+            g.w2 = second - first;
+            g.w3 = ta - second;
+        } else {
+            const float first = sid_min(s.Tb, ta);
+            g.v1 = ld(s.off);
+            g.v2 = ld(first < ta ? s.off + s.db : 0u);
+            g.v3 = T(0);
+            g.w1 = first - s.t;
+            g.w2 = ta - first;
+            g.w3 = 0.0f;
+        }
+        s.off += (sb ? s.db : 0u) + (sc ? s.dc : 0u);
+        s.kb = kb;
+        s.kc = kc;
+        s.Tb = Tb;
+        s.Tc = Tc;
+        s.t = ta;
+        s.ka += 1.0f;
+        return g;
+    }
+
+    // The exit of the ray's next plane and its crossing state after the plane, one crossing per
+    // transverse axis. (An axis that does not move has kb = 0 and dt = T0 = kSidMax: its T stays kSidMax.)
+    template <int D, int A>
+    EHP_HD inline void sid_plane_next(const SidRec& r, const SidSpan& s, float& ta, float& kb, float& kc, float& Tb,
+                                      float& Tc)
+    {
+        constexpr int b1 = TileAxes<D, A>::b1, b2 = TileAxes<D, A>::b2;
+        ta = __builtin_fmaf(s.ka, r.dt[A], r.T0[A]);
+        kb = s.kb + (s.Tb <= ta ? 1.0f : 0.0f);
+        kc = D == 3 ? s.kc + (s.Tc <= ta ? 1.0f : 0.0f) : 0.0f;
+        Tb = __builtin_fmaf(kb, r.dt[b1], r.T0[b1]);
+        Tc = D == 3 ? __builtin_fmaf(kc, r.dt[b2], r.T0[b2]) : kSidMax;
+    }
+
+    // The segments of the next plane of a ray that crosses no axis twice on it (sid_may_cross_twice
+    // says so). After the ray has left the volume (t >= tend) the caller stops; until the end of that
+    // plane it reads the padding's zeros.
+    template <int D, int A, class T, class Ld>
+    EHP_HD inline SidSegments<T> sid_plane_segments(const SidRec& r, SidSpan& s, Ld ld)
+    {
+        float ta, kb, kc, Tb, Tc;
+        sid_plane_next<D, A>(r, s, ta, kb, kc, Tb, Tc);
+        return sid_plane_once<D, T>(s, ta, kb, kc, Tb, Tc, ld);
+    }
+
+    // acc plus the crossings of the next plane of any ray: a plane with two crossings of one axis
+    // (rays at 45 degrees, by rounding) is walked step by step.
+    template <int D, int A, class T, class Ld>
+    EHP_HD inline T sid_plane_add(const SidRec& r, SidSpan& s, T acc, Ld ld)
+    {
+        constexpr int b1 = TileAxes<D, A>::b1, b2 = TileAxes<D, A>::b2;
+        float ta, kb, kc, Tb, Tc;
+        sid_plane_next<D, A>(r, s, ta, kb, kc, Tb, Tc);
+        if (sid_min(Tb, Tc) > ta)
+            return sid_segments_add<D>(sid_plane_once<D, T>(s, ta, kb, kc, Tb, Tc, ld), acc);
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll 1
+#endif
+        for (int g = 0; g < kSidPlaneSteps; ++g) {
+            const float tm = sid_min3(s.Tb, s.Tc, ta);
+            const bool mb = s.Tb <= tm, mc = D == 3 && s.Tc <= tm;
+            acc += ld(s.off) * (T) (tm - s.t);
+            s.t = tm;
+            if (mb) {
+                s.kb += 1.0f;
+                s.Tb = __builtin_fmaf(s.kb, r.dt[b1], r.T0[b1]);
+                s.off += s.db;
+            }
+            if (mc) {
+                s.kc += 1.0f;
+                s.Tc = __builtin_fmaf(s.kc, r.dt[b2], r.T0[b2]);
+                s.off += s.dc;
+            }
+            if (ta <= tm)
+                break;
+        }
+        s.t = ta;
+        s.ka += 1.0f;
+        return acc;
+    }
+
     // The part of the traversal inside the voxel box lo[i] <= c[i] <= hi[i]: fn(c0, c1, c2, w)
     // for exactly the crossings of siddon_traverse whose voxel lies in the box, with the same
     // w. The ray is restarted at the last face crossing before the box: for each axis the step

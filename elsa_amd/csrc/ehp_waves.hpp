@@ -13,7 +13,7 @@ namespace ehp
     // 8 x 8, against 77 % for a 64 x 1 row), while a wider patch reads fewer rows of a plane per
     // step. 8 x 8 for views with one element per voxel (the Joseph forward over them: 7.84 ms
     // at 256^3, 16 x 4: 7.95 ms); 16 x 4 for row-pair views, whose rows are twice as long (the
-    // same forward: 5.7 ms, 8 x 8: 6.9 ms, 32 x 2: 6.0 ms). 2D: 64 pixels of the row per
+    // same forward: 5.7 ms, 8 x 8: 6.9 ms, 32 x 2: 6.0 ms). The Siddon forward has its own (ehp_siddon_planes.hip). 2D: 64 pixels of the row per
     // wavefront, 256 per block.
     constexpr int kFwdWU = 8;
     constexpr int kFwdWUPairs = 16;
