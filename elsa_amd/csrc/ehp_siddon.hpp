@@ -537,6 +537,142 @@ namespace ehp
         }
     }
 
+    // ---------------------------------------------------------------------------------
+    // The back projection's traversal of a tile: the planes of the driving axis in ray order, each
+    // with its segments from the sorted crossing parameters as in the forward, restarted at the
+    // tile's first plane.
+
+    // Number of steps of axis i up to parameter t (T_i(k) <= t), as a float: estimated with an
+    // approximate reciprocal, then stepped to the exact count.
+    EHP_HD inline float sid_steps_until(const SidRec& r, int i, float t)
+    {
+        const float est = (t - r.T0[i]) * ehp_rcp(r.dt[i]);
+        float k = floorf(est) + 1.0f;
+        k = k > 0.0f ? (k < 1.0e7f ? k : 1.0e7f) : 0.0f;
+        // (an axis that does not move has T = kSidMax at k = 0)
+        while (__builtin_fmaf(k, r.dt[i], r.T0[i]) <= t)
+            k += 1.0f;
+        while (k > 0.0f && __builtin_fmaf(k - 1.0f, r.dt[i], r.T0[i]) > t)
+            k -= 1.0f;
+        return k;
+    }
+
+    // Bytes per row of a tile's slots along b1 (8 bytes each): an odd number of slots where the LDS
+    // allows it, so that neighbouring rows fall on different banks.
+    EHP_HD inline int sid_row_slots(const TileCfg& tc, int dim)
+    {
+        const int rows = tc.LA * (dim == 3 ? tc.TC : 1);
+        return dim == 3 && (int64_t) rows * (tc.TB | 1) * 8 + (int64_t) batch_lds_bytes(kMaxPoseBatch) <= 65536
+                   ? (tc.TB | 1)
+                   : tc.TB;
+    }
+
+    // Slot offsets of a tile in bytes: voxel (a, b, c) of the tile's axes at base + (a - A0) plane +
+    // oc + ob with ob = 8 b + nb < maxb and oc = c cs + nc < maxc as unsigned numbers (2D: ob only).
+    struct SidTileOff {
+        uint32_t nb, maxb;
+        int nc, cs;
+        uint32_t maxc, plane, base;
+    };
+
+    template <int D>
+    EHP_HD inline SidTileOff sid_tile_offsets(const TileBox& t, const TileCfg& tc, uint32_t base = 0)
+    {
+        SidTileOff o;
+        o.cs = 8 * sid_row_slots(tc, D);
+        o.nb = (uint32_t) (-8 * t.B0);
+        o.maxb = (uint32_t) (8 * (t.B1 - t.B0));
+        o.nc = -t.C0 * o.cs;
+        o.maxc = (uint32_t) ((t.C1 - t.C0) * o.cs);
+        o.plane = (uint32_t) (o.cs * (D == 3 ? tc.TC : 1));
+        o.base = base;
+        return o;
+    }
+
+    // add(off, w) for exactly the crossings of siddon_traverse whose voxel lies in the tile and whose
+    // length w is not 0, off the byte offset of the voxel's slot. r drives along A and hits the volume.
+    // A ray that has left the volume is outside every tile, as no voxel it would meet comes back.
+    template <int D, int A, class Add>
+    EHP_HD inline void sid_tile_ray(const SidRec& r, const TileBox& t, const SidTileOff& to, Add add)
+    {
+        constexpr int b1 = TileAxes<D, A>::b1, b2 = TileAxes<D, A>::b2;
+        const bool neg = sid_step(r, A) < 0;
+        const int cA = r.cur0[A];
+        // steps along A before the tile's first plane in ray order (negative: the ray starts later)
+        const int d = neg ? cA - (t.A1 - 1) : t.A0 - cA;
+        const int ja = d > 0 ? d : 0;
+        const int p = (neg ? cA - ja : cA + ja) - t.A0; // the first plane to visit, in the tile
+        int n = neg ? p + 1 : t.A1 - t.A0 - p;
+        if (n <= 0)
+            return;
+        float ka = (float) ja;
+        const float tlast = __builtin_fmaf(ka + (float) (n - 1), r.dt[A], r.T0[A]);
+        if (sid_may_cross_twice<D, A>(r, tlast)) {
+            int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
+            lo[A] = t.A0;
+            hi[A] = t.A1 - 1;
+            lo[b1] = t.B0;
+            hi[b1] = t.B1 - 1;
+            if (D == 3) {
+                lo[b2] = t.C0;
+                hi[b2] = t.C1 - 1;
+            }
+            siddon_box<D>(r, lo, hi, [&](int c0, int c1, int c2, float w) {
+                const int ca = A == 0 ? c0 : (A == 1 ? c1 : c2), cb = b1 == 0 ? c0 : c1;
+                const int cc = D == 3 ? (b2 == 1 ? c1 : c2) : 0;
+                if (w != 0.0f)
+                    add(to.base + (uint32_t) (ca - t.A0) * to.plane + (uint32_t) (8 * cb) + to.nb +
+                            (D == 3 ? (uint32_t) (cc * to.cs + to.nc) : 0u),
+                        w);
+            });
+            return;
+        }
+        float t0 = 0.0f, kb = 0.0f, kc = 0.0f;
+        if (ja > 0) {
+            t0 = __builtin_fmaf(ka - 1.0f, r.dt[A], r.T0[A]);
+            kb = sid_steps_until(r, b1, t0);
+            if (D == 3)
+                kc = sid_steps_until(r, b2, t0);
+        }
+        const int sb1 = sid_step(r, b1), sb2 = D == 3 ? sid_step(r, b2) : 0;
+        uint32_t ob = (uint32_t) (8 * ((int) r.cur0[b1] + sb1 * (int) kb)) + to.nb;
+        uint32_t oc = D == 3 ? (uint32_t) (((int) r.cur0[b2] + sb2 * (int) kc) * to.cs + to.nc) : 0u;
+        const uint32_t db = (uint32_t) (8 * sb1), dc = (uint32_t) (sb2 * to.cs);
+        uint32_t poff = to.base + (uint32_t) p * to.plane;
+        const uint32_t dp = neg ? 0u - to.plane : to.plane;
+        float Tb = __builtin_fmaf(kb, r.dt[b1], r.T0[b1]);
+        float Tc = D == 3 ? __builtin_fmaf(kc, r.dt[b2], r.T0[b2]) : kSidMax;
+        for (; n > 0; --n, poff += dp) {
+            const float ta = __builtin_fmaf(ka, r.dt[A], r.T0[A]);
+            const bool sb = Tb <= ta, sc = D == 3 && Tc <= ta;
+            const float first = D == 3 ? sid_min3(Tb, Tc, ta) : sid_min(Tb, ta);
+            const float second = D == 3 ? sid_min(sid_med3(Tb, Tc, ta), ta) : ta;
+            const float w1 = first - t0, w2 = second - first, w3 = ta - second;
+            if (ob < to.maxb && (D == 2 || oc < to.maxc) && w1 != 0.0f)
+                add(poff + ob + oc, w1);
+            // the second segment lies past the axis crossed first, the third past both
+            const bool bf = D == 2 || Tb <= Tc;
+            const uint32_t ob2 = ob + (bf ? db : 0u), oc2 = oc + (bf ? 0u : dc);
+            if (ob2 < to.maxb && (D == 2 || oc2 < to.maxc) && w2 != 0.0f)
+                add(poff + ob2 + oc2, w2);
+            if (D == 3) {
+                const uint32_t ob3 = ob + db, oc3 = oc + dc;
+                if (ob3 < to.maxb && oc3 < to.maxc && w3 != 0.0f)
+                    add(poff + ob3 + oc3, w3);
+            }
+            ob += sb ? db : 0u;
+            oc += sc ? dc : 0u;
+            kb += sb ? 1.0f : 0.0f;
+            Tb = __builtin_fmaf(kb, r.dt[b1], r.T0[b1]);
+            if (D == 3) {
+                kc += sc ? 1.0f : 0.0f;
+                Tc = __builtin_fmaf(kc, r.dt[b2], r.T0[b2]);
+            }
+            t0 = ta;
+            ka += 1.0f;
+        }
+    }
+
     // Slot of voxel c in a tile of the Siddon back projection (no halo: the tile's own voxels,
     // b1 fastest, then b2, then the driving axis).
     template <int D, int A>

@@ -4,9 +4,18 @@
 // :119-120) without global atomics, on the scheme of the tiled Joseph back projection: the
 // volume is cut into tiles long along one driving axis, one workgroup owns a tile for all
 // poses and sums in LDS every crossing of every ray (driving along that axis) that passes
-// through it, then adds the tile to the volume once; one launch per driving axis. A ray
-// enters a tile through siddon_box, which restarts its traversal exactly at the tile's
-// boundary, so every crossing -- voxel and length -- is the one the forward visits.
+// through it, then adds the tile to the volume once; one launch per driving axis.
+//
+// A ray takes the tile's planes in its own order (sid_tile_ray): its state at the first plane
+// follows from the step counts there, and each plane's segments from sorting two crossing
+// parameters, as in the forward, with every lane doing the same work. Restarting the traversal at
+// the tile's boundary and stepping through it crossing by crossing (siddon_box, kept for rays that may cross an axis
+// twice on a plane) took 111 vector instructions a crossing, most of them masked updates of the three axes:
+// 256^3, 360 poses, 384^2 pixels 20.0 -> 10.6 ms; 128^3 2.12 -> 0.94 ms; 2D 256^2 0.131 -> 0.078 ms.
+// The crossings, voxels and lengths are the forward's. Rows of slots are an odd number long
+// (sid_row_slots). Tiles: 8 x 16 x 16 (8 x 17 x 17 11.1 ms, 8 x 15 x 15 11.5, 12 x 16 x 16 11.3, 16 x 16 x 16
+// 12.0, 8 x 24 x 24 12.2, 4 x 32 x 32 13.0). VALU issue and the 64-bit LDS atomics (three a
+// plane) bound it.
 //
 // Sums are 64-bit fixed point as in the Joseph kernel: one exponent per call from max|y|
 // and the slot bound, each contribution y * length rounded once to the unit (fixed_round; in
@@ -18,6 +27,9 @@ namespace ehp
     namespace
     {
         constexpr int kThreads = 256;
+        // LDS (address space 3) pointers: 32-bit byte addresses
+        typedef __attribute__((address_space(3))) unsigned long long lds_u64;
+        typedef __attribute__((address_space(3))) char lds_char;
     } // namespace
 
     template <int D>
@@ -63,7 +75,8 @@ namespace ehp
 
     size_t siddon_tile_lds_bytes(const Dims& dims, const TileCfg& tc, int batch)
     {
-        return (size_t) tc.LA * tc.TB * (dims.dim == 3 ? tc.TC : 1) * sizeof(long long) + batch_lds_bytes(batch);
+        return (size_t) tc.LA * sid_row_slots(tc, dims.dim) * (dims.dim == 3 ? tc.TC : 1) * sizeof(long long) +
+               batch_lds_bytes(batch);
     }
 
     // One tile of the back projection along driving axis A (tile < ntA * ntB * ntC); T = float or
@@ -81,7 +94,9 @@ namespace ehp
 
         const int tid = threadIdx.x;
         const TileBox t = make_tile<D, A>(dims, tc, tile % ntA, (tile / ntA) % ntB, tile / (ntA * ntB));
-        const int nslots = tc.LA * tc.TB * (D == 3 ? tc.TC : 1);
+        const SidTileOff to = sid_tile_offsets<D>(t, tc, (uint32_t) (uintptr_t) (lds_char*) lds);
+        const int row = to.cs / 8; // slots per row
+        const int nslots = tc.LA * row * (D == 3 ? tc.TC : 1);
         long long* iacc = lds;
         const BatchLds bl = batch_lds(lds, nslots, batch);
         CandRect* s_rect = bl.rect;
@@ -89,20 +104,14 @@ namespace ehp
         for (int i = tid; i < nslots; i += kThreads)
             iacc[i] = 0;
         // the tile's voxel box
-        int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
-        lo[A] = t.A0;
-        hi[A] = t.A1 - 1;
-        lo[b1] = t.B0;
-        hi[b1] = t.B1 - 1;
-        if (D == 3) {
-            lo[b2] = t.C0;
-            hi[b2] = t.C1 - 1;
-        }
         float flo[3] = {0.0f, 0.0f, 0.0f}, fhi[3] = {0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int i = 0; i < D; ++i) {
-            flo[i] = (float) lo[i];
-            fhi[i] = (float) (hi[i] + 1);
+        flo[A] = (float) t.A0;
+        fhi[A] = (float) t.A1;
+        flo[b1] = (float) t.B0;
+        fhi[b1] = (float) t.B1;
+        if (D == 3) {
+            flo[b2] = (float) t.C0;
+            fhi[b2] = (float) t.C1;
         }
         const int eg = fixexp[0];
         __syncthreads();
@@ -131,51 +140,60 @@ namespace ehp
             }
             __syncthreads();
             const int total = s_pref[batch];
-            // ray index of candidate k of this batch: pixel (col, row) of its pose's rectangle
-            auto cand_ray = [&](int k) -> int64_t {
-                const int j = batch_pose_slot(s_pref, batch, k);
-                const CandRect cr = s_rect[j];
-                int row, col;
-                rect_split(k - s_pref[j], cr.nu, cr.rnu, row, col);
-                return cr.base + (int64_t) (mul24((uint32_t) row, (uint32_t) dims.det[0]) + (uint32_t) col);
-            };
-            T yv_next = T(0);
-            SidRec r_next{};
-            if (tid < total) {
-                const int64_t ray = cand_ray(tid);
-                yv_next = sino[ray];
-                r_next = table[ray];
-            }
-            for (int k = tid; k < total; k += kThreads) {
-                const T yv = yv_next;
-                const SidRec r = r_next;
-                if (k + kThreads < total) {
-                    const int64_t ray = cand_ray(k + kThreads);
-                    yv_next = sino[ray];
-                    r_next = table[ray];
+            // Candidate k of this batch is entry k - pref[j] of pose j's rectangle, j the last pose with
+            // pref[j] <= k; each lane takes k = tid, tid + kThreads, ... in order, keeping j in
+            // registers. The next candidate is loaded while the current one is added (two register
+            // sets taken in turn).
+            int j = 0, pj = 0, pn = s_pref[1];
+            CandRect cr = s_rect[0];
+            auto fetch = [&](int k, SidRec& r, T& yv) {
+                while (k >= pn) {
+                    ++j;
+                    pj = pn;
+                    pn = s_pref[j + 1];
+                    cr = s_rect[j];
                 }
-                if (yv == T(0) || sid_axis(r) != A)
-                    continue;
+                int rrow, col;
+                rect_split(k - pj, cr.nu, cr.rnu, rrow, col);
+                const int64_t ray = cr.base + (int64_t) (mul24((uint32_t) rrow, (uint32_t) dims.det[0]) + (uint32_t) col);
+                yv = sino[ray];
+                r = table[ray];
+            };
+            auto process = [&](const SidRec& r, T yv) {
+                if (yv == T(0) || !sid_hit(r) || sid_axis(r) != A)
+                    return;
                 // y in units of q (a power-of-two scaling, exact); each crossing adds
                 // y * length rounded once to an integer (|y * length| < 2^51 units: the slot
                 // bound is at least 4096 and lengths are below 2)
                 const double yq = ldexp((double) yv, 62 - eg);
-                siddon_box<D>(r, lo, hi, [&](int c0, int c1, int c2, float w) {
-                    if (w != 0.0f) {
-                        const int slot = sid_slot<D, A>(t, tc, c0, c1, c2);
-                        atomicAdd(reinterpret_cast<unsigned long long*>(iacc + slot), fixed_round(yq, (double) w));
-                    }
+                sid_tile_ray<D, A>(r, t, to, [&](uint32_t off, float w) {
+                    __hip_atomic_fetch_add((lds_u64*) (uintptr_t) off, fixed_round(yq, (double) w), __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_WORKGROUP);
                 });
+            };
+            SidRec ra{}, rb{};
+            T ya = T(0), yb = T(0);
+            if (tid < total)
+                fetch(tid, ra, ya);
+            for (int k = tid; k < total; k += 2 * kThreads) {
+                const int k1 = k + kThreads, k2 = k + 2 * kThreads;
+                if (k1 < total)
+                    fetch(k1, rb, yb);
+                process(ra, ya);
+                if (k2 < total)
+                    fetch(k2, ra, ya);
+                if (k1 < total)
+                    process(rb, yb);
             }
             __syncthreads();
         }
 
         // add the tile to the volume
         const double q = eg == kNonFinite ? __longlong_as_double(0x7ff8000000000000ll) : ldexp(1.0, eg - 62);
-        const int TBe = tc.TB, TCe = D == 3 ? tc.TC : 1;
+        const int TCe = D == 3 ? tc.TC : 1;
         for (int i = tid; i < nslots; i += kThreads) {
-            const int xb = i % TBe;
-            const int rest = i / TBe;
+            const int xb = i % row;
+            const int rest = i / row;
             const int xc = rest % TCe;
             const int xa = rest / TCe;
             const int ca = t.A0 + xa, cb = t.B0 + xb, cc = t.C0 + xc;

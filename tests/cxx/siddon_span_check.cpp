@@ -3,13 +3,16 @@
 // Built with g++ against elsa_amd/csrc/ehp_siddon.hpp (the functions the HIP kernel calls): rays
 // given by origin and direction walk a zero-padded plane-major view (sid_span_init, sid_plane_add)
 // of a volume whose voxels off the ray are NaN. The sum must equal siddon_traverse's bit for bit,
-// and every read must lie in the ray's plane. Used by tests/test_siddon_span.py.
+// and every read must lie in the ray's plane. The same rays through the tiles of the back
+// projection (sid_tile_ray) must give each of the traversal's crossings of nonzero length once, in
+// its slot and with its length. Used by tests/test_siddon_span.py.
 #include "ehp_siddon.hpp"
 
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
 #include <limits>
+#include <map>
 #include <vector>
 
 using namespace ehp;
@@ -64,6 +67,45 @@ namespace
         return 0;
     }
 
+    // every tile of the pass along A: the crossings of ray r by voxel
+    template <int D, int A>
+    int tiles(const Dims& dims, const SidRec& r, const TileCfg& tc)
+    {
+        constexpr int b1 = TileAxes<D, A>::b1, b2 = TileAxes<D, A>::b2;
+        std::map<int64_t, float> full, got;
+        siddon_traverse<D>(r, dims.vol, [&](int c0, int c1, int c2, float w) {
+            if (w != 0.0f)
+                full[c0 + c1 * dims.strides[1] + c2 * dims.strides[2]] = w;
+        });
+        int ntA, ntB, ntC, rc = 0;
+        tile_counts(dims, tc, A, ntA, ntB, ntC);
+        const int row = sid_row_slots(tc, D);
+        for (int tile = 0; tile < ntA * ntB * ntC && !rc; ++tile) {
+            const TileBox t = make_tile<D, A>(dims, tc, tile % ntA, (tile / ntA) % ntB, tile / (ntA * ntB));
+            sid_tile_ray<D, A>(r, t, sid_tile_offsets<D>(t, tc), [&](uint32_t off, float w) {
+                const int slot = (int) (off / 8), xb = slot % row, rest = slot / row;
+                const int xc = D == 3 ? rest % tc.TC : 0, xa = D == 3 ? rest / tc.TC : rest;
+                int c[3] = {0, 0, 0};
+                c[A] = t.A0 + xa;
+                c[b1] = t.B0 + xb;
+                if (D == 3)
+                    c[b2] = t.C0 + xc;
+                if (off % 8 || xa >= t.A1 - t.A0 || c[b1] >= t.B1 || (D == 3 && c[b2] >= t.C1)) {
+                    rc = 4; // outside the tile
+                    return;
+                }
+                const int64_t lin = c[0] + c[1] * dims.strides[1] + c[2] * dims.strides[2];
+                if (!got.emplace(lin, w).second)
+                    rc = 5; // a voxel twice
+            });
+        }
+        if (!rc && got != full) {
+            std::fprintf(stderr, "%zu crossings in the tiles, %zu in the traversal (axis %d)\n", got.size(), full.size(), A);
+            rc = 6;
+        }
+        return rc;
+    }
+
     template <int D, class T>
     int all(const int64_t* n, const float* od, int nrays, const T* data, int64_t* per_axis)
     {
@@ -93,6 +135,10 @@ namespace
                 if (!rc && D == 3)
                     rc = run<D, D - 1, true, T>(d, r, vol);
             }
+            const TileCfg cfgs[] = {{8, 16, 16}, {3, 5, 4}, {1, 2, 1}, {64, 64, 64}};
+            for (const TileCfg& tc : cfgs)
+                if (!rc && sid_hit(r))
+                    rc = a == 0 ? tiles<D, 0>(d, r, tc) : (a == 1 ? tiles<D, 1>(d, r, tc) : tiles<D, D - 1>(d, r, tc));
             if (rc) {
                 std::fprintf(stderr, "ray %d\n", k);
                 return rc;

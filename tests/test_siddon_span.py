@@ -1,5 +1,5 @@
-"""The plane-by-plane Siddon forward against the whole traversal, bit for bit (CPU, the functions the
-HIP kernel calls): random rays and rays that meet edges, corners and faces exactly (ties), drive
+"""The plane-by-plane Siddon forward and the tiles of the back projection against the whole traversal,
+bit for bit (CPU, the functions the HIP kernels call): random rays and rays that meet edges, corners and faces exactly (ties), drive
 along every axis both ways, at 45 degrees (two crossings of one axis on a plane), and along
 faces; voxels off the ray hold NaN, so a read of one shows."""
 import ctypes
