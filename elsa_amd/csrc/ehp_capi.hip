@@ -148,6 +148,12 @@ namespace
     }
 } // namespace
 
+ehp::TileCfg joseph_tile2d(int64_t nvox, int cus)
+{
+    const int t = nvox >= (int64_t) 1024 * cus ? 32 : (nvox >= (int64_t) 256 * cus ? 16 : 8);
+    return ehp::TileCfg{t, t, 1};
+}
+
 extern "C" {
 
 const char* ehp_last_error(void) { return g_last_error.c_str(); }
@@ -248,13 +254,19 @@ namespace
     // cus: compute units of the device. A 3D back projection launch is one workgroup per tile; a
     // small volume gets thinner tiles (fewer planes each) until a launch has about 8 workgroups
     // per CU, which keeps the device busy (128^3: 1024 tiles of 8 planes, 2048 of 4).
+    // 2D Joseph: squares, the largest of 32, 16 and 8 that give every CU a tile (large tiles spend less on their
+    // halo and on rays that only pass a corner; with fewer tiles than CUs the launch waits for its
+    // slowest tile): 512^2 / 360 poses 32: 109 us, 16: 123; 256^2 / 180 16: 34, 32: 59, 8: 41;
+    // 128^2 / 180 8: 26, 16: 34; 64^2 / 90 8: 19, 16: 24.
     ehp::TileCfg default_tile(int kind, const ehp::Dims& dims, int max_lds, int cus)
     {
         ehp::TileCfg tc;
         if (kind == KIND_SIDDON)
             tc = dims.dim == 3 ? ehp::TileCfg{8, 16, 16} : ehp::TileCfg{4, 16, 1};
+        else if (dims.dim == 3)
+            tc = ehp::TileCfg{8, 17, 17};
         else
-            tc = dims.dim == 3 ? ehp::TileCfg{8, 17, 17} : ehp::TileCfg{4, 15, 1};
+            return joseph_tile2d(dims.nvox, cus);
         while (tc.LA > 1 && (int) tile_lds_bytes(kind, dims, tc) > max_lds)
             tc.LA /= 2;
         while (dims.dim == 3 && tc.LA > 2) {
@@ -369,6 +381,8 @@ namespace
             e = hipMalloc((void**) &op->d_maxbits, ehp::kAbsmaxBlocks * sizeof(unsigned long long));
         if (e == hipSuccess)
             e = hipMalloc((void**) &op->d_fixexp, 2 * sizeof(int));
+        if (e == hipSuccess)
+            e = ehp::launch_fill<int>(op->d_fixexp, 2, 0, nullptr); // the exponent's block counter starts at 0
         if (e != hipSuccess)
             return fail(EHP_ERR_ALLOC, "hipMalloc of the Joseph state failed: %s", hipGetErrorString(e));
         e = ehp::joseph_ray_table(op->d_geo, dm, op->d_table, nullptr);
@@ -441,6 +455,8 @@ namespace
             e = hipMalloc((void**) &op->d_maxbits, ehp::kAbsmaxBlocks * sizeof(unsigned long long));
         if (e == hipSuccess)
             e = hipMalloc((void**) &op->d_fixexp, 2 * sizeof(int));
+        if (e == hipSuccess)
+            e = ehp::launch_fill<int>(op->d_fixexp, 2, 0, nullptr); // the exponent's block counter starts at 0
         if (e != hipSuccess)
             return fail(EHP_ERR_ALLOC, "hipMalloc of the Siddon state failed: %s", hipGetErrorString(e));
         e = ehp::siddon_ray_table(op->d_geo, dm, op->d_sidtable, op->d_pose_axes, nullptr);
@@ -510,6 +526,8 @@ namespace
             e = hipMalloc((void**) &op->d_maxbits, ehp::kAbsmaxBlocks * sizeof(unsigned long long));
         if (e == hipSuccess)
             e = hipMalloc((void**) &op->d_fixexp, 2 * sizeof(int));
+        if (e == hipSuccess)
+            e = ehp::launch_fill<int>(op->d_fixexp, 2, 0, nullptr); // the exponent's block counter starts at 0
         if (e != hipSuccess)
             return fail(EHP_ERR_ALLOC, "hipMalloc of the voxel projector state failed: %s", hipGetErrorString(e));
         e = hipMemcpy(op->d_pose_axes, axis.data(), n * sizeof(int), hipMemcpyHostToDevice);
@@ -708,6 +726,11 @@ int ehp_adjoint_noalloc(ehp_op* op, const void* d_sino, void* d_vol, void* strea
     if (e != hipSuccess)
         return hip_fail(e, "ordering after the previous call on this operator");
     const ehp::Dims& dm = op->dims;
+    // the exponent's block counter is shared by every call on the GPU: calls that overlapped against
+    // the contract must not leave it for later ones
+    e = ehp::launch_fill<int>(d_fixexp, 2, 0, s);
+    if (e != hipSuccess)
+        return hip_fail(e, "adjoint launch");
     if (siddon && op->dtype == EHP_F32)
         e = ehp::siddon_adjoint_tiled<float>(op->d_geo, op->d_sidtable, dm, op->d_pose_axes, op->axes_present,
                                              op->tile, op->batch, op->slot_bound, d_maxbits, d_fixexp,

@@ -17,7 +17,7 @@
 // operators keep row-pair views (each element holds a voxel and the one in the next row), so
 // that a sample's four taps are one load (16 bytes in FP32, 8 in bfloat16).
 //
-// Blocks of 256 lanes cover 32 x 8 pixels (64 x 4 with 16 x 4 wavefronts; 2D: 256 x 1) of one
+// Blocks of 256 lanes cover 32 x 8 pixels (64 x 4 with 16 x 4 wavefronts; 2D: fwd2d_block) of one
 // pose. Tiles are ordered detector-row band first, then pose, then column, and each XCD
 // (consecutive workgroups go to different XCDs, so the block index is remapped) takes a
 // contiguous run: the poses of a band then run together on one XCD. For a rotation about y a band of rows sees the same
@@ -104,10 +104,12 @@ namespace ehp
         }
 
         // The rays of group K = 2 * axis + direction of a wavefront share one plane loop over the
-        // group's span. Called with every lane active; `keys` holds the groups present.
+        // group's span, or over parts seg, seg + par, ... of the nseg equal parts of it, the parts summed
+        // apart and then in order. Called with every lane active; `keys` holds the groups present.
         template <int D, int K, bool V16, bool F64>
         __device__ __forceinline__ void fwd_group(int keys, int key, const RayRec& r, const Dims& dims,
-                                                  const ViewSet& vs, int tfirst, int tlast, int s0, double& val)
+                                                  const ViewSet& vs, int tfirst, int tlast, int s0, double& val,
+                                                  int seg = 0, int par = 1, int nseg = 1)
         {
             if (!((keys >> K) & 1))
                 return;
@@ -117,24 +119,44 @@ namespace ehp
             const int ta = wave_max(mine ? tfirst : -0x7fffffff); // every ray of the group has a sample
             const int tb = wave_min(mine ? tlast : 0x7fffffff);   // in [ta, tb]
             const int full0 = ta - t0, full1 = tb - t0 + 1 > full0 ? tb - t0 + 1 : full0;
-            if (mine)
-                val = fwd_span<D, K / 2, (K & 1) != 0, V16, F64>(r, dims, vs, t0, t1 - t0 + 1, s0 + t0 - tfirst,
-                                                                 full0, full1);
+            const int niter = t1 - t0 + 1;
+            if (!mine)
+                return;
+            for (int g = seg; g < nseg; g += par) {
+                const int i0 = niter * g / nseg, i1 = niter * (g + 1) / nseg; // iterations [i0, i1) of the span
+                if (i0 == i1)
+                    continue;
+                const int f0 = min(max(full0 - i0, 0), i1 - i0), f1 = min(max(full1 - i0, f0), i1 - i0);
+                val += fwd_span<D, K / 2, (K & 1) != 0, V16, F64>(r, dims, vs, t0 + i0, i1 - i0,
+                                                                  s0 + t0 + i0 - tfirst, f0, f1);
+            }
         }
+
+        // The views of a volume, copied in one launch: view a takes the blocks from b0[a] on (INT64_MAX:
+        // there is no such view).
+        template <class E>
+        struct CopySet {
+            E* view[3];
+            PadLayout L[3];
+            int gx[3], gy[3];
+            int64_t b0[3];
+        };
 
         template <class E>
         __global__ void __launch_bounds__(256)
-            view_copy_rows_kernel(const E* __restrict__ in, E* __restrict__ out, const Dims dims, const PadLayout L)
+            view_copy_set_kernel(const E* __restrict__ in, const Dims dims, const CopySet<E> cs)
         {
-            view_copy_rows<E>(in, out, dims, L, blockIdx.x);
-        }
-
-        template <class E>
-        __global__ void __launch_bounds__(256)
-            view_copy_transpose_kernel(const E* __restrict__ in, E* __restrict__ out, const Dims dims,
-                                       const PadLayout L)
-        {
-            view_copy_transpose<E>(in, out, dims, L, blockIdx.x, blockIdx.y, blockIdx.z);
+            const int64_t blk = blockIdx.x;
+            const int a = blk >= cs.b0[2] ? 2 : (blk >= cs.b0[1] ? 1 : 0);
+            const PadLayout& L = cs.L[a];
+            const int64_t b = blk - cs.b0[a];
+            if (L.f == 0) {
+                view_copy_rows<E>(in, cs.view[a], dims, L, b);
+            } else {
+                const int64_t gxy = (int64_t) cs.gx[a] * cs.gy[a];
+                const int bz = (int) (b / gxy), r = (int) (b - bz * gxy);
+                view_copy_transpose<E>(in, cs.view[a], dims, L, r % cs.gx[a], r / cs.gx[a], bz);
+            }
         }
 
         // Block id of one pose-band tile of the forward: id = (band * nposes + pose) * tiles_u + tu.
@@ -184,6 +206,75 @@ namespace ehp
             }
         }
 
+        // 2D: a launch has few wavefronts and each ray a long chain of dependent steps, so latency bounds
+        // it: four samples in flight per wavefront (plane_span_forward) and up to four wavefronts per
+        // 64 rays. 64^2 / 90 poses 21.5 -> 5.4 us, 256^2 / 180 59.7 -> 15.8 (kernel), 512^2 / 360
+        // 149 -> 72 (with the view copies).
+        // Block of the 2D forward whose wavefronts sum `par` of the nseg parts of their rays' spans each
+        // at once (par wavefronts share 64 rays; 1 or nseg): the parts' FP64 sums are added in order
+        // either way, so par does not change the result. id = pose * tiles_u + tu, kThreads / par
+        // pixels a block.
+        template <class OT>
+        __device__ __forceinline__ void fwd2d_block(const PoseGeom* __restrict__ geo, const Dims& dims,
+                                                    const ViewSet& views, const int nseg, const int par,
+                                                    const int tiles_u, const int64_t id, OT* __restrict__ sino)
+        {
+            __shared__ double part[kThreads];
+            const int lane = (int) threadIdx.x % 64, w = (int) threadIdx.x / 64;
+            const int pose = (int) (id / tiles_u), seg = w % par;
+            const int u = (int) (id % tiles_u) * (kThreads / par) + (w / par) * 64 + lane;
+            const bool inside = u < dims.det[0];
+            RayRec r{};
+            int key = -1, tfirst = 0, tlast = 0, s0 = 0;
+            if (inside) {
+                float o[3], d[3];
+                make_ray_px<2>(geo[pose], dims, u, 0, o, d);
+                JRay jr;
+                joseph_setup<2>(o, d, dims.vol, jr);
+                r = make_ray_rec<2>(jr);
+                if (plane_ray_span(r, dims.vol[jr.axis], tfirst, tlast, s0))
+                    key = 2 * jr.axis + ((r.meta & 4) ? 1 : 0);
+            }
+            constexpr bool V16 = sizeof(OT) == 2, F64 = sizeof(OT) == 8;
+            const int keys = wave_or(key >= 0 ? 1 << key : 0);
+            double sum = 0.0;
+            fwd_group<2, 0, V16, F64>(keys, key, r, dims, views, tfirst, tlast, s0, sum, seg, par, nseg);
+            fwd_group<2, 1, V16, F64>(keys, key, r, dims, views, tfirst, tlast, s0, sum, seg, par, nseg);
+            fwd_group<2, 2, V16, F64>(keys, key, r, dims, views, tfirst, tlast, s0, sum, seg, par, nseg);
+            fwd_group<2, 3, V16, F64>(keys, key, r, dims, views, tfirst, tlast, s0, sum, seg, par, nseg);
+            if (par > 1) {
+                part[threadIdx.x] = sum;
+                __syncthreads();
+                if (seg == 0)
+                    for (int g = 1; g < par; ++g)
+                        sum += part[threadIdx.x + 64 * g];
+            }
+            if (inside && seg == 0) {
+                OT* out = sino + (int64_t) pose * dims.pix_per_pose + u;
+                if constexpr (F64)
+                    *out = sum;
+                else
+                    *out = down<OT>((float) sum);
+            }
+        }
+
+        template <class OT>
+        __global__ void __launch_bounds__(kThreads)
+            joseph_fwd2d_kernel(const PoseGeom* __restrict__ geo, const Dims dims, const ViewSet views, const int nseg,
+                                const int tiles_u, OT* __restrict__ sino)
+        {
+            fwd2d_block<OT>(geo, dims, views, nseg, nseg, tiles_u, blockIdx.x, sino);
+        }
+
+        // Parts of a 2D ray's span summed apart, a property of the operator (its launches alone and in
+        // a batch give the same sums): as many as four wavefronts per 64 rays while the launch has
+        // few wavefronts for the device's 1024 SIMDs. FP64 operators sum in elsa's order, one part.
+        inline int fwd2d_parts(const Dims& dims, size_t esize)
+        {
+            const int64_t waves = (int64_t) dims.nposes * ((dims.det[0] + 63) / 64);
+            return esize == 8 ? 1 : (waves <= 4096 ? 4 : (waves <= 8192 ? 2 : 1));
+        }
+
         template <int D, class OT, int WU = kFwdWU>
         __global__ void __launch_bounds__(kThreads)
             joseph_fwd_planes_kernel(const PoseGeom* __restrict__ geo, const Dims dims, const ViewSet views,
@@ -225,27 +316,45 @@ namespace ehp
             if (id >= total)
                 return;
             const FwdJob& J = jobs[block_job[id]];
-            fwd_planes_block<D, float>(J.geo, J.dims, J.views, J.tiles_u, id - J.block0, sinos + J.sino_off);
+            if constexpr (D == 2)
+                fwd2d_block<float>(J.geo, J.dims, J.views, J.parts, 1, J.tiles_u, id - J.block0, sinos + J.sino_off);
+            else
+                fwd_planes_block<D, float>(J.geo, J.dims, J.views, J.tiles_u, id - J.block0, sinos + J.sino_off);
         }
     } // namespace
 
+    // The views of every axis present (layouts[a], views[a]) from one volume
     template <class E>
-    hipError_t joseph_view_copy(const Dims& dims, const PadLayout& L, const E* vol, E* view, hipStream_t s)
+    hipError_t joseph_view_copies(const Dims& dims, const PadLayout* layouts, void* const* views, int axes_present,
+                                  const E* vol, hipStream_t s)
     {
-        if (L.f < 0 || L.f > 2 || L.f == L.A)
-            return hipErrorInvalidValue;
-        if (L.f == 0) {
-            const int64_t blocks = (dims.nvox + 255) / 256;
-            hipLaunchKernelGGL((view_copy_rows_kernel<E>), dim3((unsigned) blocks), dim3(256), 0, s, vol, view, dims,
-                               L);
-        } else {
-            const int t = 3 - L.f;
-            const dim3 grid((unsigned) ((dims.vol[0] + kTile - 1) / kTile),
-                            (unsigned) ((dims.vol[L.f] + kTile - 1) / kTile), (unsigned) dims.vol[t]);
-            hipLaunchKernelGGL((view_copy_transpose_kernel<E>), grid, dim3(256), 0, s, vol, view, dims, L);
+        CopySet<E> cs{};
+        int64_t blocks = 0;
+        int n = 0;
+        for (int a = 0; a < dims.dim; ++a) {
+            if (!(axes_present & (1 << a)))
+                continue;
+            if (layouts[a].f < 0 || layouts[a].f > 2 || layouts[a].f == layouts[a].A)
+                return hipErrorInvalidValue;
+            cs.view[n] = (E*) views[a];
+            cs.L[n] = layouts[a];
+            cs.b0[n] = blocks;
+            blocks += view_copy_blocks(dims, layouts[a], cs.gx[n], cs.gy[n]);
+            ++n;
         }
+        for (; n < 3; ++n)
+            cs.b0[n] = INT64_MAX;
+        if (blocks > (int64_t) 0x7fffffff)
+            return hipErrorInvalidValue;
+        if (blocks > 0)
+            hipLaunchKernelGGL((view_copy_set_kernel<E>), dim3((unsigned) blocks), dim3(256), 0, s, vol, dims, cs);
         return hipGetLastError();
     }
+
+    template hipError_t joseph_view_copies<float>(const Dims&, const PadLayout*, void* const*, int, const float*,
+                                                  hipStream_t);
+    template hipError_t joseph_view_copies<double>(const Dims&, const PadLayout*, void* const*, int, const double*,
+                                                   hipStream_t);
 
     // T = float (FP32 operators), bf16 (bfloat16 storage: bfloat16 volume, views and sinogram,
     // FP32 arithmetic) or double (FP64 operators: FP64 views, elsa's FP64 sums)
@@ -255,13 +364,13 @@ namespace ehp
     {
         constexpr uint32_t es = sizeof(T);
         ViewSet vs{};
+        hipError_t e = joseph_view_copies<T>(dims, layouts, views, axes_present, vol, s);
+        if (e != hipSuccess)
+            return e;
         for (int a = 0; a < dims.dim; ++a) {
             if (!(axes_present & (1 << a)))
                 continue;
             const PadLayout& L = layouts[a];
-            hipError_t e = joseph_view_copy<T>(dims, L, vol, (T*) views[a], s);
-            if (e != hipSuccess)
-                return e;
             vs.v[a] = PadView{views[a], L.PS * es, L.RS * es, L.size};
             const int b2 = dims.dim == 3 ? (a == 2 ? 1 : 2) : -1;
             if (L.f == b2)
@@ -269,18 +378,25 @@ namespace ehp
             if (L.pairs)
                 vs.pairs |= 1 << a;
         }
+        if (dims.dim == 2) {
+            const int parts = fwd2d_parts(dims, es);
+            const int tu = (dims.det[0] + kThreads / parts - 1) / (kThreads / parts);
+            const int64_t blocks = (int64_t) tu * dims.nposes;
+            if (blocks > (int64_t) 0x7fffffff)
+                return hipErrorInvalidValue;
+            hipLaunchKernelGGL((joseph_fwd2d_kernel<T>), dim3((unsigned) blocks), dim3(kThreads), 0, s, geo, dims, vs,
+                               parts, tu, sino);
+            return hipGetLastError();
+        }
         // row-pair views (3D) run with wider wavefronts
-        const bool pairs = dims.dim == 3 && vs.pairs != 0;
+        const bool pairs = vs.pairs != 0;
         const FwdGrid fg = fwd_grid(dims, pairs ? kFwdWUPairs : kFwdWU);
         const int tiles_u = fg.tiles_u;
         const int64_t total = fg.total, per_xcd = fg.per_xcd;
         if (per_xcd * 8 > (int64_t) 0x7fffffff)
             return hipErrorInvalidValue;
         const dim3 grid((unsigned) (per_xcd * 8));
-        if (dims.dim == 2)
-            hipLaunchKernelGGL((joseph_fwd_planes_kernel<2, T>), grid, dim3(kThreads), 0, s, geo, dims, vs, tiles_u,
-                               (int) per_xcd, total, sino);
-        else if (pairs)
+        if (pairs)
             hipLaunchKernelGGL((joseph_fwd_planes_kernel<3, T, kFwdWUPairs>), grid, dim3(kThreads), 0, s, geo, dims,
                                vs, tiles_u, (int) per_xcd, total, sino);
         else
@@ -289,9 +405,6 @@ namespace ehp
         return hipGetLastError();
     }
 
-    template hipError_t joseph_view_copy<float>(const Dims&, const PadLayout&, const float*, float*, hipStream_t);
-    template hipError_t joseph_view_copy<bf16>(const Dims&, const PadLayout&, const bf16*, bf16*, hipStream_t);
-    template hipError_t joseph_view_copy<double>(const Dims&, const PadLayout&, const double*, double*, hipStream_t);
     template hipError_t joseph_forward_planes<float>(const PoseGeom*, const Dims&, const PadLayout*, void* const*, int,
                                                      const float*, float*, hipStream_t);
     template hipError_t joseph_forward_planes<bf16>(const PoseGeom*, const Dims&, const PadLayout*, void* const*, int,
@@ -336,6 +449,7 @@ namespace ehp
             }
             const FwdGrid fg = fwd_grid(it.dims);
             fj.tiles_u = fg.tiles_u;
+            fj.parts = it.dims.dim == 2 ? fwd2d_parts(it.dims, sizeof(float)) : 1;
             const int64_t nb = fg.total;
             fj.block0 = (int64_t) fblocks.size();
             fblocks.insert(fblocks.end(), (size_t) nb, (int) fjobs.size());

@@ -1231,6 +1231,14 @@ namespace ehp
         return true;
     }
 
+    // compile-time flags for generic lambdas
+    struct TagTrue {
+        static constexpr bool value = true;
+    };
+    struct TagFalse {
+        static constexpr bool value = false;
+    };
+
     // plane_ray_forward with the plane loop shared by a group of rays of one driving axis and
     // direction (a wavefront, on the GPU): iteration it visits the plane at traversal coordinate
     // t0 + it, the same plane for every ray of the group, so their reads fall on neighbouring
@@ -1253,6 +1261,53 @@ namespace ehp
         const double len = r.len;
         double acc = 0.0;
         int it = 0;
+        if constexpr (D == 2) {
+            // A 2D launch has few wavefronts: four samples are fetched before the first is added, also
+            // where only some rays have a sample (the others read the plane's padding or a voxel, and
+            // add 0)
+            auto four = [&](auto masked) {
+                constexpr bool MASKED = decltype(masked)::value;
+                if constexpr (F64) {
+                    SampleTaps64 T[4];
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+#endif
+                    for (uint32_t k = 0; k < 4; ++k) {
+                        T[k] = plane_sample_taps64<D, A, FB2>(r, dims, V, poff + k * dp, fs + (float) k);
+                        if (MASKED && !(j + k < n))
+                            T[k].v00 = T[k].v10 = 0.0;
+                    }
+                    for (int k = 0; k < 4; ++k)
+                        acc = plane_taps_add64<D, A>(T[k], len, acc);
+                } else {
+                    SampleTaps T[4];
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+#endif
+                    for (uint32_t k = 0; k < 4; ++k) {
+                        T[k] = plane_sample_taps<D, A, FB2, V16, PR>(r, dims, V, poff + k * dp, fs + (float) k);
+                        if (MASKED && !(j + k < n))
+                            T[k].v00 = T[k].v10 = 0.0f;
+                    }
+                    for (int k = 0; k < 4; ++k)
+                        acc = plane_taps_add<D>(T[k], len, acc);
+                }
+                it += 4;
+                j += 4;
+                fs += 4.0f;
+                poff += 4u * dp;
+            };
+            while (it + 4 <= niter) {
+                if (it >= full0 && it + 4 <= full1)
+                    four(TagFalse{});
+                else
+                    four(TagTrue{});
+            }
+            for (; it < niter; ++it, ++j, fs += 1.0f, poff += dp)
+                if (j < n)
+                    acc = plane_sample_add<D, A, FB2, V16, PR, F64>(r, dims, V, poff, fs, len, acc);
+            return acc;
+        }
         for (; it < full0; ++it, ++j, fs += 1.0f, poff += dp)
             if (j < n)
                 acc = plane_sample_add<D, A, FB2, V16, PR, F64>(r, dims, V, poff, fs, len, acc);

@@ -6,15 +6,13 @@
 // tile for all poses: it accumulates in LDS every sample of every ray whose driving axis is
 // a and whose bilinear footprint touches the tile, then adds the tile to the volume once.
 // One launch per driving axis that occurs in the trajectory ("pass"); each voxel is owned by
-// exactly one tile per pass, so passes are plain read-modify-write.
+// exactly one tile per pass, so passes are plain read-modify-write. In 2D a tile takes the rays of
+// both axes (adj2d_block) and one launch writes the volume.
 //
 // Accumulation: LDS float atomics are slow on this part (a ds_add_f32 wave operation costs
 // about 15 times a ds_add_u64), so the tile is summed with 64-bit integer atomics in fixed
 // point: units of q = 2^(eg - 62), eg chosen per call from max|y| and a bound on what one slot
-// can receive, so that no sum can overflow. Each ray rounds its contributions to int32 in its
-// own power-of-two scale (error at most 2^-30 of y * len) and shifts them into units of q: a
-// conversion, a sign extension and a 64-bit shift per tap instead of a float-to-int64
-// conversion. Integer sums do not depend on the order of the additions, so the result is
+// can receive, so that no sum can overflow, each contribution rounded once (fixed_round). Integer sums do not depend on the order of the additions, so the result is
 // bitwise reproducible, whatever the tile shape, and more accurate than a sequential FP32
 // accumulation. A non-finite y makes the whole output NaN (the fixed-point sums cannot carry
 // it to just the voxels it touches).
@@ -87,62 +85,63 @@ namespace ehp
         return m; // valid in thread 0
     }
 
+    // Bit pattern of |x| (FP32 and bfloat16: of its FP32 value), whose integer order is the values'
+    template <class T>
+    __device__ __forceinline__ auto abs_bits(T x)
+    {
+        if constexpr (sizeof(T) == 8)
+            return (unsigned long long) __double_as_longlong(fabs(x));
+        else
+            return __float_as_uint(fabsf(up(x)));
+    }
+
+    __device__ inline double bits_value(unsigned int u) { return __uint_as_float(u); }
+    __device__ inline double bits_value(unsigned long long u) { return __longlong_as_double((long long) u); }
+
+    // fixexp[0] = the fixed-point exponent eg for the slot bound of the operator. Each block reduces its
+    // share of x; the block that finishes last (fixexp[1] counts them and is 0 between launches)
+    // reduces the blocks' maxima, so that the exponent takes one launch.
     template <class T>
     __global__ void __launch_bounds__(256)
-        absmax_kernel(const T* __restrict__ x, int64_t n, unsigned int* __restrict__ partial)
+        absmax_scale_kernel(const T* __restrict__ x, int64_t n, double bound, unsigned long long* __restrict__ partial,
+                            int* __restrict__ fixexp)
     {
-        unsigned int m = 0u;
+        using U = decltype(abs_bits(x[0]));
+        U m = 0;
         const int64_t stride = (int64_t) gridDim.x * blockDim.x;
         for (int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-            const unsigned int u = __float_as_uint(fabsf(up(x[i])));
+            const U u = abs_bits(x[i]);
             m = u > m ? u : m;
         }
         m = block_max_bits(m);
-        if (threadIdx.x == 0)
-            partial[blockIdx.x] = m;
-    }
-
-    // the fixed-point exponent eg for the slot bound of the operator, from the partial maxima
-    __global__ void __launch_bounds__(256)
-        scale_kernel(const unsigned int* __restrict__ partial, int nblocks, double bound, int* __restrict__ fixexp)
-    {
-        unsigned int m = 0u;
-        for (int i = threadIdx.x; i < nblocks; i += blockDim.x)
-            m = partial[i] > m ? partial[i] : m;
-        m = block_max_bits(m);
-        if (threadIdx.x == 0)
-            fixexp[0] = fixed_point_exponent(__uint_as_float(m), bound);
-    }
-
-    // The same in FP64: the bit patterns of non-negative doubles order as the values do.
-    __global__ void __launch_bounds__(256)
-        absmax64_kernel(const double* __restrict__ x, int64_t n, unsigned long long* __restrict__ partial)
-    {
-        unsigned long long m = 0ull;
-        const int64_t stride = (int64_t) gridDim.x * blockDim.x;
-        for (int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-            const unsigned long long u = (unsigned long long) __double_as_longlong(fabs(x[i]));
-            m = u > m ? u : m;
+        __shared__ bool last;
+        if (gridDim.x > 1) {
+            if (threadIdx.x == 0) {
+                __hip_atomic_store(partial + blockIdx.x, (unsigned long long) m, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+                // release of the maximum, acquire of the others' by the block that counts last
+                last = __hip_atomic_fetch_add(fixexp + 1, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
+                       (int) gridDim.x - 1;
+            }
+            __syncthreads();
+            if (!last)
+                return;
+            m = 0;
+            for (int i = threadIdx.x; i < (int) gridDim.x; i += blockDim.x) {
+                const U u = (U) __hip_atomic_load(partial + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                m = u > m ? u : m;
+            }
+            __syncthreads(); // block_max_bits' LDS is read again
+            m = block_max_bits(m);
+            if (threadIdx.x == 0)
+                fixexp[1] = 0;
         }
-        m = block_max_bits(m);
         if (threadIdx.x == 0)
-            partial[blockIdx.x] = m;
+            fixexp[0] = fixed_point_exponent(bits_value(m), bound);
     }
 
-    __global__ void __launch_bounds__(256)
-        scale64_kernel(const unsigned long long* __restrict__ partial, int nblocks, double bound,
-                       int* __restrict__ fixexp)
-    {
-        unsigned long long m = 0ull;
-        for (int i = threadIdx.x; i < nblocks; i += blockDim.x)
-            m = partial[i] > m ? partial[i] : m;
-        m = block_max_bits(m);
-        if (threadIdx.x == 0)
-            fixexp[0] = fixed_point_exponent(__longlong_as_double((long long) m), bound);
-    }
-
-    // d_maxbits holds kAbsmaxBlocks 64-bit partial maxima (FP32 and bfloat16 use its first half
-    // as 32-bit ones)
+    // d_maxbits holds kAbsmaxBlocks 64-bit partial maxima, d_fixexp the exponent and a counter that is
+    // 0 between launches
     template <class T>
     hipError_t fixed_point_exponent_launch(const T* y, int64_t n, double slot_bound, unsigned int* d_maxbits,
                                            int* d_fixexp, hipStream_t s)
@@ -150,14 +149,8 @@ namespace ehp
         // 16 elements per thread at least
         int64_t blocks = (n + 256 * 16 - 1) / (256 * 16);
         blocks = blocks > kAbsmaxBlocks ? kAbsmaxBlocks : (blocks < 1 ? 1 : blocks);
-        if constexpr (sizeof(T) == 8) {
-            unsigned long long* part = reinterpret_cast<unsigned long long*>(d_maxbits);
-            hipLaunchKernelGGL(absmax64_kernel, dim3((unsigned) blocks), dim3(256), 0, s, y, n, part);
-            hipLaunchKernelGGL(scale64_kernel, dim3(1), dim3(256), 0, s, part, (int) blocks, slot_bound, d_fixexp);
-        } else {
-            hipLaunchKernelGGL((absmax_kernel<T>), dim3((unsigned) blocks), dim3(256), 0, s, y, n, d_maxbits);
-            hipLaunchKernelGGL(scale_kernel, dim3(1), dim3(256), 0, s, d_maxbits, (int) blocks, slot_bound, d_fixexp);
-        }
+        hipLaunchKernelGGL((absmax_scale_kernel<T>), dim3((unsigned) blocks), dim3(256), 0, s, y, n, slot_bound,
+                           reinterpret_cast<unsigned long long*>(d_maxbits), d_fixexp);
         return hipGetLastError();
     }
 
@@ -171,13 +164,29 @@ namespace ehp
     // ---------------------------------------------------------------------------------
     // the tiled back projection
 
-    // The candidate rays of one pose batch of one tile, all added into the tile's slots.
+    // The ray value in units of the fixed-point unit q = 2^(eg - 62): FP64 y * len as elsa's FP64
+    // operator forms it, else elsa's FP32 product (both scaled by a power of two, exactly).
+    template <class YT>
+    __device__ __forceinline__ double ray_units(YT yv, float len, int eg)
+    {
+        if constexpr (sizeof(YT) == 8)
+            return ldexp(yv * (double) len, 62 - eg);
+        else
+            return ldexp((double) (yv * len), 62 - eg);
+    }
+
+    __device__ __forceinline__ void lds_add(uint32_t off, unsigned long long v)
+    {
+        __hip_atomic_fetch_add((lds_u64*) (uintptr_t) off, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+
+    // The candidate rays of one pose batch of one 3D tile, all added into the tile's slots.
     // Candidate k (k < total) is pixel k - pref[j] of pose j's rectangle, j the last pose with
     // pref[j] <= k. Each lane walks its candidates k = tid, tid + 256, ... in order, so it keeps
     // its pose j (and j's rectangle) in registers and moves on when k passes pref[j + 1]. The
     // ray state and y of the next candidate are loaded while the current one is added (two
     // register sets taken in turn).
-    template <int D, int A, bool LOW, class ST>
+    template <int A, bool LOW, class ST>
     __device__ __forceinline__ void adj_tile_batch(const RayRec* __restrict__ table, const ST* __restrict__ sino,
                                                    const int det0, const CandRect* s_rect, const int* s_pref,
                                                    const int total, const TileBox& t, const TileOff& to,
@@ -201,24 +210,18 @@ namespace ehp
             r = table[ray];
         };
         auto process = [&](const RayRec& r, YT yv) {
+            const double yq = ray_units(yv, r.len, eg);
             if constexpr (sizeof(YT) == 8) {
                 // FP64: each contribution is elsa's (y * len) * weight in FP64 (the weight in FP32,
                 // as the one-thread-per-ray FP64 kernel forms it), rounded to the nearest multiple of
                 // q; yq is y * len in units of q (a power-of-two scaling, exact)
-                const double yq = ldexp(yv * (double) r.len, 62 - eg);
-                tile_candidate_fx<D, A, LOW, TAP_WEIGHT>(r, t, to, yq, [&](uint32_t off, float w) {
-                    __hip_atomic_fetch_add((lds_u64*) (uintptr_t) off, fixed_round(yq, (double) w), __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_WORKGROUP);
-                });
+                tile_candidate_fx<3, A, LOW, TAP_WEIGHT>(
+                    r, t, to, yq, [&](uint32_t off, float w) { lds_add(off, fixed_round(yq, (double) w)); });
             } else {
                 // FP32 (and bfloat16, widened): elsa's FP32 product y * len in units of q (exact),
                 // times the exact weights, rounded once to the nearest multiple of q
-                const double yq = ldexp((double) (yv * r.len), 62 - eg);
                 // off: the slot's LDS byte address (the tile's base included)
-                tile_candidate_fx<D, A, LOW, TAP_FIXED>(r, t, to, yq, [&](uint32_t off, unsigned long long v) {
-                    __hip_atomic_fetch_add((lds_u64*) (uintptr_t) off, v, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_WORKGROUP);
-                });
+                tile_candidate_fx<3, A, LOW, TAP_FIXED>(r, t, to, yq, lds_add);
             }
         };
         RayRec ra{}, rb{};
@@ -235,6 +238,201 @@ namespace ehp
             if (k1 < total)
                 process(rb, yb);
         }
+    }
+
+    // ---------------------------------------------------------------------------------
+    // 2D: a workgroup owns LA x TB voxels (x by y) for the rays of both driving axes, each with its own
+    // slots, and writes each voxel once: one launch per back projection, with no volume to clear and
+    // none to add to. Few rays of a pose meet a tile, so one step takes many poses at once; while a
+    // launch has few tiles its workgroups are large, as nothing but the number of
+    // wavefronts per tile hides the latency of the ray table and the LDS. Latency bounds the small
+    // problems, the 64-bit LDS atomics and VALU the large ones. Against one launch per axis over 4 x 15 tiles (the pass with the
+    // exponent's launch): 64^2 / 90 poses 42 -> 19 us, 256^2 / 180 73 -> 34, 512^2 / 360 309 -> 109; 64 problems
+    // of 128^2..512^2 in one launch 4635 -> 1129 us.
+
+    constexpr int kPoses2d = 512; // poses per step at most
+
+    // The rays of one pose that can meet the tile: pixels [base, base + count) of the sinogram
+    struct Rays2d {
+        long long base;
+        int cnt, pref;
+    };
+
+    // The tile the 2D back projection runs for the tile tc of the operator: halved until both axes'
+    // slots and a step of poses fit 64 KB.
+    TileCfg tile2d(const TileCfg& tc)
+    {
+        TileCfg t = tc;
+        auto bytes = [&] {
+            return ((int64_t) t.LA * (t.TB + 2) + (int64_t) t.TB * (t.LA + 2)) * 8 + kPoses2d * (int64_t) sizeof(Rays2d);
+        };
+        while (bytes() > 65536 && (t.LA > 1 || t.TB > 1)) {
+            int& m = t.LA >= t.TB ? t.LA : t.TB;
+            m = (m + 1) / 2;
+        }
+        return t;
+    }
+
+    size_t lds2d(const TileCfg& t, int steps)
+    {
+        return ((size_t) t.LA * (t.TB + 2) + (size_t) t.TB * (t.LA + 2)) * 8 + (size_t) (steps + 1) * sizeof(Rays2d);
+    }
+
+    // Poses per step: 16 pose batches, at most the operator's poses
+    int steps2d(const Dims& dims, int batch)
+    {
+        const int s = 16 * batch < kPoses2d ? 16 * batch : kPoses2d;
+        return s < dims.nposes ? s : dims.nposes;
+    }
+
+    template <int NT, class ST>
+    __device__ __forceinline__ void adj2d_block(const PoseGeom* __restrict__ geo, const RayRec* __restrict__ table,
+                                                const Dims& dims, const int* __restrict__ pose_axes, const TileCfg& tc,
+                                                const int ntx, const int tile, const int steps,
+                                                const int* __restrict__ fixexp, const ST* __restrict__ sino,
+                                                typename Acc<ST>::type* __restrict__ vol)
+    {
+        using YT = typename Acc<ST>::type;
+        extern __shared__ long long lds[];
+        const int tid = threadIdx.x;
+        const int ix = tile % ntx, iy = tile / ntx;
+        const TileBox t0 = make_tile<2, 0>(dims, tc, ix, iy, 0);
+        const TileBox t1 = make_tile<2, 1>(dims, TileCfg{tc.TB, tc.LA, 1}, iy, ix, 0);
+        const uint32_t lds0 = (uint32_t) (uintptr_t) (lds_char*) lds;
+        const TileOff o0 = tile_offsets(t0, lds0), o1 = tile_offsets(t1, lds0 + 8u * (uint32_t) t0.nslots);
+        Rays2d* rays = reinterpret_cast<Rays2d*>(lds + t0.nslots + t1.nslots);
+        for (int i = tid; i < t0.nslots + t1.nslots; i += NT)
+            lds[i] = 0;
+        const int eg = fixexp[0];
+        const bool low = tile_low_face<2>(t0) || tile_low_face<2>(t1);
+
+        for (int pbase = 0; eg != kNonFinite && pbase < dims.nposes; pbase += steps) {
+            __syncthreads();
+            for (int i = tid; i < steps; i += NT) {
+                const int p = pbase + i;
+                int u0 = dims.det[0], u1 = -1;
+                if (p < dims.nposes) {
+                    int a0, a1, v0, v1;
+                    if ((pose_axes[p] & 1) && tile_bbox<2, 0>(geo[p], t0, dims, a0, a1, v0, v1)) {
+                        u0 = a0;
+                        u1 = a1;
+                    }
+                    if ((pose_axes[p] & 2) && tile_bbox<2, 1>(geo[p], t1, dims, a0, a1, v0, v1)) {
+                        u0 = a0 < u0 ? a0 : u0;
+                        u1 = a1 > u1 ? a1 : u1;
+                    }
+                }
+                rays[i].base = (long long) p * dims.pix_per_pose + u0;
+                rays[i].cnt = u1 >= u0 ? u1 - u0 + 1 : 0;
+            }
+            __syncthreads();
+            if (tid < 64) {
+                // exclusive prefix of the counts, kPoses2d / 64 consecutive ones a lane
+                constexpr int per = kPoses2d / 64;
+                int sum = 0;
+                for (int i = 0; i < per; ++i)
+                    sum += tid * per + i < steps ? rays[tid * per + i].cnt : 0;
+                int pre = sum;
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int v = __shfl_up(pre, o, 64);
+                    pre += tid >= o ? v : 0;
+                }
+                pre -= sum;
+                for (int i = 0; i < per; ++i)
+                    if (tid * per + i < steps) {
+                        rays[tid * per + i].pref = pre;
+                        pre += rays[tid * per + i].cnt;
+                    }
+                if (tid == 63)
+                    rays[steps].pref = pre;
+            }
+            __syncthreads();
+            const int total = rays[steps].pref;
+            // ray k is pixel k - pref[j] of pose j's pixels, j the last pose with pref[j] <= k; each lane
+            // takes k = tid, tid + NT, ... in order, keeping j in registers
+            int j = 0, pj = 0, pn = rays[1].pref;
+            int64_t base = rays[0].base;
+            auto fetch = [&](int k, RayRec& r, YT& yv) {
+                while (k >= pn) {
+                    ++j;
+                    pj = pn;
+                    pn = rays[j + 1].pref;
+                    base = rays[j].base;
+                }
+                const int64_t ray = base + (k - pj);
+                yv = up(sino[ray]);
+                r = table[ray];
+            };
+            auto walk = [&](auto lw) {
+                constexpr bool LOW = decltype(lw)::value;
+                auto process = [&](const RayRec& r, YT yv) {
+                    const double yq = ray_units(yv, r.len, eg);
+                    if constexpr (sizeof(YT) == 8) {
+                        auto add = [&](uint32_t off, float w) { lds_add(off, fixed_round(yq, (double) w)); };
+                        if ((r.meta & 3) == 0)
+                            tile_candidate_fx<2, 0, LOW, TAP_WEIGHT>(r, t0, o0, yq, add);
+                        else
+                            tile_candidate_fx<2, 1, LOW, TAP_WEIGHT>(r, t1, o1, yq, add);
+                    } else if ((r.meta & 3) == 0) {
+                        tile_candidate_fx<2, 0, LOW, TAP_FIXED>(r, t0, o0, yq, lds_add);
+                    } else {
+                        tile_candidate_fx<2, 1, LOW, TAP_FIXED>(r, t1, o1, yq, lds_add);
+                    }
+                };
+                RayRec ra{}, rb{};
+                YT ya = 0, yb = 0;
+                if (tid < total)
+                    fetch(tid, ra, ya);
+                for (int k = tid; k < total; k += 2 * NT) {
+                    const int k1 = k + NT, k2 = k + 2 * NT;
+                    if (k1 < total)
+                        fetch(k1, rb, yb);
+                    process(ra, ya);
+                    if (k2 < total)
+                        fetch(k2, ra, ya);
+                    if (k1 < total)
+                        process(rb, yb);
+                }
+            };
+            if (low)
+                walk(TagTrue{});
+            else
+                walk(TagFalse{});
+        }
+        __syncthreads();
+
+        // the voxels: the sum of both axes' slots (each axis keeps its own halo)
+        const double q = eg == kNonFinite ? __longlong_as_double(0x7ff8000000000000ll) : ldexp(1.0, eg - 62);
+        const int nx = t0.A1 - t0.A0, ny = t0.B1 - t0.B0;
+        for (int i = tid; i < nx * ny; i += NT) {
+            const int x = i % nx, y = i / nx;
+            const long long sum = lds[x * t0.PB + y + 1] + lds[t0.nslots + y * t1.PB + x + 1];
+            vol[(int64_t) (t0.B0 + y) * dims.strides[1] + t0.A0 + x] = (YT) ((double) sum * q);
+        }
+    }
+
+    template <int NT, class ST>
+    __global__ void __launch_bounds__(NT)
+        joseph_adj2d_kernel(const PoseGeom* __restrict__ geo, const RayRec* __restrict__ table, const Dims dims,
+                            const int* __restrict__ pose_axes, const TileCfg tc, const int ntx, const int steps,
+                            const int* __restrict__ fixexp, const ST* __restrict__ sino,
+                            typename Acc<ST>::type* __restrict__ vol)
+    {
+        adj2d_block<NT, ST>(geo, table, dims, pose_axes, tc, ntx, (int) blockIdx.x, steps, fixexp, sino, vol);
+    }
+
+    // the tiles of many 2D operators in one launch (block b: tile b - job.block0 of job block_job[b])
+    __global__ void __launch_bounds__(256)
+        joseph_adj2d_batch_kernel(const AdjJob* __restrict__ jobs, const int* __restrict__ block_job,
+                                  const int per_xcd, const int64_t total, const int* __restrict__ fixexp,
+                                  const float* __restrict__ sinos, float* __restrict__ vols)
+    {
+        const int64_t id = (int64_t) (blockIdx.x % 8u) * per_xcd + (blockIdx.x / 8u);
+        if (id >= total)
+            return;
+        const AdjJob& J = jobs[block_job[id]];
+        adj2d_block<256, float>(J.geo, J.table, J.dims, J.pose_axes, J.tc, J.ntA, (int) (id - J.block0), J.batch,
+                                fixexp + J.item, sinos + J.sino_off, vols + J.vol_off);
     }
 
     // One tile of the back projection along driving axis A (tile < ntA * ntB * ntC).
@@ -286,9 +484,9 @@ namespace ehp
             __syncthreads();
             const int total = s_pref[batch];
             if (low)
-                adj_tile_batch<D, A, true>(table, sino, dims.det[0], s_rect, s_pref, total, t, to, eg);
+                adj_tile_batch<A, true>(table, sino, dims.det[0], s_rect, s_pref, total, t, to, eg);
             else
-                adj_tile_batch<D, A, false>(table, sino, dims.det[0], s_rect, s_pref, total, t, to, eg);
+                adj_tile_batch<A, false>(table, sino, dims.det[0], s_rect, s_pref, total, t, to, eg);
             __syncthreads();
         }
 
@@ -409,9 +607,27 @@ namespace ehp
         using VT = typename Acc<ST>::type;
         if (batch < 1 || batch > kMaxPoseBatch)
             return hipErrorInvalidValue;
-        hipError_t e = launch_fill<VT>(vol, dims.nvox, VT(0), s);
-        if (e == hipSuccess)
-            e = fixed_point_exponent_launch(sino, dims.nrays, slot_bound, d_maxbits, d_fixexp, s);
+        hipError_t e = fixed_point_exponent_launch(sino, dims.nrays, slot_bound, d_maxbits, d_fixexp, s);
+        if (e != hipSuccess)
+            return e;
+        if (dims.dim == 2) {
+            const TileCfg t = tile2d(tc);
+            const int ntx = (dims.vol[0] + t.LA - 1) / t.LA;
+            const int64_t tiles = (int64_t) ntx * ((dims.vol[1] + t.TB - 1) / t.TB);
+            if (tiles > 0x7fffffff)
+                return hipErrorInvalidValue;
+            const int steps = steps2d(dims, batch);
+            const size_t lds = lds2d(t, steps);
+            // up to two tiles per CU: large workgroups
+            if (tiles <= 512)
+                hipLaunchKernelGGL((joseph_adj2d_kernel<1024, ST>), dim3((unsigned) tiles), dim3(1024), lds, s, geo,
+                                   table, dims, pose_axes, t, ntx, steps, d_fixexp, sino, vol);
+            else
+                hipLaunchKernelGGL((joseph_adj2d_kernel<256, ST>), dim3((unsigned) tiles), dim3(256), lds, s, geo,
+                                   table, dims, pose_axes, t, ntx, steps, d_fixexp, sino, vol);
+            return hipGetLastError();
+        }
+        e = launch_fill<VT>(vol, dims.nvox, VT(0), s);
         if (e != hipSuccess)
             return e;
         const size_t lds = joseph_tile_lds_bytes(dims, tc, batch);
@@ -422,22 +638,15 @@ namespace ehp
             tile_counts(dims, tc, a, ntA, ntB, ntC);
             const int per_xcd = (ntA * ntB * ntC + 7) / 8;
             const dim3 grid((unsigned) (per_xcd * 8));
-#define EHP_ADJ_TILED(Dv, Av)                                                                                      \
-    hipLaunchKernelGGL((joseph_adj_tiled_kernel<Dv, Av, ST>), grid, dim3(kThreads), lds, s, geo, table, dims,         \
-                       pose_axes, tc, ntA, ntB, ntC, per_xcd, batch, d_fixexp, sino, vol)
-            if (dims.dim == 2) {
-                if (a == 0)
-                    EHP_ADJ_TILED(2, 0);
-                else
-                    EHP_ADJ_TILED(2, 1);
-            } else {
-                if (a == 0)
-                    EHP_ADJ_TILED(3, 0);
-                else if (a == 1)
-                    EHP_ADJ_TILED(3, 1);
-                else
-                    EHP_ADJ_TILED(3, 2);
-            }
+#define EHP_ADJ_TILED(Av)                                                                                          \
+    hipLaunchKernelGGL((joseph_adj_tiled_kernel<3, Av, ST>), grid, dim3(kThreads), lds, s, geo, table, dims, pose_axes, \
+                       tc, ntA, ntB, ntC, per_xcd, batch, d_fixexp, sino, vol)
+            if (a == 0)
+                EHP_ADJ_TILED(0);
+            else if (a == 1)
+                EHP_ADJ_TILED(1);
+            else
+                EHP_ADJ_TILED(2);
 #undef EHP_ADJ_TILED
             e = hipGetLastError();
             if (e != hipSuccess)
@@ -508,6 +717,27 @@ namespace ehp
         }
         for (int j = 0; j < n; ++j) {
             const JosephBatchItem& it = items[j];
+            if (it.dims.dim == 2) {
+                // one list for both axes
+                AdjJob aj{};
+                aj.geo = it.geo;
+                aj.table = it.table;
+                aj.pose_axes = it.pose_axes;
+                aj.dims = it.dims;
+                aj.tc = tile2d(it.tile);
+                aj.batch = steps2d(it.dims, it.batch);
+                aj.item = j;
+                aj.sino_off = it.sino_off;
+                aj.vol_off = it.vol_off;
+                aj.ntA = (it.dims.vol[0] + aj.tc.LA - 1) / aj.tc.LA;
+                const int nty = (it.dims.vol[1] + aj.tc.TB - 1) / aj.tc.TB;
+                aj.block0 = (int64_t) ablocks[0].size();
+                ablocks[0].insert(ablocks[0].end(), (size_t) aj.ntA * nty, (int) ajobs[0].size());
+                ajobs[0].push_back(aj);
+                const size_t need = lds2d(aj.tc, aj.batch);
+                lds[0] = need > lds[0] ? need : lds[0];
+                continue;
+            }
             for (int a = 0; a < it.dims.dim; ++a) {
                 if (!(it.axes_present & (1 << a)))
                     continue;
@@ -538,7 +768,7 @@ namespace ehp
                                     unsigned int* d_maxbits, int* d_fixexp, const float* sinos, float* vols,
                                     hipStream_t s)
     {
-        hipError_t e = launch_fill<float>(vols, nvol_total, 0.0f, s);
+        hipError_t e = dim == 2 ? hipSuccess : launch_fill<float>(vols, nvol_total, 0.0f, s); // 2D tiles write every voxel
         if (e == hipSuccess)
             e = fixed_point_exponent_batch(nitems, segs, sblocks, nsblocks, bounds, d_maxbits, d_fixexp, sinos, s);
         if (e != hipSuccess)
@@ -551,22 +781,18 @@ namespace ehp
             if (per_xcd * 8 > (int64_t) 0x7fffffff)
                 return hipErrorInvalidValue;
             const dim3 grid((unsigned) (per_xcd * 8));
-#define EHP_ADJ_BATCH(Dv, Av)                                                                                      \
-    hipLaunchKernelGGL((joseph_adj_tiled_batch_kernel<Dv, Av>), grid, dim3(kThreads), lds[a], s, ajobs[a], ablocks[a], \
+#define EHP_ADJ_BATCH(Av)                                                                                          \
+    hipLaunchKernelGGL((joseph_adj_tiled_batch_kernel<3, Av>), grid, dim3(kThreads), lds[a], s, ajobs[a], ablocks[a],   \
                        (int) per_xcd, total, d_fixexp, sinos, vols)
-            if (dim == 2) {
-                if (a == 0)
-                    EHP_ADJ_BATCH(2, 0);
-                else
-                    EHP_ADJ_BATCH(2, 1);
-            } else {
-                if (a == 0)
-                    EHP_ADJ_BATCH(3, 0);
-                else if (a == 1)
-                    EHP_ADJ_BATCH(3, 1);
-                else
-                    EHP_ADJ_BATCH(3, 2);
-            }
+            if (dim == 2)
+                hipLaunchKernelGGL(joseph_adj2d_batch_kernel, grid, dim3(256), lds[a], s, ajobs[a], ablocks[a],
+                                   (int) per_xcd, total, d_fixexp, sinos, vols);
+            else if (a == 0)
+                EHP_ADJ_BATCH(0);
+            else if (a == 1)
+                EHP_ADJ_BATCH(1);
+            else
+                EHP_ADJ_BATCH(2);
 #undef EHP_ADJ_BATCH
             e = hipGetLastError();
             if (e != hipSuccess)

@@ -53,18 +53,19 @@ namespace ehp
         ViewSet views;
         Dims dims;
         int tiles_u;
+        int parts; // 2D: parts of a ray's span summed apart
         int64_t sino_off;
         int64_t block0;
     };
 
-    struct AdjJob { // the tiles of one operator along one driving axis
+    struct AdjJob { // the tiles of one operator along one driving axis (2D: its tiles, both axes)
         const PoseGeom* geo;
         const RayRec* table;
         const int* pose_axes;
         Dims dims;
         TileCfg tc;
         int ntA, ntB;
-        int batch;
+        int batch; // poses per step
         int item; // index of the operator in the batch (its fixed-point exponent)
         int64_t sino_off, vol_off;
         int64_t block0;
@@ -225,9 +226,10 @@ namespace ehp
     template <class T>
     hipError_t joseph_forward_planes(const PoseGeom* geo, const Dims& dims, const PadLayout* layouts,
                                      void* const* views, int axes_present, const T* vol, T* sino, hipStream_t s);
-    // the volume copied into the interior of its plane-major view (float or bfloat16 elements)
+    // the volume copied into the interiors of its plane-major views, in one launch
     template <class E>
-    hipError_t joseph_view_copy(const Dims& dims, const PadLayout& L, const E* vol, E* view, hipStream_t s);
+    hipError_t joseph_view_copies(const Dims& dims, const PadLayout* layouts, void* const* views, int axes_present,
+                                  const E* vol, hipStream_t s);
     // Siddon forward over plane-major views (FP32, FP64), from the per-ray table
     template <class T>
     hipError_t siddon_forward_planes(const SidRec* table, const Dims& dims, const PadLayout* layouts,

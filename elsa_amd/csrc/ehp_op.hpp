@@ -53,3 +53,7 @@ struct ehp_op {
     size_t stage_bytes = 0;
     ehp::OrderGuard order;   // calls on this operator run one after another on the device
 };
+
+// The 2D Joseph back projection's tile for a launch over nvox voxels (one problem's, or all of a
+// batch's) on a device of cus compute units
+ehp::TileCfg joseph_tile2d(int64_t nvox, int cus);

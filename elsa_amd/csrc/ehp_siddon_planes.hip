@@ -191,14 +191,14 @@ namespace ehp
             const PadLayout& L = layouts[a];
             if (L.pairs)
                 return hipErrorInvalidValue; // the Siddon walk reads single voxels of plain views
-            hipError_t e = joseph_view_copy<T>(dims, L, vol, (T*) views[a], s);
-            if (e != hipSuccess)
-                return e;
             vs.v[a] = PadView{views[a], L.PS * es, L.RS * es, L.size};
             const int b2 = dims.dim == 3 ? (a == 2 ? 1 : 2) : -1;
             if (L.f == b2)
                 vs.fb2 |= 1 << a;
         }
+        hipError_t e = joseph_view_copies<T>(dims, layouts, views, axes_present, vol, s);
+        if (e != hipSuccess)
+            return e;
         const FwdGrid fg = fwd_grid(dims, kSidWU);
         if (fg.per_xcd * 8 > (int64_t) 0x7fffffff)
             return hipErrorInvalidValue;

@@ -161,15 +161,16 @@ int ehp_op_sizes(const ehp_op* op, int64_t* n_vol, int64_t* n_sino);
 int ehp_sample_count(const ehp_op* op, uint64_t* samples);
 
 /* Tile shape of the operator's LDS-tiled kernel (FP32). Joseph and Siddon back projections:
- * la planes along the driving axis, tb x tc voxels across (tc ignored in 2D). Voxel forward
+ * la planes along the driving axis, tb x tc voxels across (tc ignored in 2D; Joseph in 2D: la x tb
+ * voxels along x and y, halved by the kernel until they fit its LDS). Voxel forward
  * projection: la x tb detector pixels (tb ignored in 2D, tc ignored). No counterpart in elsa;
  * it is the knob the tile autotuner turns. Fails with EHP_ERR_ARGUMENT if the tile does not
  * fit the device's LDS or the operator has no tiled kernel. Queries only when out pointers
  * are given and la <= 0. */
 int ehp_tile(ehp_op* op, int la, int tb, int tc, int* la_out, int* tb_out, int* tc_out);
 
-/* Poses per step of the tiled back projections (Joseph, Siddon; 1-32, default 8): each step
- * gathers the candidate rays of that many poses for one tile, so larger steps keep more lanes
+/* Poses per step of the tiled back projections (Joseph, Siddon; 1-32, default 32; Joseph in 2D takes
+ * 16 times as many): each step gathers the candidate rays of that many poses for one tile, so larger steps keep more lanes
  * busy where few rays meet a tile (2D). No counterpart in elsa; a knob of the tile autotuner.
  * Queries only when batch <= 0. */
 int ehp_pose_batch(ehp_op* op, int batch, int* batch_out);
