@@ -32,6 +32,7 @@ struct ehp_batch {
     ehp::SidAdjJob* d_sajobs[3] = {nullptr, nullptr, nullptr};
     // fused voxel passes (the forward's blocks in d_fblocks, its segments over the volumes)
     ehp::VoxFwdJob* d_vfjobs = nullptr;
+    int vox_cols = 0; // the columns of the voxel forward's kernel, 0: the general one
     ehp::VoxAdjJob* d_vajobs = nullptr;
     int* d_vablocks = nullptr;
     int64_t nvablocks = 0;
@@ -156,12 +157,13 @@ namespace
                 v.pose_axes = op->d_pose_axes;
                 v.pose_margin = op->d_pose_margin;
                 v.tile = op->tile;
+                v.plan = op->vox;
                 v.vol_off = b->vol_off[j];
                 v.sino_off = b->sino_off[j];
                 offs[j] = b->vol_off[j];
                 sizes[j] = op->dims.nvox;
             }
-            ehp::voxel_forward_batch_jobs(vitems.data(), n, vfj, fb, b->lds[0]);
+            ehp::voxel_forward_batch_jobs(vitems.data(), n, vfj, fb, b->lds[0], b->vox_cols);
             ehp::batch_segments(offs.data(), sizes.data(), n, sg, sb);
             ehp::voxel_adjoint_batch_jobs(vitems.data(), n, vaj, vab);
         } else if (sid) {
@@ -281,8 +283,8 @@ namespace
             e = ehp::fixed_point_exponent_batch((int) b->ops.size(), b->d_segs, b->d_sblocks, b->nsblocks,
                                                 b->d_bounds, b->d_maxbits, b->d_fixexp, (const float*) in, s);
             if (e == hipSuccess)
-                e = ehp::voxel_forward_batch(b->dim, b->d_vfjobs, b->d_fblocks, b->nfblocks, b->lds[0], b->d_fixexp,
-                                             (const float*) in, (float*) out, s);
+                e = ehp::voxel_forward_batch(b->dim, b->vox_cols, b->d_vfjobs, b->d_fblocks, b->nfblocks, b->lds[0],
+                                             b->d_fixexp, (const float*) in, (float*) out, s);
         } else if (adjoint && b->kind == KIND_VOXEL) {
             e = ehp::voxel_adjoint_batch(b->dim, b->d_vajobs, b->d_vablocks, b->nvablocks, (const float*) in,
                                          (float*) out, s);

@@ -8,6 +8,7 @@
 #include "ehp_kernels.hpp"
 #include "ehp_solvers.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -484,6 +485,46 @@ namespace
         op->tiled = true;
         return EHP_OK;
     }
+    // The 3D voxel kernels' plan: footprints of at most kVoxMaxCols columns, a table in their reach that fits the LDS
+    // array of the general kernels, 32-bit voxel indices with 24-bit strides.
+    void plan_voxel(ehp_op* op, const std::vector<int>& axis, double smax)
+    {
+        const ehp::Dims& dm = op->dims;
+        op->vox = ehp::VoxPlan{};
+        if (dm.dim != 3 || dm.nvox >= (1ll << 31) || dm.strides[1] >= (1 << 24) || dm.strides[2] >= (1 << 24))
+            return;
+        double smin = smax;
+        std::vector<int> bits(axis.size());
+        for (size_t p = 0; p < axis.size(); ++p) {
+            bits[p] = 1 << axis[p];
+            smin = std::min(smin, ehp::voxel_min_scaling(op->host_geo[p], dm));
+        }
+        const int cols = ehp::footprint_cols(op->support, smax);
+        const double span = op->dtype == EHP_F64 ? op->n_lut + 1.0
+                                                 : ehp::column_table_span(op->n_lut, op->support, smin,
+                                                                          ehp::kernel_cols(cols));
+        if (cols > ehp::kVoxMaxCols || !(smin > 0.0) || !(span <= ehp::kVoxLutSpan))
+            return;
+        op->vox.cols = cols;
+        op->vox.span = (int) span;
+        for (int a = 0; a < 3; ++a)
+            op->vox.fan[a] = fan_axis(op, bits, a);
+    }
+
+    // Tiles of the 3D voxel forward by columns: about 96 x 16 pixels, widths evened over the detector, so
+    // that most candidates of a tile lie in it and no tile is a sliver; lower ones (down to 5 rows) while
+    // the launch has fewer than three blocks a CU. 131 x 125 x 119 blobs on 193 x 187, 180 poses: 5.60 ms
+    // with 97 x 16 tiles, 6.10 with 65 x 16, 8.05 with 32 x 32, 6.80 with 193 x 24; 40^3 on 60^2, 60 poses:
+    // 132 us with 60 x 5, 180 with 60 x 15.
+    ehp::TileCfg voxel_tile3d(const ehp::Dims& dm, int cus)
+    {
+        const int d0 = dm.det[0], d1 = dm.det[1];
+        const int nu = std::max(1, (d0 + 48) / 96);
+        const int64_t want = (3ll * cus + (int64_t) nu * dm.nposes - 1) / ((int64_t) nu * dm.nposes);
+        const int nv = std::max({1, (d1 + 8) / 16, (int) std::min<int64_t>(want, (d1 + 4) / 5)});
+        return ehp::TileCfg{(d0 + nu - 1) / nu, (d1 + nv - 1) / nv, 1};
+    }
+
     // Voxel projectors (FP32, bfloat16, FP64): the detector-tiled forward, when every source lies
     // outside the volume (the footprint scaling is then bounded).
     int setup_voxel_tiled(ehp_op* op, const void* host_lut)
@@ -519,6 +560,7 @@ namespace
         while (ls < lutmax)
             ls *= 2.0;
         op->slot_bound = ehp::voxel_slot_bound(dm, op->support, smax_all, ls);
+        plan_voxel(op, axis, smax_all);
         hipError_t e = hipMalloc((void**) &op->d_pose_axes, n * sizeof(int));
         if (e == hipSuccess)
             e = hipMalloc((void**) &op->d_pose_margin, n * sizeof(float));
@@ -536,6 +578,8 @@ namespace
         if (e != hipSuccess)
             return hip_fail(e, "voxel projector state");
         op->tile = dm.dim == 3 ? ehp::TileCfg{32, 32, 1} : ehp::TileCfg{256, 1, 1};
+        if (op->vox.cols > 0)
+            op->tile = voxel_tile3d(dm, device_cus(op->device));
         op->tiled = true;
         return EHP_OK;
     }
@@ -868,8 +912,9 @@ static hipError_t launch(ehp_op* op, const void* in, void* out, hipStream_t s, b
         if (!adjoint)
             e = ehp::voxel_forward_tiled<ehp::bf16, float>(op->d_geo, dm, (const float*) op->d_lut, op->n_lut,
                                                            op->support, op->differential, op->d_pose_axes,
-                                                           op->d_pose_margin, op->tile, op->slot_bound, op->d_maxbits,
-                                                           op->d_fixexp, (const ehp::bf16*) in, (ehp::bf16*) out, s);
+                                                           op->d_pose_margin, op->vox, op->tile, op->slot_bound,
+                                                           op->d_maxbits, op->d_fixexp, (const ehp::bf16*) in,
+                                                           (ehp::bf16*) out, s);
         else
             e = ehp::voxel_adjoint_fast<ehp::bf16>(op->d_geo, dm, (const float*) op->d_lut, op->n_lut, op->support,
                                                    op->differential, (const ehp::bf16*) in, (ehp::bf16*) out, s);
@@ -907,8 +952,8 @@ static hipError_t launch(ehp_op* op, const void* in, void* out, hipStream_t s, b
         else if (!adjoint && op->tiled)
             e = ehp::voxel_forward_tiled<float, float>(op->d_geo, dm, (const float*) op->d_lut, op->n_lut,
                                                        op->support, op->differential, op->d_pose_axes,
-                                                       op->d_pose_margin, op->tile, op->slot_bound, op->d_maxbits,
-                                                       op->d_fixexp, x, y, s);
+                                                       op->d_pose_margin, op->vox, op->tile, op->slot_bound,
+                                                       op->d_maxbits, op->d_fixexp, x, y, s);
         else if (adjoint && op->tiled)
             e = ehp::voxel_adjoint_fast<float>(op->d_geo, dm, (const float*) op->d_lut, op->n_lut, op->support,
                                                op->differential, x, y, s);
@@ -940,8 +985,8 @@ static hipError_t launch(ehp_op* op, const void* in, void* out, hipStream_t s, b
         else if (!adjoint && op->tiled)
             e = ehp::voxel_forward_tiled<double, double>(op->d_geo, dm, (const double*) op->d_lut, op->n_lut,
                                                          op->support, op->differential, op->d_pose_axes,
-                                                         op->d_pose_margin, op->tile, op->slot_bound, op->d_maxbits,
-                                                         op->d_fixexp, x, y, s);
+                                                         op->d_pose_margin, op->vox, op->tile, op->slot_bound,
+                                                         op->d_maxbits, op->d_fixexp, x, y, s);
         else
             e = adjoint ? ehp::voxel_adjoint<double>(op->d_geo, dm, (const double*) op->d_lut, op->n_lut, op->support,
                                                      op->differential, x, y, s)

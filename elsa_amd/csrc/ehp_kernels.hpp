@@ -136,6 +136,15 @@ namespace ehp
                                     const int64_t nablocks[3], const size_t lds[3], const int* d_fixexp,
                                     const float* sinos, float* vols, hipStream_t s);
 
+    // What the 3D voxel kernels know of an operator: the most pixels a footprint is wide (0: the
+    // general kernels run), the entries of the forward's table in LDS, and per driving axis the
+    // transverse axis along which the voxels of a plane fan out over a detector row.
+    struct VoxPlan {
+        int cols;
+        int span;
+        int fan[3];
+    };
+
     // ---- batches of voxel projectors (FP32 fast kernels): the tiled forward and the gather
     struct VoxBatchItem {
         const PoseGeom* geo;
@@ -147,6 +156,7 @@ namespace ehp
         const int* pose_axes;
         const float* pose_margin;
         TileCfg tile;
+        VoxPlan plan;
         int64_t vol_off, sino_off;
     };
 
@@ -159,6 +169,7 @@ namespace ehp
         int diff;
         const int* pose_axis;
         const float* pose_margin;
+        VoxPlan plan;
         int TU, TV, ntu;
         int item;
         int64_t vol_off, sino_off;
@@ -177,9 +188,9 @@ namespace ehp
     };
 
     void voxel_forward_batch_jobs(const VoxBatchItem* items, int n, std::vector<VoxFwdJob>& jobs,
-                                  std::vector<int>& blocks, size_t& lds);
-    hipError_t voxel_forward_batch(int dim, const VoxFwdJob* jobs, const int* blocks, int64_t nblocks, size_t lds,
-                                   const int* d_fixexp, const float* vols, float* sinos, hipStream_t s);
+                                  std::vector<int>& blocks, size_t& lds, int& cols);
+    hipError_t voxel_forward_batch(int dim, int cols, const VoxFwdJob* jobs, const int* blocks, int64_t nblocks,
+                                   size_t lds, const int* d_fixexp, const float* vols, float* sinos, hipStream_t s);
     void voxel_adjoint_batch_jobs(const VoxBatchItem* items, int n, std::vector<VoxAdjJob>& jobs,
                                   std::vector<int>& blocks);
     hipError_t voxel_adjoint_batch(int dim, const VoxAdjJob* jobs, const int* blocks, int64_t nblocks,
@@ -220,9 +231,9 @@ namespace ehp
     int voxel_max_lut();
     template <class ST, class LT>
     hipError_t voxel_forward_tiled(const PoseGeom* geo, const Dims& dims, const LT* lut, int n_lut, float support,
-                                   int diff, const int* pose_axis, const float* pose_margin, const TileCfg& tc,
-                                   double slot_bound, unsigned int* d_maxbits, int* d_fixexp, const ST* vol, ST* sino,
-                                   hipStream_t s);
+                                   int diff, const int* pose_axis, const float* pose_margin, const VoxPlan& plan,
+                                   const TileCfg& tc, double slot_bound, unsigned int* d_maxbits, int* d_fixexp,
+                                   const ST* vol, ST* sino, hipStream_t s);
     template <class T>
     hipError_t joseph_forward_planes(const PoseGeom* geo, const Dims& dims, const PadLayout* layouts,
                                      void* const* views, int axes_present, const T* vol, T* sino, hipStream_t s);

@@ -43,6 +43,7 @@ struct ehp_op {
     ehp::TileCfg tile{};
     ehp::RayRec* d_table = nullptr;   // per-ray traversal state (Joseph)
     ehp::SidRec* d_sidtable = nullptr; // per-ray traversal state (Siddon)
+    ehp::VoxPlan vox{};                // voxel projectors (3D)
     float* d_pose_margin = nullptr;    // voxel forward: frustum margin per pose (pixels)
     unsigned int* d_maxbits = nullptr; // per-block maxima of |y| of the current back projection (kAbsmaxBlocks)
     int* d_fixexp = nullptr;           // fixed-point exponent of the current back projection

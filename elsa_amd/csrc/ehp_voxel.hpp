@@ -240,6 +240,136 @@ namespace ehp
         return w * d0;
     }
 
+    // ---------------------------------------------------------------------------------
+    // The 3D kernels' footprints by columns: a footprint is at most `cols` pixels wide (a property of
+    // the operator), so a voxel's column distances are formed once and every row of taps is straight
+    // code over them, with no loop over columns.
+
+    // Most columns of the 3D kernels' footprints; wider ones take the general kernels.
+    constexpr int kVoxMaxCols = 8;
+
+    // Pixels across the widest footprint: floor(2 r s) + 1 for the radius r and the largest scaling s,
+    // with room for the rounding of its ends.
+    inline int footprint_cols(double support, double smax)
+    {
+        const double w = 2.0 * support * smax * (1.0 + 1.0e-5) + 1.0e-4;
+        return w < 1.0e6 ? (int) w + 1 : 1 << 20;
+    }
+
+    // The kernels' column counts: the next of 4, 5, 6 and 8
+    inline int kernel_cols(int cols)
+    {
+        return cols <= 4 ? 4 : (cols <= 6 ? cols : 8);
+    }
+
+    // Entries of the pair table (lerp_table_entry) that taps reach when columns past the footprint's end
+    // are not masked: the first of nc columns lies at least r s - 1 before the centre, so the last less
+    // than nc - r s past it: (nc / (r s) - 1) (n - 1) in table units, and at least n - 1; rows at most n - 1.
+    inline double column_table_span(int n, double support, double smin, int nc)
+    {
+        const double far = nc / (support * smin) - 1.0, e = far > 1.0 ? far : 1.0;
+        return sqrt(e * e + 1.0) * 1.0001 * (n - 1) + 4.0;
+    }
+
+    // Smallest footprint scaling of a pose over the volume: sdd over the largest distance from the
+    // source to a corner of the volume.
+    inline double voxel_min_scaling(const PoseGeom& g, const Dims& dims)
+    {
+        double dist2 = 0.0;
+        for (int i = 0; i < dims.dim; ++i) {
+            const double c = g.C[i], far = c < 0.5 * dims.vol[i] ? dims.vol[i] - c : c;
+            dist2 += far * far;
+        }
+        return dist2 > 0.0 ? (double) g.sdd / sqrt(dist2) : -1.0;
+    }
+
+    // a / b, correctly rounded, from rb = 1 / b correctly rounded: the quotient estimate with one
+    // correction (Markstein, Computation of elementary functions on the IBM RISC System/6000, 1990,
+    // theorem on division); b's mantissa is not all ones, quotients far from underflow.
+    EHP_HD inline float div_rounded(float a, float b, float rb)
+    {
+        const float q = a * rb;
+        return __builtin_fmaf(__builtin_fmaf(-b, q, a), rb, q);
+    }
+
+    // The FP64 weight at table position index (tap_weight's interpolation t fb + (1 - t) fa), 0 past
+    // n - 1; tab holds n entries and a zero.
+    EHP_HD inline double lut_weight64(const double* __restrict__ tab, int n, float index)
+    {
+        const int ia = (int) index; // index >= 0
+        const int a = ia < n - 1 ? ia : n - 1;
+        const double t = (double) (index - (float) a);
+        const double w = t * tab[a + 1] + (1.0 - t) * tab[a];
+        return index <= (float) (n - 1) ? w : 0.0;
+    }
+
+    // The weight of an FP32 tap as the tiled forward forms it, from the distances in table units: d0k =
+    // (c0 - i) rsk and d1s = ((c1 - j) rsk)^2 (2D: 0) with rsk = (n - 1) / (support scaling), so that
+    // the square root is the table index; du = d0 in footprint radii (diff in 3D only).
+    template <int D, bool TZ>
+    EHP_HD inline float tap_weight_units(const float* __restrict__ tab, int n, float d0k, float d1s, float du,
+                                         bool diff)
+    {
+        if (D == 2)
+            return tap_weight_fast<2, TZ>(tab, n, 1.0f, 0.0f, d0k, diff);
+        const float w = tap_weight_fast<3, TZ>(tab, n, 1.0f, __builtin_fmaf(d0k, d0k, d1s), 0.0f, false);
+        return diff ? w * du : w;
+    }
+
+    // Columns l0 .. l0 + NC - 1 of an FP32 footprint of columns l0 .. h0: the distances in table units and,
+    // for the phase-contrast weights, in footprint radii. A table that ends in 0 (TZ) gives the columns
+    // past h0 weight 0 by itself (column_table_span); others put them past its end.
+    template <int NC, bool TZ>
+    EHP_HD inline void column_units(float c0, int l0, int h0, float rs, float rsk, bool diff, float* d0k, float* du)
+    {
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            const float d = c0 - (float) (l0 + i);
+            d0k[i] = d * rsk;
+            if (!TZ)
+                d0k[i] = l0 + i <= h0 ? d0k[i] : 1.0e6f;
+            du[i] = diff ? d * rs : 1.0f;
+        }
+    }
+
+    // The weights of row j over those columns
+    template <int NC, bool TZ>
+    EHP_HD inline void row_units(const float* __restrict__ tab, int n, float c1, int j, float rsk, const float* d0k,
+                                 const float* du, bool diff, float* w)
+    {
+        const float d1 = (c1 - (float) j) * rsk;
+        const float d1s = d1 * d1;
+#pragma unroll
+        for (int i = 0; i < NC; ++i)
+            w[i] = tap_weight_units<3, TZ>(tab, n, d0k[i], d1s, du[i], diff);
+    }
+
+    // The same for FP64 tables: the distances and weights of visit() and tap_weight bit for bit, their
+    // divisions from correctly rounded reciprocals (rsc = 1 / scaling, rsupport = 1 / support).
+    template <int NC>
+    EHP_HD inline void column_units64(float c0, int l0, int h0, float scaling, float rsc, float* d0)
+    {
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            d0[i] = div_rounded(c0 - (float) (l0 + i), scaling, rsc);
+            d0[i] = l0 + i <= h0 ? d0[i] : 1.0e6f;
+        }
+    }
+
+    template <int NC>
+    EHP_HD inline void row_units64(const double* __restrict__ tab, int n, float support, float rsupport, float c1,
+                                   int j, float scaling, float rsc, const float* d0, bool diff, double* w)
+    {
+        const float d1 = div_rounded(c1 - (float) j, scaling, rsc);
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            const float dist = sqrtf(d0[i] * d0[i] + d1 * d1);
+            w[i] = lut_weight64(tab, n, div_rounded(dist, support, rsupport) * (float) (n - 1));
+            if (diff)
+                w[i] = w[i] * (double) d0[i];
+        }
+    }
+
     // Row stride (slots) of a detector tile's LDS sums in the tiled voxel forward: odd in 3D, so
     // that the 8-byte slots of neighbouring detector rows fall on different LDS banks.
     EHP_HD inline int vox_acc_stride(int TU, int TV)
