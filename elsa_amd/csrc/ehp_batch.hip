@@ -32,7 +32,7 @@ struct ehp_batch {
     ehp::SidAdjJob* d_sajobs[3] = {nullptr, nullptr, nullptr};
     // fused voxel passes (the forward's blocks in d_fblocks, its segments over the volumes)
     ehp::VoxFwdJob* d_vfjobs = nullptr;
-    int vox_cols = 0; // the columns of the voxel forward's kernel, 0: the general one
+    int vox_cols = 0, vox_gather_cols = 0, vox_gather_threads = 256; // the columns of the voxel kernels, 0: the general ones
     ehp::VoxAdjJob* d_vajobs = nullptr;
     int* d_vablocks = nullptr;
     int64_t nvablocks = 0;
@@ -165,7 +165,8 @@ namespace
             }
             ehp::voxel_forward_batch_jobs(vitems.data(), n, vfj, fb, b->lds[0], b->vox_cols);
             ehp::batch_segments(offs.data(), sizes.data(), n, sg, sb);
-            ehp::voxel_adjoint_batch_jobs(vitems.data(), n, vaj, vab);
+            ehp::voxel_gather_batch_jobs(vitems.data(), n, vaj, vab, b->lds[1], b->vox_gather_cols,
+                                         b->vox_gather_threads);
         } else if (sid) {
             std::vector<int64_t> offs(n), sizes(n);
             for (int j = 0; j < n; ++j) {
@@ -286,8 +287,8 @@ namespace
                 e = ehp::voxel_forward_batch(b->dim, b->vox_cols, b->d_vfjobs, b->d_fblocks, b->nfblocks, b->lds[0],
                                              b->d_fixexp, (const float*) in, (float*) out, s);
         } else if (adjoint && b->kind == KIND_VOXEL) {
-            e = ehp::voxel_adjoint_batch(b->dim, b->d_vajobs, b->d_vablocks, b->nvablocks, (const float*) in,
-                                         (float*) out, s);
+            e = ehp::voxel_gather_batch(b->dim, b->vox_gather_cols, b->d_vajobs, b->d_vablocks, b->nvablocks, b->lds[1],
+                                        b->vox_gather_threads, (const float*) in, (float*) out, s);
         } else if (!adjoint && b->kind == KIND_SIDDON) {
             e = ehp::siddon_forward_batch(b->dim, b->d_cjobs, b->d_cblocks, b->ncblocks, b->d_sfjobs, b->d_fblocks,
                                           b->nfblocks, (const float*) in, (float*) out, s);

@@ -486,12 +486,14 @@ namespace
         return EHP_OK;
     }
     // The 3D voxel kernels' plan: footprints of at most kVoxMaxCols columns, a table in their reach that fits the LDS
-    // array of the general kernels, 32-bit voxel indices with 24-bit strides.
+    // array of the general kernels, 32-bit voxel indices with 24-bit strides and 30-bit byte offsets of a pose's
+    // pixels.
     void plan_voxel(ehp_op* op, const std::vector<int>& axis, double smax)
     {
         const ehp::Dims& dm = op->dims;
         op->vox = ehp::VoxPlan{};
-        if (dm.dim != 3 || dm.nvox >= (1ll << 31) || dm.strides[1] >= (1 << 24) || dm.strides[2] >= (1 << 24))
+        if (dm.dim != 3 || dm.nvox >= (1ll << 31) || dm.strides[1] >= (1 << 24) || dm.strides[2] >= (1 << 24) ||
+            dm.pix_per_pose >= (1 << 27))
             return;
         double smin = smax;
         std::vector<int> bits(axis.size());
@@ -916,8 +918,9 @@ static hipError_t launch(ehp_op* op, const void* in, void* out, hipStream_t s, b
                                                            op->d_maxbits, op->d_fixexp, (const ehp::bf16*) in,
                                                            (ehp::bf16*) out, s);
         else
-            e = ehp::voxel_adjoint_fast<ehp::bf16>(op->d_geo, dm, (const float*) op->d_lut, op->n_lut, op->support,
-                                                   op->differential, (const ehp::bf16*) in, (ehp::bf16*) out, s);
+            e = ehp::voxel_gather<ehp::bf16, float>(op->d_geo, dm, (const float*) op->d_lut, op->n_lut, op->support,
+                                                    op->differential, op->vox, (const ehp::bf16*) in,
+                                                    (ehp::bf16*) out, s);
     } else if (op->dtype == EHP_BF16) {
         // bfloat16 storage, FP32 arithmetic: the forward reads bfloat16 views and rounds each ray
         // sum once; the back projection sums in fixed point into FP32 and rounds each voxel once
@@ -955,8 +958,8 @@ static hipError_t launch(ehp_op* op, const void* in, void* out, hipStream_t s, b
                                                        op->d_pose_margin, op->vox, op->tile, op->slot_bound,
                                                        op->d_maxbits, op->d_fixexp, x, y, s);
         else if (adjoint && op->tiled)
-            e = ehp::voxel_adjoint_fast<float>(op->d_geo, dm, (const float*) op->d_lut, op->n_lut, op->support,
-                                               op->differential, x, y, s);
+            e = ehp::voxel_gather<float, float>(op->d_geo, dm, (const float*) op->d_lut, op->n_lut, op->support,
+                                                op->differential, op->vox, x, y, s);
         else
             e = adjoint ? ehp::voxel_adjoint<float>(op->d_geo, dm, (const float*) op->d_lut, op->n_lut, op->support,
                                                     op->differential, x, y, s)
@@ -987,6 +990,9 @@ static hipError_t launch(ehp_op* op, const void* in, void* out, hipStream_t s, b
                                                          op->support, op->differential, op->d_pose_axes,
                                                          op->d_pose_margin, op->vox, op->tile, op->slot_bound,
                                                          op->d_maxbits, op->d_fixexp, x, y, s);
+        else if (adjoint && op->tiled)
+            e = ehp::voxel_gather<double, double>(op->d_geo, dm, (const double*) op->d_lut, op->n_lut, op->support,
+                                                  op->differential, op->vox, x, y, s);
         else
             e = adjoint ? ehp::voxel_adjoint<double>(op->d_geo, dm, (const double*) op->d_lut, op->n_lut, op->support,
                                                      op->differential, x, y, s)

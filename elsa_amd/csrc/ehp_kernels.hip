@@ -225,15 +225,14 @@ namespace ehp
     // ---------------------------------------------------------------------------------
     // Voxel-driven blob / B-spline projector.
 
-    // Adjoint: one thread per voxel gathers over all poses (no atomics). ST is the storage type
-    // (bfloat16 storage: widened exactly, summed in FP32, each voxel rounded once).
-    template <int D, class T, class ST>
+    // Adjoint: one thread per voxel gathers over all poses (no atomics).
+    template <int D, class T>
     __global__ void __launch_bounds__(256)
         voxel_adj_kernel(const PoseGeom* __restrict__ geo, const Dims dims, const T* __restrict__ lut, int n_lut,
-                         float support, const int diff, const int per_xcd, const ST* __restrict__ sino,
-                         ST* __restrict__ vol)
+                         float support, const int diff, const int per_xcd, const T* __restrict__ sino,
+                         T* __restrict__ vol)
     {
-        // the FP32 gather's order (voxel_adj_fast_kernel): in 3D y slowest and a contiguous run of
+        // the default gather's order (voxel_gather_kernel): in 3D y slowest and a contiguous run of
         // blocks per XCD, so that an XCD's detector rows stay in its L2; each voxel's sum is the same
         const int64_t blk = (int64_t) (blockIdx.x % 8u) * per_xcd + (blockIdx.x / 8u);
         const int64_t vox = blk * blockDim.x + threadIdx.x;
@@ -252,162 +251,13 @@ namespace ehp
         for (int p = 0; p < dims.nposes; ++p) {
             Footprint fp;
             footprint<D>(geo[p], dims, x, y, z, support, fp);
-            const ST* sp = sino + (int64_t) p * dims.pix_per_pose;
+            const T* sp = sino + (int64_t) p * dims.pix_per_pose;
             visit<D, T>(fp, dims, [&](int64_t pix, float dist, float d0) {
-                acc += tap_weight<D, T>(lut, n_lut, support, dist, d0, diff != 0) * up(sp[pix]);
+                acc += tap_weight<D, T>(lut, n_lut, support, dist, d0, diff != 0) * sp[pix];
             });
         }
-        vol[x + (int64_t) y * dims.strides[1] + (int64_t) z * dims.strides[2]] = down<ST>(acc);
+        vol[x + (int64_t) y * dims.strides[1] + (int64_t) z * dims.strides[2]] = acc;
     }
-
-    // The default FP32 gather: the footprints and taps of the tiled forward (footprint_fast, one
-    // reciprocal of the scaling per voxel and pose instead of a division per tap,
-    // tap_weight_fast's square root and table index), so forward and back projection weigh every
-    // tap alike. The pair table of the n_lut <=
-    // kVoxMaxLut entries (lerp_table_entry) is read from LDS. ST: float or bfloat16 storage.
-    // YSLOW: the thread's index vox counts the voxels with y slowest (x fastest, then z), else in
-    // the volume's order.
-    template <int D, class ST, bool YSLOW = false>
-    __device__ __forceinline__ void vox_adj_fast(const PoseGeom* __restrict__ geo, const Dims& dims,
-                                                 const float* __restrict__ lut, int n_lut, float support,
-                                                 const int diff, const ST* __restrict__ sino, ST* __restrict__ vol,
-                                                 const int64_t vox)
-    {
-        __shared__ float s_lut[2 * kVoxLutSpan];
-        for (int i = threadIdx.x; i < lerp_table_size(n_lut); i += blockDim.x)
-            lerp_table_entry(lut, n_lut, i, s_lut);
-        __syncthreads();
-        if (vox >= dims.nvox)
-            return;
-        const int x = (int) (vox % dims.vol[0]);
-        int y, z;
-        if (YSLOW) {
-            z = (int) ((vox / dims.vol[0]) % dims.vol[2]);
-            y = (int) (vox / ((int64_t) dims.vol[0] * dims.vol[2]));
-        } else {
-            y = (int) ((vox / dims.vol[0]) % dims.vol[1]);
-            z = (int) (vox / ((int64_t) dims.vol[0] * dims.vol[1]));
-        }
-        const float kidx = (float) (n_lut - 1) / support;
-        // a table ending in 0 takes tap_weight_fast's TZ form
-        auto gather = [&](auto tzc) {
-            constexpr bool TZ = decltype(tzc)::value;
-            float acc = 0.0f;
-            for (int p = 0; p < dims.nposes; ++p) {
-                Footprint fp;
-                float rs;
-                footprint_fast<D>(geo[p], dims, x, y, z, support, fp, rs);
-                const ST* sp = sino + (int64_t) p * dims.pix_per_pose;
-                for (int j = fp.lo[1]; j <= fp.hi[1]; ++j) {
-                    const float d1 = D == 3 ? (fp.center[1] - (float) j) * rs : 0.0f;
-                    const float d1s = d1 * d1;
-                    float fi = (float) fp.lo[0]; // i as a float (exact), without a conversion per tap
-                    for (int i = fp.lo[0]; i <= fp.hi[0]; ++i, fi += 1.0f) {
-                        const float d0 = (fp.center[0] - fi) * rs;
-                        // one FMA per tap: the sum of the taps in pose and pixel order, each product
-                        // unrounded
-                        acc = __builtin_fmaf(tap_weight_fast<D, TZ>(s_lut, n_lut, kidx, __builtin_fmaf(d0, d0, d1s),
-                                                                    d0, diff != 0),
-                                             up(sp[(int64_t) j * dims.det[0] + i]), acc);
-                    }
-                }
-            }
-            return acc;
-        };
-        const float acc = lut[n_lut - 1] == 0.0f ? gather(std::true_type{}) : gather(std::false_type{});
-        vol[x + (int64_t) y * dims.strides[1] + (int64_t) z * dims.strides[2]] = down<ST>(acc);
-    }
-
-    // DIFF: the phase-contrast projectors' weights (a compile-time flag, so that the taps of the
-    // others carry no select). In 3D the voxels are taken with y slowest and each XCD gets a
-    // contiguous run of blocks (consecutive blocks land on different XCDs): a slab of y, whose
-    // detector rows over all poses stay in that XCD's L2 when the trajectory turns about y.
-    template <int D, class ST, bool DIFF>
-    __global__ void __launch_bounds__(256)
-        voxel_adj_fast_kernel(const PoseGeom* __restrict__ geo, const Dims dims, const float* __restrict__ lut,
-                              int n_lut, float support, const int per_xcd, const ST* __restrict__ sino,
-                              ST* __restrict__ vol)
-    {
-        const int64_t blk = (int64_t) (blockIdx.x % 8u) * per_xcd + (blockIdx.x / 8u);
-        if (blk * blockDim.x >= dims.nvox)
-            return; // the whole block
-        vox_adj_fast<D, ST, D == 3>(geo, dims, lut, n_lut, support, DIFF ? 1 : 0, sino, vol,
-                                    blk * blockDim.x + threadIdx.x);
-    }
-
-    // the gathers of many operators in one launch (block b: block b - job.block0 of job
-    // block_job[b])
-    template <int D>
-    __global__ void __launch_bounds__(256)
-        voxel_adj_fast_batch_kernel(const VoxAdjJob* __restrict__ jobs, const int* __restrict__ block_job,
-                                    const float* __restrict__ sinos, float* __restrict__ vols)
-    {
-        const VoxAdjJob& J = jobs[block_job[blockIdx.x]];
-        vox_adj_fast<D, float>(J.geo, J.dims, J.lut, J.n_lut, J.support, J.diff, sinos + J.sino_off,
-                               vols + J.vol_off, ((int64_t) blockIdx.x - J.block0) * blockDim.x + threadIdx.x);
-    }
-
-    void voxel_adjoint_batch_jobs(const VoxBatchItem* items, int n, std::vector<VoxAdjJob>& jobs,
-                                  std::vector<int>& blocks)
-    {
-        jobs.clear();
-        blocks.clear();
-        for (int j = 0; j < n; ++j) {
-            const VoxBatchItem& it = items[j];
-            VoxAdjJob J{};
-            J.geo = it.geo;
-            J.dims = it.dims;
-            J.lut = it.lut;
-            J.n_lut = it.n_lut;
-            J.support = it.support;
-            J.diff = it.diff;
-            J.vol_off = it.vol_off;
-            J.sino_off = it.sino_off;
-            J.block0 = (int64_t) blocks.size();
-            blocks.insert(blocks.end(), (size_t) ((it.dims.nvox + 255) / 256), (int) jobs.size());
-            jobs.push_back(J);
-        }
-    }
-
-    hipError_t voxel_adjoint_batch(int dim, const VoxAdjJob* jobs, const int* blocks, int64_t nblocks,
-                                   const float* sinos, float* vols, hipStream_t s)
-    {
-        if (nblocks > 0x7fffffff)
-            return hipErrorInvalidValue;
-        if (nblocks == 0)
-            return hipSuccess;
-        if (dim == 2)
-            hipLaunchKernelGGL((voxel_adj_fast_batch_kernel<2>), dim3((unsigned) nblocks), dim3(256), 0, s, jobs,
-                               blocks, sinos, vols);
-        else
-            hipLaunchKernelGGL((voxel_adj_fast_batch_kernel<3>), dim3((unsigned) nblocks), dim3(256), 0, s, jobs,
-                               blocks, sinos, vols);
-        return hipGetLastError();
-    }
-
-    template <class ST>
-    hipError_t voxel_adjoint_fast(const PoseGeom* geo, const Dims& dims, const float* lut, int n_lut, float support,
-                                  int diff, const ST* sino, ST* vol, hipStream_t s)
-    {
-        const int64_t per_xcd = ((dims.nvox + 255) / 256 + 7) / 8;
-        if (per_xcd * 8 > (int64_t) 0x7fffffff)
-            return hipErrorInvalidValue;
-        const dim3 grid((unsigned) (per_xcd * 8));
-        auto launch = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, geo, dims, lut, n_lut, support, (int) per_xcd, sino,
-                               vol);
-        };
-        if (dims.dim == 2)
-            diff ? launch(voxel_adj_fast_kernel<2, ST, true>) : launch(voxel_adj_fast_kernel<2, ST, false>);
-        else
-            diff ? launch(voxel_adj_fast_kernel<3, ST, true>) : launch(voxel_adj_fast_kernel<3, ST, false>);
-        return hipGetLastError();
-    }
-
-    template hipError_t voxel_adjoint_fast<float>(const PoseGeom*, const Dims&, const float*, int, float, int,
-                                                  const float*, float*, hipStream_t);
-    template hipError_t voxel_adjoint_fast<bf16>(const PoseGeom*, const Dims&, const float*, int, float, int,
-                                                 const bf16*, bf16*, hipStream_t);
 
     // Forward: one thread per (voxel, pose) scatters into the detector.
     template <int D, class T>
@@ -570,19 +420,19 @@ namespace ehp
         return hipGetLastError();
     }
 
-    template <class T, class ST>
+    template <class T>
     hipError_t voxel_adjoint(const PoseGeom* geo, const Dims& dims, const T* lut, int n_lut, float support,
-                             int diff, const ST* sino, ST* vol, hipStream_t s)
+                             int diff, const T* sino, T* vol, hipStream_t s)
     {
         const int64_t per_xcd = ((dims.nvox + 255) / 256 + 7) / 8;
         if (per_xcd * 8 > (int64_t) 0x7fffffff)
             return hipErrorInvalidValue;
         const dim3 grid((unsigned) (per_xcd * 8));
         if (dims.dim == 2)
-            hipLaunchKernelGGL((voxel_adj_kernel<2, T, ST>), grid, dim3(256), 0, s, geo, dims, lut, n_lut, support,
+            hipLaunchKernelGGL((voxel_adj_kernel<2, T>), grid, dim3(256), 0, s, geo, dims, lut, n_lut, support,
                                diff, (int) per_xcd, sino, vol);
         else
-            hipLaunchKernelGGL((voxel_adj_kernel<3, T, ST>), grid, dim3(256), 0, s, geo, dims, lut, n_lut, support,
+            hipLaunchKernelGGL((voxel_adj_kernel<3, T>), grid, dim3(256), 0, s, geo, dims, lut, n_lut, support,
                                diff, (int) per_xcd, sino, vol);
         return hipGetLastError();
     }
@@ -606,7 +456,7 @@ namespace ehp
     template hipError_t siddon_adjoint<T>(const PoseGeom*, const Dims&, const T*, T*, hipStream_t);              \
     template hipError_t voxel_forward<T>(const PoseGeom*, const Dims&, const T*, int, float, int, const T*, T*,   \
                                          hipStream_t);                                                           \
-    template hipError_t voxel_adjoint<T, T>(const PoseGeom*, const Dims&, const T*, int, float, int, const T*,    \
+    template hipError_t voxel_adjoint<T>(const PoseGeom*, const Dims&, const T*, int, float, int, const T*,    \
                                             T*, hipStream_t);
 
     EHP_INSTANTIATE(float)

@@ -183,6 +183,7 @@ namespace ehp
         int n_lut;
         float support;
         int diff;
+        int parts;
         int64_t vol_off, sino_off;
         int64_t block0;
     };
@@ -191,10 +192,11 @@ namespace ehp
                                   std::vector<int>& blocks, size_t& lds, int& cols);
     hipError_t voxel_forward_batch(int dim, int cols, const VoxFwdJob* jobs, const int* blocks, int64_t nblocks,
                                    size_t lds, const int* d_fixexp, const float* vols, float* sinos, hipStream_t s);
-    void voxel_adjoint_batch_jobs(const VoxBatchItem* items, int n, std::vector<VoxAdjJob>& jobs,
-                                  std::vector<int>& blocks);
-    hipError_t voxel_adjoint_batch(int dim, const VoxAdjJob* jobs, const int* blocks, int64_t nblocks,
-                                   const float* sinos, float* vols, hipStream_t s);
+    int voxel_gather_parts(const Dims& dims);
+    void voxel_gather_batch_jobs(const VoxBatchItem* items, int n, std::vector<VoxAdjJob>& jobs,
+                                 std::vector<int>& blocks, size_t& lds, int& cols, int& threads);
+    hipError_t voxel_gather_batch(int dim, int cols, const VoxAdjJob* jobs, const int* blocks, int64_t nblocks,
+                                  size_t lds, int threads, const float* sinos, float* vols, hipStream_t s);
 
     template <class T>
     hipError_t launch_fill(T* p, int64_t n, T value, hipStream_t s);
@@ -255,14 +257,14 @@ namespace ehp
     template <class T>
     hipError_t voxel_forward(const PoseGeom* geo, const Dims& dims, const T* lut, int n_lut, float support,
                              int diff, const T* vol, T* sino, hipStream_t s);
-    // elsa's tap arithmetic (a division per tap): the one-thread-per-voxel kernels and FP64
-    template <class T, class ST = T>
+    // elsa's tap arithmetic (a division per tap): the one-thread-per-voxel kernels
+    template <class T>
     hipError_t voxel_adjoint(const PoseGeom* geo, const Dims& dims, const T* lut, int n_lut, float support,
-                             int diff, const ST* sino, ST* vol, hipStream_t s);
-    // the default FP32 gather, with the tiled forward's tap arithmetic (ST: float or bfloat16)
-    template <class ST>
-    hipError_t voxel_adjoint_fast(const PoseGeom* geo, const Dims& dims, const float* lut, int n_lut, float support,
-                                  int diff, const ST* sino, ST* vol, hipStream_t s);
+                             int diff, const T* sino, T* vol, hipStream_t s);
+    // the default gather, with the tiled forward's tap arithmetic
+    template <class ST, class LT>
+    hipError_t voxel_gather(const PoseGeom* geo, const Dims& dims, const LT* lut, int n_lut, float support, int diff,
+                            const VoxPlan& plan, const ST* sino, ST* vol, hipStream_t s);
     hipError_t voxel_count(const PoseGeom* geo, const Dims& dims, float support, unsigned long long* total,
                            hipStream_t s);
 

@@ -131,15 +131,23 @@ namespace ehp
     // footprint). The homogeneous division is the quotient q = p rcp(w) with one correction,
     // q + (p - q w) rcp(w) (two FMAs): within about half an ulp of p / w, as the centre, a
     // coordinate of hundreds of pixels from which the taps' pixel indices are subtracted, needs.
-    // The scaling sdd / |ext x| = sdd rsq(|ext x|^2) and rs = 1 / scaling come within an ulp or
+    // The scaling sdd / |ext x| = sdd rsq(|ext x|^2), by FMAs, and rs = 1 / scaling come within an ulp or
     // two (relative errors of 1e-7 in the tap distances). Forward and back projection share it, so
     // they stay each other's adjoint.
     template <int D>
     EHP_HD inline void footprint_fast(const PoseGeom& g, const Dims& dims, int x, int y, int z, float radius,
                                       Footprint& fp, float& rs)
     {
-        float pc[3], ce[3];
-        voxel_project<D>(g, x, y, z, pc, ce);
+        float pc[3], ce[3], unused[3];
+        voxel_project<D>(g, x, y, z, pc, unused);
+        const float h[3] = {(float) x + 0.5f, (float) y + 0.5f, (float) z + 0.5f};
+#pragma unroll
+        for (int i = 0; i < D; ++i) {
+            ce[i] = g.ext[i + D * D];
+#pragma unroll
+            for (int j = D - 1; j >= 0; --j)
+                ce[i] = __builtin_fmaf(g.ext[i + j * D], h[j], ce[i]);
+        }
         const float w = pc[D - 1];
         const float rw = fast_rcp(w);
 #pragma unroll
@@ -150,7 +158,7 @@ namespace ehp
         float n2 = ce[0] * ce[0];
 #pragma unroll
         for (int i = 1; i < D; ++i)
-            n2 = n2 + ce[i] * ce[i];
+            n2 = __builtin_fmaf(ce[i], ce[i], n2);
         fp.scaling = g.sdd * fast_rsq(n2);
         rs = fast_rcp(fp.scaling);
         footprint_rect<D>(dims, radius, fp);
@@ -303,7 +311,7 @@ namespace ehp
         return index <= (float) (n - 1) ? w : 0.0;
     }
 
-    // The weight of an FP32 tap as the tiled forward forms it, from the distances in table units: d0k =
+    // The weight of an FP32 tap as every FP32 kernel forms it, from the distances in table units: d0k =
     // (c0 - i) rsk and d1s = ((c1 - j) rsk)^2 (2D: 0) with rsk = (n - 1) / (support scaling), so that
     // the square root is the table index; du = d0 in footprint radii (diff in 3D only).
     template <int D, bool TZ>
@@ -328,6 +336,21 @@ namespace ehp
             d0k[i] = d * rsk;
             if (!TZ)
                 d0k[i] = l0 + i <= h0 ? d0k[i] : 1.0e6f;
+            du[i] = diff ? d * rs : 1.0f;
+        }
+    }
+
+    // The same for NC columns from lo, of which those past the last lie just past the end of the table
+    // (index at least n - 1 + 1/16, below lerp_table_size(n) on every row), so that every table gives them 0.
+    template <int NC>
+    EHP_HD inline void column_units_clipped(float c0, int lo, int last, int n, float rs, float rsk, bool diff,
+                                            float* d0k, float* du)
+    {
+        const float past = (float) (n - 1) + 0.0625f;
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            const float d = c0 - (float) (lo + i);
+            d0k[i] = i <= last ? d * rsk : past;
             du[i] = diff ? d * rs : 1.0f;
         }
     }

@@ -285,9 +285,9 @@ namespace ehp
     // columns (VoxFan), as lanes whose voxels fall on one pixel add to one LDS word in turn.
     //
     // Bound by vector instructions and LDS together: a tap is 13 instructions (the square root counts as
-    // four issues) and two LDS operations, a voxel another 150 (projection, scaling, rectangle). At
-    // 131 x 125 x 119 blobs on 193 x 187, 180 poses: 2.55e9 wavefront instructions (0.69 a cycle and CU, with
-    // the square roots 0.8), the LDS active 0.6 of the time; 5.60 ms against 11.42 ms for loops over the
+    // four issues) and two LDS operations, a voxel another 140 (projection, scaling, rectangle). At
+    // 131 x 125 x 119 blobs on 193 x 187, 180 poses: 2.69e9 wavefront instructions (0.78 a cycle and CU), the
+    // LDS active 0.65 of the time; 5.48 ms against 11.42 ms for loops over the
     // clipped rectangle in 32 x 32 tiles, which ran 26 instructions a tap and left lanes idle in the
     // loops over columns. FP64 B-splines 96^3 on 144^2, 90 poses: 2.39 ms against 5.33 ms (correctly rounded
     // divisions from reciprocals that are formed once, div_rounded).

@@ -59,6 +59,19 @@ namespace
                 row_units<NC, TZ>(tab.data(), n, fp.center[1], j, rsk, d0k, du, diff, w);
                 row_units64<NC>(tab64.data(), n, support, 1.0f / support, fp.center[1], j, fp.scaling,
                                 1.0f / fp.scaling, d0, diff, w64);
+                // clipped to columns of the footprint's middle (the detector's edge): the same weights
+                // inside, 0 past the last from entries of the pair table
+                float dc[NC], uc[NC], wc[NC];
+                const int lo = l0 + (k & 1), last = h0 - lo - (k >> 1 & 1);
+                column_units_clipped<NC>(fp.center[0], lo, last, n, rs, rsk, diff, dc, uc);
+                row_units<NC, TZ>(tab.data(), n, fp.center[1], j, rsk, dc, uc, diff, wc);
+                for (int i = 0; i < NC; ++i) {
+                    const float d1c = (fp.center[1] - (float) j) * rsk;
+                    if ((int) std::sqrt(std::fma(dc[i], dc[i], d1c * d1c)) >= lerp_table_size(n))
+                        return 6;
+                    if (i <= last ? wc[i] != w[i + (k & 1)] : wc[i] != 0.0f)
+                        return 7;
+                }
                 for (int i = 0; i < NC; ++i) {
                     const float d1k = (fp.center[1] - (float) j) * rsk;
                     if (TZ && (int) std::sqrt(std::fma(d0k[i], d0k[i], d1k * d1k)) >= span)

@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 # basis function, detector distance over source distance: 4 (B-spline) and 5, 6, 8, 9, 13 columns
 CASES = [("bspline", 0.05), ("blob", 0.05), ("blob", 0.35), ("bspline", 1.2), ("blob", 0.8), ("blob", 1.2),
          ("blob", 2.0)]
-SIZES = [((13, 9, 11), (23, 17), 7), ((1, 1, 3), (5, 4), 3), ((33, 40, 7), (41, 3), 5)]
+# (with 150 and 40 poses the gather sums in sixteen and four parts)
+SIZES = [((13, 9, 11), (23, 17), 7), ((1, 1, 3), (5, 4), 150), ((33, 40, 7), (41, 3), 40)]
 
 
 def rel_l2(a, b):
@@ -52,6 +53,26 @@ def test_voxel_columns(kind, ratio, size, dtype):
         np.testing.assert_array_equal(op.apply(x), got, err_msg=str(tile))
     x.reshape(-1)[1] = np.inf
     assert np.isnan(op.apply(x)).all()
+    # an infinite pixel reaches the voxels whose footprints hold it and no others
+    y[:] = 0
+    y.reshape(-1)[y.size // 2] = 1
+    held = op.applyAdjoint(y) != 0
+    y.reshape(-1)[y.size // 2] = np.inf
+    got = op.applyAdjoint(y)
+    near = oracle.voxel(g, y, lut, 1.01 * sup, adjoint=True, acc64=True)
+    assert not np.isfinite(got[held]).any() and np.isfinite(got[np.isfinite(near)]).all()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("vol,det,poses", [((1, 5), 9, 7), ((31, 17), 40, 33), ((24, 40), 61, 140)])
+def test_gather_parts_2d(vol, det, poses, dtype):
+    import elsa_amd as E
+
+    g = oracle.circle_geometry(2, vol, poses, 360, 200.0, 60.0, det=(det,))
+    op = E.BlobVoxelProjectorCUDA(*geom_to_descriptors(g), dtype=dtype)
+    y = np.random.default_rng(6).random(g.sino_shape).astype(dtype)
+    ref = oracle.voxel(g, y, oracle.blob_lut(2.0, 10.83, 2, 100, dtype), 2.0, adjoint=True, acc64=True)
+    assert rel_l2(op.applyAdjoint(y), ref) <= (1e-6 if dtype == np.float32 else 1e-13)
 
 
 @pytest.mark.parametrize("second", [("blob", 0.1), ("blob", 0.35), ("bspline", 1.2)])
