@@ -242,9 +242,7 @@ int ehp_geometry_set_pixel_coords(ehp_geometry* g, const float* coords)
 namespace
 {
     // Tile shape of the LDS-privatised back projections, shrunk until it fits the device's LDS
-    // per workgroup. Joseph 3D: 8 x 17 x 17 (9.15 ms against 9.3 ms for 8 x 15 x 15 and 9.7 ms for
-    // 8 x 19 x 19 at 256^3 / 360 poses; odd widths, as an even slot row stride costs LDS bank
-    // conflicts: 12.6 ms for 8 x 18 x 18).
+    // per workgroup.
     size_t tile_lds_bytes(int kind, const ehp::Dims& dims, const ehp::TileCfg& tc, int dtype = EHP_F32)
     {
         if (kind == KIND_VOXEL)
@@ -252,9 +250,41 @@ namespace
         return kind == KIND_SIDDON ? ehp::siddon_tile_lds_bytes(dims, tc) : ehp::joseph_tile_lds_bytes(dims, tc);
     }
 
-    // cus: compute units of the device. A 3D back projection launch is one workgroup per tile; a
-    // small volume gets thinner tiles (fewer planes each) until a launch has about 8 workgroups
-    // per CU, which keeps the device busy (128^3: 1024 tiles of 8 planes, 2048 of 4).
+    // 3D Joseph tiles: four planes of up to 32 x 32 voxels, the widths evened over the volume (a large
+    // cross-section spends less on the halo and on rays that leave sideways, few planes leave four
+    // workgroups of 512 a CU). While a launch of two axes has fewer than three tiles a CU, cross-sections
+    // of 24 and 16; below one a CU two planes. Back projections, us (512 threads, both axes in one launch):
+    //   256^3 / 360 poses  4x32x32 7547  8x24x24 8160  8x22x22 7647  8x17x17 8450
+    //   128^3 / 180        4x32x32  607  8x16x16  613  4x22x22  635  4x16x16  667
+    //   96^3 / 120         4x24x24  226  8x16x16  236  4x16x16  243  2x16x16  267
+    //   64^3 / 90          4x16x16   81  4x24x24  120  2x16x16  101
+    ehp::TileCfg joseph_tile3d(const ehp::Dims& dims, int cus)
+    {
+        ehp::TileCfg tc{4, 32, 32};
+        auto tiles = [&] {
+            int64_t n = 0;
+            for (int a = 0; a < 3; a += 2) {
+                int nA, nB, nC;
+                ehp::tile_counts(dims, tc, a, nA, nB, nC);
+                n += (int64_t) nA * nB * nC;
+            }
+            return n;
+        };
+        for (int w = 32; w >= 16; w -= 8) {
+            auto even = [&](int n) { return (n + (n + w - 1) / w - 1) / ((n + w - 1) / w); };
+            tc.TB = std::max(even(dims.vol[0]), even(dims.vol[1]));
+            tc.TC = std::max(even(dims.vol[1]), even(dims.vol[2]));
+            if (tiles() >= 3 * (int64_t) cus)
+                break;
+        }
+        if (tiles() < cus)
+            tc.LA = 2;
+        return tc;
+    }
+
+    // cus: compute units of the device. A 3D Siddon launch is one workgroup per tile; a small volume
+    // gets thinner tiles (fewer planes each) until a launch has about 8 workgroups per CU, which
+    // keeps the device busy (128^3: 1024 tiles of 8 planes, 2048 of 4).
     // 2D Joseph: squares, the largest of 32, 16 and 8 that give every CU a tile (large tiles spend less on their
     // halo and on rays that only pass a corner; with fewer tiles than CUs the launch waits for its
     // slowest tile): 512^2 / 360 poses 32: 109 us, 16: 123; 256^2 / 180 16: 34, 32: 59, 8: 41;
@@ -265,12 +295,12 @@ namespace
         if (kind == KIND_SIDDON)
             tc = dims.dim == 3 ? ehp::TileCfg{8, 16, 16} : ehp::TileCfg{4, 16, 1};
         else if (dims.dim == 3)
-            tc = ehp::TileCfg{8, 17, 17};
+            tc = joseph_tile3d(dims, cus);
         else
             return joseph_tile2d(dims.nvox, cus);
         while (tc.LA > 1 && (int) tile_lds_bytes(kind, dims, tc) > max_lds)
             tc.LA /= 2;
-        while (dims.dim == 3 && tc.LA > 2) {
+        while (kind == KIND_SIDDON && dims.dim == 3 && tc.LA > 2) {
             int ntA, ntB, ntC;
             ehp::tile_counts(dims, tc, 0, ntA, ntB, ntC);
             if ((int64_t) ntA * ntB * ntC >= (int64_t) 8 * cus)

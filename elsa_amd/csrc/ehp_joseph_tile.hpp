@@ -111,6 +111,13 @@ namespace ehp
         static constexpr int b2 = (D == 2) ? 0 : (A == 2 ? 1 : 2);
     };
 
+    // Slots of a tile's row: its voxels and the halo, in 3D odd (the atomics of neighbouring rows then
+    // fall on different LDS banks)
+    EHP_HD inline int tile_row_slots(int dim, int TB)
+    {
+        return dim == 3 ? (TB + 2) | 1 : TB + 2;
+    }
+
     template <int D, int A>
     EHP_HD inline TileBox make_tile(const Dims& dims, const TileCfg& tc, int ia, int ib, int ic)
     {
@@ -122,7 +129,7 @@ namespace ehp
         t.B1 = dims.vol[b1] < t.B0 + tc.TB ? dims.vol[b1] : t.B0 + tc.TB;
         t.C0 = (D == 3) ? ic * tc.TC : 0;
         t.C1 = (D == 3) ? (dims.vol[b2] < t.C0 + tc.TC ? dims.vol[b2] : t.C0 + tc.TC) : 1;
-        t.PB = tc.TB + 2;
+        t.PB = tile_row_slots(D, tc.TB);
         t.PC = (D == 3) ? tc.TC + 2 : 1;
         t.nslots = tc.LA * t.PC * t.PB;
         t.B0m1f = (float) (t.B0 - 1);
@@ -552,8 +559,7 @@ namespace ehp
     };
     // Dynamic LDS of a tiled back projection after the tile's 8-byte slots: the rectangles,
     // candidate counts and their prefix sums of a batch of `batch` poses, sized by the launch's
-    // batch (at 8 x 17 x 17 tiles and 8 poses that keeps a workgroup under a seventh of the
-    // CU's 160 KB, where 32 poses' worth would allow only six workgroups per CU).
+    // batch.
     EHP_HD constexpr size_t batch_lds_bytes(int batch)
     {
         return ((size_t) batch * sizeof(CandRect) + (size_t) (2 * batch + 1) * sizeof(int) + 7) & ~(size_t) 7;

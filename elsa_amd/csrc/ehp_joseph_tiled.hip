@@ -5,9 +5,11 @@
 // long along one driving axis a (LA planes) and TB x TC voxels across. One workgroup owns a
 // tile for all poses: it accumulates in LDS every sample of every ray whose driving axis is
 // a and whose bilinear footprint touches the tile, then adds the tile to the volume once.
-// One launch per driving axis that occurs in the trajectory ("pass"); each voxel is owned by
-// exactly one tile per pass, so passes are plain read-modify-write. In 2D a tile takes the rays of
-// both axes (adj2d_block) and one launch writes the volume.
+// Each voxel is owned by exactly one tile per driving axis that occurs in the trajectory. With two
+// such axes, as about any axis of rotation, one launch runs the tiles of both (joseph_adj_pair_kernel:
+// a voxel gets two sums, added by whichever workgroup comes second); otherwise one launch per axis
+// adds to the volume in plain read-modify-write. In 2D a tile takes the rays of both axes
+// (adj2d_block) and one launch writes the volume.
 //
 // Accumulation: LDS float atomics are slow on this part (a ds_add_f32 wave operation costs
 // about 15 times a ds_add_u64), so the tile is summed with 64-bit integer atomics in fixed
@@ -22,11 +24,13 @@
 // same arithmetic as joseph_sample, so they are bit-identical to the forward's.
 #include "ehp_kernels.hpp"
 
+#include <type_traits>
+
 namespace ehp
 {
     namespace
     {
-        constexpr int kThreads = 256;
+        constexpr int kThreads = 512; // of the 3D back projection's workgroups
         // LDS (address space 3) pointers: 32-bit byte addresses
         typedef __attribute__((address_space(3))) unsigned long long lds_u64;
         typedef __attribute__((address_space(3))) char lds_char;
@@ -435,8 +439,19 @@ namespace ehp
                                 fixexp + J.item, sinos + J.sino_off, vols + J.vol_off);
     }
 
+    // Adds v to a voxel that starts at 0 and gets two sums in all, from workgroups in any order: whichever
+    // comes second finds the first's sum in exchange for its own and stores both, so the result is the
+    // two sums' rounded sum either way.
+    template <class T>
+    __device__ __forceinline__ void add_second(T* p, T v)
+    {
+        const T first = __hip_atomic_exchange(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (first != T(0))
+            __hip_atomic_store(p, first + v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+
     // One tile of the back projection along driving axis A (tile < ntA * ntB * ntC).
-    template <int D, int A, class ST = float>
+    template <int D, int A, bool PAIR, class ST = float>
     __device__ __forceinline__ void adj_tiled_block(const PoseGeom* __restrict__ geo,
                                                     const RayRec* __restrict__ table, const Dims& dims,
                                                     const int* __restrict__ pose_axes, const TileCfg& tc,
@@ -490,17 +505,22 @@ namespace ehp
             __syncthreads();
         }
 
-        // add the owned voxels of the tile to the volume
+        // add the owned voxels of the tile to the volume (PAIR: the other axis' tiles may add theirs now)
         const double q = eg == kNonFinite ? __longlong_as_double(0x7ff8000000000000ll) : ldexp(1.0, eg - 62);
         for (int i = tid; i < t.nslots; i += kThreads) {
             const int64_t lin = tile_slot_voxel<D, A>(t, dims, i);
-            if (lin >= 0)
-                vol[lin] += (typename Acc<ST>::type) ((double) iacc[i] * q);
+            if (lin < 0)
+                continue;
+            const typename Acc<ST>::type sum = (typename Acc<ST>::type) ((double) iacc[i] * q);
+            if (PAIR)
+                add_second(vol + lin, sum);
+            else
+                vol[lin] += sum;
         }
     }
 
     template <int D, int A, class ST>
-    __global__ void __launch_bounds__(kThreads)
+    __global__ void __launch_bounds__(kThreads, 8)
         joseph_adj_tiled_kernel(const PoseGeom* __restrict__ geo, const RayRec* __restrict__ table, const Dims dims,
                                 const int* __restrict__ pose_axes, const TileCfg tc, const int ntA, const int ntB,
                                 const int ntC, const int tiles_per_xcd, const int batch,
@@ -511,24 +531,101 @@ namespace ehp
         const int tile = (int) (blockIdx.x % 8u) * tiles_per_xcd + (int) (blockIdx.x / 8u);
         if (tile >= ntA * ntB * ntC)
             return;
-        adj_tiled_block<D, A, ST>(geo, table, dims, pose_axes, tc, ntA, ntB, tile, batch, fixexp, sino, vol);
+        adj_tiled_block<D, A, false, ST>(geo, table, dims, pose_axes, tc, ntA, ntB, tile, batch, fixexp, sino, vol);
+    }
+
+    // The tiles of two driving axes A0 < A1 in one launch: the counts along A, b1 and b2 of either axis
+    struct TileCounts {
+        int nA, nB, n, per_xcd;
+    };
+
+    // One launch leaves the device waiting for its last workgroups once instead of twice. Bound by the
+    // LDS and VALU together (64-bit atomics, four a sample: the LDS is busy 0.97 of the time, vector
+    // instructions 0.85 a cycle and CU). Workgroups of 512 threads over tiles of four planes
+    // (64 VGPRs, so that 32 wavefronts a CU fit), against one launch of 256 threads per axis over 8 x 17 x 17 and 4 x 17 x
+    // 17 tiles: 256^3 / 360 poses 8.61 -> 7.55 ms, 128^3 / 180 0.79 -> 0.61, 96^3 / 120 0.33 -> 0.23, 64^3 / 90
+    // 0.142 -> 0.081, FP64 97 x 61 x 113 / 77 0.195 -> 0.17.
+    template <int A0, int A1, class ST>
+    __global__ void __launch_bounds__(kThreads, 8)
+        joseph_adj_pair_kernel(const PoseGeom* __restrict__ geo, const RayRec* __restrict__ table, const Dims dims,
+                               const int* __restrict__ pose_axes, const TileCfg tc, const TileCounts c0,
+                               const TileCounts c1, const int batch, const int* __restrict__ fixexp,
+                               const ST* __restrict__ sino, typename Acc<ST>::type* __restrict__ vol)
+    {
+        const int xcd = (int) (blockIdx.x % 8u), k = (int) (blockIdx.x / 8u);
+        if (k < c0.per_xcd) {
+            const int tile = xcd * c0.per_xcd + k;
+            if (tile < c0.n)
+                adj_tiled_block<3, A0, true, ST>(geo, table, dims, pose_axes, tc, c0.nA, c0.nB, tile, batch, fixexp,
+                                                 sino, vol);
+        } else {
+            const int tile = xcd * c1.per_xcd + k - c0.per_xcd;
+            if (tile < c1.n)
+                adj_tiled_block<3, A1, true, ST>(geo, table, dims, pose_axes, tc, c1.nA, c1.nB, tile, batch, fixexp,
+                                                 sino, vol);
+        }
     }
 
     // the tiles of axis A of many operators in one launch (block b: tile b - job.block0 of job
     // block_job[b])
-    template <int D, int A>
-    __global__ void __launch_bounds__(kThreads)
+    template <int A, bool PAIR>
+    __device__ __forceinline__ void adj_batch_block(const AdjJob* __restrict__ jobs, const int* __restrict__ block_job,
+                                                    const int64_t id, const int* __restrict__ fixexp,
+                                                    const float* __restrict__ sinos, float* __restrict__ vols)
+    {
+        const AdjJob& J = jobs[block_job[id]];
+        adj_tiled_block<3, A, PAIR, float>(J.geo, J.table, J.dims, J.pose_axes, J.tc, J.ntA, J.ntB,
+                                           (int) (id - J.block0), J.batch, fixexp + J.item, sinos + J.sino_off,
+                                           vols + J.vol_off);
+    }
+
+    template <int A>
+    __global__ void __launch_bounds__(kThreads, 8)
         joseph_adj_tiled_batch_kernel(const AdjJob* __restrict__ jobs, const int* __restrict__ block_job,
                                       const int per_xcd, const int64_t total, const int* __restrict__ fixexp,
                                       const float* __restrict__ sinos, float* __restrict__ vols)
     {
         const int64_t id = (int64_t) (blockIdx.x % 8u) * per_xcd + (blockIdx.x / 8u);
-        if (id >= total)
-            return;
-        const int j = block_job[id];
-        const AdjJob& J = jobs[j];
-        adj_tiled_block<D, A, float>(J.geo, J.table, J.dims, J.pose_axes, J.tc, J.ntA, J.ntB, (int) (id - J.block0),
-                                     J.batch, fixexp + J.item, sinos + J.sino_off, vols + J.vol_off);
+        if (id < total)
+            adj_batch_block<A, false>(jobs, block_job, id, fixexp, sinos, vols);
+    }
+
+    struct BatchTiles { // the tiles of one driving axis
+        const AdjJob* jobs;
+        const int* block_job;
+        int64_t total;
+        int per_xcd;
+    };
+
+    template <int A0, int A1>
+    __global__ void __launch_bounds__(kThreads, 8)
+        joseph_adj_pair_batch_kernel(const BatchTiles t0, const BatchTiles t1, const int* __restrict__ fixexp,
+                                     const float* __restrict__ sinos, float* __restrict__ vols)
+    {
+        const int64_t xcd = blockIdx.x % 8u;
+        const int k = (int) (blockIdx.x / 8u);
+        if (k < t0.per_xcd) {
+            const int64_t id = xcd * t0.per_xcd + k;
+            if (id < t0.total)
+                adj_batch_block<A0, true>(t0.jobs, t0.block_job, id, fixexp, sinos, vols);
+        } else {
+            const int64_t id = xcd * t1.per_xcd + k - t0.per_xcd;
+            if (id < t1.total)
+                adj_batch_block<A1, true>(t1.jobs, t1.block_job, id, fixexp, sinos, vols);
+        }
+    }
+
+    // fn(first, second) of two of three axes, as constants
+    template <class Fn>
+    void with_axis_pair(int axes, Fn fn)
+    {
+        using std::integral_constant;
+        if (axes == 3)
+            fn(integral_constant<int, 0>{}, integral_constant<int, 1>{});
+        else if (axes == 5)
+            fn(integral_constant<int, 0>{}, integral_constant<int, 2>{});
+        else
+            fn(integral_constant<int, 1>{}, integral_constant<int, 2>{});
     }
 
     // max|y| per operator of a batch: block b writes the maximum of its share of segment
@@ -593,7 +690,7 @@ namespace ehp
     size_t joseph_tile_lds_bytes(const Dims& dims, const TileCfg& tc, int batch)
     {
         const int PC = dims.dim == 3 ? tc.TC + 2 : 1;
-        return (size_t) tc.LA * PC * (tc.TB + 2) * sizeof(long long) + batch_lds_bytes(batch);
+        return (size_t) tc.LA * PC * tile_row_slots(dims.dim, tc.TB) * sizeof(long long) + batch_lds_bytes(batch);
     }
 
     // ST: the sinogram's storage type (float, or bf16 for bfloat16 operators); the volume is
@@ -631,6 +728,28 @@ namespace ehp
         if (e != hipSuccess)
             return e;
         const size_t lds = joseph_tile_lds_bytes(dims, tc, batch);
+        if (axes_present == 3 || axes_present == 5 || axes_present == 6) {
+            with_axis_pair(axes_present, [&](auto a0, auto a1) {
+                auto counts = [&](int a) {
+                    TileCounts c;
+                    int nC;
+                    tile_counts(dims, tc, a, c.nA, c.nB, nC);
+                    c.n = c.nA * c.nB * nC;
+                    c.per_xcd = (c.n + 7) / 8;
+                    return c;
+                };
+                const TileCounts c0 = counts(a0), c1 = counts(a1);
+                if ((int64_t) (c0.per_xcd + c1.per_xcd) * 8 > (int64_t) 0x7fffffff) {
+                    e = hipErrorInvalidValue;
+                    return;
+                }
+                hipLaunchKernelGGL((joseph_adj_pair_kernel<decltype(a0)::value, decltype(a1)::value, ST>),
+                                   dim3((unsigned) (c0.per_xcd + c1.per_xcd) * 8), dim3(kThreads), lds, s, geo, table,
+                                   dims, pose_axes, tc, c0, c1, batch, d_fixexp, sino, vol);
+                e = hipGetLastError();
+            });
+            return e;
+        }
         for (int a = 0; a < dims.dim; ++a) {
             if (!(axes_present & (1 << a)))
                 continue;
@@ -773,6 +892,26 @@ namespace ehp
             e = fixed_point_exponent_batch(nitems, segs, sblocks, nsblocks, bounds, d_maxbits, d_fixexp, sinos, s);
         if (e != hipSuccess)
             return e;
+        int axes = 0;
+        for (int a = 0; a < dim; ++a)
+            axes |= nablocks[a] > 0 ? 1 << a : 0;
+        if (dim == 3 && (axes == 3 || axes == 5 || axes == 6)) {
+            with_axis_pair(axes, [&](auto a0, auto a1) {
+                const int64_t p0 = (nablocks[a0] + 7) / 8, p1 = (nablocks[a1] + 7) / 8;
+                if ((p0 + p1) * 8 > (int64_t) 0x7fffffff) {
+                    e = hipErrorInvalidValue;
+                    return;
+                }
+                const BatchTiles t0{ajobs[a0], ablocks[a0], nablocks[a0], (int) p0};
+                const BatchTiles t1{ajobs[a1], ablocks[a1], nablocks[a1], (int) p1};
+                const size_t need = lds[a0] > lds[a1] ? lds[a0] : lds[a1];
+                hipLaunchKernelGGL((joseph_adj_pair_batch_kernel<decltype(a0)::value, decltype(a1)::value>),
+                                   dim3((unsigned) (p0 + p1) * 8), dim3(kThreads), need, s, t0, t1, d_fixexp, sinos,
+                                   vols);
+                e = hipGetLastError();
+            });
+            return e;
+        }
         for (int a = 0; a < dim; ++a) {
             const int64_t total = nablocks[a];
             if (total == 0)
@@ -782,7 +921,7 @@ namespace ehp
                 return hipErrorInvalidValue;
             const dim3 grid((unsigned) (per_xcd * 8));
 #define EHP_ADJ_BATCH(Av)                                                                                          \
-    hipLaunchKernelGGL((joseph_adj_tiled_batch_kernel<3, Av>), grid, dim3(kThreads), lds[a], s, ajobs[a], ablocks[a],   \
+    hipLaunchKernelGGL((joseph_adj_tiled_batch_kernel<Av>), grid, dim3(kThreads), lds[a], s, ajobs[a], ablocks[a],   \
                        (int) per_xcd, total, d_fixexp, sinos, vols)
             if (dim == 2)
                 hipLaunchKernelGGL(joseph_adj2d_batch_kernel, grid, dim3(256), lds[a], s, ajobs[a], ablocks[a],
