@@ -250,6 +250,26 @@ namespace
         return kind == KIND_SIDDON ? ehp::siddon_tile_lds_bytes(dims, tc) : ehp::joseph_tile_lds_bytes(dims, tc);
     }
 
+    // la planes of at most w x w voxels, the widths evened over the volume
+    ehp::TileCfg even_tile(const ehp::Dims& dims, int la, int w)
+    {
+        auto even = [&](int n) { return (n + (n + w - 1) / w - 1) / ((n + w - 1) / w); };
+        return ehp::TileCfg{la, std::max(even(dims.vol[0]), even(dims.vol[1])),
+                            std::max(even(dims.vol[1]), even(dims.vol[2]))};
+    }
+
+    // Tiles of a launch over two driving axes (the first and the last, as about any axis of rotation)
+    int64_t two_axis_tiles(const ehp::Dims& dims, const ehp::TileCfg& tc)
+    {
+        int64_t n = 0;
+        for (int a = 0; a < 3; a += 2) {
+            int nA, nB, nC;
+            ehp::tile_counts(dims, tc, a, nA, nB, nC);
+            n += (int64_t) nA * nB * nC;
+        }
+        return n;
+    }
+
     // 3D Joseph tiles: four planes of up to 32 x 32 voxels, the widths evened over the volume (a large
     // cross-section spends less on the halo and on rays that leave sideways, few planes leave four
     // workgroups of 512 a CU). While a launch of two axes has fewer than three tiles a CU, cross-sections
@@ -260,53 +280,52 @@ namespace
     //   64^3 / 90          4x16x16   81  4x24x24  120  2x16x16  101
     ehp::TileCfg joseph_tile3d(const ehp::Dims& dims, int cus)
     {
-        ehp::TileCfg tc{4, 32, 32};
-        auto tiles = [&] {
-            int64_t n = 0;
-            for (int a = 0; a < 3; a += 2) {
-                int nA, nB, nC;
-                ehp::tile_counts(dims, tc, a, nA, nB, nC);
-                n += (int64_t) nA * nB * nC;
-            }
-            return n;
-        };
+        ehp::TileCfg tc{};
         for (int w = 32; w >= 16; w -= 8) {
-            auto even = [&](int n) { return (n + (n + w - 1) / w - 1) / ((n + w - 1) / w); };
-            tc.TB = std::max(even(dims.vol[0]), even(dims.vol[1]));
-            tc.TC = std::max(even(dims.vol[1]), even(dims.vol[2]));
-            if (tiles() >= 3 * (int64_t) cus)
+            tc = even_tile(dims, 4, w);
+            if (two_axis_tiles(dims, tc) >= 3 * (int64_t) cus)
                 break;
         }
-        if (tiles() < cus)
+        if (two_axis_tiles(dims, tc) < cus)
             tc.LA = 2;
         return tc;
     }
 
-    // cus: compute units of the device. A 3D Siddon launch is one workgroup per tile; a small volume
-    // gets thinner tiles (fewer planes each) until a launch has about 8 workgroups per CU, which
-    // keeps the device busy (128^3: 1024 tiles of 8 planes, 2048 of 4).
+    // 3D Siddon tiles: eight planes of up to 22 x 22 voxels, evened; of 16 x 16 while a launch of two
+    // axes has fewer than eight tiles a CU, and below two a CU fewer planes. Back projections, us:
+    //   256^3 / 360 poses  8x22x22 9874  8x24x24 10036  8x16x16 10317  4x32x32 10817
+    //   128^3 / 180        8x16x16  782  8x22x22   852  4x16x16   871
+    //   50 x 36 x 38 / 62  2x16x16   56  4x16x16    57  8x16x16    77
+    ehp::TileCfg siddon_tile3d(const ehp::Dims& dims, int cus)
+    {
+        ehp::TileCfg tc = even_tile(dims, 8, 22);
+        if (two_axis_tiles(dims, tc) < 8 * (int64_t) cus)
+            tc = even_tile(dims, 8, 16);
+        while (tc.LA > 2 && two_axis_tiles(dims, tc) < 2 * (int64_t) cus)
+            tc.LA /= 2;
+        return tc;
+    }
+
+    // cus: compute units of the device.
     // 2D Joseph: squares, the largest of 32, 16 and 8 that give every CU a tile (large tiles spend less on their
     // halo and on rays that only pass a corner; with fewer tiles than CUs the launch waits for its
     // slowest tile): 512^2 / 360 poses 32: 109 us, 16: 123; 256^2 / 180 16: 34, 32: 59, 8: 41;
     // 128^2 / 180 8: 26, 16: 34; 64^2 / 90 8: 19, 16: 24.
+    // 2D Siddon, in the same way: 500 x 420 / 500 poses 8 x 32: 177 us, 8 x 16: 230, 4 x 16: 336; 320^2 / 300
+    // 92, 89, 120; 256^2 / 180 61, 54, 53.
     ehp::TileCfg default_tile(int kind, const ehp::Dims& dims, int max_lds, int cus)
     {
         ehp::TileCfg tc;
-        if (kind == KIND_SIDDON)
-            tc = dims.dim == 3 ? ehp::TileCfg{8, 16, 16} : ehp::TileCfg{4, 16, 1};
-        else if (dims.dim == 3)
-            tc = joseph_tile3d(dims, cus);
-        else
+        if (dims.dim == 2 && kind == KIND_JOSEPH)
             return joseph_tile2d(dims.nvox, cus);
+        if (dims.dim == 2)
+            tc = dims.nvox >= 512 * (int64_t) cus ? ehp::TileCfg{8, 32, 1}
+                                                  : (dims.nvox >= 320 * (int64_t) cus ? ehp::TileCfg{8, 16, 1}
+                                                                                      : ehp::TileCfg{4, 16, 1});
+        else
+            tc = kind == KIND_SIDDON ? siddon_tile3d(dims, cus) : joseph_tile3d(dims, cus);
         while (tc.LA > 1 && (int) tile_lds_bytes(kind, dims, tc) > max_lds)
             tc.LA /= 2;
-        while (kind == KIND_SIDDON && dims.dim == 3 && tc.LA > 2) {
-            int ntA, ntB, ntC;
-            ehp::tile_counts(dims, tc, 0, ntA, ntB, ntC);
-            if ((int64_t) ntA * ntB * ntC >= (int64_t) 8 * cus)
-                break;
-            tc.LA /= 2;
-        }
         return tc;
     }
 

@@ -23,6 +23,7 @@
 // the one-thread-per-ray kernels (make_ray, joseph_setup), and the per-sample weights use the
 // same arithmetic as joseph_sample, so they are bit-identical to the forward's.
 #include "ehp_kernels.hpp"
+#include "ehp_tile_pair.hpp"
 
 #include <type_traits>
 
@@ -439,17 +440,6 @@ namespace ehp
                                 fixexp + J.item, sinos + J.sino_off, vols + J.vol_off);
     }
 
-    // Adds v to a voxel that starts at 0 and gets two sums in all, from workgroups in any order: whichever
-    // comes second finds the first's sum in exchange for its own and stores both, so the result is the
-    // two sums' rounded sum either way.
-    template <class T>
-    __device__ __forceinline__ void add_second(T* p, T v)
-    {
-        const T first = __hip_atomic_exchange(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (first != T(0))
-            __hip_atomic_store(p, first + v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-
     // One tile of the back projection along driving axis A (tile < ntA * ntB * ntC).
     template <int D, int A, bool PAIR, class ST = float>
     __device__ __forceinline__ void adj_tiled_block(const PoseGeom* __restrict__ geo,
@@ -534,11 +524,6 @@ namespace ehp
         adj_tiled_block<D, A, false, ST>(geo, table, dims, pose_axes, tc, ntA, ntB, tile, batch, fixexp, sino, vol);
     }
 
-    // The tiles of two driving axes A0 < A1 in one launch: the counts along A, b1 and b2 of either axis
-    struct TileCounts {
-        int nA, nB, n, per_xcd;
-    };
-
     // One launch leaves the device waiting for its last workgroups once instead of twice. Bound by the
     // LDS and VALU together (64-bit atomics, four a sample: the LDS is busy 0.97 of the time, vector
     // instructions 0.85 a cycle and CU). Workgroups of 512 threads over tiles of four planes
@@ -590,16 +575,9 @@ namespace ehp
             adj_batch_block<A, false>(jobs, block_job, id, fixexp, sinos, vols);
     }
 
-    struct BatchTiles { // the tiles of one driving axis
-        const AdjJob* jobs;
-        const int* block_job;
-        int64_t total;
-        int per_xcd;
-    };
-
     template <int A0, int A1>
     __global__ void __launch_bounds__(kThreads, 8)
-        joseph_adj_pair_batch_kernel(const BatchTiles t0, const BatchTiles t1, const int* __restrict__ fixexp,
+        joseph_adj_pair_batch_kernel(const BatchTiles<AdjJob> t0, const BatchTiles<AdjJob> t1, const int* __restrict__ fixexp,
                                      const float* __restrict__ sinos, float* __restrict__ vols)
     {
         const int64_t xcd = blockIdx.x % 8u;
@@ -613,19 +591,6 @@ namespace ehp
             if (id < t1.total)
                 adj_batch_block<A1, true>(t1.jobs, t1.block_job, id, fixexp, sinos, vols);
         }
-    }
-
-    // fn(first, second) of two of three axes, as constants
-    template <class Fn>
-    void with_axis_pair(int axes, Fn fn)
-    {
-        using std::integral_constant;
-        if (axes == 3)
-            fn(integral_constant<int, 0>{}, integral_constant<int, 1>{});
-        else if (axes == 5)
-            fn(integral_constant<int, 0>{}, integral_constant<int, 2>{});
-        else
-            fn(integral_constant<int, 1>{}, integral_constant<int, 2>{});
     }
 
     // max|y| per operator of a batch: block b writes the maximum of its share of segment
@@ -728,17 +693,9 @@ namespace ehp
         if (e != hipSuccess)
             return e;
         const size_t lds = joseph_tile_lds_bytes(dims, tc, batch);
-        if (axes_present == 3 || axes_present == 5 || axes_present == 6) {
+        if (two_axes(axes_present)) {
             with_axis_pair(axes_present, [&](auto a0, auto a1) {
-                auto counts = [&](int a) {
-                    TileCounts c;
-                    int nC;
-                    tile_counts(dims, tc, a, c.nA, c.nB, nC);
-                    c.n = c.nA * c.nB * nC;
-                    c.per_xcd = (c.n + 7) / 8;
-                    return c;
-                };
-                const TileCounts c0 = counts(a0), c1 = counts(a1);
+                const TileCounts c0 = axis_tiles(dims, tc, a0), c1 = axis_tiles(dims, tc, a1);
                 if ((int64_t) (c0.per_xcd + c1.per_xcd) * 8 > (int64_t) 0x7fffffff) {
                     e = hipErrorInvalidValue;
                     return;
@@ -895,15 +852,15 @@ namespace ehp
         int axes = 0;
         for (int a = 0; a < dim; ++a)
             axes |= nablocks[a] > 0 ? 1 << a : 0;
-        if (dim == 3 && (axes == 3 || axes == 5 || axes == 6)) {
+        if (dim == 3 && two_axes(axes)) {
             with_axis_pair(axes, [&](auto a0, auto a1) {
                 const int64_t p0 = (nablocks[a0] + 7) / 8, p1 = (nablocks[a1] + 7) / 8;
                 if ((p0 + p1) * 8 > (int64_t) 0x7fffffff) {
                     e = hipErrorInvalidValue;
                     return;
                 }
-                const BatchTiles t0{ajobs[a0], ablocks[a0], nablocks[a0], (int) p0};
-                const BatchTiles t1{ajobs[a1], ablocks[a1], nablocks[a1], (int) p1};
+                const BatchTiles<AdjJob> t0{ajobs[a0], ablocks[a0], nablocks[a0], (int) p0};
+                const BatchTiles<AdjJob> t1{ajobs[a1], ablocks[a1], nablocks[a1], (int) p1};
                 const size_t need = lds[a0] > lds[a1] ? lds[a0] : lds[a1];
                 hipLaunchKernelGGL((joseph_adj_pair_batch_kernel<decltype(a0)::value, decltype(a1)::value>),
                                    dim3((unsigned) (p0 + p1) * 8), dim3(kThreads), need, s, t0, t1, d_fixexp, sinos,

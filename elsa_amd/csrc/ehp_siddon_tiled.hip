@@ -4,7 +4,8 @@
 // :119-120) without global atomics, on the scheme of the tiled Joseph back projection: the
 // volume is cut into tiles long along one driving axis, one workgroup owns a tile for all
 // poses and sums in LDS every crossing of every ray (driving along that axis) that passes
-// through it, then adds the tile to the volume once; one launch per driving axis.
+// through it, then adds the tile to the volume once; one launch for the tiles of two driving axes
+// (siddon_adj_pair_kernel), one per axis otherwise.
 //
 // A ray takes the tile's planes in its own order (sid_tile_ray): its state at the first plane
 // follows from the step counts there, and each plane's segments from sorting two crossing
@@ -13,20 +14,25 @@
 // twice on a plane) took 111 vector instructions a crossing, most of them masked updates of the three axes:
 // 256^3, 360 poses, 384^2 pixels 20.0 -> 10.6 ms; 128^3 2.12 -> 0.94 ms; 2D 256^2 0.131 -> 0.078 ms.
 // The crossings, voxels and lengths are the forward's. Rows of slots are an odd number long
-// (sid_row_slots). Tiles: 8 x 16 x 16 (8 x 17 x 17 11.1 ms, 8 x 15 x 15 11.5, 12 x 16 x 16 11.3, 16 x 16 x 16
-// 12.0, 8 x 24 x 24 12.2, 4 x 32 x 32 13.0). VALU issue and the 64-bit LDS atomics (three a
-// plane) bound it.
+// (sid_row_slots). VALU issue and the 64-bit LDS atomics (three a plane) bound it.
+//
+// Both axes in one launch and 512 threads in 64 VGPRs, against one launch of 256 threads per axis:
+// 256^3 10.6 -> 9.96 ms, 128^3 0.94 -> 0.79, FP64 96 x 64 x 112 / 77 poses 0.23 -> 0.185; 2D (256
+// threads) 256^2 78 -> 54 us.
 //
 // Sums are 64-bit fixed point as in the Joseph kernel: one exponent per call from max|y|
 // and the slot bound, each contribution y * length rounded once to the unit (fixed_round; in
 // FP32 the product is exact in FP64).
 #include "ehp_kernels.hpp"
+#include "ehp_tile_pair.hpp"
 
 namespace ehp
 {
     namespace
     {
-        constexpr int kThreads = 256;
+        // threads of a workgroup
+        template <int D>
+        constexpr int kNT = D == 3 ? 512 : 256;
         // LDS (address space 3) pointers: 32-bit byte addresses
         typedef __attribute__((address_space(3))) unsigned long long lds_u64;
         typedef __attribute__((address_space(3))) char lds_char;
@@ -81,7 +87,8 @@ namespace ehp
 
     // One tile of the back projection along driving axis A (tile < ntA * ntB * ntC); T = float or
     // double (sinogram and volume).
-    template <int D, int A, class T>
+    // PAIR: the other axis' tiles may add to the volume now
+    template <int D, int A, bool PAIR, class T>
     __device__ __forceinline__ void sid_adj_tiled_block(const PoseGeom* __restrict__ geo,
                                                         const SidRec* __restrict__ table, const Dims& dims,
                                                         const int* __restrict__ pose_axes, const TileCfg& tc,
@@ -90,6 +97,7 @@ namespace ehp
                                                         T* __restrict__ vol)
     {
         constexpr int b1 = TileAxes<D, A>::b1, b2 = TileAxes<D, A>::b2;
+        constexpr int kThreads = kNT<D>;
         extern __shared__ long long lds[];
 
         const int tid = threadIdx.x;
@@ -205,39 +213,120 @@ namespace ehp
             if (D == 3)
                 c[b2] = cc;
             const int64_t lin = c[0] + c[1] * dims.strides[1] + (int64_t) c[2] * dims.strides[2];
-            vol[lin] += (T) ((double) iacc[i] * q);
+            const T sum = (T) ((double) iacc[i] * q);
+            if (PAIR)
+                add_second(vol + lin, sum);
+            else
+                vol[lin] += sum;
         }
     }
 
     template <int D, int A, class T>
-    __global__ void __launch_bounds__(kThreads)
+    __global__ void __launch_bounds__(kNT<D>, 8)
         siddon_adj_tiled_kernel(const PoseGeom* __restrict__ geo, const SidRec* __restrict__ table, const Dims dims,
-                                const int* __restrict__ pose_axes, const TileCfg tc, const int ntA, const int ntB,
-                                const int ntC, const int tiles_per_xcd, const int batch,
-                                const int* __restrict__ fixexp, const T* __restrict__ sino, T* __restrict__ vol)
+                                const int* __restrict__ pose_axes, const TileCfg tc, const TileCounts c,
+                                const int batch, const int* __restrict__ fixexp, const T* __restrict__ sino,
+                                T* __restrict__ vol)
     {
         // consecutive workgroups land on different XCDs: give each XCD a contiguous block of tiles
-        const int tile = (int) (blockIdx.x % 8u) * tiles_per_xcd + (int) (blockIdx.x / 8u);
-        if (tile >= ntA * ntB * ntC)
-            return;
-        sid_adj_tiled_block<D, A, T>(geo, table, dims, pose_axes, tc, ntA, ntB, tile, batch, fixexp, sino, vol);
+        const int tile = (int) (blockIdx.x % 8u) * c.per_xcd + (int) (blockIdx.x / 8u);
+        if (tile < c.n)
+            sid_adj_tiled_block<D, A, false, T>(geo, table, dims, pose_axes, tc, c.nA, c.nB, tile, batch, fixexp, sino,
+                                                vol);
     }
 
-    // the tiles of axis A of many operators in one launch (block b: tile b - job.block0 of job
-    // block_job[b])
+    // the tiles of two driving axes
+    template <int D, int A0, int A1, class T>
+    __global__ void __launch_bounds__(kNT<D>, 8)
+        siddon_adj_pair_kernel(const PoseGeom* __restrict__ geo, const SidRec* __restrict__ table, const Dims dims,
+                               const int* __restrict__ pose_axes, const TileCfg tc, const TileCounts c0,
+                               const TileCounts c1, const int batch, const int* __restrict__ fixexp,
+                               const T* __restrict__ sino, T* __restrict__ vol)
+    {
+        const int xcd = (int) (blockIdx.x % 8u), k = (int) (blockIdx.x / 8u);
+        if (k < c0.per_xcd) {
+            const int tile = xcd * c0.per_xcd + k;
+            if (tile < c0.n)
+                sid_adj_tiled_block<D, A0, true, T>(geo, table, dims, pose_axes, tc, c0.nA, c0.nB, tile, batch, fixexp,
+                                                    sino, vol);
+        } else {
+            const int tile = xcd * c1.per_xcd + k - c0.per_xcd;
+            if (tile < c1.n)
+                sid_adj_tiled_block<D, A1, true, T>(geo, table, dims, pose_axes, tc, c1.nA, c1.nB, tile, batch, fixexp,
+                                                    sino, vol);
+        }
+    }
+
+    // the tiles of many operators in one launch (block b: tile b - job.block0 of job block_job[b])
+    template <int D, int A, bool PAIR>
+    __device__ __forceinline__ void sid_batch_block(const SidAdjJob* __restrict__ jobs,
+                                                    const int* __restrict__ block_job, const int64_t id,
+                                                    const int* __restrict__ fixexp, const float* __restrict__ sinos,
+                                                    float* __restrict__ vols)
+    {
+        const SidAdjJob& J = jobs[block_job[id]];
+        sid_adj_tiled_block<D, A, PAIR, float>(J.geo, J.table, J.dims, J.pose_axes, J.tc, J.ntA, J.ntB,
+                                               (int) (id - J.block0), J.batch, fixexp + J.item, sinos + J.sino_off,
+                                               vols + J.vol_off);
+    }
+
     template <int D, int A>
-    __global__ void __launch_bounds__(kThreads)
-        siddon_adj_tiled_batch_kernel(const SidAdjJob* __restrict__ jobs, const int* __restrict__ block_job,
-                                      const int per_xcd, const int64_t total, const int* __restrict__ fixexp,
+    __global__ void __launch_bounds__(kNT<D>, 8)
+        siddon_adj_tiled_batch_kernel(const BatchTiles<SidAdjJob> t, const int* __restrict__ fixexp,
                                       const float* __restrict__ sinos, float* __restrict__ vols)
     {
-        const int64_t id = (int64_t) (blockIdx.x % 8u) * per_xcd + (blockIdx.x / 8u);
-        if (id >= total)
-            return;
-        const SidAdjJob& J = jobs[block_job[id]];
-        sid_adj_tiled_block<D, A, float>(J.geo, J.table, J.dims, J.pose_axes, J.tc, J.ntA, J.ntB,
-                                         (int) (id - J.block0), J.batch, fixexp + J.item, sinos + J.sino_off,
-                                         vols + J.vol_off);
+        const int64_t id = (int64_t) (blockIdx.x % 8u) * t.per_xcd + (blockIdx.x / 8u);
+        if (id < t.total)
+            sid_batch_block<D, A, false>(t.jobs, t.block_job, id, fixexp, sinos, vols);
+    }
+
+    template <int D, int A0, int A1>
+    __global__ void __launch_bounds__(kNT<D>, 8)
+        siddon_adj_pair_batch_kernel(const BatchTiles<SidAdjJob> t0, const BatchTiles<SidAdjJob> t1,
+                                     const int* __restrict__ fixexp, const float* __restrict__ sinos,
+                                     float* __restrict__ vols)
+    {
+        const int64_t xcd = blockIdx.x % 8u;
+        const int k = (int) (blockIdx.x / 8u);
+        if (k < t0.per_xcd) {
+            const int64_t id = xcd * t0.per_xcd + k;
+            if (id < t0.total)
+                sid_batch_block<D, A0, true>(t0.jobs, t0.block_job, id, fixexp, sinos, vols);
+        } else {
+            const int64_t id = xcd * t1.per_xcd + k - t0.per_xcd;
+            if (id < t1.total)
+                sid_batch_block<D, A1, true>(t1.jobs, t1.block_job, id, fixexp, sinos, vols);
+        }
+    }
+
+    // fn(D, axis) or fn(D, first, second) as constants
+    template <class Fn>
+    void with_axis(int dim, int a, Fn fn)
+    {
+        using std::integral_constant;
+        if (dim == 2) {
+            if (a == 0)
+                fn(integral_constant<int, 2>{}, integral_constant<int, 0>{});
+            else
+                fn(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+        } else {
+            if (a == 0)
+                fn(integral_constant<int, 3>{}, integral_constant<int, 0>{});
+            else if (a == 1)
+                fn(integral_constant<int, 3>{}, integral_constant<int, 1>{});
+            else
+                fn(integral_constant<int, 3>{}, integral_constant<int, 2>{});
+        }
+    }
+
+    template <class Fn>
+    void with_pair(int dim, int axes, Fn fn)
+    {
+        using std::integral_constant;
+        if (dim == 2)
+            fn(integral_constant<int, 2>{}, integral_constant<int, 0>{}, integral_constant<int, 1>{});
+        else
+            with_axis_pair(axes, [&](auto a0, auto a1) { fn(integral_constant<int, 3>{}, a0, a1); });
     }
 
     template <class T>
@@ -253,35 +342,34 @@ namespace ehp
         if (e != hipSuccess)
             return e;
         const size_t lds = siddon_tile_lds_bytes(dims, tc, batch);
-        for (int a = 0; a < dims.dim; ++a) {
+        if (two_axes(axes_present)) {
+            with_pair(dims.dim, axes_present, [&](auto d, auto a0, auto a1) {
+                constexpr int D = decltype(d)::value;
+                const TileCounts c0 = axis_tiles(dims, tc, a0), c1 = axis_tiles(dims, tc, a1);
+                if ((int64_t) (c0.per_xcd + c1.per_xcd) * 8 > (int64_t) 0x7fffffff) {
+                    e = hipErrorInvalidValue;
+                    return;
+                }
+                hipLaunchKernelGGL((siddon_adj_pair_kernel<D, decltype(a0)::value, decltype(a1)::value, T>),
+                                   dim3((unsigned) (c0.per_xcd + c1.per_xcd) * 8), dim3(kNT<D>), lds, s, geo, table,
+                                   dims, pose_axes, tc, c0, c1, batch, d_fixexp, sino, vol);
+                e = hipGetLastError();
+            });
+            return e;
+        }
+        for (int a = 0; e == hipSuccess && a < dims.dim; ++a) {
             if (!(axes_present & (1 << a)))
                 continue;
-            int ntA, ntB, ntC;
-            tile_counts(dims, tc, a, ntA, ntB, ntC);
-            const int per_xcd = (ntA * ntB * ntC + 7) / 8;
-            const dim3 grid((unsigned) (per_xcd * 8));
-#define EHP_SID_TILED(Dv, Av)                                                                                      \
-    hipLaunchKernelGGL((siddon_adj_tiled_kernel<Dv, Av, T>), grid, dim3(kThreads), lds, s, geo, table, dims,         \
-                       pose_axes, tc, ntA, ntB, ntC, per_xcd, batch, d_fixexp, sino, vol)
-            if (dims.dim == 2) {
-                if (a == 0)
-                    EHP_SID_TILED(2, 0);
-                else
-                    EHP_SID_TILED(2, 1);
-            } else {
-                if (a == 0)
-                    EHP_SID_TILED(3, 0);
-                else if (a == 1)
-                    EHP_SID_TILED(3, 1);
-                else
-                    EHP_SID_TILED(3, 2);
-            }
-#undef EHP_SID_TILED
-            e = hipGetLastError();
-            if (e != hipSuccess)
-                return e;
+            with_axis(dims.dim, a, [&](auto d, auto ax) {
+                constexpr int D = decltype(d)::value;
+                const TileCounts c = axis_tiles(dims, tc, a);
+                hipLaunchKernelGGL((siddon_adj_tiled_kernel<D, decltype(ax)::value, T>),
+                                   dim3((unsigned) c.per_xcd * 8), dim3(kNT<D>), lds, s, geo, table, dims, pose_axes, tc,
+                                   c, batch, d_fixexp, sino, vol);
+                e = hipGetLastError();
+            });
         }
-        return hipSuccess;
+        return e;
     }
 
     template hipError_t siddon_adjoint_tiled<float>(const PoseGeom*, const SidRec*, const Dims&, const int*, int,
@@ -333,35 +421,41 @@ namespace ehp
                                     const int64_t nablocks[3], const size_t lds[3], const int* d_fixexp,
                                     const float* sinos, float* vols, hipStream_t s)
     {
+        hipError_t e = hipSuccess;
+        auto tiles = [&](int a) {
+            return BatchTiles<SidAdjJob>{ajobs[a], ablocks[a], nablocks[a], (int) ((nablocks[a] + 7) / 8)};
+        };
+        int axes = 0;
+        int64_t most = 0;
         for (int a = 0; a < dim; ++a) {
-            const int64_t total = nablocks[a];
-            if (total == 0)
-                continue;
-            const int64_t per_xcd = (total + 7) / 8;
-            if (per_xcd * 8 > (int64_t) 0x7fffffff)
-                return hipErrorInvalidValue;
-            const dim3 grid((unsigned) (per_xcd * 8));
-#define EHP_SID_BATCH(Dv, Av)                                                                                      \
-    hipLaunchKernelGGL((siddon_adj_tiled_batch_kernel<Dv, Av>), grid, dim3(kThreads), lds[a], s, ajobs[a], ablocks[a], \
-                       (int) per_xcd, total, d_fixexp, sinos, vols)
-            if (dim == 2) {
-                if (a == 0)
-                    EHP_SID_BATCH(2, 0);
-                else
-                    EHP_SID_BATCH(2, 1);
-            } else {
-                if (a == 0)
-                    EHP_SID_BATCH(3, 0);
-                else if (a == 1)
-                    EHP_SID_BATCH(3, 1);
-                else
-                    EHP_SID_BATCH(3, 2);
-            }
-#undef EHP_SID_BATCH
-            const hipError_t e = hipGetLastError();
-            if (e != hipSuccess)
-                return e;
+            axes |= nablocks[a] > 0 ? 1 << a : 0;
+            most += nablocks[a] + 8;
         }
-        return hipSuccess;
+        if (most > (int64_t) 0x7fffffff)
+            return hipErrorInvalidValue;
+        if (two_axes(axes)) {
+            with_pair(dim, axes, [&](auto d, auto a0, auto a1) {
+                constexpr int D = decltype(d)::value;
+                const BatchTiles<SidAdjJob> t0 = tiles(a0), t1 = tiles(a1);
+                const size_t need = lds[a0] > lds[a1] ? lds[a0] : lds[a1];
+                hipLaunchKernelGGL((siddon_adj_pair_batch_kernel<D, decltype(a0)::value, decltype(a1)::value>),
+                                   dim3((unsigned) (t0.per_xcd + t1.per_xcd) * 8), dim3(kNT<D>), need, s, t0, t1,
+                                   d_fixexp, sinos, vols);
+                e = hipGetLastError();
+            });
+            return e;
+        }
+        for (int a = 0; e == hipSuccess && a < dim; ++a) {
+            if (nablocks[a] == 0)
+                continue;
+            with_axis(dim, a, [&](auto d, auto ax) {
+                constexpr int D = decltype(d)::value;
+                const BatchTiles<SidAdjJob> t = tiles(a);
+                hipLaunchKernelGGL((siddon_adj_tiled_batch_kernel<D, decltype(ax)::value>),
+                                   dim3((unsigned) t.per_xcd * 8), dim3(kNT<D>), lds[a], s, t, d_fixexp, sinos, vols);
+                e = hipGetLastError();
+            });
+        }
+        return e;
     }
 } // namespace ehp
