@@ -143,8 +143,8 @@ int ehp_adjoint(ehp_op* op, const void* d_sino, void* d_vol, void* stream);
 /* ehp_adjoint for callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc). No counterpart in elsa. The same
  * kernels and result, bit for bit, but the scratch of the back projection (the fixed-point
- * scale: per-block maxima of |y| and the exponent, 16.6 KB) lives in one static device array
- * of the library, 16.6 KB per GPU held until the process ends, instead of the operator's; the
+ * scale: per-block maxima of |y| and the exponent, 2.3 KB) lives in one static device array
+ * of the library, 2.3 KB per GPU held until the process ends, instead of the operator's; the
  * call allocates nothing. Takes FP32 and FP64 Joseph and Siddon operators with a tiled back
  * projection (EHP_ERR_UNSUPPORTED otherwise: bfloat16, voxel or EHP_SIMPLE_KERNELS operators,
  * and geometries without a tiled back projection). Every call on a GPU shares that GPU's array: calls that overlap
