@@ -102,11 +102,53 @@ namespace ehp
             }
         }
 
+        // What a solver does with a dot product once it has it (dot_final_kernel; a launch of its own for
+        // these few scalars took 5 us)
+        struct Then {
+            enum Op { NOTHING, CGLS_STEP, ALPHA, BETA, APGD_CHECK } op = NOTHING;
+            double a = 0.0, b = 0.0;
+        };
+
+        __device__ __forceinline__ void scalar_step(double* sc, int seg, const Then& t)
+        {
+            const bool done = scal(sc, seg, S_DONE) != 0.0;
+            switch (t.op) {
+                case Then::CGLS_STEP: // start of a CGLS iteration: stop when kold < tol (CGLS.cpp:54-58), else count it
+                    if (!done && scal(sc, seg, S_KOLD) < t.b)
+                        scal(sc, seg, S_DONE) = 1.0;
+                    else if (!done)
+                        scal(sc, seg, S_ITERS) += 1.0;
+                    [[fallthrough]];
+                case Then::ALPHA: { // a: the damping
+                    const double d =
+                        t.a == 0.0 ? scal(sc, seg, S_DELTA) : scal(sc, seg, S_DELTA) + t.a * scal(sc, seg, S_CN);
+                    scal(sc, seg, S_ALPHA) = scal(sc, seg, S_KOLD) / d;
+                    break;
+                }
+                case Then::BETA:
+                    if (done) {
+                        scal(sc, seg, S_BETA) = 0.0;
+                        break;
+                    }
+                    scal(sc, seg, S_BETA) = scal(sc, seg, S_K) / scal(sc, seg, S_KOLD);
+                    scal(sc, seg, S_KOLD) = scal(sc, seg, S_K);
+                    break;
+                case Then::APGD_CHECK: // ||grad||^2 <= a ends the method after this iteration (APGD.cpp:83-87)
+                    if (done)
+                        break;
+                    scal(sc, seg, S_ITERS) += 1.0;
+                    if (scal(sc, seg, S_SN) <= t.a)
+                        scal(sc, seg, S_DONE) = 1.0;
+                    break;
+                default: break;
+            }
+        }
+
         // per problem (one block each): slot = sum of its partial sums in a fixed order; hist, when
         // given, gets a copy at index iters of the problem's row (only while not converged)
         __global__ void __launch_bounds__(kThreads)
             dot_final_kernel(const double* __restrict__ partial, const SegSpace S, double* __restrict__ sc, int slot,
-                             double* __restrict__ hist, int nh)
+                             double* __restrict__ hist, int nh, const Then then)
         {
             const int seg = blockIdx.x;
             __shared__ double red[kThreads];
@@ -124,6 +166,7 @@ namespace ehp
                 scal(sc, seg, slot) = red[0];
                 if (hist && scal(sc, seg, S_DONE) == 0.0)
                     hist[(int64_t) seg * nh + (int) scal(sc, seg, S_ITERS)] = red[0];
+                scalar_step(sc, seg, then);
             }
         }
 
@@ -187,40 +230,6 @@ namespace ehp
             c[i] = down<T>(up(r[i]) + beta * up(c[i]));
         }
 
-        // start of a CGLS iteration: stop when kold < tol (CGLS.cpp:54-58), else count it
-        __global__ void cgls_check_kernel(double* sc, int nseg, double tol)
-        {
-            const int seg = blockIdx.x * blockDim.x + threadIdx.x;
-            if (seg >= nseg)
-                return;
-            if (scal(sc, seg, S_DONE) == 0.0 && scal(sc, seg, S_KOLD) < tol)
-                scal(sc, seg, S_DONE) = 1.0;
-            if (scal(sc, seg, S_DONE) == 0.0)
-                scal(sc, seg, S_ITERS) += 1.0;
-        }
-
-        __global__ void cgls_alpha_kernel(double* sc, int nseg, double damp)
-        {
-            const int seg = blockIdx.x * blockDim.x + threadIdx.x;
-            if (seg >= nseg)
-                return;
-            const double d = damp == 0.0 ? scal(sc, seg, S_DELTA) : scal(sc, seg, S_DELTA) + damp * scal(sc, seg, S_CN);
-            scal(sc, seg, S_ALPHA) = scal(sc, seg, S_KOLD) / d;
-        }
-
-        __global__ void cgls_beta_kernel(double* sc, int nseg)
-        {
-            const int seg = blockIdx.x * blockDim.x + threadIdx.x;
-            if (seg >= nseg)
-                return;
-            if (scal(sc, seg, S_DONE) != 0.0) {
-                scal(sc, seg, S_BETA) = 0.0;
-                return;
-            }
-            scal(sc, seg, S_BETA) = scal(sc, seg, S_K) / scal(sc, seg, S_KOLD);
-            scal(sc, seg, S_KOLD) = scal(sc, seg, S_K);
-        }
-
         __global__ void set_scalar_kernel(double* sc, int nseg, int slot, double v)
         {
             const int seg = blockIdx.x * blockDim.x + threadIdx.x;
@@ -280,18 +289,6 @@ namespace ehp
             xprev[i] = xi;
         }
 
-        // APGD convergence: ||grad||^2 <= epsilon ends the method after this iteration
-        // (APGD.cpp:83-87)
-        __global__ void apgd_check_kernel(double* sc, int nseg, double eps)
-        {
-            const int seg = blockIdx.x * blockDim.x + threadIdx.x;
-            if (seg >= nseg || scal(sc, seg, S_DONE) != 0.0)
-                return;
-            scal(sc, seg, S_ITERS) += 1.0;
-            if (scal(sc, seg, S_SN) <= eps)
-                scal(sc, seg, S_DONE) = 1.0;
-        }
-
         // u = u / sqrt(||u||^2) per problem
         template <class T>
         __global__ void __launch_bounds__(kThreads)
@@ -315,11 +312,11 @@ namespace ehp
 
         template <class T>
         hipError_t dot(const T* a, const T* b, const SegSpace& S, int nseg, double* partial, double* sc, int slot,
-                       double* hist, int nh, hipStream_t s)
+                       double* hist, int nh, hipStream_t s, const Then& then = Then{})
         {
             hipLaunchKernelGGL((dot_partial_kernel<T>), dim3((unsigned) S.nrb), dim3(kThreads), 0, s, a, b, S, partial);
             hipLaunchKernelGGL(dot_final_kernel, dim3((unsigned) nseg), dim3(kThreads), 0, s, partial, S, sc, slot,
-                               hist, nh);
+                               hist, nh, then);
             return hipGetLastError();
         }
 
@@ -556,15 +553,14 @@ namespace ehp
                 return rc;
 
             auto body = [&]() -> int {
-                hipLaunchKernelGGL(cgls_check_kernel, dim3(seg_blocks(nseg)), dim3(64), 0, s, sc, nseg, tol);
                 int r2 = A.fwd(c, q, s); // q = A c
                 if (r2 != EHP_OK)
                     return r2;
-                if (dot<T>(q, q, R, nseg, partial, sc, S_DELTA, nullptr, nh, s) != hipSuccess)
+                const Then step{Then::CGLS_STEP, damp, tol};
+                if (dot<T>(q, q, R, nseg, partial, sc, S_DELTA, nullptr, nh, s, damp == 0.0 ? step : Then{}) != hipSuccess)
                     return EHP_ERR_HIP;
-                if (damp != 0.0 && dot<T>(c, c, D, nseg, partial, sc, S_CN, nullptr, nh, s) != hipSuccess)
+                if (damp != 0.0 && dot<T>(c, c, D, nseg, partial, sc, S_CN, nullptr, nh, s, step) != hipSuccess)
                     return EHP_ERR_HIP;
-                hipLaunchKernelGGL(cgls_alpha_kernel, dim3(seg_blocks(nseg)), dim3(64), 0, s, sc, nseg, damp);
                 hipLaunchKernelGGL((cgls_update_kernel<T>), dim3((unsigned) D.neb), dim3(kThreads), 0, s, x, c, D, sc, 0);
                 hipLaunchKernelGGL((cgls_update_kernel<T>), dim3((unsigned) R.neb), dim3(kThreads), 0, s, sres, q, R, sc,
                                    1);
@@ -574,9 +570,8 @@ namespace ehp
                 if (damp != 0.0)
                     hipLaunchKernelGGL((axpy_kernel<T>), dim3(blocks(nd)), dim3(kThreads), 0, s, (typename Acc<T>::type) -damp, x,
                                    r, nd);
-                if (dot<T>(r, r, D, nseg, partial, sc, S_K, nullptr, nh, s) != hipSuccess)
+                if (dot<T>(r, r, D, nseg, partial, sc, S_K, nullptr, nh, s, Then{Then::BETA}) != hipSuccess)
                     return EHP_ERR_HIP;
-                hipLaunchKernelGGL(cgls_beta_kernel, dim3(seg_blocks(nseg)), dim3(64), 0, s, sc, nseg);
                 hipLaunchKernelGGL((cgls_direction_kernel<T>), dim3((unsigned) D.neb), dim3(kThreads), 0, s, r, c, D, sc);
                 // ||s||^2 of this iteration, recorded at index iters while not converged
                 if (dot<T>(sres, sres, R, nseg, partial, sc, S_SN, hist, nh, s) != hipSuccess)
@@ -716,9 +711,9 @@ namespace ehp
                 hipLaunchKernelGGL((apgd_t_kernel<T>), dim3(seg_blocks(nseg)), dim3(64), 0, s, sc, nseg);
                 hipLaunchKernelGGL((apgd_momentum_kernel<T>), dim3((unsigned) D.neb), dim3(kThreads), 0, s, x, xprev, y,
                                    D, sc);
-                if (dot<T>(grad, grad, D, nseg, partial, sc, S_SN, hist, nh, s) != hipSuccess)
+                if (dot<T>(grad, grad, D, nseg, partial, sc, S_SN, hist, nh, s, Then{Then::APGD_CHECK, epsilon}) !=
+                    hipSuccess)
                     return EHP_ERR_HIP;
-                hipLaunchKernelGGL(apgd_check_kernel, dim3(seg_blocks(nseg)), dim3(64), 0, s, sc, nseg, epsilon);
                 const int r2 = gradient();
                 if (r2 != EHP_OK)
                     return r2;
@@ -902,7 +897,7 @@ namespace ehp
             hipLaunchKernelGGL(refine_residual_kernel, dim3((unsigned) sv.R.nrb), dim3(kThreads), 0, s, b, q, r, sv.R,
                                sv.partial);
             hipLaunchKernelGGL(dot_final_kernel, dim3((unsigned) sv.nseg), dim3(kThreads), 0, s, sv.partial, sv.R,
-                               sv.sc, (int) S_SN, (double*) nullptr, 0);
+                               sv.sc, (int) S_SN, (double*) nullptr, 0, Then{});
             double rr = 0.0;
             hipError_t e = hipMemcpyAsync(&rr, sv.sc + S_SN, sizeof(double), hipMemcpyDeviceToHost, s);
             if (e == hipSuccess)
@@ -1058,16 +1053,15 @@ namespace ehp
                     r2 = normal(c, ac);
                     if (r2 != EHP_OK)
                         return r2;
-                    if (dot<T>(c, ac, D, nseg, sv.partial, sv.sc, S_DELTA, nullptr, nh, s) != hipSuccess)
+                    if (dot<T>(c, ac, D, nseg, sv.partial, sv.sc, S_DELTA, nullptr, nh, s, Then{Then::ALPHA}) !=
+                        hipSuccess)
                         return EHP_ERR_HIP;
-                    hipLaunchKernelGGL(cgls_alpha_kernel, dim3(seg_blocks(nseg)), dim3(64), 0, s, sv.sc, nseg, 0.0);
                     hipLaunchKernelGGL((cgls_update_kernel<T>), dim3((unsigned) D.neb), dim3(kThreads), 0, s, x, c, D,
                                        sv.sc, 0);
                     hipLaunchKernelGGL((cgls_update_kernel<T>), dim3((unsigned) D.neb), dim3(kThreads), 0, s, r, ac, D,
                                        sv.sc, 1);
-                    if (dot<T>(r, r, D, nseg, sv.partial, sv.sc, S_K, nullptr, nh, s) != hipSuccess)
+                    if (dot<T>(r, r, D, nseg, sv.partial, sv.sc, S_K, nullptr, nh, s, Then{Then::BETA}) != hipSuccess)
                         return EHP_ERR_HIP;
-                    hipLaunchKernelGGL(cgls_beta_kernel, dim3(seg_blocks(nseg)), dim3(64), 0, s, sv.sc, nseg);
                     hipLaunchKernelGGL((cgls_direction_kernel<T>), dim3((unsigned) D.neb), dim3(kThreads), 0, s, r, c, D,
                                        sv.sc);
                 }
