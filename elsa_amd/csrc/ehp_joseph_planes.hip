@@ -166,13 +166,11 @@ namespace ehp
         // per-lane loop would put rays that enter through a side face of the volume, each at its
         // own plane, on a cache line of their own at every step. Every lane of the block takes
         // part in the wavefront reductions; lanes past the detector edge join no group.
-        template <int D, class OT = float, int WU = kFwdWU>
-        __device__ __forceinline__ void fwd_planes_block(const PoseGeom* __restrict__ geo, const Dims& dims,
-                                                         const ViewSet& views, const int tiles_u, const int64_t id,
-                                                         OT* __restrict__ sino)
+        template <int D, class OT>
+        __device__ __forceinline__ void fwd_planes_ray(const PoseGeom* __restrict__ geo, const Dims& dims,
+                                                       const ViewSet& views, const int u, const int v, const int pose,
+                                                       OT* __restrict__ sino)
         {
-            int u, v, pose;
-            fwd_pixel<D, WU>(dims, tiles_u, id, u, v, pose);
             const bool inside = u < dims.det[0] && v < dims.det[1];
             RayRec r{};
             int key = -1, tfirst = 0, tlast = 0, s0 = 0;
@@ -284,7 +282,9 @@ namespace ehp
             const int64_t id = (int64_t) (blockIdx.x % 8u) * per_xcd + (blockIdx.x / 8u);
             if (id >= total)
                 return;
-            fwd_planes_block<D, OT, WU>(geo, dims, views, tiles_u, id, sino);
+            int u, v, pose;
+            fwd_pixel<D, WU>(dims, tiles_u, id, u, v, pose);
+            fwd_planes_ray<D, OT>(geo, dims, views, u, v, pose, sino);
         }
 
         // ---- batches: one launch over the jobs of many operators; block b runs block
@@ -316,10 +316,16 @@ namespace ehp
             if (id >= total)
                 return;
             const FwdJob& J = jobs[block_job[id]];
-            if constexpr (D == 2)
+            if constexpr (D == 2) {
                 fwd2d_block<float>(J.geo, J.dims, J.views, J.parts, 1, J.tiles_u, id - J.block0, sinos + J.sino_off);
-            else
-                fwd_planes_block<D, float>(J.geo, J.dims, J.views, J.tiles_u, id - J.block0, sinos + J.sino_off);
+            } else {
+                int u, v, pose;
+                if (J.views.pairs) // the wavefronts of the operator's own launch
+                    fwd_pixel<D, kFwdWUPairs>(J.dims, J.tiles_u, id - J.block0, u, v, pose);
+                else
+                    fwd_pixel<D, kFwdWU>(J.dims, J.tiles_u, id - J.block0, u, v, pose);
+                fwd_planes_ray<D, float>(J.geo, J.dims, J.views, u, v, pose, sinos + J.sino_off);
+            }
         }
     } // namespace
 
@@ -447,7 +453,7 @@ namespace ehp
                 if (L.pairs)
                     fj.views.pairs |= 1 << a;
             }
-            const FwdGrid fg = fwd_grid(it.dims);
+            const FwdGrid fg = fwd_grid(it.dims, fj.views.pairs ? kFwdWUPairs : kFwdWU);
             fj.tiles_u = fg.tiles_u;
             fj.parts = it.dims.dim == 2 ? fwd2d_parts(it.dims, sizeof(float)) : 1;
             const int64_t nb = fg.total;
