@@ -18,7 +18,7 @@ CANDIDATES = {
     ("siddon", 3): [(8, 22, 22), (8, 16, 16), (4, 16, 16), (6, 16, 16), (8, 24, 24), (2, 16, 16)],
     ("siddon", 2): [(8, 32, 1), (4, 16, 1), (8, 16, 1), (4, 32, 1), (2, 16, 1), (4, 8, 1), (16, 32, 1)],
     ("voxel", 3): [(96, 16, 1), (64, 16, 1), (32, 32, 1), (128, 16, 1), (96, 8, 1), (32, 16, 1)],
-    ("voxel", 2): [(256, 1, 1), (128, 1, 1), (512, 1, 1), (64, 1, 1)],
+    ("voxel", 2): [(256, 1, 1), (128, 1, 1), (64, 1, 1), (32, 1, 1), (16, 1, 1)],
 }
 POSE_BATCHES = (4, 8, 16, 32)
 

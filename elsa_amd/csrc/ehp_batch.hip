@@ -144,6 +144,9 @@ namespace
         if (vox) {
             // the forward's fixed-point scale comes from each problem's volume
             std::vector<ehp::VoxBatchItem> vitems(n);
+            int64_t poses = 0;
+            for (int j = 0; j < n; ++j)
+                poses += b->ops[j]->dims.nposes;
             std::vector<int64_t> offs(n), sizes(n);
             for (int j = 0; j < n; ++j) {
                 const ehp_op* op = b->ops[j];
@@ -156,7 +159,10 @@ namespace
                 v.diff = op->differential;
                 v.pose_axes = op->d_pose_axes;
                 v.pose_margin = op->d_pose_margin;
+                // 2D tiles left at the problem's own default follow the whole batch's poses
                 v.tile = op->tile;
+                if (b->dim == 2 && v.tile.LA == voxel_tile2d(op->dims.det[0], op->dims.nposes, cus).LA)
+                    v.tile = voxel_tile2d(op->dims.det[0], poses, cus);
                 v.plan = op->vox;
                 v.vol_off = b->vol_off[j];
                 v.sino_off = b->sino_off[j];

@@ -58,3 +58,4 @@ struct ehp_op {
 // The 2D Joseph back projection's tile for a launch over nvox voxels (one problem's, or all of a
 // batch's) on a device of cus compute units
 ehp::TileCfg joseph_tile2d(int64_t nvox, int cus);
+ehp::TileCfg voxel_tile2d(int det, int64_t poses, int cus);

@@ -75,6 +75,23 @@ def test_gather_parts_2d(vol, det, poses, dtype):
     assert rel_l2(op.applyAdjoint(y), ref) <= (1e-6 if dtype == np.float32 else 1e-13)
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("vol,det,poses", [((1, 5), 9, 7), ((31, 17), 40, 33), ((50, 60), 300, 1100)])
+def test_forward_tiles_2d(vol, det, poses, dtype):
+    """Tiles by the launch's size: narrow ones for few poses, up to 256 pixels for many."""
+    import elsa_amd as E
+
+    g = oracle.circle_geometry(2, vol, poses, 360, 200.0, 60.0, det=(det,))
+    op = E.BlobVoxelProjectorCUDA(*geom_to_descriptors(g), dtype=dtype)
+    x = np.random.default_rng(7).random(g.vol_shape).astype(dtype)
+    got = op.apply(x)
+    ref = oracle.voxel(g, x, oracle.blob_lut(2.0, 10.83, 2, 100, dtype), 2.0, acc64=True)
+    assert rel_l2(got, ref) <= (1e-6 if dtype == np.float32 else 1e-13)
+    for tile in (1, 16, 37, 256, 512):
+        op.tile(tile, 1, 1)
+        np.testing.assert_array_equal(op.apply(x), got, err_msg=str(tile))
+
+
 @pytest.mark.parametrize("second", [("blob", 0.1), ("blob", 0.35), ("bspline", 1.2)])
 def test_batch_of_columns(second):
     """Operators of one column count share the kernel by columns, others the general one."""
