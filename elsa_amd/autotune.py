@@ -13,7 +13,7 @@ import numpy as np
 from .projectors import BlobVoxelProjectorCUDA, BSplineVoxelProjectorCUDA, JosephsMethodCUDA, SiddonsMethodCUDA
 
 CANDIDATES = {
-    ("joseph", 3): [(4, 32, 32), (8, 22, 22), (8, 24, 24), (4, 24, 24), (8, 16, 16), (4, 16, 16), (5, 20, 20)],
+    ("joseph", 3): [(8, 26, 26), (4, 32, 32), (8, 22, 22), (8, 24, 24), (4, 24, 24), (8, 16, 16), (4, 16, 16), (5, 20, 20)],
     ("joseph", 2): [(16, 16, 1), (8, 8, 1), (32, 32, 1), (24, 24, 1), (16, 32, 1), (12, 12, 1)],
     ("siddon", 3): [(8, 22, 22), (8, 16, 16), (4, 16, 16), (6, 16, 16), (8, 24, 24), (2, 16, 16)],
     ("siddon", 2): [(8, 32, 1), (4, 16, 1), (8, 16, 1), (4, 32, 1), (2, 16, 1), (4, 8, 1), (16, 32, 1)],

@@ -280,17 +280,22 @@ namespace
         return n;
     }
 
-    // 3D Joseph tiles: four planes of up to 32 x 32 voxels, the widths evened over the volume (a large
-    // cross-section spends less on the halo and on rays that leave sideways, few planes leave four
-    // workgroups of 512 a CU). While a launch of two axes has fewer than three tiles a CU, cross-sections
-    // of 24 and 16; below one a CU two planes. Back projections, us (512 threads, both axes in one launch):
-    //   256^3 / 360 poses  4x32x32 7547  8x24x24 8160  8x22x22 7647  8x17x17 8450
+    // 3D Joseph tiles: eight planes of up to 26 x 26 voxels, the widths evened over the volume (a large
+    // cross-section spends less on the halo and on rays that leave sideways); while a launch of two axes has fewer
+    // than eight such tiles a CU, four planes of 32 x 32, below three a CU of 24 x 24 and 16 x 16, and
+    // below one a CU two planes. Back projections, us (512 threads, both axes in one launch):
+    //   256^3 / 360 poses  8x26x26 8015  4x32x32 7978  8x22x22 8080  8x24x24 8626  8x17x17 8873
+    //   the same at magnification 1.05, after a forward each
+    //                      8x26x26 6833  4x32x32 7133  8x22x22 6850  8x24x24 7493  8x17x17 7706
+    //   192^3 / 270        8x24x24 2558  4x32x32 2715  8x22x22 2839  8x17x17 3045
     //   128^3 / 180        4x32x32  607  8x16x16  613  4x22x22  635  4x16x16  667
     //   96^3 / 120         4x24x24  226  8x16x16  236  4x16x16  243  2x16x16  267
     //   64^3 / 90          4x16x16   81  4x24x24  120  2x16x16  101
     ehp::TileCfg joseph_tile3d(const ehp::Dims& dims, int cus)
     {
-        ehp::TileCfg tc{};
+        ehp::TileCfg tc = even_tile(dims, 8, 26);
+        if (two_axis_tiles(dims, tc) >= 8 * (int64_t) cus)
+            return tc;
         for (int w = 32; w >= 16; w -= 8) {
             tc = even_tile(dims, 4, w);
             if (two_axis_tiles(dims, tc) >= 3 * (int64_t) cus)

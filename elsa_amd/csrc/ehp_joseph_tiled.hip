@@ -569,10 +569,11 @@ namespace ehp
 
     // One launch leaves the device waiting for its last workgroups once instead of twice. Bound by the
     // LDS and VALU together (64-bit atomics, four a sample: the LDS is busy 0.97 of the time, vector
-    // instructions 0.85 a cycle and CU). Workgroups of 512 threads over tiles of four planes
-    // (64 VGPRs, so that 32 wavefronts a CU fit), against one launch of 256 threads per axis over 8 x 17 x 17 and 4 x 17 x
-    // 17 tiles: 256^3 / 360 poses 8.61 -> 7.55 ms, 128^3 / 180 0.79 -> 0.61, 96^3 / 120 0.33 -> 0.23, 64^3 / 90
-    // 0.142 -> 0.081, FP64 97 x 61 x 113 / 77 0.195 -> 0.17.
+    // instructions 0.85 a cycle and CU), close to the card's power limit: after it the next kernel's clock is a few
+    // percent lower. Workgroups of 512 threads over tiles of 8 x 26 x 26 or 4 x 32 x 32 (64 VGPRs, so that
+    // 32 wavefronts a CU fit), against one launch of 256 threads per axis over 8 x 17 x 17 and 4 x 17 x 17 tiles:
+    // 256^3 / 360 poses 8.9 -> 8.0 ms, 192^3 / 270 3.05 -> 2.56, 128^3 / 180 0.79 -> 0.61, 96^3 / 120 0.33 -> 0.23,
+    // 64^3 / 90 0.142 -> 0.081, FP64 97 x 61 x 113 / 77 0.195 -> 0.17.
     template <int A0, int A1, class ST>
     __global__ void __launch_bounds__(kThreads, 8)
         joseph_adj_pair_kernel(const PoseGeom* __restrict__ geo, const RayRec* __restrict__ table, const Dims dims,
