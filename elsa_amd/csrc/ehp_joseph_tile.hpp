@@ -1245,6 +1245,9 @@ namespace ehp
         static constexpr bool value = false;
     };
 
+    // Longest row (bytes) of a 3D view over which plane_span_forward takes four samples at once
+    constexpr uint32_t kFourSampleRow = 2304;
+
     // plane_ray_forward with the plane loop shared by a group of rays of one driving axis and
     // direction (a wavefront, on the GPU): iteration it visits the plane at traversal coordinate
     // t0 + it, the same plane for every ray of the group, so their reads fall on neighbouring
@@ -1317,11 +1320,14 @@ namespace ehp
         for (; it < full0; ++it, ++j, fs += 1.0f, poff += dp)
             if (j < n)
                 acc = plane_sample_add<D, A, FB2, V16, PR, F64>(r, dims, V, poff, fs, len, acc);
-        // Four samples per step (FP64 views: two, in as many registers), all fetched before the first is added.
-        // 256^3 / 360 poses 5.02 ms with two samples, 4.82 with four (55 VGPRs, still eight wavefronts a
-        // SIMD); bfloat16 384^3 / 200 9.05 and 8.52. The rays' common middle holds most samples: pairs
-        // of samples in the masked ends as well took 4.90 and 8.63.
-        if constexpr (!F64) {
+        // Four samples per step (FP64 views and views of long rows: two), all fetched before the first is
+        // added. FP64 has no registers for more (55 VGPRs with four FP32 samples, still eight wavefronts a SIMD);
+        // over rows past 2.3 KB, whose planes the caches hold less of, the further loads only displace each
+        // other. ms with two / four: 256^3 / 360 poses (rows of 2080 bytes) 5.02 / 4.82, 192^3 / 270 1.64 / 1.62,
+        // 384^3 / 200 (3104) 10.7 / 11.0, 512^3 / 180 (4128) 26.6 / 29.2; bfloat16 384^3 / 200 (1552) 9.05 / 8.52,
+        // 512^3 / 120 (2064) 14.2 / 13.0. The rays' common middle holds most samples: pairs of samples
+        // in the masked ends as well took 4.90 at 256^3.
+        if (!F64 && V.RS4 <= kFourSampleRow) {
             for (; it + 3 < full1; it += 4, fs += 4.0f, poff += 4u * dp) {
                 SampleTaps T[4];
 #if defined(__HIP_DEVICE_COMPILE__)

@@ -7,6 +7,7 @@ import pytest
 
 import oracle
 from backends import geom_to_descriptors
+from fp32_bounds import check_forward
 
 pytestmark = pytest.mark.gpu
 
@@ -48,6 +49,21 @@ def test_back_projection(name, dtype):
         np.testing.assert_array_equal(op.applyAdjoint(y), got, err_msg=str(tile))
     y[:] = 0
     assert not op.applyAdjoint(y).any()
+
+
+@pytest.mark.parametrize("vol", [(40, 6, 37), (284, 5, 9), (285, 5, 9), (9, 4, 330), (3, 300, 2)], ids=str)
+def test_forward_of_short_and_long_rows(vol):
+    """Four samples at once over view rows up to 2304 bytes (284 voxels), two over longer ones; spans that
+    leave one to three samples over."""
+    import elsa_amd as E
+
+    n = max(vol)
+    angles = np.array([0.0, 20.0, 45.0, 71.0, 90.0, 200.0], np.float32)
+    g = oracle.circle_geometry(3, vol, len(angles), 360, 10.0 * n, 3.0 * n, det=(int(1.5 * n), 12),
+                               angles_deg=angles)
+    op = E.JosephsMethodCUDA(*geom_to_descriptors(g), dtype=np.float32)
+    x = np.random.default_rng(12).standard_normal(g.vol_shape).astype(np.float32)
+    check_forward(op.apply(x), g, x)
 
 
 @pytest.mark.parametrize("names", [("two", "two_small", "one"), ("two", "three"), ("one", "one")])
