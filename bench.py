@@ -12,8 +12,9 @@ Prints ONE JSON line:
               profiles/, over its mean duration from HIP events on the launch stream) against
               the VALU's published 78.6 T lane operations/s (157.3 TFLOP/s FP32); beside it the
               counter-measured HBM bytes against 8 TB/s and the algorithmic tap bytes (16 B per
-              3D sample, served from L2 / LDS). The back projection runs one launch per driving
-              axis; each is given the share of the pass's time that its samples have
+              3D sample, served from L2 / LDS). The back projection is one launch for the tiles of
+              two driving axes, or one per axis, each given the share of the pass's time that its
+              samples have
   cpu_baseline  the CPU restatement (oracle/, OpenMP over rays) on a bounded sample of the same
               workload (a subset of the poses spread over the orbit), on this host's cores: median
               of 5 runs with every thread and with one thread
@@ -657,36 +658,38 @@ def main():
     if a.projector == "joseph":
         # 4 (2D: 2) taps per sample, one value per ray
         alg_bytes = (4 if wl["dim"] == 3 else 2) * eb * S + eb * R
-        adj_name = "joseph_adj_tiled_kernel" if a.kernels == "fast" else "joseph_adj_kernel"
-        fwd_name = "joseph_fwd_planes_kernel" if a.kernels == "fast" else "joseph_fwd_kernel"
+        adj_name, fwd_name = "joseph_adj_kernel", "joseph_fwd_kernel"
+        if a.kernels == "fast":
+            adj_name = "joseph_adj_pair_kernel" if wl["dim"] == 3 else "joseph_adj2d_kernel"
+            fwd_name = "joseph_fwd_planes_kernel" if wl["dim"] == 3 else "joseph_fwd2d_kernel"
         unit, metric = "Gsamples/s", METRIC
     elif a.projector == "siddon":
         # one voxel per crossing, one value per ray
         alg_bytes = eb * S + eb * R
         fwd_name = "siddon_fwd_planes_kernel" if a.kernels == "fast" else "siddon_kernel"
-        adj_name = "siddon_adj_tiled_kernel" if a.kernels == "fast" else "siddon_kernel"
+        adj_name = "siddon_adj_pair_kernel" if a.kernels == "fast" else "siddon_kernel"
         unit, metric = "Gcrossings/s", "Siddon fwd+adj voxel crossings/s & %HBM roofline"
     else:
         # one detector value per footprint tap, one voxel per voxel and pose
         alg_bytes = eb * S + eb * nvox * wl["views"]
-        # FP64: the tiled forward and the simple kernels' gather
-        adj_name = "voxel_adj_fast_kernel" if a.kernels == "fast" and a.dtype == "f32" else "voxel_adj_kernel"
-        fwd_name = "voxel_fwd_tiled_kernel" if a.kernels == "fast" else "voxel_fwd_kernel"
+        adj_name = "voxel_gather_kernel" if a.kernels == "fast" else "voxel_adj_kernel"
+        fwd_name = "voxel_fwd_kernel"
+        if a.kernels == "fast":
+            fwd_name = "voxel_fwd_cols_kernel" if wl["dim"] == 3 else "voxel_fwd_tiled_kernel"
         unit, metric = "Gtaps/s", f"{a.projector} voxel projector fwd+adj footprint taps/s & %HBM roofline"
-    # The tiled back projections run one launch per driving axis that occurs (a "pass"), each
-    # a kernel of its own in rocprof's statistics. Their durations are not timed one by one, so
-    # each launch gets the share of the back projection's time that its samples have; the
-    # dominant kernel is the one with the longest launch.
+    # A tiled 3D back projection runs one launch for the tiles of two driving axes; with one or three
+    # axes a launch each, whose durations are not timed one by one: each gets the share of the back
+    # projection's time that its samples have. The dominant kernel is the one with the longest launch.
     adj_launches = [(adj_name, alg_bytes, t_adj)]  # one pass, timed as a whole
-    if a.kernels == "fast" and a.projector == "joseph":
+    if a.kernels == "fast" and a.projector == "joseph" and wl["dim"] == 3:
         axis, nsteps = op.ray_info()
         per_axis = [(ax, int(nsteps[axis == ax].sum()), int(np.count_nonzero((axis == ax) & (nsteps > 0))))
-                    for ax in range(wl["dim"])]
+                    for ax in range(3)]
         per_axis = [(ax, s_a, r_a) for ax, s_a, r_a in per_axis if s_a > 0]
-        s_tot = sum(s_a for _, s_a, _ in per_axis)
-        b_tap = (4 if wl["dim"] == 3 else 2) * eb
-        adj_launches = [(f"{adj_name}<{wl['dim']},{ax}>", b_tap * s_a + eb * r_a, t_adj * s_a / s_tot)
-                        for ax, s_a, r_a in per_axis]
+        if len(per_axis) != 2:
+            s_tot = sum(s_a for _, s_a, _ in per_axis)
+            adj_launches = [(f"joseph_adj_tiled_kernel<3,{ax}>", 4 * eb * s_a + eb * r_a, t_adj * s_a / s_tot)
+                            for ax, s_a, r_a in per_axis]
     adj_launch = max(adj_launches, key=lambda x: x[2])
     if adj_launch[2] >= t_fwd:
         name, launch_bytes, t_dom = adj_launch

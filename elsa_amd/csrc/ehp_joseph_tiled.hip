@@ -230,7 +230,7 @@ namespace ehp
 
     // The candidate rays of one pose batch of one 3D tile, all added into the tile's slots.
     // Candidate k (k < total) is pixel k - pref[j] of pose j's rectangle, j the last pose with
-    // pref[j] <= k. Each lane walks its candidates k = tid, tid + 256, ... in order, so it keeps
+    // pref[j] <= k. Each lane walks its candidates k = tid, tid + kThreads, ... in order, so it keeps
     // its pose j (and j's rectangle) in registers and moves on when k passes pref[j + 1]. The
     // ray state and y of the next candidate are loaded while the current one is added (two
     // register sets taken in turn).
