@@ -279,18 +279,6 @@ namespace ehp
         return sqrt(e * e + 1.0) * 1.0001 * (n - 1) + 4.0;
     }
 
-    // Smallest footprint scaling of a pose over the volume: sdd over the largest distance from the
-    // source to a corner of the volume.
-    inline double voxel_min_scaling(const PoseGeom& g, const Dims& dims)
-    {
-        double dist2 = 0.0;
-        for (int i = 0; i < dims.dim; ++i) {
-            const double c = g.C[i], far = c < 0.5 * dims.vol[i] ? dims.vol[i] - c : c;
-            dist2 += far * far;
-        }
-        return dist2 > 0.0 ? (double) g.sdd / sqrt(dist2) : -1.0;
-    }
-
     // a / b, correctly rounded, from rb = 1 / b correctly rounded: the quotient estimate with one
     // correction (Markstein, Computation of elementary functions on the IBM RISC System/6000, 1990,
     // theorem on division); b's mantissa is not all ones, quotients far from underflow.
@@ -415,9 +403,33 @@ namespace ehp
         return b > 4096.0 * ls ? b : 4096.0 * ls;
     }
 
-    // Largest footprint scaling of a pose over the volume: sdd over the smallest distance from
-    // the source to the volume box (scaling is sdd / |ext x| and |ext x| is the distance from
-    // the source to the voxel centre x).
+    // Least (sign -1) or largest (+1) stretch of the extrinsic matrix' linear part: |ext x| lies between
+    // these times the distance, in voxels, from the source to the voxel centre x. Bounds of its singular
+    // values from M^T M (Gershgorin): the voxel spacings for a rotation of them, 1 for unit spacing.
+    inline double ext_stretch(const PoseGeom& g, const Dims& dims, int sign)
+    {
+        double best = 0.0;
+        for (int i = 0; i < dims.dim; ++i) {
+            double diag = 0.0, off = 0.0;
+            for (int j = 0; j < dims.dim; ++j) {
+                double dot = 0.0;
+                for (int k = 0; k < dims.dim; ++k)
+                    dot += (double) g.ext[k + i * dims.dim] * g.ext[k + j * dims.dim];
+                if (i == j)
+                    diag = dot;
+                else
+                    off += fabs(dot);
+            }
+            const double b = diag + sign * off;
+            best = i == 0 || sign * b > sign * best ? b : best;
+        }
+        if (fabs(best - 1.0) < 1.0e-5) // the rounding of a rotation
+            return 1.0;
+        return best > 0.0 ? sqrt(best) : 0.0;
+    }
+
+    // Largest footprint scaling of a pose over the volume, sdd / |ext x|: from the smallest distance from the
+    // source to the volume box (the source inside, or ext singular: -1).
     inline double voxel_max_scaling(const PoseGeom& g, const Dims& dims)
     {
         double dist2 = 0.0;
@@ -426,7 +438,21 @@ namespace ehp
             const double e = c < 0.0 ? -c : (c > dims.vol[i] ? c - dims.vol[i] : 0.0);
             dist2 += e * e;
         }
-        return dist2 > 0.0 ? (double) g.sdd / sqrt(dist2) : -1.0;
+        const double least = ext_stretch(g, dims, -1) * sqrt(dist2);
+        return least > 0.0 ? (double) g.sdd / least : -1.0;
+    }
+
+    // Smallest footprint scaling of a pose over the volume, from the largest distance from the source to a
+    // corner of the volume.
+    inline double voxel_min_scaling(const PoseGeom& g, const Dims& dims)
+    {
+        double dist2 = 0.0;
+        for (int i = 0; i < dims.dim; ++i) {
+            const double c = g.C[i], far = c < 0.5 * dims.vol[i] ? dims.vol[i] - c : c;
+            dist2 += far * far;
+        }
+        const double most = ext_stretch(g, dims, 1) * sqrt(dist2);
+        return most > 0.0 ? (double) g.sdd / most : -1.0;
     }
 
     // Driving axis of a pose for the tiled forward: the largest component of the central ray.

@@ -64,6 +64,30 @@ def test_voxel_columns(kind, ratio, size, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
+@pytest.mark.parametrize("spacing", [(0.5, 0.5, 0.5), (0.6, 0.6, 0.6), (1.5, 1.5, 1.5), (2.0, 0.8, 1.0)], ids=str)
+@pytest.mark.parametrize("kind", ["blob", "bspline"])
+def test_voxel_spacing(kind, spacing, dtype):
+    """Footprints scale with the extrinsic matrix, which holds the voxel spacing: twice as wide (the
+    general kernels) or wider, narrower and anisotropic (other column counts and tables)."""
+    import elsa_amd as E
+
+    vol, det = (17, 12, 21), (50, 44)
+    poses = [oracle.geometry_pose(3, 300.0, 30.0, vol, det, angle_rad=a, vol_spacing=spacing)
+             for a in (0.0, 0.4, 1.1, 1.6, 3.0)]
+    g = oracle.geom_from_poses(3, vol, det, poses)
+    cls = E.BlobVoxelProjectorCUDA if kind == "blob" else E.BSplineVoxelProjectorCUDA
+    lut, sup = (oracle.blob_lut(2.0, 10.83, 2, 100, dtype), 2.0) if kind == "blob" else (
+        oracle.bspline_lut(3, 2, 100, dtype), 1.5)
+    op = cls(*geom_to_descriptors(g), dtype=dtype)
+    rng = np.random.default_rng(8)
+    x = rng.random(g.vol_shape).astype(dtype)
+    y = rng.random(g.sino_shape).astype(dtype)
+    bar = 1e-6 if dtype == np.float32 else 1e-13
+    assert rel_l2(op.applyAdjoint(y), oracle.voxel(g, y, lut, sup, adjoint=True, acc64=True)) <= bar
+    assert rel_l2(op.apply(x), oracle.voxel(g, x, lut, sup, acc64=True)) <= bar
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64], ids=["f32", "f64"])
 @pytest.mark.parametrize("vol,det,poses", [((1, 5), 9, 7), ((31, 17), 40, 33), ((24, 40), 61, 140)])
 def test_gather_parts_2d(vol, det, poses, dtype):
     import elsa_amd as E
