@@ -105,6 +105,34 @@ namespace ehp
         footprint_rect<D>(dims, radius, fp);
     }
 
+    // |ext x|^2 of voxel (x, y, z) for the FP32 kernels. 2D: elsa's order. 3D: the rotated coordinates by
+    // FMAs with the translation (the source's distance, up to a hundred times the volume) added last, so that
+    // only the last addition rounds at that size, and the squares by FMAs: eight instructions a voxel less than
+    // elsa's order, and an RMS error of the scaling against 64 bits of 4.9e-8 instead of 5.1e-8 (36 to 400 voxels
+    // a side, source 100 sides away; 4.6e-8 and 4.85e-8 at a source 1.2 sides away). An FMA chain that
+    // starts with the translation rounds at its size at every step: 5.3e-8 to 5.7e-8.
+    template <int D>
+    EHP_HD inline float source_dist2(const PoseGeom& g, int x, int y, int z)
+    {
+        if constexpr (D == 2) {
+            float pc[3], ce[3];
+            voxel_project<2>(g, x, y, z, pc, ce);
+            return ce[0] * ce[0] + ce[1] * ce[1];
+        } else {
+            const float h[3] = {(float) x + 0.5f, (float) y + 0.5f, (float) z + 0.5f};
+            float n2 = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                float c = g.ext[i] * h[0];
+                c = __builtin_fmaf(g.ext[i + 3], h[1], c);
+                c = __builtin_fmaf(g.ext[i + 6], h[2], c);
+                c = c + g.ext[i + 9];
+                n2 = i == 0 ? c * c : __builtin_fmaf(c, c, n2);
+            }
+            return n2;
+        }
+    }
+
     // Reciprocal and reciprocal square root in one instruction each (v_rcp_f32, v_rsq_f32, within
     // 1 ulp); correctly rounded on the CPU.
     EHP_HD inline float fast_rcp(float x)
@@ -131,23 +159,15 @@ namespace ehp
     // footprint). The homogeneous division is the quotient q = p rcp(w) with one correction,
     // q + (p - q w) rcp(w) (two FMAs): within about half an ulp of p / w, as the centre, a
     // coordinate of hundreds of pixels from which the taps' pixel indices are subtracted, needs.
-    // The scaling sdd / |ext x| = sdd rsq(|ext x|^2), by FMAs, and rs = 1 / scaling come within an ulp or
+    // The scaling sdd / |ext x| = sdd rsq(|ext x|^2) (source_dist2) and rs = 1 / scaling come within an ulp or
     // two (relative errors of 1e-7 in the tap distances). Forward and back projection share it, so
     // they stay each other's adjoint.
     template <int D>
     EHP_HD inline void footprint_fast(const PoseGeom& g, const Dims& dims, int x, int y, int z, float radius,
                                       Footprint& fp, float& rs)
     {
-        float pc[3], ce[3], unused[3];
+        float pc[3], unused[3];
         voxel_project<D>(g, x, y, z, pc, unused);
-        const float h[3] = {(float) x + 0.5f, (float) y + 0.5f, (float) z + 0.5f};
-#pragma unroll
-        for (int i = 0; i < D; ++i) {
-            ce[i] = g.ext[i + D * D];
-#pragma unroll
-            for (int j = D - 1; j >= 0; --j)
-                ce[i] = __builtin_fmaf(g.ext[i + j * D], h[j], ce[i]);
-        }
         const float w = pc[D - 1];
         const float rw = fast_rcp(w);
 #pragma unroll
@@ -155,11 +175,7 @@ namespace ehp
             const float q = pc[i] * rw;
             fp.center[i] = __builtin_fmaf(__builtin_fmaf(-q, w, pc[i]), rw, q) - 0.5f;
         }
-        float n2 = ce[0] * ce[0];
-#pragma unroll
-        for (int i = 1; i < D; ++i)
-            n2 = __builtin_fmaf(ce[i], ce[i], n2);
-        fp.scaling = g.sdd * fast_rsq(n2);
+        fp.scaling = g.sdd * fast_rsq(source_dist2<D>(g, x, y, z));
         rs = fast_rcp(fp.scaling);
         footprint_rect<D>(dims, radius, fp);
     }
