@@ -23,6 +23,7 @@
 // the one-thread-per-ray kernels (make_ray, joseph_setup), and the per-sample weights use the
 // same arithmetic as joseph_sample, so they are bit-identical to the forward's.
 #include "ehp_kernels.hpp"
+#include "ehp_last_block.hpp"
 #include "ehp_tile_pair.hpp"
 
 #include <type_traits>
@@ -165,9 +166,7 @@ namespace ehp
             if (threadIdx.x == 0) {
                 __hip_atomic_store(partial + blockIdx.x, (unsigned long long) m, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
-                // release of the maximum, acquire of the others' by the block that counts last
-                last = __hip_atomic_fetch_add(fixexp + 1, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
-                       (int) gridDim.x - 1;
+                last = counts_last(reinterpret_cast<unsigned int*>(fixexp + 1), gridDim.x);
             }
             __syncthreads();
             if (!last)
@@ -179,8 +178,6 @@ namespace ehp
             }
             __syncthreads(); // block_max_bits' LDS is read again
             m = block_max_bits(m);
-            if (threadIdx.x == 0)
-                fixexp[1] = 0;
         }
         if (threadIdx.x == 0)
             fixexp[0] = fixed_point_exponent(bits_value(m), bound);
