@@ -248,24 +248,12 @@ namespace
         return EHP_OK;
     }
 
-    int batch_apply(ehp_batch* b, const void* in, void* out, hipStream_t s, bool adjoint)
+    // Runs fn, which enqueues work on s that uses the operators' device state, after the previous calls on
+    // the batch and on every operator of it and before their next ones. The mutexes are taken in address order,
+    // so two callers cannot deadlock.
+    template <class Fn>
+    hipError_t ordered(ehp_batch* b, hipStream_t s, Fn fn)
     {
-        if (!b->fused) {
-            const size_t es = b->dtype == EHP_F64 ? sizeof(double) : (b->dtype == EHP_BF16 ? 2 : sizeof(float));
-            for (size_t j = 0; j < b->ops.size(); ++j) {
-                const int64_t ai = adjoint ? b->sino_off[j] : b->vol_off[j];
-                const int64_t ao = adjoint ? b->vol_off[j] : b->sino_off[j];
-                const void* pi = (const char*) in + ai * es;
-                void* po = (char*) out + ao * es;
-                const int rc = adjoint ? ehp_adjoint(b->ops[j], pi, po, s) : ehp_forward(b->ops[j], pi, po, s);
-                if (rc != EHP_OK)
-                    return rc;
-            }
-            return EHP_OK;
-        }
-        // A fused pass rewrites the operators' views and the batch's scale: it runs after the
-        // previous call on the batch and on every operator of it, and the operators' next calls
-        // run after it. The mutexes are taken in address order, so two callers cannot deadlock.
         std::vector<std::mutex*> mus{&b->order.mu};
         for (ehp_op* op : b->ops)
             mus.push_back(&op->order.mu);
@@ -284,51 +272,73 @@ namespace
             waited.push_back(g.last.get());
             e = ehp::order_begin(g, s, capturing);
         }
-        if (e != hipSuccess)
-            return bfail(EHP_ERR_HIP, "ordering after the previous calls: %s", hipGetErrorString(e));
-        if (!adjoint && b->kind == KIND_VOXEL) {
-            e = ehp::fixed_point_exponent_batch((int) b->ops.size(), b->d_segs, b->d_sblocks, b->nsblocks,
-                                                b->d_bounds, b->d_maxbits, b->d_fixexp, (const float*) in, s);
-            if (e == hipSuccess)
-                e = ehp::voxel_forward_batch(b->dim, b->vox_cols, b->d_vfjobs, b->d_fblocks, b->nfblocks, b->lds[0],
-                                             b->d_fixexp, (const float*) in, (float*) out, s);
-        } else if (adjoint && b->kind == KIND_VOXEL) {
-            e = ehp::voxel_gather_batch(b->dim, b->vox_gather_cols, b->d_vajobs, b->d_vablocks, b->nvablocks, b->lds[1],
-                                        b->vox_gather_threads, (const float*) in, (float*) out, s);
-        } else if (!adjoint && b->kind == KIND_SIDDON) {
-            e = ehp::siddon_forward_batch(b->dim, b->d_cjobs, b->d_cblocks, b->ncblocks, b->d_sfjobs, b->d_fblocks,
-                                          b->nfblocks, (const float*) in, (float*) out, s);
-        } else if (!adjoint) {
-            e = ehp::joseph_forward_batch(b->dim, b->d_cjobs, b->d_cblocks, b->ncblocks, b->d_fjobs, b->d_fblocks,
-                                          b->nfblocks, (const float*) in, (float*) out, s);
-        } else if (b->kind == KIND_SIDDON) {
-            e = ehp::launch_fill<float>((float*) out, b->vol_off.back(), 0.0f, s);
-            if (e == hipSuccess)
-                e = ehp::fixed_point_exponent_batch((int) b->ops.size(), b->d_segs, b->d_sblocks, b->nsblocks,
-                                                    b->d_bounds, b->d_maxbits, b->d_fixexp, (const float*) in, s);
-            const ehp::SidAdjJob* sj[3] = {b->d_sajobs[0], b->d_sajobs[1], b->d_sajobs[2]};
-            const int* ab[3] = {b->d_ablocks[0], b->d_ablocks[1], b->d_ablocks[2]};
-            if (e == hipSuccess)
-                e = ehp::siddon_adjoint_batch(b->dim, sj, ab, b->nablocks, b->lds, b->d_fixexp, (const float*) in,
-                                              (float*) out, s);
-        } else {
-            const ehp::AdjJob* aj[3] = {b->d_ajobs[0], b->d_ajobs[1], b->d_ajobs[2]};
-            const int* ab[3] = {b->d_ablocks[0], b->d_ablocks[1], b->d_ablocks[2]};
-            e = ehp::joseph_adjoint_batch(b->dim, (int) b->ops.size(), b->d_segs, b->d_sblocks, b->nsblocks,
-                                          b->d_bounds, aj, ab, b->nablocks, b->lds, b->vol_off.back(), b->d_maxbits,
-                                          b->d_fixexp, (const float*) in, (float*) out, s);
-        }
-        if (e != hipSuccess)
-            return bfail(EHP_ERR_HIP, "%s launch: %s", adjoint ? "batch adjoint" : "batch forward",
-                         hipGetErrorString(e));
-        e = ehp::order_end(b->order, s, capturing);
-        if (e != hipSuccess)
-            return bfail(EHP_ERR_HIP, "recording the end of the pass: %s", hipGetErrorString(e));
-        if (!capturing)
+        if (e == hipSuccess)
+            e = fn();
+        if (e == hipSuccess)
+            e = ehp::order_end(b->order, s, capturing);
+        if (e == hipSuccess && !capturing)
             for (ehp_op* op : b->ops) {
                 op->order.last = b->order.last;
                 op->order.last_stream = s;
             }
+        return e;
+    }
+
+    int batch_apply(ehp_batch* b, const void* in, void* out, hipStream_t s, bool adjoint)
+    {
+        if (!b->fused) {
+            const size_t es = b->dtype == EHP_F64 ? sizeof(double) : (b->dtype == EHP_BF16 ? 2 : sizeof(float));
+            for (size_t j = 0; j < b->ops.size(); ++j) {
+                const int64_t ai = adjoint ? b->sino_off[j] : b->vol_off[j];
+                const int64_t ao = adjoint ? b->vol_off[j] : b->sino_off[j];
+                const void* pi = (const char*) in + ai * es;
+                void* po = (char*) out + ao * es;
+                const int rc = adjoint ? ehp_adjoint(b->ops[j], pi, po, s) : ehp_forward(b->ops[j], pi, po, s);
+                if (rc != EHP_OK)
+                    return rc;
+            }
+            return EHP_OK;
+        }
+        // A fused pass rewrites the operators' views and the batch's scale.
+        const hipError_t e = ordered(b, s, [&] {
+            hipError_t e = hipSuccess;
+            if (!adjoint && b->kind == KIND_VOXEL) {
+                e = ehp::fixed_point_exponent_batch((int) b->ops.size(), b->d_segs, b->d_sblocks, b->nsblocks,
+                                                    b->d_bounds, b->d_maxbits, b->d_fixexp, (const float*) in, s);
+                if (e == hipSuccess)
+                    e = ehp::voxel_forward_batch(b->dim, b->vox_cols, b->d_vfjobs, b->d_fblocks, b->nfblocks, b->lds[0],
+                                                 b->d_fixexp, (const float*) in, (float*) out, s);
+            } else if (adjoint && b->kind == KIND_VOXEL) {
+                e = ehp::voxel_gather_batch(b->dim, b->vox_gather_cols, b->d_vajobs, b->d_vablocks, b->nvablocks, b->lds[1],
+                                            b->vox_gather_threads, (const float*) in, (float*) out, s);
+            } else if (!adjoint && b->kind == KIND_SIDDON) {
+                e = ehp::siddon_forward_batch(b->dim, b->d_cjobs, b->d_cblocks, b->ncblocks, b->d_sfjobs, b->d_fblocks,
+                                              b->nfblocks, (const float*) in, (float*) out, s);
+            } else if (!adjoint) {
+                e = ehp::joseph_forward_batch(b->dim, b->d_cjobs, b->d_cblocks, b->ncblocks, b->d_fjobs, b->d_fblocks,
+                                              b->nfblocks, (const float*) in, (float*) out, s);
+            } else if (b->kind == KIND_SIDDON) {
+                e = ehp::launch_fill<float>((float*) out, b->vol_off.back(), 0.0f, s);
+                if (e == hipSuccess)
+                    e = ehp::fixed_point_exponent_batch((int) b->ops.size(), b->d_segs, b->d_sblocks, b->nsblocks,
+                                                        b->d_bounds, b->d_maxbits, b->d_fixexp, (const float*) in, s);
+                const ehp::SidAdjJob* sj[3] = {b->d_sajobs[0], b->d_sajobs[1], b->d_sajobs[2]};
+                const int* ab[3] = {b->d_ablocks[0], b->d_ablocks[1], b->d_ablocks[2]};
+                if (e == hipSuccess)
+                    e = ehp::siddon_adjoint_batch(b->dim, sj, ab, b->nablocks, b->lds, b->d_fixexp, (const float*) in,
+                                                  (float*) out, s);
+            } else {
+                const ehp::AdjJob* aj[3] = {b->d_ajobs[0], b->d_ajobs[1], b->d_ajobs[2]};
+                const int* ab[3] = {b->d_ablocks[0], b->d_ablocks[1], b->d_ablocks[2]};
+                e = ehp::joseph_adjoint_batch(b->dim, (int) b->ops.size(), b->d_segs, b->d_sblocks, b->nsblocks,
+                                              b->d_bounds, aj, ab, b->nablocks, b->lds, b->vol_off.back(), b->d_maxbits,
+                                              b->d_fixexp, (const float*) in, (float*) out, s);
+            }
+            return e;
+        });
+        if (e != hipSuccess)
+            return bfail(EHP_ERR_HIP, "%s launch: %s", adjoint ? "batch adjoint" : "batch forward",
+                         hipGetErrorString(e));
         return EHP_OK;
     }
 
@@ -358,6 +368,7 @@ namespace
         }
         A.fwd = [b](const void* x, void* y, hipStream_t s) { return batch_apply(b, x, y, s, false); };
         A.adj = [b](const void* y, void* x, hipStream_t s) { return batch_apply(b, y, x, s, true); };
+        A.ordered = [b](hipStream_t s, const std::function<hipError_t()>& fn) { return ordered(b, s, fn); };
         return A;
     }
 } // namespace

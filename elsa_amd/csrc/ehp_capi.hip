@@ -1180,6 +1180,15 @@ namespace
             ops.shapes = {op->dims.dim, op->dims.vol[0], op->dims.vol[1], op->dims.vol[2]};
             ops.fwd = [op](const void* x, void* y, hipStream_t s) { return ehp_forward(op, x, y, s); };
             ops.adj = [op](const void* y, void* x, hipStream_t s) { return ehp_adjoint(op, y, x, s); };
+            ops.ordered = [op](hipStream_t s, const std::function<hipError_t()>& fn) {
+                std::lock_guard<std::mutex> lock(op->order.mu);
+                hipError_t e = ehp::order_begin(op->order, s, false);
+                if (e == hipSuccess)
+                    e = fn();
+                if (e == hipSuccess)
+                    e = ehp::order_end(op->order, s, false);
+                return e;
+            };
         }
     };
 } // namespace

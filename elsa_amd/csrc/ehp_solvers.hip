@@ -421,9 +421,13 @@ namespace ehp
             }
         };
 
-        // Runs body() once eagerly per iteration, or captures it into a graph and replays it.
+        // Runs body(), which launches on s, once eagerly per iteration, or captures it into a graph and replays it on
+        // s. A capture orders nothing against other streams, so the replays together take their turn among the
+        // operators' calls. It runs on a stream of its own, to which s is set meanwhile: no stream may
+        // wait for an event of a stream that is capturing, as another thread's call on the operators would for
+        // the event after their last call on s.
         template <class Body>
-        hipError_t iterate(hipStream_t s, int iterations, bool graph, Body body)
+        hipError_t iterate(const SolveOps& A, hipStream_t& s, int iterations, bool graph, Body body)
         {
             if (iterations <= 0)
                 return hipSuccess;
@@ -437,21 +441,33 @@ namespace ehp
             }
             hipGraph_t g = nullptr;
             hipGraphExec_t ge = nullptr;
-            hipError_t e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
+            const hipStream_t run = s;
+            hipStream_t cap = nullptr;
+            hipError_t e = hipStreamCreateWithFlags(&cap, hipStreamNonBlocking);
             if (e != hipSuccess)
                 return e;
-            const int rc = body();
-            e = hipStreamEndCapture(s, &g);
-            if (rc != EHP_OK) {
+            e = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
+            int rc = EHP_OK;
+            if (e == hipSuccess) {
+                s = cap;
+                rc = body();
+                s = run;
+                e = hipStreamEndCapture(cap, &g);
+            }
+            (void) hipStreamDestroy(cap);
+            if (rc != EHP_OK || e != hipSuccess) {
                 if (g)
                     (void) hipGraphDestroy(g);
-                return hipErrorLaunchFailure;
+                return rc != EHP_OK ? hipErrorLaunchFailure : e;
             }
-            if (e != hipSuccess)
-                return e;
             e = hipGraphInstantiate(&ge, g, nullptr, nullptr, 0);
-            for (int i = 0; e == hipSuccess && i < iterations; ++i)
-                e = hipGraphLaunch(ge, s);
+            if (e == hipSuccess)
+                e = A.ordered(s, [&] {
+                    hipError_t el = hipSuccess;
+                    for (int i = 0; el == hipSuccess && i < iterations; ++i)
+                        el = hipGraphLaunch(ge, s);
+                    return el;
+                });
             if (ge)
                 (void) hipGraphExecDestroy(ge);
             (void) hipGraphDestroy(g);
@@ -578,7 +594,7 @@ namespace ehp
                     return EHP_ERR_HIP;
                 return hipGetLastError() == hipSuccess ? EHP_OK : EHP_ERR_HIP;
             };
-            hipError_t e = iterate(s, iterations, graph, body);
+            hipError_t e = iterate(A, s, iterations, graph, body);
             if (e != hipSuccess)
                 return rc != EHP_OK ? rc : ehp_solver_fail(EHP_ERR_HIP, hipGetErrorString(e));
             std::vector<double> hsc, hh;
@@ -719,7 +735,7 @@ namespace ehp
                     return r2;
                 return hipGetLastError() == hipSuccess ? EHP_OK : EHP_ERR_HIP;
             };
-            hipError_t e = iterate(s, iterations, graph, body);
+            hipError_t e = iterate(A, s, iterations, graph, body);
             if (e != hipSuccess)
                 return ehp_solver_fail(EHP_ERR_HIP, hipGetErrorString(e));
             std::vector<double> hsc, hh;
@@ -1077,7 +1093,7 @@ namespace ehp
                 return hipGetLastError() == hipSuccess ? EHP_OK : EHP_ERR_HIP;
             };
             if (!residuals) {
-                hipError_t e = iterate(s, iterations, graph, body);
+                hipError_t e = iterate(A, s, iterations, graph, body);
                 if (e == hipSuccess)
                     e = hipStreamSynchronize(s);
                 return e == hipSuccess ? EHP_OK : ehp_solver_fail(EHP_ERR_HIP, hipGetErrorString(e));

@@ -17,6 +17,10 @@ namespace ehp
         const int64_t* doff = nullptr;
         const int64_t* roff = nullptr;
         std::function<int(const void*, void*, hipStream_t)> fwd, adj;
+        // Runs fn, which enqueues on s work that uses the operators outside fwd and adj (replays of a graph
+        // that captured these), after the operators' previous calls and before their next ones. fn makes
+        // no call on the operators.
+        std::function<hipError_t(hipStream_t s, const std::function<hipError_t()>& fn)> ordered;
         // per problem: number of volume axes and their sizes (dim, n0, n1, n2), for regularisers
         // defined on the volume grid
         std::vector<int> shapes;
