@@ -582,6 +582,44 @@ namespace ehp
     constexpr int kAbsmaxBlocks = 256;
     constexpr int kPoseBatch = 8;
 
+    // ---- the launches of the 2D back projection
+
+    constexpr int kPoses2d = 512; // poses per step at most
+
+    // The rays of one pose that can meet the tile: pixels [base, base + count) of the sinogram
+    struct Rays2d {
+        long long base;
+        int cnt, pref;
+    };
+
+    // LDS of a 2D workgroup: both axes' slots and a step's poses
+    inline size_t lds2d(const TileCfg& t, int steps)
+    {
+        return ((size_t) t.LA * (t.TB + 2) + (size_t) t.TB * (t.LA + 2)) * 8 + (size_t) (steps + 1) * sizeof(Rays2d);
+    }
+
+    // The tile the 2D back projection runs for the tile tc of the operator: halved until it fits 64 KB
+    // with the longest step.
+    inline TileCfg tile2d(const TileCfg& tc)
+    {
+        TileCfg t = tc;
+        while (lds2d(t, kPoses2d - 1) > 65536 && (t.LA > 1 || t.TB > 1)) {
+            int& m = t.LA >= t.TB ? t.LA : t.TB;
+            m = (m + 1) / 2;
+        }
+        return t;
+    }
+
+    // Poses per step: 16 pose batches, at most the operator's poses, and no more than 2^30 pixels in
+    // all (a step's candidate rays are counted in an int).
+    inline int steps2d(const Dims& dims, int batch)
+    {
+        const int most = (1 << 30) / dims.det[0];
+        int s = 16 * batch < kPoses2d ? 16 * batch : kPoses2d;
+        s = s < dims.nposes ? s : dims.nposes;
+        return s < most ? s : most;
+    }
+
     // Upper bound of sum |len * weight| over the contributions one LDS slot can receive from
     // all poses. Per pose a slot receives one sample of each ray whose crossing point with the
     // slot's plane lies within the slot's 2x2 (2D: 2) interpolation footprint; with

@@ -295,41 +295,6 @@ namespace ehp
     // exponent's launch): 64^2 / 90 poses 42 -> 19 us, 256^2 / 180 73 -> 34, 512^2 / 360 309 -> 109; 64 problems
     // of 128^2..512^2 in one launch 4635 -> 1129 us.
 
-    constexpr int kPoses2d = 512; // poses per step at most
-
-    // The rays of one pose that can meet the tile: pixels [base, base + count) of the sinogram
-    struct Rays2d {
-        long long base;
-        int cnt, pref;
-    };
-
-    // The tile the 2D back projection runs for the tile tc of the operator: halved until both axes'
-    // slots and a step of poses fit 64 KB.
-    TileCfg tile2d(const TileCfg& tc)
-    {
-        TileCfg t = tc;
-        auto bytes = [&] {
-            return ((int64_t) t.LA * (t.TB + 2) + (int64_t) t.TB * (t.LA + 2)) * 8 + kPoses2d * (int64_t) sizeof(Rays2d);
-        };
-        while (bytes() > 65536 && (t.LA > 1 || t.TB > 1)) {
-            int& m = t.LA >= t.TB ? t.LA : t.TB;
-            m = (m + 1) / 2;
-        }
-        return t;
-    }
-
-    size_t lds2d(const TileCfg& t, int steps)
-    {
-        return ((size_t) t.LA * (t.TB + 2) + (size_t) t.TB * (t.LA + 2)) * 8 + (size_t) (steps + 1) * sizeof(Rays2d);
-    }
-
-    // Poses per step: 16 pose batches, at most the operator's poses
-    int steps2d(const Dims& dims, int batch)
-    {
-        const int s = 16 * batch < kPoses2d ? 16 * batch : kPoses2d;
-        return s < dims.nposes ? s : dims.nposes;
-    }
-
     template <int NT, class ST>
     __device__ __forceinline__ void adj2d_block(const PoseGeom* __restrict__ geo, const RayRec* __restrict__ table,
                                                 const Dims& dims, const int* __restrict__ pose_axes, const TileCfg& tc,

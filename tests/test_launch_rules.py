@@ -1,0 +1,27 @@
+"""The rules that size the back projections' launches (CPU, the functions that the library calls)."""
+import ctypes
+import os
+
+import pytest
+
+from test_tile_logic import ROOT, SFX, _build
+
+SRC = os.path.join(ROOT, "tests", "cxx", "launch_rules_check.cpp")
+OUT = os.path.join(ROOT, "tests", "cxx", "_build", f"liblaunch_rules{SFX}.so")
+
+
+@pytest.fixture(scope="module")
+def lib():
+    _build(SRC, OUT)
+    return ctypes.CDLL(OUT)
+
+
+@pytest.mark.parametrize("det", [1, 1000, (1 << 21) - 1, 1 << 21, (1 << 22) + 5, (1 << 23) - 1])
+@pytest.mark.parametrize("poses,batch", [(1, 1), (37, 32), (100000, 1), (100000, 8), (100000, 32)])
+def test_rays_of_a_2d_step_count_in_an_int(lib, det, poses, batch):
+    """Up to the widest detector that the tiled back projections take (2^23 - 1), with room for the
+    workgroup's strides past the last ray."""
+    s = lib.steps_2d(det, poses, batch)
+    assert 1 <= s <= min(poses, 16 * batch, 512)
+    assert s * det + 4 * 1024 < 2 ** 31
+    assert s == min(poses, 16 * batch, 512) or det > (1 << 30) // 512
