@@ -603,7 +603,7 @@ namespace ehp
     inline TileCfg tile2d(const TileCfg& tc)
     {
         TileCfg t = tc;
-        while (lds2d(t, kPoses2d - 1) > 65536 && (t.LA > 1 || t.TB > 1)) {
+        while (lds2d(t, kPoses2d) > 65536 && (t.LA > 1 || t.TB > 1)) {
             int& m = t.LA >= t.TB ? t.LA : t.TB;
             m = (m + 1) / 2;
         }

@@ -13,7 +13,9 @@ OUT = os.path.join(ROOT, "tests", "cxx", "_build", f"liblaunch_rules{SFX}.so")
 @pytest.fixture(scope="module")
 def lib():
     _build(SRC, OUT)
-    return ctypes.CDLL(OUT)
+    L = ctypes.CDLL(OUT)
+    L.most_lds_2d.restype = ctypes.c_int64
+    return L
 
 
 @pytest.mark.parametrize("det", [1, 1000, (1 << 21) - 1, 1 << 21, (1 << 22) + 5, (1 << 23) - 1])
@@ -25,3 +27,7 @@ def test_rays_of_a_2d_step_count_in_an_int(lib, det, poses, batch):
     assert 1 <= s <= min(poses, 16 * batch, 512)
     assert s * det + 4 * 1024 < 2 ** 31
     assert s == min(poses, 16 * batch, 512) or det > (1 << 30) // 512
+
+
+def test_2d_tiles_fit_64_kb(lib):
+    assert lib.most_lds_2d(300, 1300) <= 65536
