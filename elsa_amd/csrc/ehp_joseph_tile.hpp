@@ -111,11 +111,17 @@ namespace ehp
         static constexpr int b2 = (D == 2) ? 0 : (A == 2 ? 1 : 2);
     };
 
-    // Slots of a tile's row: its voxels and the halo, in 3D odd (the atomics of neighbouring rows then
-    // fall on different LDS banks)
-    EHP_HD inline int tile_row_slots(int dim, int TB)
+    constexpr int kMaxPoseBatch = 32;
+    EHP_HD constexpr size_t batch_lds_bytes(int batch);
+
+    // Slots of a tile's row: its voxels and the halo, in 3D an odd number (the atomics of neighbouring rows
+    // then fall on different LDS banks) where the tile fits 64 KB with it.
+    EHP_HD inline int tile_row_slots(int dim, const TileCfg& tc)
     {
-        return dim == 3 ? (TB + 2) | 1 : TB + 2;
+        const int odd = (tc.TB + 2) | 1;
+        return dim == 3 && (int64_t) tc.LA * (tc.TC + 2) * odd * 8 + (int64_t) batch_lds_bytes(kMaxPoseBatch) <= 65536
+                   ? odd
+                   : tc.TB + 2;
     }
 
     template <int D, int A>
@@ -129,7 +135,7 @@ namespace ehp
         t.B1 = dims.vol[b1] < t.B0 + tc.TB ? dims.vol[b1] : t.B0 + tc.TB;
         t.C0 = (D == 3) ? ic * tc.TC : 0;
         t.C1 = (D == 3) ? (dims.vol[b2] < t.C0 + tc.TC ? dims.vol[b2] : t.C0 + tc.TC) : 1;
-        t.PB = tile_row_slots(D, tc.TB);
+        t.PB = tile_row_slots(D, tc);
         t.PC = (D == 3) ? tc.TC + 2 : 1;
         t.nslots = tc.LA * t.PC * t.PB;
         t.B0m1f = (float) (t.B0 - 1);
@@ -547,8 +553,6 @@ namespace ehp
         }
         return lo;
     }
-
-    constexpr int kMaxPoseBatch = 32;
 
     // Candidate rectangle of one pose of a batch in the tiled back projections: rnu = 1 / width,
     // nu = width, base = ray index of its first pixel.

@@ -676,7 +676,7 @@ namespace ehp
     size_t joseph_tile_lds_bytes(const Dims& dims, const TileCfg& tc, int batch)
     {
         const int PC = dims.dim == 3 ? tc.TC + 2 : 1;
-        return (size_t) tc.LA * PC * tile_row_slots(dims.dim, tc.TB) * sizeof(long long) + batch_lds_bytes(batch);
+        return (size_t) tc.LA * PC * tile_row_slots(dims.dim, tc) * sizeof(long long) + batch_lds_bytes(batch);
     }
 
     // ST: the sinogram's storage type (float, or bf16 for bfloat16 operators); the volume is

@@ -26,3 +26,21 @@ extern "C" int64_t most_lds_2d(int la, int tb)
             most = std::max(most, lds2d(tile2d(TileCfg{a, b, 1}), kPoses2d));
     return (int64_t) most;
 }
+
+// Tiles of 3D back projections that a device with `limit` bytes of LDS per workgroup took with rows as
+// long as the voxels need, and does not take with the rows that they have.
+extern "C" int refused_tiles_3d(int64_t limit)
+{
+    int refused = 0;
+    for (int la = 1; la <= 40; ++la)
+        for (int tb = 1; tb <= 150; ++tb)
+            for (int c = 1; c <= 150; ++c) {
+                const TileCfg t{la, tb, c};
+                const int64_t rest = (int64_t) batch_lds_bytes(kMaxPoseBatch), rows = (int64_t) la * (c + 2) * 8;
+                const int slots = tile_row_slots(3, t);
+                if (slots != tb + 2 && slots != ((tb + 2) | 1))
+                    return -1;
+                refused += rows * (tb + 2) + rest <= limit && rows * slots + rest > limit;
+            }
+    return refused;
+}

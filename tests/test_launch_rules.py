@@ -31,3 +31,8 @@ def test_rays_of_a_2d_step_count_in_an_int(lib, det, poses, batch):
 
 def test_2d_tiles_fit_64_kb(lib):
     assert lib.most_lds_2d(300, 1300) <= 65536
+
+
+@pytest.mark.parametrize("limit", [65536, 163840])
+def test_row_padding_refuses_no_3d_tile(lib, limit):
+    assert lib.refused_tiles_3d(ctypes.c_int64(limit)) == 0
