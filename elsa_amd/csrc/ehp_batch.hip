@@ -10,6 +10,7 @@
 #include "elsa_hip.h"
 #include "ehp_op.hpp"
 #include "ehp_solvers.hpp"
+#include "ehp_tile_rules.hpp"
 
 #include <algorithm>
 #include <cstdarg>
@@ -115,14 +116,11 @@ namespace
                 it.layouts[a] = op->layouts[a];
             }
             it.dims = op->dims;
-            // 2D Joseph tiles that were left at the problem's own default follow the whole batch's size
+            // 2D Joseph tiles that no caller chose follow the whole batch's size
             // (64 problems of 128^2..512^2: 1129 us a pass with 32 x 32 tiles, 1446 with 16 x 16)
             it.tile = op->tile;
-            if (b->kind == KIND_JOSEPH && b->dim == 2) {
-                const ehp::TileCfg own = joseph_tile2d(op->dims.nvox, cus);
-                if (op->tile.LA == own.LA && op->tile.TB == own.TB)
-                    it.tile = joseph_tile2d(b->vol_off.back(), cus);
-            }
+            if (b->kind == KIND_JOSEPH && b->dim == 2)
+                it.tile = ehp::batch_tile(op->tile, op->tile_set, ehp::joseph_tile2d(b->vol_off.back(), cus));
             it.axes_present = op->axes_present;
             it.batch = op->batch;
             it.vol_off = b->vol_off[j];
@@ -159,10 +157,11 @@ namespace
                 v.diff = op->differential;
                 v.pose_axes = op->d_pose_axes;
                 v.pose_margin = op->d_pose_margin;
-                // 2D tiles left at the problem's own default follow the whole batch's poses
+                // 2D tiles that no caller chose follow the whole batch's poses
                 v.tile = op->tile;
-                if (b->dim == 2 && v.tile.LA == voxel_tile2d(op->dims.det[0], op->dims.nposes, cus).LA)
-                    v.tile = voxel_tile2d(op->dims.det[0], poses, cus);
+                if (b->dim == 2)
+                    v.tile = ehp::batch_tile(op->tile, op->tile_set,
+                                             ehp::voxel_tile2d(op->dims.det[0], poses, cus));
                 v.plan = op->vox;
                 v.vol_off = b->vol_off[j];
                 v.sino_off = b->sino_off[j];

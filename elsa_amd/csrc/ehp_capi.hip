@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "ehp_op.hpp"
+#include "ehp_tile_rules.hpp"
 
 namespace
 {
@@ -148,22 +149,6 @@ namespace
         return EHP_OK;
     }
 } // namespace
-
-// Tiles of the 2D voxel forward: up to 256 pixels, narrower ones (down to 16, widths evened) until a
-// launch over `poses` poses has four blocks a CU. Blobs, us: 92 x 80 / 70 poses 16: 26.7, 256: 41; 150^2 in
-// FP64 / 150 32: 101, 256: 154; 256^2 / 180 64: 125, 256: 206; 300 x 380 / 524 256: 322, 64: 431.
-ehp::TileCfg voxel_tile2d(int det, int64_t poses, int cus)
-{
-    const int64_t most = (det + 15) / 16, want = (4 * (int64_t) cus + poses - 1) / poses;
-    const int nt = (int) std::max<int64_t>((det + 255) / 256, std::min(most, want));
-    return ehp::TileCfg{(det + nt - 1) / nt, 1, 1};
-}
-
-ehp::TileCfg joseph_tile2d(int64_t nvox, int cus)
-{
-    const int t = nvox >= (int64_t) 1024 * cus ? 32 : (nvox >= (int64_t) 256 * cus ? 16 : 8);
-    return ehp::TileCfg{t, t, 1};
-}
 
 extern "C" {
 
@@ -332,7 +317,7 @@ namespace
     {
         ehp::TileCfg tc;
         if (dims.dim == 2 && kind == KIND_JOSEPH)
-            return joseph_tile2d(dims.nvox, cus);
+            return ehp::joseph_tile2d(dims.nvox, cus);
         if (dims.dim == 2)
             tc = dims.nvox >= 512 * (int64_t) cus ? ehp::TileCfg{8, 32, 1}
                                                   : (dims.nvox >= 320 * (int64_t) cus ? ehp::TileCfg{8, 16, 1}
@@ -645,7 +630,7 @@ namespace
             return hip_fail(e, "voxel projector state");
         const int cus = device_cus(op->device);
         if (dm.dim == 2)
-            op->tile = voxel_tile2d(dm.det[0], dm.nposes, cus);
+            op->tile = ehp::voxel_tile2d(dm.det[0], dm.nposes, cus);
         else
             op->tile = op->vox.cols > 0 ? voxel_tile3d(dm, cus) : ehp::TileCfg{32, 32, 1};
         op->tiled = true;
@@ -1099,6 +1084,7 @@ int ehp_tile(ehp_op* op, int la, int tb, int tc, int* la_out, int* tb_out, int* 
         if ((int64_t) need > max_lds)
             return fail(EHP_ERR_ARGUMENT, "tile needs %zu bytes of LDS, the device allows %d", need, max_lds);
         op->tile = t;
+        op->tile_set = true;
     }
     if (la_out)
         *la_out = op->tile.LA;

@@ -41,6 +41,7 @@ struct ehp_op {
     int* d_pose_axes = nullptr;
     int axes_present = 0;
     ehp::TileCfg tile{};
+    bool tile_set = false;             // tile() chose it (else the default)
     ehp::RayRec* d_table = nullptr;   // per-ray traversal state (Joseph)
     ehp::SidRec* d_sidtable = nullptr; // per-ray traversal state (Siddon)
     ehp::VoxPlan vox{};                // voxel projectors (3D)
@@ -54,8 +55,3 @@ struct ehp_op {
     size_t stage_bytes = 0;
     ehp::OrderGuard order;   // calls on this operator run one after another on the device
 };
-
-// The 2D Joseph back projection's tile for a launch over nvox voxels (one problem's, or all of a
-// batch's) on a device of cus compute units
-ehp::TileCfg joseph_tile2d(int64_t nvox, int cus);
-ehp::TileCfg voxel_tile2d(int det, int64_t poses, int cus);

@@ -1,7 +1,7 @@
 // launch_rules_check.cpp -- the rules that size the back projections' launches, on the CPU.
 //
 // Built with g++ against the headers that the library's host code uses. Used by tests/test_launch_rules.py.
-#include "ehp_joseph_tile.hpp"
+#include "ehp_tile_rules.hpp"
 
 #include <algorithm>
 
@@ -43,4 +43,13 @@ extern "C" int refused_tiles_3d(int64_t limit)
                 refused += rows * (tb + 2) + rest <= limit && rows * slots + rest > limit;
             }
     return refused;
+}
+
+// Side of the 2D Joseph tile of an n x n problem in a batch of `total` voxels: its own default tile, left
+// alone (0) or chosen by the caller (1)
+extern "C" int batch_tile_2d(int n, int64_t total, int set_by_caller)
+{
+    const int cus = 256;
+    const TileCfg own = joseph_tile2d((int64_t) n * n, cus);
+    return batch_tile(own, set_by_caller != 0, joseph_tile2d(total, cus)).LA;
 }

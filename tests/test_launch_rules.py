@@ -36,3 +36,10 @@ def test_2d_tiles_fit_64_kb(lib):
 @pytest.mark.parametrize("limit", [65536, 163840])
 def test_row_padding_refuses_no_3d_tile(lib, limit):
     assert lib.refused_tiles_3d(ctypes.c_int64(limit)) == 0
+
+
+def test_a_tile_that_the_caller_chose_stays_in_a_batch(lib):
+    """Also when it equals the tile that the operator would have by itself."""
+    total = ctypes.c_int64(64 * 512 * 512)
+    assert lib.batch_tile_2d(64, total, 0) == 32
+    assert lib.batch_tile_2d(64, total, 1) == 8
