@@ -159,6 +159,7 @@ namespace
                 v.pose_margin = op->d_pose_margin;
                 // 2D tiles that no caller chose follow the whole batch's poses
                 v.tile = op->tile;
+                v.tile_set = op->tile_set;
                 if (b->dim == 2)
                     v.tile = ehp::batch_tile(op->tile, op->tile_set,
                                              ehp::voxel_tile2d(op->dims.det[0], poses, cus));

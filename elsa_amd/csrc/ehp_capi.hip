@@ -558,6 +558,7 @@ namespace
             return;
         op->vox.cols = cols;
         op->vox.span = (int) span;
+        op->vox.smin = smin;
         for (int a = 0; a < 3; ++a)
             op->vox.fan[a] = fan_axis(op, bits, a);
     }
@@ -632,7 +633,7 @@ namespace
         if (dm.dim == 2)
             op->tile = ehp::voxel_tile2d(dm.det[0], dm.nposes, cus);
         else
-            op->tile = op->vox.cols > 0 ? voxel_tile3d(dm, cus) : ehp::TileCfg{32, 32, 1};
+            op->tile = op->vox.cols > 0 ? voxel_tile3d(dm, cus) : ehp::kVoxGeneralTile;
         op->tiled = true;
         return EHP_OK;
     }

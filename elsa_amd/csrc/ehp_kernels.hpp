@@ -142,6 +142,7 @@ namespace ehp
     struct VoxPlan {
         int cols;
         int span;
+        double smin; // least footprint scaling
         int fan[3];
     };
 
@@ -156,6 +157,7 @@ namespace ehp
         const int* pose_axes;
         const float* pose_margin;
         TileCfg tile;
+        bool tile_set; // the caller chose it
         VoxPlan plan;
         int64_t vol_off, sino_off;
     };

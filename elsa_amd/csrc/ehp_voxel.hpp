@@ -280,6 +280,9 @@ namespace ehp
         return w < 1.0e6 ? (int) w + 1 : 1 << 20;
     }
 
+    // Detector tile of the general 3D forward
+    constexpr TileCfg kVoxGeneralTile{32, 32, 1};
+
     // The kernels' column counts: the next of 4, 5, 6 and 8
     inline int kernel_cols(int cols)
     {
@@ -293,6 +296,31 @@ namespace ehp
     {
         const double far = nc / (support * smin) - 1.0, e = far > 1.0 ? far : 1.0;
         return sqrt(e * e + 1.0) * 1.0001 * (n - 1) + 4.0;
+    }
+
+    // What fixes an operator's columns: its footprints' (0: none), its table and its least scaling
+    struct ColumnNeeds {
+        int cols, n_lut;
+        double support, smin;
+    };
+
+    // Entries of the pair table in the reach of a kernel of nc columns (as a number that may be too large)
+    inline double column_table_span(const ColumnNeeds& c, int nc)
+    {
+        return column_table_span(c.n_lut, c.support, c.smin, nc);
+    }
+
+    // Columns of the kernel that takes all of n operators: the widest one's (the further columns of the others
+    // add nothing where their tables reach as far), 0 if one has none or its table would not fit.
+    inline int common_cols(const ColumnNeeds* ops, int n)
+    {
+        int nc = 0;
+        for (int j = 0; j < n; ++j)
+            nc = kernel_cols(ops[j].cols) > nc ? kernel_cols(ops[j].cols) : nc;
+        for (int j = 0; j < n; ++j)
+            if (ops[j].cols <= 0 || !(column_table_span(ops[j], nc) <= kVoxLutSpan))
+                return 0;
+        return nc;
     }
 
     // a / b, correctly rounded, from rb = 1 / b correctly rounded: the quotient estimate with one

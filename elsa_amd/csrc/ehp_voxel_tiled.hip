@@ -563,9 +563,9 @@ namespace ehp
     // plane tables it has to fit 64 KB.
     constexpr size_t kColsLds = 65536 - kPlaneLds;
 
-    size_t cols_lds_bytes(const VoxPlan& plan, const TileCfg& tc)
+    size_t cols_lds_bytes(int nc, int span, const TileCfg& tc)
     {
-        return ((size_t) cols_stride(tc.LA, kernel_cols(plan.cols)) * tc.TB + (size_t) plan.span) * 8;
+        return ((size_t) cols_stride(tc.LA, nc) * tc.TB + (size_t) span) * 8;
     }
 
     int voxel_max_lut()
@@ -593,7 +593,7 @@ namespace ehp
         if (per_xcd * 8 > (int64_t) 0x7fffffff)
             return hipErrorInvalidValue;
         const dim3 grid((unsigned) (per_xcd * 8));
-        const size_t clds = plan.cols > 0 ? cols_lds_bytes(plan, tc) : 0;
+        const size_t clds = plan.cols > 0 ? cols_lds_bytes(kernel_cols(plan.cols), plan.span, tc) : 0;
         if (clds > 0 && clds <= kColsLds) {
             const VoxFan fan{{plan.fan[0], plan.fan[1], plan.fan[2]}};
             auto cols = [&](auto kernel) {
@@ -644,18 +644,22 @@ namespace ehp
                                                             hipStream_t);
 
     // Jobs of a batched voxel forward: one per operator, its tile-pose blocks back to back; the
-    // launch's dynamic LDS is the largest tile's. cols: the columns of the operators' kernel by columns
-    // if they all have one of the same width, else 0 (the general kernel).
+    // launch's dynamic LDS is the largest tile's. cols: the columns of the widest operator's kernel by columns
+    // (the further columns of the others add nothing; their tables reach as far), or 0 where one has none: all
+    // take the general kernel, in its tiles unless the caller chose others. A batch of 96^3 blobs and B-splines,
+    // 90 poses each, us: general kernel in 96 x 16 tiles 5017, in 32 x 32 4172, by columns 2502.
     void voxel_forward_batch_jobs(const VoxBatchItem* items, int n, std::vector<VoxFwdJob>& jobs,
                                   std::vector<int>& blocks, size_t& lds, int& cols)
     {
         jobs.clear();
         blocks.clear();
         lds = 0;
-        cols = n > 0 && items[0].plan.cols > 0 ? kernel_cols(items[0].plan.cols) : 0;
+        std::vector<ColumnNeeds> needs(n);
         for (int j = 0; j < n; ++j)
-            if (items[j].plan.cols <= 0 || kernel_cols(items[j].plan.cols) != cols ||
-                cols_lds_bytes(items[j].plan, items[j].tile) > kColsLds)
+            needs[j] = ColumnNeeds{items[j].plan.cols, items[j].n_lut, items[j].support, items[j].plan.smin};
+        cols = common_cols(needs.data(), n);
+        for (int j = 0; j < n && cols > 0; ++j)
+            if (cols_lds_bytes(cols, (int) column_table_span(needs[j], cols), items[j].tile) > kColsLds)
                 cols = 0;
         for (int j = 0; j < n; ++j) {
             const VoxBatchItem& it = items[j];
@@ -669,8 +673,13 @@ namespace ehp
             J.pose_axis = it.pose_axes;
             J.pose_margin = it.pose_margin;
             J.plan = it.plan;
-            J.TU = it.tile.LA;
-            J.TV = it.dims.dim == 3 ? it.tile.TB : 1;
+            TileCfg tile = it.tile;
+            if (cols > 0)
+                J.plan.span = (int) column_table_span(needs[j], cols);
+            else if (it.dims.dim == 3 && !it.tile_set)
+                tile = kVoxGeneralTile;
+            J.TU = tile.LA;
+            J.TV = it.dims.dim == 3 ? tile.TB : 1;
             J.ntu = (it.dims.det[0] + J.TU - 1) / J.TU;
             const int ntv = (it.dims.det[1] + J.TV - 1) / J.TV;
             J.item = j;
@@ -679,7 +688,7 @@ namespace ehp
             J.block0 = (int64_t) blocks.size();
             blocks.insert(blocks.end(), (size_t) J.ntu * ntv * it.dims.nposes, (int) jobs.size());
             jobs.push_back(J);
-            const size_t need = cols > 0 ? cols_lds_bytes(it.plan, it.tile)
+            const size_t need = cols > 0 ? cols_lds_bytes(cols, J.plan.span, tile)
                                          : (size_t) vox_acc_stride(J.TU, J.TV) * J.TV * sizeof(long long);
             lds = need > lds ? need : lds;
         }

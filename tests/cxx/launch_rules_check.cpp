@@ -2,6 +2,7 @@
 //
 // Built with g++ against the headers that the library's host code uses. Used by tests/test_launch_rules.py.
 #include "ehp_tile_rules.hpp"
+#include "ehp_voxel.hpp"
 
 #include <algorithm>
 
@@ -52,4 +53,19 @@ extern "C" int batch_tile_2d(int n, int64_t total, int set_by_caller)
     const int cus = 256;
     const TileCfg own = joseph_tile2d((int64_t) n * n, cus);
     return batch_tile(own, set_by_caller != 0, joseph_tile2d(total, cus)).LA;
+}
+
+// Columns of the kernel for two voxel projectors in one batch: supports, least and largest scalings, table
+// entries; alone: of the first's own kernel (0: the general one)
+extern "C" int common_columns(const double* support, const double* smin, const double* smax, const int* n_lut,
+                              int* alone)
+{
+    ColumnNeeds c[2];
+    for (int j = 0; j < 2; ++j) {
+        const int cols = footprint_cols(support[j], smax[j]);
+        c[j] = ColumnNeeds{cols <= kVoxMaxCols ? cols : 0, n_lut[j], support[j], smin[j]};
+        if (c[j].cols > 0)
+            alone[j] = kernel_cols(cols);
+    }
+    return common_cols(c, 2);
 }

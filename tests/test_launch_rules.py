@@ -43,3 +43,20 @@ def test_a_tile_that_the_caller_chose_stays_in_a_batch(lib):
     total = ctypes.c_int64(64 * 512 * 512)
     assert lib.batch_tile_2d(64, total, 0) == 32
     assert lib.batch_tile_2d(64, total, 1) == 8
+
+
+@pytest.mark.parametrize("ops,alone,both", [
+    # support, least and largest scaling, table entries of each
+    (((2.0, 1.04, 1.06, 100), (2.0, 1.04, 1.06, 100)), (5, 5), 5),
+    (((2.0, 1.04, 1.06, 100), (1.5, 1.04, 1.06, 100)), (5, 4), 5),
+    (((1.5, 1.04, 1.06, 100), (2.0, 1.4, 1.9, 100)), (4, 8), 8),
+    (((2.0, 1.04, 1.06, 100), (2.0, 1.5, 2.5, 100)), (5, 0), 0),  # a footprint wider than eight
+    (((1.0, 0.9, 1.1, 1000), (2.0, 1.4, 1.9, 100)), (4, 8), 0),  # the first's table would not reach as far
+], ids=str)
+def test_columns_of_a_batch_of_voxel_projectors(lib, ops, alone, both):
+    """Operators of different widths share the widest one's kernel."""
+    f = lambda i, c: (c * 2)(*(op[i] for op in ops))
+    own = (ctypes.c_int * 2)(0, 0)
+    got = lib.common_columns(f(0, ctypes.c_double), f(1, ctypes.c_double), f(2, ctypes.c_double),
+                             f(3, ctypes.c_int), own)
+    assert tuple(own) == alone and got == both
