@@ -3,6 +3,7 @@
 #pragma once
 
 #include "ehp_kernels.hpp"
+#include "ehp_tile_rules.hpp"
 
 namespace ehp
 {
@@ -55,8 +56,8 @@ namespace ehp
         constexpr int TU = (D == 3) ? FwdShape<WU3>::TU : kFwdThreads;
         constexpr int TV = kFwdThreads / TU;
         constexpr int WU = (D == 3) ? WU3 : 64, WV = 64 / WU;
-        const int tu = (int) (id % tiles_u);
         const int64_t bp = id / tiles_u;
+        const int tu = D == 3 ? turned_column(id, bp, tiles_u) : (int) (id - bp * tiles_u);
         pose = (int) (bp % dims.nposes);
         const int band = (int) (bp / dims.nposes);
         const int lane = (int) threadIdx.x % 64, w = (int) threadIdx.x / 64;

@@ -5,6 +5,7 @@
 #include "ehp_voxel.hpp"
 
 #include <algorithm>
+#include <vector>
 
 using namespace ehp;
 
@@ -68,4 +69,23 @@ extern "C" int common_columns(const double* support, const double* smin, const d
             alone[j] = kernel_cols(cols);
     }
     return common_cols(c, 2);
+}
+
+// Whether the columns of `rows` rows of tiles are each taken once, and the most by which the four shader
+// engines' blocks of one column differ in number over the rows (-1: not each taken once)
+extern "C" int column_spread(int tiles_u, int rows)
+{
+    std::vector<int> seen((size_t) tiles_u * rows, 0), engine((size_t) tiles_u * 4, 0);
+    for (int64_t id = 0; id < (int64_t) tiles_u * rows; ++id) {
+        const int c = turned_column(id, id / tiles_u, tiles_u);
+        if (c < 0 || c >= tiles_u || seen[(id / tiles_u) * tiles_u + c]++)
+            return -1;
+        ++engine[c * 4 + id % 4];
+    }
+    int most = 0;
+    for (int c = 0; c < tiles_u; ++c) {
+        const auto e = std::minmax_element(&engine[c * 4], &engine[c * 4] + 4);
+        most = std::max(most, *e.second - *e.first);
+    }
+    return most;
 }

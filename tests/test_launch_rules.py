@@ -60,3 +60,11 @@ def test_columns_of_a_batch_of_voxel_projectors(lib, ops, alone, both):
     got = lib.common_columns(f(0, ctypes.c_double), f(1, ctypes.c_double), f(2, ctypes.c_double),
                              f(3, ctypes.c_int), own)
     assert tuple(own) == alone and got == both
+
+
+@pytest.mark.parametrize("tiles", list(range(1, 26)) + [64, 97])
+def test_columns_of_a_forward_launch(lib, tiles):
+    """Every row takes each of its tiles once, and over many rows the four shader engines take each column
+    equally often (up to the rows of an unfinished turn)."""
+    rows = 4 * tiles * 30
+    assert 0 <= lib.column_spread(tiles, rows) <= 1
