@@ -288,7 +288,8 @@ namespace ehp
         }
 
         // ---- batches: one launch over the jobs of many operators; block b runs block
-        // b - job.block0 of job block_job[b], exactly as the single-operator launch would
+        // b - job.block0 of job block_job[b]; each ray's sum is that of the operator's own launch, whatever
+        // wavefront it lies in
 
         __global__ void __launch_bounds__(256)
             view_copy_batch_kernel(const CopyJob* __restrict__ jobs, const int* __restrict__ block_job,
@@ -320,7 +321,7 @@ namespace ehp
                 fwd2d_block<float>(J.geo, J.dims, J.views, J.parts, 1, J.tiles_u, id - J.block0, sinos + J.sino_off);
             } else {
                 int u, v, pose;
-                if (J.views.pairs) // the wavefronts of the operator's own launch
+                if (J.wu == kFwdWUPairs)
                     fwd_pixel<D, kFwdWUPairs>(J.dims, J.tiles_u, id - J.block0, u, v, pose);
                 else
                     fwd_pixel<D, kFwdWU>(J.dims, J.tiles_u, id - J.block0, u, v, pose);
@@ -453,7 +454,8 @@ namespace ehp
                 if (L.pairs)
                     fj.views.pairs |= 1 << a;
             }
-            const FwdGrid fg = fwd_grid(it.dims, fj.views.pairs ? kFwdWUPairs : kFwdWU);
+            fj.wu = fj.views.pairs && batch_wave_width(it.dims) == kFwdWUPairs ? kFwdWUPairs : kFwdWU;
+            const FwdGrid fg = fwd_grid(it.dims, fj.wu);
             fj.tiles_u = fg.tiles_u;
             fj.parts = it.dims.dim == 2 ? fwd2d_parts(it.dims, sizeof(float)) : 1;
             const int64_t nb = fg.total;

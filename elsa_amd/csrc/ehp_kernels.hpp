@@ -54,6 +54,7 @@ namespace ehp
         Dims dims;
         int tiles_u;
         int parts; // 2D: parts of a ray's span summed apart
+        int wu;    // 3D: wavefront width
         int64_t sino_off;
         int64_t block0;
     };

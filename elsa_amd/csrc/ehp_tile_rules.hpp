@@ -37,6 +37,17 @@ namespace ehp
         return (int) ((id - bp * tiles_u + turn) % tiles_u);
     }
 
+    // Wavefront width (pixels; 64 in all) of an operator's 3D Joseph forward in a batch, from row-pair views: 16 x 4 as
+    // in the operator's own launch, 8 x 8 for volumes below 112 voxels, whose detectors the wider blocks (64 x 4
+    // pixels) overlap by up to a third and whose rays differ more across a wavefront. Batches, us, 8 x 8 / 16 x 4:
+    // four of 64^3 / 64 poses on 95 x 73 90.6 / 94.4, three of 56^3 / 56 on 134 x 64 54.0 / 59.8, three of 72^3 / 48
+    // at magnification 2 183 / 200, three of 96^3 / 72 195 / 198, three of 100^3 / 64 at magnification 2 499 / 515,
+    // two of 112^3 / 48 153 / 143, three of 160^3 / 72 843 / 742.
+    inline int batch_wave_width(const Dims& dims)
+    {
+        return std::max({dims.vol[0], dims.vol[1], dims.vol[2]}) < 112 ? 8 : 16;
+    }
+
     // The tile of one of a batch's operators: the caller's where tile() chose it, else the rule's for the launch
     // over the whole batch.
     inline TileCfg batch_tile(const TileCfg& own, bool set_by_caller, const TileCfg& whole)

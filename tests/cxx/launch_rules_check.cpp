@@ -89,3 +89,14 @@ extern "C" int column_spread(int tiles_u, int rows)
     }
     return most;
 }
+
+// Wavefront width of a batch's 3D Joseph forward over x x y x z voxels
+extern "C" int wave_width(int x, int y, int z)
+{
+    Dims d{};
+    d.dim = 3;
+    d.vol[0] = x;
+    d.vol[1] = y;
+    d.vol[2] = z;
+    return batch_wave_width(d);
+}

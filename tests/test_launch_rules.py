@@ -68,3 +68,10 @@ def test_columns_of_a_forward_launch(lib, tiles):
     equally often (up to the rows of an unfinished turn)."""
     rows = 4 * tiles * 30
     assert 0 <= lib.column_spread(tiles, rows) <= 1
+
+
+@pytest.mark.parametrize("vol,width", [((64, 64, 64), 8), ((1, 1, 1), 8), ((111, 111, 111), 8), ((112, 5, 5), 16),
+                                       ((5, 112, 5), 16), ((5, 5, 300), 16)], ids=str)
+def test_wavefronts_of_a_batch_of_3d_joseph_forwards(lib, vol, width):
+    """Narrow ones for small volumes, which 64-pixel blocks overlap too far."""
+    assert lib.wave_width(*vol) == width
