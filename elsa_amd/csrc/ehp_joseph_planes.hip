@@ -378,7 +378,7 @@ namespace ehp
             if (!(axes_present & (1 << a)))
                 continue;
             const PadLayout& L = layouts[a];
-            vs.v[a] = PadView{views[a], L.PS * es, L.RS * es, L.size};
+            vs.v[a] = PadView{views[a], L.PS * es, L.RS * es, L.size, L.four};
             const int b2 = dims.dim == 3 ? (a == 2 ? 1 : 2) : -1;
             if (L.f == b2)
                 vs.fb2 |= 1 << a;
@@ -447,7 +447,7 @@ namespace ehp
                 const int64_t nb = view_copy_blocks(it.dims, L, cj.gx, cj.gy);
                 cblocks.insert(cblocks.end(), (size_t) nb, (int) cjobs.size());
                 cjobs.push_back(cj);
-                fj.views.v[a] = PadView{it.views[a], L.PS * 4u, L.RS * 4u, L.size};
+                fj.views.v[a] = PadView{it.views[a], L.PS * 4u, L.RS * 4u, L.size, L.four};
                 const int b2 = it.dims.dim == 3 ? (a == 2 ? 1 : 2) : -1;
                 if (L.f == b2)
                     fj.views.fb2 |= 1 << a;

@@ -846,6 +846,10 @@ namespace ehp
     // (m, f), (m + 1, f), (m, f + 1), (m + 1, f + 1), is 16 contiguous bytes (8 in bfloat16): one
     // load instead of two. Each voxel is stored twice (slot 0 of its own row, slot 1 of the row
     // before).
+    // Longest row (bytes) of a 3D view over which plane_span_forward takes four samples at once: flat is for
+    // trajectories whose detector rows each see one slab of the volume (flat_trajectory).
+    constexpr uint32_t kFourSampleRow = 800, kFourSampleRowFlat = 2304;
+
     struct PadLayout {
         int A, m, f;
         int mpad;      // 2 in 3D, 0 in 2D
@@ -853,11 +857,13 @@ namespace ehp
         uint32_t RS;   // row stride in elements ((n_f + 4, rounded up to even) times 1 + pairs)
         uint32_t PS;   // plane stride
         int64_t size;  // elements in the view
+        uint32_t four; // longest row of a view for four samples at once
     };
 
-    inline PadLayout pad_layout(const Dims& dims, int A, int f, bool pairs = false)
+    inline PadLayout pad_layout(const Dims& dims, int A, int f, bool pairs = false, bool flat = true)
     {
         PadLayout L{};
+        L.four = flat ? kFourSampleRowFlat : kFourSampleRow;
         L.A = A;
         L.f = f;
         L.m = 3 - A - f; // in 2D the third axis has one voxel
@@ -901,6 +907,7 @@ namespace ehp
         const void* base;
         uint32_t PS4, RS4;
         int64_t size; // elements in the view (bounds checks of the CPU build)
+        uint32_t four = kFourSampleRowFlat; // longest row for four samples at once
     };
 
 #if defined(EHP_VIEW_CHECK)
@@ -1287,9 +1294,6 @@ namespace ehp
         static constexpr bool value = false;
     };
 
-    // Longest row (bytes) of a 3D view over which plane_span_forward takes four samples at once
-    constexpr uint32_t kFourSampleRow = 2304;
-
     // plane_ray_forward with the plane loop shared by a group of rays of one driving axis and
     // direction (a wavefront, on the GPU): iteration it visits the plane at traversal coordinate
     // t0 + it, the same plane for every ray of the group, so their reads fall on neighbouring
@@ -1367,9 +1371,12 @@ namespace ehp
         // over rows past 2.3 KB, whose planes the caches hold less of, the further loads only displace each
         // other. ms with two / four: 256^3 / 360 poses (rows of 2080 bytes) 5.02 / 4.82, 192^3 / 270 1.64 / 1.62,
         // 384^3 / 200 (3104) 10.7 / 11.0, 512^3 / 180 (4128) 26.6 / 29.2; bfloat16 384^3 / 200 (1552) 9.05 / 8.52,
-        // 512^3 / 120 (2064) 14.2 / 13.0. The rays' common middle holds most samples: pairs of samples
+        // 512^3 / 120 (2064) 14.2 / 13.0. Where a detector row's rays cross the volume's slabs (a tilted trajectory)
+        // the caches hold less of a plane from 0.8 KB on: 90 poses, tilted by up to 46 degrees, 96^3 (800 bytes)
+        // 0.256 / 0.243, 128^3 (1056) 0.679 / 0.690, 192^3 2.19 / 2.78, 256^3 7.5 / 9.4; by up to 86 degrees 128^3
+        // 0.456 / 0.530. The rays' common middle holds most samples: pairs of samples
         // in the masked ends as well took 4.90 at 256^3.
-        if (!F64 && V.RS4 <= kFourSampleRow) {
+        if (!F64 && V.RS4 <= V.four) {
             for (; it + 3 < full1; it += 4, fs += 4.0f, poff += 4u * dp) {
                 SampleTaps T[4];
 #if defined(__HIP_DEVICE_COMPILE__)

@@ -4,6 +4,7 @@
 #include "ehp_joseph_tile.hpp"
 
 #include <algorithm>
+#include <cmath>
 
 namespace ehp
 {
@@ -23,6 +24,26 @@ namespace ehp
     {
         const int t = nvox >= (int64_t) 1024 * cus ? 32 : (nvox >= (int64_t) 256 * cus ? 16 : 8);
         return TileCfg{t, t, 1};
+    }
+
+    // Whether the detector's columns run along one volume axis in every pose (3D), up to 0.02: the rays of a detector
+    // row then stay in one slab of the volume over the whole trajectory.
+    inline bool flat_trajectory(const PoseGeom* poses, int n)
+    {
+        int axis = -1;
+        for (int p = 0; p < n; ++p) {
+            const float* v = poses[p].Pinv + 4; // the ray direction's change from row to row
+            int k = 0;
+            double off = 0.0;
+            for (int i = 1; i < 3; ++i)
+                k = std::fabs(v[i]) > std::fabs(v[k]) ? i : k;
+            for (int i = 0; i < 3; ++i)
+                off += i == k ? 0.0 : (double) v[i] * v[i];
+            if (!(std::sqrt(off) <= 0.02 * std::fabs(v[k])) || (axis >= 0 && k != axis))
+                return false;
+            axis = k;
+        }
+        return true;
     }
 
     // Tile column of block id of a forward launch with tiles_u tiles across, in row bp = id / tiles_u of them. An XCD

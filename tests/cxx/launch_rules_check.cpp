@@ -100,3 +100,12 @@ extern "C" int wave_width(int x, int y, int z)
     d.vol[2] = z;
     return batch_wave_width(d);
 }
+
+// Whether the trajectory of n poses with the inverse projections pinv (3D, column-major 4 x 3) is flat
+extern "C" int is_flat(int n, const float* pinv)
+{
+    std::vector<PoseGeom> g(n);
+    for (int p = 0; p < n; ++p)
+        std::copy(pinv + 12 * p, pinv + 12 * p + 12, g[p].Pinv);
+    return flat_trajectory(g.data(), n);
+}

@@ -2,8 +2,10 @@
 import ctypes
 import os
 
+import numpy as np
 import pytest
 
+from backends import OracleBackend
 from test_tile_logic import ROOT, SFX, _build
 
 SRC = os.path.join(ROOT, "tests", "cxx", "launch_rules_check.cpp")
@@ -75,3 +77,13 @@ def test_columns_of_a_forward_launch(lib, tiles):
 def test_wavefronts_of_a_batch_of_3d_joseph_forwards(lib, vol, width):
     """Narrow ones for small volumes, which 64-pixel blocks overlap too far."""
     assert lib.wave_width(*vol) == width
+
+
+@pytest.mark.parametrize("beta,flat", [(0.0, 1), (0.015, 1), (0.03, 0), (0.8, 0), (np.pi / 2, 0)])
+def test_flat_trajectories(lib, beta, flat):
+    """A circle about y is flat, also slightly tilted; one tilted further, in turn either way, is not."""
+    poses = [dict(s2c=400.0, c2d=100.0, gamma=a, beta=beta * np.sin(2.0 * a)) for a in np.linspace(0.0, 6.0, 25)]
+    g = OracleBackend().setup((40, 50, 60), (70, 60), poses)
+    pinv = np.ascontiguousarray(g.Pinv, np.float32)
+    assert pinv.size == 25 * 12
+    assert lib.is_flat(25, pinv.ctypes.data_as(ctypes.POINTER(ctypes.c_float))) == flat
