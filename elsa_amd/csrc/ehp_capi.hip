@@ -245,52 +245,6 @@ namespace
         return kind == KIND_SIDDON ? ehp::siddon_tile_lds_bytes(dims, tc) : ehp::joseph_tile_lds_bytes(dims, tc);
     }
 
-    // la planes of at most w x w voxels, the widths evened over the volume
-    ehp::TileCfg even_tile(const ehp::Dims& dims, int la, int w)
-    {
-        auto even = [&](int n) { return (n + (n + w - 1) / w - 1) / ((n + w - 1) / w); };
-        return ehp::TileCfg{la, std::max(even(dims.vol[0]), even(dims.vol[1])),
-                            std::max(even(dims.vol[1]), even(dims.vol[2]))};
-    }
-
-    // Tiles of a launch over two driving axes (the first and the last, as about any axis of rotation)
-    int64_t two_axis_tiles(const ehp::Dims& dims, const ehp::TileCfg& tc)
-    {
-        int64_t n = 0;
-        for (int a = 0; a < 3; a += 2) {
-            int nA, nB, nC;
-            ehp::tile_counts(dims, tc, a, nA, nB, nC);
-            n += (int64_t) nA * nB * nC;
-        }
-        return n;
-    }
-
-    // 3D Joseph tiles: eight planes of up to 26 x 26 voxels, the widths evened over the volume (a large
-    // cross-section spends less on the halo and on rays that leave sideways); while a launch of two axes has fewer
-    // than eight such tiles a CU, four planes of 32 x 32, below three a CU of 24 x 24 and 16 x 16, and
-    // below one a CU two planes. Back projections, us (512 threads, both axes in one launch):
-    //   256^3 / 360 poses  8x26x26 8015  4x32x32 7978  8x22x22 8080  8x24x24 8626  8x17x17 8873
-    //   the same at magnification 1.05, after a forward each
-    //                      8x26x26 6833  4x32x32 7133  8x22x22 6850  8x24x24 7493  8x17x17 7706
-    //   192^3 / 270        8x24x24 2558  4x32x32 2715  8x22x22 2839  8x17x17 3045
-    //   128^3 / 180        4x32x32  607  8x16x16  613  4x22x22  635  4x16x16  667
-    //   96^3 / 120         4x24x24  226  8x16x16  236  4x16x16  243  2x16x16  267
-    //   64^3 / 90          4x16x16   81  4x24x24  120  2x16x16  101
-    ehp::TileCfg joseph_tile3d(const ehp::Dims& dims, int cus)
-    {
-        ehp::TileCfg tc = even_tile(dims, 8, 26);
-        if (two_axis_tiles(dims, tc) >= 8 * (int64_t) cus)
-            return tc;
-        for (int w = 32; w >= 16; w -= 8) {
-            tc = even_tile(dims, 4, w);
-            if (two_axis_tiles(dims, tc) >= 3 * (int64_t) cus)
-                break;
-        }
-        if (two_axis_tiles(dims, tc) < cus)
-            tc.LA = 2;
-        return tc;
-    }
-
     // 3D Siddon tiles: eight planes of up to 22 x 22 voxels, evened; of 16 x 16 while a launch of two
     // axes has fewer than eight tiles a CU, and below two a CU fewer planes. Back projections, us:
     //   256^3 / 360 poses  8x22x22 9874  8x24x24 10036  8x16x16 10317  4x32x32 10817
@@ -298,22 +252,22 @@ namespace
     //   50 x 36 x 38 / 62  2x16x16   56  4x16x16    57  8x16x16    77
     ehp::TileCfg siddon_tile3d(const ehp::Dims& dims, int cus)
     {
-        ehp::TileCfg tc = even_tile(dims, 8, 22);
-        if (two_axis_tiles(dims, tc) < 8 * (int64_t) cus)
-            tc = even_tile(dims, 8, 16);
-        while (tc.LA > 2 && two_axis_tiles(dims, tc) < 2 * (int64_t) cus)
+        ehp::TileCfg tc = ehp::even_tile(dims, 8, 22);
+        if (ehp::two_axis_tiles(dims, tc) < 8 * (int64_t) cus)
+            tc = ehp::even_tile(dims, 8, 16);
+        while (tc.LA > 2 && ehp::two_axis_tiles(dims, tc) < 2 * (int64_t) cus)
             tc.LA /= 2;
         return tc;
     }
 
-    // cus: compute units of the device.
+    // axes: the driving axes that occur; cus: compute units of the device.
     // 2D Joseph: squares, the largest of 32, 16 and 8 that give every CU a tile (large tiles spend less on their
     // halo and on rays that only pass a corner; with fewer tiles than CUs the launch waits for its
     // slowest tile): 512^2 / 360 poses 32: 109 us, 16: 123; 256^2 / 180 16: 34, 32: 59, 8: 41;
     // 128^2 / 180 8: 26, 16: 34; 64^2 / 90 8: 19, 16: 24.
     // 2D Siddon, in the same way: 500 x 420 / 500 poses 8 x 32: 177 us, 8 x 16: 230, 4 x 16: 336; 320^2 / 300
     // 92, 89, 120; 256^2 / 180 61, 54, 53.
-    ehp::TileCfg default_tile(int kind, const ehp::Dims& dims, int max_lds, int cus)
+    ehp::TileCfg default_tile(int kind, const ehp::Dims& dims, int axes, int max_lds, int cus)
     {
         ehp::TileCfg tc;
         if (dims.dim == 2 && kind == KIND_JOSEPH)
@@ -323,7 +277,7 @@ namespace
                                                   : (dims.nvox >= 320 * (int64_t) cus ? ehp::TileCfg{8, 16, 1}
                                                                                       : ehp::TileCfg{4, 16, 1});
         else
-            tc = kind == KIND_SIDDON ? siddon_tile3d(dims, cus) : joseph_tile3d(dims, cus);
+            tc = kind == KIND_SIDDON ? siddon_tile3d(dims, cus) : ehp::joseph_tile3d(dims, axes, cus);
         while (tc.LA > 1 && (int) tile_lds_bytes(kind, dims, tc) > max_lds)
             tc.LA /= 2;
         return tc;
@@ -479,7 +433,7 @@ namespace
         int max_lds = 65536;
         if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, op->device) != hipSuccess)
             max_lds = 65536;
-        op->tile = default_tile(KIND_JOSEPH, dm, max_lds, device_cus(op->device));
+        op->tile = default_tile(KIND_JOSEPH, dm, op->axes_present, max_lds, device_cus(op->device));
         op->batch = default_pose_batch(dm);
         op->tiled = true;
         return EHP_OK;
@@ -530,7 +484,7 @@ namespace
         int max_lds = 65536;
         if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, op->device) != hipSuccess)
             max_lds = 65536;
-        op->tile = default_tile(KIND_SIDDON, dm, max_lds, device_cus(op->device));
+        op->tile = default_tile(KIND_SIDDON, dm, op->axes_present, max_lds, device_cus(op->device));
         op->batch = default_pose_batch(dm);
         op->tiled = true;
         return EHP_OK;

@@ -26,6 +26,86 @@ namespace ehp
         return TileCfg{t, t, 1};
     }
 
+    // la planes of at most w x w voxels, the widths evened over the volume
+    inline TileCfg even_tile(const Dims& dims, int la, int w)
+    {
+        auto even = [&](int n) { return (n + (n + w - 1) / w - 1) / ((n + w - 1) / w); };
+        return TileCfg{la, std::max(even(dims.vol[0]), even(dims.vol[1])),
+                            std::max(even(dims.vol[1]), even(dims.vol[2]))};
+    }
+
+    // Tiles of a launch over two driving axes (the first and the last, as about any axis of rotation)
+    inline int64_t two_axis_tiles(const Dims& dims, const TileCfg& tc)
+    {
+        int64_t n = 0;
+        for (int a = 0; a < 3; a += 2) {
+            int nA, nB, nC;
+            tile_counts(dims, tc, a, nA, nB, nC);
+            n += (int64_t) nA * nB * nC;
+        }
+        return n;
+    }
+
+    // Tiles of the smallest launch of a 3D back projection with these driving axes: two run in one launch, one or
+    // three in a launch each
+    inline int64_t least_launch_tiles(const Dims& dims, const TileCfg& tc, int axes)
+    {
+        if (axes == 3 || axes == 5 || axes == 6)
+            return two_axis_tiles(dims, tc);
+        int64_t least = 0;
+        for (int a = 0; a < 3; ++a) {
+            if (!(axes & (1 << a)))
+                continue;
+            int nA, nB, nC;
+            tile_counts(dims, tc, a, nA, nB, nC);
+            const int64_t n = (int64_t) nA * nB * nC;
+            least = least == 0 || n < least ? n : least;
+        }
+        return least;
+    }
+
+    // 3D Joseph tiles: eight planes of up to 26 x 26 voxels, the widths evened over the volume (a large
+    // cross-section spends less on the halo and on rays that leave sideways); while a launch of two axes has fewer
+    // than eight such tiles a CU, four planes of 32 x 32, below three a CU of 24 x 24 and 16 x 16, and
+    // below one a CU two planes. A launch of one axis: either from 15/16 of four a CU, as four workgroups of
+    // 512 threads run on a CU and each launch drains by itself. Back projections, us (512 threads):
+    //   two axes
+    //   256^3 / 360 poses  8x26x26 8015  4x32x32 7978  8x22x22 8080  8x24x24 8626  8x17x17 8873
+    //   the same at magnification 1.05, after a forward each
+    //                      8x26x26 6833  4x32x32 7133  8x22x22 6850  8x24x24 7493  8x17x17 7706
+    //   192^3 / 270        8x24x24 2558  4x32x32 2715  8x22x22 2839  8x17x17 3045
+    //   128^3 / 180        4x32x32  607  8x16x16  613  4x22x22  635  4x16x16  667
+    //   96^3 / 120         4x24x24  226  8x16x16  236  4x16x16  243  2x16x16  267
+    //   64^3 / 90          4x16x16   81  4x24x24  120  2x16x16  101
+    //   three axes, 90 poses
+    //   192^3              8x24x24 4777  4x32x32 5030  8x22x22 5125  4x24x24 4839
+    //   176^3              8x26x26 4231  4x30x30 4538
+    //   160^3              8x23x23 2899  4x32x32 2932  4x23x23 2985  4x16x16 3149
+    //   144^3              4x24x24 2395  4x29x29 2744  4x18x18 2211  8x16x16 2311
+    //   128^3              4x22x22 1691  4x32x32 1840  4x16x16 1641  8x16x16 1760
+    //   112^3              4x16x16 1184  4x28x28 1567  4x23x23 1210  4x19x19 1096
+    //   96^3               4x16x16  854  4x24x24 1054  2x24x24  826
+    //   one axis, 60 poses
+    //   128^3              4x22x22  234  4x32x32  236  4x16x16  214
+    //   112^3              4x16x16  170  4x28x28  187  4x19x19  158
+    inline TileCfg joseph_tile3d(const Dims& dims, int axes, int cus)
+    {
+        const bool pair = axes == 3 || axes == 5 || axes == 6;
+        const int64_t alone = 15 * (int64_t) cus / 4;
+        const int64_t deep = pair ? 8 * (int64_t) cus : alone, enough = pair ? 3 * (int64_t) cus : alone;
+        TileCfg tc = even_tile(dims, 8, 26);
+        if (least_launch_tiles(dims, tc, axes) >= deep)
+            return tc;
+        for (int w = 32; w >= 16; w -= 8) {
+            tc = even_tile(dims, 4, w);
+            if (least_launch_tiles(dims, tc, axes) >= enough)
+                break;
+        }
+        if (least_launch_tiles(dims, tc, axes) < cus)
+            tc.LA = 2;
+        return tc;
+    }
+
     // Whether the detector's columns run along one volume axis in every pose (3D), up to 0.02: the rays of a detector
     // row then stay in one slab of the volume over the whole trajectory.
     inline bool flat_trajectory(const PoseGeom* poses, int n)

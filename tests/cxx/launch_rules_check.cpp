@@ -109,3 +109,13 @@ extern "C" int is_flat(int n, const float* pinv)
         std::copy(pinv + 12 * p, pinv + 12 * p + 12, g[p].Pinv);
     return flat_trajectory(g.data(), n);
 }
+
+// The 3D Joseph back projection's tile of an n^3 volume, as la * 1000 + width, on 256 compute units
+extern "C" int joseph_tile(int n, int axes)
+{
+    Dims d{};
+    d.dim = 3;
+    d.vol[0] = d.vol[1] = d.vol[2] = n;
+    const TileCfg t = joseph_tile3d(d, axes, 256);
+    return t.TB == t.TC ? t.LA * 1000 + t.TB : -1;
+}

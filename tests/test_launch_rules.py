@@ -87,3 +87,12 @@ def test_flat_trajectories(lib, beta, flat):
     pinv = np.ascontiguousarray(g.Pinv, np.float32)
     assert pinv.size == 25 * 12
     assert lib.is_flat(25, pinv.ctypes.data_as(ctypes.POINTER(ctypes.c_float))) == flat
+
+
+@pytest.mark.parametrize("n,two,one", [(256, 8026, 8026), (192, 8024, 8024), (176, 8026, 8026), (160, 4032, 8023), (144, 4029, 4024),
+                                       (128, 4032, 4022), (112, 4028, 4016), (96, 4024, 4016), (64, 4016, 4016),
+                                       (32, 2016, 2016)])
+def test_3d_joseph_tiles(lib, n, two, one):
+    """By the tiles of one launch: two driving axes run in one, one or three axes in a launch each."""
+    assert all(lib.joseph_tile(n, axes) == two for axes in (3, 5, 6))
+    assert all(lib.joseph_tile(n, axes) == one for axes in (1, 2, 4, 7))
