@@ -119,9 +119,13 @@ namespace ehp
     EHP_HD inline int tile_row_slots(int dim, const TileCfg& tc)
     {
         const int odd = (tc.TB + 2) | 1;
-        return dim == 3 && (int64_t) tc.LA * (tc.TC + 2) * odd * 8 + (int64_t) batch_lds_bytes(kMaxPoseBatch) <= 65536
-                   ? odd
-                   : tc.TB + 2;
+#if defined(__HIP_DEVICE_COMPILE__)
+        typedef uint32_t slots_t; // the host has checked that the tile fits the LDS
+#else
+        typedef uint64_t slots_t;
+#endif
+        const slots_t most = (65536 - batch_lds_bytes(kMaxPoseBatch)) / 8;
+        return dim == 3 && (slots_t) tc.LA * (slots_t) (tc.TC + 2) * (slots_t) odd <= most ? odd : tc.TB + 2;
     }
 
     template <int D, int A>
