@@ -33,7 +33,7 @@ struct ehp_batch {
     ehp::SidAdjJob* d_sajobs[3] = {nullptr, nullptr, nullptr};
     // fused voxel passes (the forward's blocks in d_fblocks, its segments over the volumes)
     ehp::VoxFwdJob* d_vfjobs = nullptr;
-    int vox_cols = 0, vox_gather_cols = 0, vox_gather_threads = 256; // the columns of the voxel kernels, 0: the general ones
+    int vox_cols = 0, vox_gather_cols = 0, vox_gather_threads = 256; // the columns of the voxel kernels, 0 (gather: or less): the general ones
     ehp::VoxAdjJob* d_vajobs = nullptr;
     int* d_vablocks = nullptr;
     int64_t nvablocks = 0;

@@ -496,6 +496,8 @@ namespace
     {
         const ehp::Dims& dm = op->dims;
         op->vox = ehp::VoxPlan{};
+        const int cols = ehp::footprint_cols(op->support, smax);
+        op->vox.width = cols;
         if (dm.dim != 3 || dm.nvox >= (1ll << 31) || dm.strides[1] >= (1 << 24) || dm.strides[2] >= (1 << 24) ||
             dm.pix_per_pose >= (1 << 27))
             return;
@@ -505,7 +507,6 @@ namespace
             bits[p] = 1 << axis[p];
             smin = std::min(smin, ehp::voxel_min_scaling(op->host_geo[p], dm));
         }
-        const int cols = ehp::footprint_cols(op->support, smax);
         const double span = op->dtype == EHP_F64 ? op->n_lut + 1.0
                                                  : ehp::column_table_span(op->n_lut, op->support, smin,
                                                                           ehp::kernel_cols(cols));

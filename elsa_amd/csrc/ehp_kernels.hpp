@@ -139,9 +139,11 @@ namespace ehp
 
     // What the 3D voxel kernels know of an operator: the most pixels a footprint is wide (0: the
     // general kernels run), the entries of the forward's table in LDS, and per driving axis the
-    // transverse axis along which the voxels of a plane fan out over a detector row.
+    // transverse axis along which the voxels of a plane fan out over a detector row. width: the most
+    // pixels a footprint is wide, whatever kernels run.
     struct VoxPlan {
         int cols;
+        int width;
         int span;
         double smin; // least footprint scaling
         int fan[3];
@@ -186,7 +188,7 @@ namespace ehp
         int n_lut;
         float support;
         int diff;
-        int parts;
+        int parts, waves; // of a voxel's sum
         int64_t vol_off, sino_off;
         int64_t block0;
     };
@@ -195,7 +197,6 @@ namespace ehp
                                   std::vector<int>& blocks, size_t& lds, int& cols);
     hipError_t voxel_forward_batch(int dim, int cols, const VoxFwdJob* jobs, const int* blocks, int64_t nblocks,
                                    size_t lds, const int* d_fixexp, const float* vols, float* sinos, hipStream_t s);
-    int voxel_gather_parts(const Dims& dims);
     void voxel_gather_batch_jobs(const VoxBatchItem* items, int n, std::vector<VoxAdjJob>& jobs,
                                  std::vector<int>& blocks, size_t& lds, int& cols, int& threads);
     hipError_t voxel_gather_batch(int dim, int cols, const VoxAdjJob* jobs, const int* blocks, int64_t nblocks,

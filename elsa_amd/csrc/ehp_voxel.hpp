@@ -323,6 +323,38 @@ namespace ehp
         return nc;
     }
 
+    // Parts that a voxel's poses are summed in by the gather, added in order (a property of the operator: its launches
+    // alone and in a batch give the same sums): as many (a power of two, at most 16, at least four poses each) as
+    // bring a launch with a wavefront for each part to six wavefronts a SIMD of a device of 1024.
+    inline int gather_part_count(const Dims& dims)
+    {
+        int parts = 1;
+        while (parts < 16 && dims.nvox * parts < (int64_t) 6144 * 64 && dims.nposes >= 8 * parts)
+            parts *= 2;
+        return parts;
+    }
+
+    // Wavefronts that share a voxel's parts: all of them apart, which one sum a voxel would leave most of the
+    // device idle for on small volumes: 92 x 80 blobs, 70 poses 48.3 -> 11.9 us, 300 x 380 / 524 poses 319 -> 147,
+    // 36 x 33 x 40 / 40 poses 125 -> 25. In 3D wide footprints (`width` pixels at most) fill the caches: further
+    // wavefronts, at other poses, displace the detector rows that a wavefront comes back to. Up to four a SIMD past eight
+    // pixels, one and a half from sixteen on. (FP64's divisions weigh more than its loads: blobs 64^3 / 60 poses, width 13
+    // 2782 us with one, 2493 with two wavefronts.) Blobs in FP32, us, with 1 / 2 / 4 / 8 wavefronts:
+    //   width 11  64^3 / 60 poses  883  926 1032 1019   48^3 / 60  542  422  381  386   40^3 / 40  359  199  176  171
+    //   width 25  64^3 / 60       5312 7706    -    -   48^3 / 60 2704 2981 3893 3704   40^3 / 40 1587  922 1146 1270
+    //             33^3 / 50       2603 1467  886  810   24^3 / 24  920  483  341  192
+    inline int gather_waves(const Dims& dims, int width, bool f64)
+    {
+        const int64_t simd = 1024 * 64; // a wavefront each
+        const int parts = gather_part_count(dims);
+        if (f64 || dims.dim == 2 || width <= kVoxMaxCols)
+            return parts;
+        int waves = 1;
+        while (waves < parts && dims.nvox * waves < (width < 16 ? 4 * simd : 3 * simd / 2))
+            waves *= 2;
+        return waves;
+    }
+
     // a / b, correctly rounded, from rb = 1 / b correctly rounded: the quotient estimate with one
     // correction (Markstein, Computation of elementary functions on the IBM RISC System/6000, 1990,
     // theorem on division); b's mantissa is not all ones, quotients far from underflow.

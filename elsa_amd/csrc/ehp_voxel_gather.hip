@@ -14,12 +14,11 @@ namespace ehp
     namespace
     {
         constexpr int kMaxThreads = 1024;
-        constexpr int kMaxParts = 16;
 
-        // Threads of a block: 256, or one wavefront a part
-        int gather_threads(int parts)
+        // Threads of a block: 256, or one wavefront for each of a voxel's
+        int gather_threads(int waves)
         {
-            return parts > 4 ? 64 * parts : 256;
+            return waves > 4 ? 64 * waves : 256;
         }
 
         typedef __amdgpu_buffer_rsrc_t buf_t;
@@ -47,28 +46,16 @@ namespace ehp
         }
     } // namespace
 
-    // Parts a voxel's poses are summed in, each by a wavefront of its own and added in order (a property of
-    // the operator: its launches alone and in a batch give the same sums): as many (a power of two, at
-    // most 16, at least four poses each) as bring the launch to six wavefronts a SIMD of a device of
-    // 1024. One sum a voxel left most of the device idle on small volumes: 92 x 80 blobs,
-    // 70 poses 48.3 -> 11.9 us, 300 x 380 / 524 poses 319 -> 147, 36 x 33 x 40 / 40 poses 125 -> 25.
-    int voxel_gather_parts(const Dims& dims)
+    // The voxels of a block: threads / waves (at least 64), lane t taking parts (t / voxels) * parts / waves onwards of
+    // voxel t % voxels; one part unless MORE. gather(p0, p1, x, y, z): the sum over poses p0 .. p1 - 1, the same in a
+    // wavefront. sums: LDS for the parts of each of the block's voxels (waves > 1). YSLOW: voxels are counted with y
+    // slowest (x fastest, then z), else in the volume's order.
+    template <bool YSLOW, bool MORE, class AT, class ST, class Fn>
+    __device__ __forceinline__ void gather_parts(const Dims& dims, const int parts, const int waves, const int64_t blk,
+                                                 AT* sums, ST* __restrict__ vol, Fn gather)
     {
-        int parts = 1;
-        while (parts < kMaxParts && dims.nvox * parts < (int64_t) 6144 * 64 && dims.nposes >= 8 * parts)
-            parts *= 2;
-        return parts;
-    }
-
-    // The voxels of a block: threads / parts (at least 64), lane t taking part t / voxels of voxel t % voxels.
-    // gather(p0, p1, x, y, z): the sum over poses p0 .. p1 - 1, the same in a wavefront. sums: LDS for a sum
-    // per thread. YSLOW: voxels are counted with y slowest (x fastest, then z), else in the volume's order.
-    template <bool YSLOW, class AT, class ST, class Fn>
-    __device__ __forceinline__ void gather_parts(const Dims& dims, const int parts, const int64_t blk, AT* sums,
-                                                 ST* __restrict__ vol, Fn gather)
-    {
-        const int nv = (int) blockDim.x / parts;
-        const int part = __builtin_amdgcn_readfirstlane((int) threadIdx.x / nv);
+        const int nv = (int) blockDim.x / waves;
+        const int wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x / nv);
         const int64_t vox = blk * nv + (int) threadIdx.x % nv;
         const bool in = vox < dims.nvox;
         int x = 0, y = 0, z = 0;
@@ -82,31 +69,43 @@ namespace ehp
                 y = (int) ((vox / dims.vol[0]) % dims.vol[1]);
                 z = (int) (vox / ((int64_t) dims.vol[0] * dims.vol[1]));
             }
-            acc = gather((int) ((int64_t) dims.nposes * part / parts),
-                         (int) ((int64_t) dims.nposes * (part + 1) / parts), x, y, z);
+            if constexpr (MORE) {
+                const int each = parts / waves;
+                for (int q = wave * each; q < (wave + 1) * each; ++q) {
+                    const AT sum = gather((int) ((int64_t) dims.nposes * q / parts),
+                                          (int) ((int64_t) dims.nposes * (q + 1) / parts), x, y, z);
+                    acc = q == wave * each ? sum : acc + sum;
+                    if (waves > 1)
+                        sums[q * nv + (int) threadIdx.x % nv] = sum;
+                }
+            } else {
+                acc = gather((int) ((int64_t) dims.nposes * wave / parts),
+                             (int) ((int64_t) dims.nposes * (wave + 1) / parts), x, y, z);
+            }
         }
-        if (parts > 1) {
-            sums[threadIdx.x] = acc;
+        if (waves > 1) {
+            if (!MORE)
+                sums[threadIdx.x] = acc;
             __syncthreads();
-            if (part == 0)
-                for (int q = 1; q < parts; ++q)
+            if (wave == 0) // whose own parts are added already
+                for (int q = MORE ? parts / waves : 1; q < parts; ++q)
                     acc = acc + sums[threadIdx.x + q * nv];
         }
-        if (in && part == 0)
+        if (in && wave == 0)
             vol[x + (int64_t) y * dims.strides[1] + (int64_t) z * dims.strides[2]] = down<ST>(acc);
     }
 
     // The general gather, a loop over the clipped rectangle of every footprint. FP32 tables (at most
     // kVoxMaxLut entries) are read as pairs from LDS.
-    template <int D, class ST, class LT, bool YSLOW>
+    template <int D, class ST, class LT, bool YSLOW, bool MORE>
     __device__ __forceinline__ void vox_gather_block(const PoseGeom* __restrict__ geo, const Dims& dims,
                                                      const LT* __restrict__ lut, const int n_lut, const float support,
-                                                     const int diff, const int parts, const int64_t blk,
+                                                     const int diff, const int parts, const int waves, const int64_t blk,
                                                      const ST* __restrict__ sino, ST* __restrict__ vol)
     {
         extern __shared__ long long lds[];
         if constexpr (sizeof(LT) == 8) {
-            gather_parts<YSLOW, double>(dims, parts, blk, reinterpret_cast<double*>(lds), vol, [&](int p0, int p1, int x, int y, int z) {
+            auto gather = [&](int p0, int p1, int x, int y, int z) {
                 double acc = 0.0;
                 for (int p = p0; p < p1; ++p) {
                     Footprint fp;
@@ -117,7 +116,8 @@ namespace ehp
                     });
                 }
                 return acc;
-            });
+            };
+            gather_parts<YSLOW, MORE>(dims, parts, waves, blk, reinterpret_cast<double*>(lds), vol, gather);
         } else {
             float* s_lut = reinterpret_cast<float*>(lds);
             for (int i = threadIdx.x; i < lerp_table_size(n_lut); i += blockDim.x)
@@ -125,7 +125,7 @@ namespace ehp
             __syncthreads();
             const float kidx = (float) (n_lut - 1) / support;
             const bool tail_zero = lut[n_lut - 1] == 0.0f;
-            gather_parts<YSLOW, float>(dims, parts, blk, s_lut + 2 * lerp_table_size(n_lut), vol, [&](int p0, int p1, int x, int y, int z) {
+            auto gather = [&](int p0, int p1, int x, int y, int z) {
                 // a table ending in 0 takes tap_weight_fast's TZ form
                 auto sum = [&](auto tzc) {
                     constexpr bool TZ = decltype(tzc)::value;
@@ -153,7 +153,9 @@ namespace ehp
                     return acc;
                 };
                 return tail_zero ? sum(std::true_type{}) : sum(std::false_type{});
-            });
+            };
+            float* sums = s_lut + 2 * lerp_table_size(n_lut);
+            gather_parts<YSLOW, MORE>(dims, parts, waves, blk, sums, vol, gather);
         }
     }
 
@@ -192,7 +194,7 @@ namespace ehp
         const uint32_t rowb = (uint32_t) dims.det[0] * es;
         typedef typename std::conditional<F64, double, float>::type AT;
         AT* sums = s_lut + (F64 ? n_lut + 1 : 2 * lerp_table_size(n_lut));
-        gather_parts<YSLOW, AT>(dims, parts, blk, sums, vol, [&](const int p0, const int p1, int x, int y, int z) {
+        gather_parts<YSLOW, false, AT>(dims, parts, parts, blk, sums, vol, [&](const int p0, const int p1, int x, int y, int z) {
             auto sum = [&](auto tzc) {
                 constexpr bool TZ = decltype(tzc)::value;
                 AT acc = AT(0);
@@ -256,27 +258,29 @@ namespace ehp
     }
 
     // NC 0: the general gather. DIFF: the phase-contrast projectors' weights (a compile-time flag, so
-    // that the taps of the others carry no select). In 3D the voxels are taken with y slowest and each
+    // that the taps of the others carry no select). split: the parts of a voxel's sum, a wavefront each; MORE: a
+    // wavefront takes more than one (gather_waves), their number is in split's upper bits. In 3D the voxels are taken with y slowest and each
     // XCD gets a contiguous run of blocks (consecutive blocks land on different XCDs): a slab of y, whose
     // detector rows over all poses stay in that XCD's L2 when the trajectory turns about y.
-    template <int D, int NC, class ST, class LT, int DIFF>
+    template <int D, int NC, class ST, class LT, int DIFF, bool MORE = false>
     __global__ void __launch_bounds__(kMaxThreads)
         voxel_gather_kernel(const PoseGeom* __restrict__ geo, const Dims dims, const LT* __restrict__ lut,
-                            const int n_lut, const float support, const int parts, const int per_xcd,
+                            const int n_lut, const float support, const int split, const int per_xcd,
                             const ST* __restrict__ sino, ST* __restrict__ vol)
     {
         const int64_t blk = (int64_t) (blockIdx.x % 8u) * per_xcd + (blockIdx.x / 8u);
-        if (blk * ((int) blockDim.x / parts) >= dims.nvox)
+        const int parts = MORE ? split & 255 : split, waves = MORE ? split >> 8 : split;
+        if (blk * ((int) blockDim.x / waves) >= dims.nvox)
             return; // the whole block
         if constexpr (NC == 0)
-            vox_gather_block<D, ST, LT, D == 3>(geo, dims, lut, n_lut, support, DIFF, parts, blk, sino, vol);
+            vox_gather_block<D, ST, LT, D == 3, MORE>(geo, dims, lut, n_lut, support, DIFF, parts, waves, blk, sino, vol);
         else
             vox_gather_cols_block<NC, ST, LT, DIFF, true>(geo, dims, lut, n_lut, support, DIFF, parts, blk, sino, vol);
     }
 
     // the gathers of many operators in one launch (block b: block b - job.block0 of job block_job[b]);
     // NC: the columns of the widest operator's kernel (a wider kernel's extra columns add nothing), 0: the general one
-    template <int D, int NC>
+    template <int D, int NC, bool MORE = false>
     __global__ void __launch_bounds__(kMaxThreads)
         voxel_gather_batch_kernel(const VoxAdjJob* __restrict__ jobs, const int* __restrict__ block_job,
                                   const float* __restrict__ sinos, float* __restrict__ vols)
@@ -284,7 +288,8 @@ namespace ehp
         const VoxAdjJob& J = jobs[block_job[blockIdx.x]];
         const int64_t blk = (int64_t) blockIdx.x - J.block0;
         if constexpr (NC == 0)
-            vox_gather_block<D, float, float, false>(J.geo, J.dims, J.lut, J.n_lut, J.support, J.diff, J.parts, blk,
+            vox_gather_block<D, float, float, false, MORE>(J.geo, J.dims, J.lut, J.n_lut, J.support, J.diff, J.parts,
+                                                           MORE ? J.waves : J.parts, blk,
                                                      sinos + J.sino_off, vols + J.vol_off);
         else
             vox_gather_cols_block<NC, float, float, 2, false>(J.geo, J.dims, J.lut, J.n_lut, J.support, J.diff,
@@ -293,11 +298,11 @@ namespace ehp
 
     namespace
     {
-        // dynamic LDS: the table and the threads' sums
+        // dynamic LDS: the table and the sums of a block's voxels' parts
         template <class LT>
-        size_t gather_lds(int n_lut, bool cols, int threads)
+        size_t gather_lds(int n_lut, bool cols, int parts, int waves, int threads)
         {
-            const size_t sums = (size_t) threads * sizeof(LT);
+            const size_t sums = waves > 1 ? (size_t) threads / waves * parts * sizeof(LT) : 0;
             if (sizeof(LT) == 8)
                 return (cols ? (size_t) (n_lut + 1) * 8 : 0) + sums;
             return (size_t) lerp_table_size(n_lut) * 8 + sums;
@@ -325,7 +330,7 @@ namespace ehp
         lds = 0;
         threads = 256;
         for (int j = 0; j < n; ++j) {
-            const int t = gather_threads(voxel_gather_parts(items[j].dims));
+            const int t = gather_threads(gather_waves(items[j].dims, items[j].plan.width, false));
             threads = t > threads ? t : threads;
         }
         cols = kVoxMaxCols;
@@ -345,14 +350,17 @@ namespace ehp
             J.n_lut = it.n_lut;
             J.support = it.support;
             J.diff = it.diff;
-            J.parts = voxel_gather_parts(it.dims);
+            J.parts = gather_part_count(it.dims);
+            J.waves = gather_waves(it.dims, it.plan.width, false);
             J.vol_off = it.vol_off;
             J.sino_off = it.sino_off;
             J.block0 = (int64_t) blocks.size();
-            const int nv = threads / J.parts;
+            const int nv = threads / J.waves;
             blocks.insert(blocks.end(), (size_t) ((it.dims.nvox + nv - 1) / nv), (int) jobs.size());
             jobs.push_back(J);
-            const size_t need = gather_lds<float>(it.n_lut, cols > 0, threads);
+            if (J.waves < J.parts)
+                cols = -1; // the general kernel in any case: its footprints are too wide for columns
+            const size_t need = gather_lds<float>(it.n_lut, cols > 0, J.parts, J.waves, threads);
             lds = need > lds ? need : lds;
         }
     }
@@ -369,6 +377,8 @@ namespace ehp
         };
         if (dim == 2)
             launch(voxel_gather_batch_kernel<2, 0>);
+        else if (cols < 0)
+            launch(voxel_gather_batch_kernel<3, 0, true>);
         else
             with_columns(cols, [&](auto nc) { launch(voxel_gather_batch_kernel<3, decltype(nc)::value>); });
         return hipGetLastError();
@@ -380,24 +390,31 @@ namespace ehp
     {
         if (n_lut < 2 || n_lut > kVoxMaxLut)
             return hipErrorInvalidValue;
-        const int parts = voxel_gather_parts(dims);
-        const int threads = gather_threads(parts), nv = threads / parts;
+        const int parts = gather_part_count(dims), waves = gather_waves(dims, plan.width, sizeof(LT) == 8);
+        const int threads = gather_threads(waves), nv = threads / waves;
         const int64_t per_xcd = ((dims.nvox + nv - 1) / nv + 7) / 8;
         if (per_xcd * 8 > (int64_t) 0x7fffffff)
             return hipErrorInvalidValue;
         const dim3 grid((unsigned) (per_xcd * 8));
-        const size_t lds = gather_lds<LT>(n_lut, plan.cols > 0, parts > 1 ? threads : 0);
+        const int split = waves < parts ? waves << 8 | parts : parts;
+        const size_t lds = gather_lds<LT>(n_lut, plan.cols > 0, parts, waves, threads);
         auto launch = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, grid, dim3((unsigned) threads), lds, s, geo, dims, lut, n_lut, support, parts,
+            hipLaunchKernelGGL(kernel, grid, dim3((unsigned) threads), lds, s, geo, dims, lut, n_lut, support, split,
                                (int) per_xcd, sino, vol);
         };
-        if (dims.dim == 2)
+        if (dims.dim == 2) {
             diff ? launch(voxel_gather_kernel<2, 0, ST, LT, 1>) : launch(voxel_gather_kernel<2, 0, ST, LT, 0>);
-        else
-            with_columns(plan.cols, [&](auto nc) {
-                constexpr int NC = decltype(nc)::value;
-                diff ? launch(voxel_gather_kernel<3, NC, ST, LT, 1>) : launch(voxel_gather_kernel<3, NC, ST, LT, 0>);
-            });
+            return hipGetLastError();
+        }
+        if constexpr (sizeof(LT) == 4)
+            if (waves < parts) { // footprints too wide for columns
+                diff ? launch(voxel_gather_kernel<3, 0, ST, LT, 1, true>) : launch(voxel_gather_kernel<3, 0, ST, LT, 0, true>);
+                return hipGetLastError();
+            }
+        with_columns(plan.cols, [&](auto nc) {
+            constexpr int NC = decltype(nc)::value;
+            diff ? launch(voxel_gather_kernel<3, NC, ST, LT, 1>) : launch(voxel_gather_kernel<3, NC, ST, LT, 0>);
+        });
         return hipGetLastError();
     }
 

@@ -119,3 +119,13 @@ extern "C" int joseph_tile(int n, int axes)
     const TileCfg t = joseph_tile3d(d, axes, 256);
     return t.TB == t.TC ? t.LA * 1000 + t.TB : -1;
 }
+
+// Parts of the voxel gather's sums and the wavefronts that share them, as parts * 100 + waves
+extern "C" int gather_split(int dim, int64_t nvox, int poses, int width, int f64)
+{
+    Dims d{};
+    d.dim = dim;
+    d.nvox = nvox;
+    d.nposes = poses;
+    return gather_part_count(d) * 100 + gather_waves(d, width, f64 != 0);
+}
