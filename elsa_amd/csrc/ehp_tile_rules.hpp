@@ -9,10 +9,14 @@
 namespace ehp
 {
     // Tiles of the 2D voxel forward: up to 256 pixels, narrower ones (down to 16, widths evened) until a
-    // launch over `poses` poses has four blocks a CU. Blobs, us: 92 x 80 / 70 poses 16: 26.7, 256: 41; 150^2 in
-    // FP64 / 150 32: 101, 256: 154; 256^2 / 180 64: 125, 256: 206; 300 x 380 / 524 256: 322, 64: 431.
+    // launch over `poses` poses has four blocks a CU; a detector that fits one tile is left whole from three and a
+    // half. Blobs, us: 92 x 80 / 70 poses 16: 26.7, 256: 41; 150^2 in FP64 / 150 32: 101, 256: 154; 256^2 / 180
+    // 64: 125, 256: 206; 300 x 380 / 524 256: 322, 64: 431; 128^2 on 190 / 960 190: 84, 95: 90; 64^2 on 95 / 960 95: 31,
+    // 48: 38; 128^2 on 190 / 480 95: 55, 190: 69.
     inline TileCfg voxel_tile2d(int det, int64_t poses, int cus)
     {
+        if (det <= 256 && 2 * poses >= 7 * (int64_t) cus)
+            return TileCfg{det, 1, 1};
         const int64_t most = (det + 15) / 16, want = (4 * (int64_t) cus + poses - 1) / poses;
         const int nt = (int) std::max<int64_t>((det + 255) / 256, std::min(most, want));
         return TileCfg{(det + nt - 1) / nt, 1, 1};

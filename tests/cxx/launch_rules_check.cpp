@@ -129,3 +129,9 @@ extern "C" int gather_split(int dim, int64_t nvox, int poses, int width, int f64
     d.nposes = poses;
     return gather_part_count(d) * 100 + gather_waves(d, width, f64 != 0);
 }
+
+// Width of the 2D voxel forward's tiles on 256 compute units
+extern "C" int voxel_tile(int det, int64_t poses)
+{
+    return voxel_tile2d(det, poses, 256).LA;
+}

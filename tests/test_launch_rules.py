@@ -108,3 +108,11 @@ def test_parts_of_the_voxel_gather(lib, dim, n, poses, width, parts, waves):
     pixels the caches hold for few poses at once."""
     assert lib.gather_split(dim, ctypes.c_int64(n ** dim), poses, width, 0) == parts * 100 + waves
     assert lib.gather_split(dim, ctypes.c_int64(n ** dim), poses, width, 1) == parts * 101
+
+
+@pytest.mark.parametrize("det,poses,width", [(190, 960, 190), (95, 960, 95), (256, 896, 256), (190, 895, 95),
+                                             (257, 960, 129), (190, 480, 64), (1, 1, 1), (1, 5000, 1), (381, 180, 64),
+                                             (763, 360, 255), (300, 5000, 150)])
+def test_2d_voxel_forward_tiles(lib, det, poses, width):
+    """A detector that fits one tile is left whole while the launch has three and a half blocks a CU."""
+    assert lib.voxel_tile(det, ctypes.c_int64(poses)) == width
