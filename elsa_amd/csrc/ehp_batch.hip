@@ -117,10 +117,9 @@ namespace
             }
             it.dims = op->dims;
             // 2D Joseph tiles that no caller chose follow the whole batch's size
-            // (64 problems of 128^2..512^2: 1129 us a pass with 32 x 32 tiles, 1446 with 16 x 16)
             it.tile = op->tile;
             if (b->kind == KIND_JOSEPH && b->dim == 2)
-                it.tile = ehp::batch_tile(op->tile, op->tile_set, ehp::joseph_tile2d(b->vol_off.back(), cus));
+                it.tile = ehp::batch_tile(op->tile, op->tile_set, ehp::joseph_batch_tile2d(b->vol_off.back(), cus));
             it.axes_present = op->axes_present;
             it.batch = op->batch;
             it.vol_off = b->vol_off[j];

@@ -22,11 +22,21 @@ namespace ehp
         return TileCfg{(det + nt - 1) / nt, 1, 1};
     }
 
-    // Tiles of the 2D Joseph back projection for a launch over nvox voxels (one problem's, or all of a batch's) on
-    // a device of cus compute units
+    // Tiles of an operator's 2D Joseph back projection over nvox voxels on a device of cus compute units
     inline TileCfg joseph_tile2d(int64_t nvox, int cus)
     {
         const int t = nvox >= (int64_t) 1024 * cus ? 32 : (nvox >= (int64_t) 256 * cus ? 16 : 8);
+        return TileCfg{t, t, 1};
+    }
+
+    // Tiles of a batch's over nvox voxels in all, whose workgroups have 256 threads (an operator's few tiles have 1024):
+    // smaller ones for longer, as a CU needs several. Back projections, us, with 8 / 16 / 32: 64 problems of 32^2 /
+    // 48 poses (256 voxels a CU) 22 / 31 / 60, 16 of 64^2 / 90 (256) 29 / 40 / 82, 24 of 100^2 / 100 (937) 66 / 50 / 91, 16 of
+    // 128^2 / 180 (1024) 109 / 71 / 148 and at magnification 3 304 / 283 / 406, 32 of them (2048) 202 / 125 / 156, 64 (4096)
+    // 376 / 200 / 195; 64 of 128^2 .. 512^2 16: 1446, 32: 1129.
+    inline TileCfg joseph_batch_tile2d(int64_t nvox, int cus)
+    {
+        const int t = nvox >= (int64_t) 4096 * cus ? 32 : (nvox >= (int64_t) 512 * cus ? 16 : 8);
         return TileCfg{t, t, 1};
     }
 

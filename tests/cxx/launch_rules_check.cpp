@@ -53,7 +53,7 @@ extern "C" int batch_tile_2d(int n, int64_t total, int set_by_caller)
 {
     const int cus = 256;
     const TileCfg own = joseph_tile2d((int64_t) n * n, cus);
-    return batch_tile(own, set_by_caller != 0, joseph_tile2d(total, cus)).LA;
+    return batch_tile(own, set_by_caller != 0, joseph_batch_tile2d(total, cus)).LA;
 }
 
 // Columns of the kernel for two voxel projectors in one batch: supports, least and largest scalings, table

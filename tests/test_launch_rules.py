@@ -116,3 +116,10 @@ def test_parts_of_the_voxel_gather(lib, dim, n, poses, width, parts, waves):
 def test_2d_voxel_forward_tiles(lib, det, poses, width):
     """A detector that fits one tile is left whole while the launch has three and a half blocks a CU."""
     assert lib.voxel_tile(det, ctypes.c_int64(poses)) == width
+
+
+@pytest.mark.parametrize("problems,n,side", [(64, 32, 8), (16, 64, 8), (32, 64, 16), (24, 100, 16), (16, 128, 16),
+                                             (32, 128, 16), (63, 128, 16), (64, 128, 32), (64, 512, 32)])
+def test_2d_joseph_tiles_of_a_batch(lib, problems, n, side):
+    """Several tiles a compute unit before they grow."""
+    assert lib.batch_tile_2d(n, ctypes.c_int64(problems * n * n), 0) == side
