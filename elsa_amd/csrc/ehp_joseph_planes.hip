@@ -104,7 +104,7 @@ namespace ehp
         }
 
         // The rays of group K = 2 * axis + direction of a wavefront share one plane loop over the
-        // group's span, or over parts seg, seg + par, ... of the nseg equal parts of it, the parts summed
+        // group's span, in 2D over parts seg, seg + par, ... of the nseg equal parts of it, the parts summed
         // apart and then in order. Called with every lane active; `keys` holds the groups present.
         template <int D, int K, bool V16, bool F64>
         __device__ __forceinline__ void fwd_group(int keys, int key, const RayRec& r, const Dims& dims,
@@ -122,6 +122,10 @@ namespace ehp
             const int niter = t1 - t0 + 1;
             if (!mine)
                 return;
+            if constexpr (D == 3) { // one part
+                val = fwd_span<D, K / 2, (K & 1) != 0, V16, F64>(r, dims, vs, t0, niter, s0 + t0 - tfirst, full0, full1);
+                return;
+            }
             for (int g = seg; g < nseg; g += par) {
                 const int i0 = niter * g / nseg, i1 = niter * (g + 1) / nseg; // iterations [i0, i1) of the span
                 if (i0 == i1)
