@@ -541,23 +541,6 @@ namespace ehp
         return c[0] * dims.strides[0] + c[1] * dims.strides[1] + c[2] * dims.strides[2];
     }
 
-    // Poses whose candidate rays one workgroup gathers between two barriers (at most
-    // kMaxPoseBatch).
-    // Pose j of candidate k of a pose batch: the largest j with pref[j] <= k (pref is the
-    // prefix sum of the batch's per-pose candidate counts, pref[0] = 0, k < pref[batch]).
-    EHP_HD inline int batch_pose_slot(const int* pref, int batch, int k)
-    {
-        int lo = 0, hi = batch - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (pref[mid] <= k)
-                lo = mid;
-            else
-                hi = mid - 1;
-        }
-        return lo;
-    }
-
     // Candidate rectangle of one pose of a batch in the tiled back projections: rnu = 1 / width,
     // nu = width, base = ray index of its first pixel.
     struct CandRect {
@@ -803,28 +786,6 @@ namespace ehp
     {
         return fixed_point_exponent((double) maxabs, bound);
     }
-
-    // Per-ray scale of the contributions: with |yl| < 2^er (er raised to at least eg - 32),
-    // ys = yl * 2^(30 - er), so every contribution ys * w (w <= 1) truncates to an int32 of
-    // magnitude at most 2^30, and shifting it left by sh = er - eg + 32 (0..32) puts it in units
-    // of q. The truncation error of a contribution is below 2^(er - 30), at most 2^-29 |yl|
-    // (2^-30 of the bound 2^er): far below an FP32 rounding of the sums it enters.
-    EHP_HD inline void ray_scale(float yl, int eg, float& ys, int& sh)
-    {
-        int er;
-        frexpf(yl, &er);
-        er = er < eg - 32 ? eg - 32 : er;
-        ys = ldexpf(yl, 30 - er);
-        sh = er - eg + 32;
-    }
-
-    // The 64-bit fixed-point value of one contribution.
-    // Truncation (one conversion instruction) rather than rounding to nearest (two).
-    EHP_HD inline unsigned long long fixed_contrib(float t, int sh)
-    {
-        return (unsigned long long) (long long) (int) t << sh;
-    }
-
 
     inline void tile_counts(const Dims& dims, const TileCfg& tc, int a, int& ntA, int& ntB, int& ntC)
     {

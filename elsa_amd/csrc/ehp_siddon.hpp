@@ -151,7 +151,8 @@ namespace ehp
         }
     }
 
-    // A Siddon traversal that can pause between the planes of one axis: the state of
+    // The traversal plane by plane in single steps, which the CPU checks of the views run; the kernels form a
+    // plane's segments by sorting (sid_plane_segments). It can pause between the planes of one axis: the state of
     // siddon_traverse after some of its steps (voxel, step direction and count per axis as a
     // float -- exact, as counts stay below 2^24 -- next crossing per axis, the last crossing).
     struct SidWalk {
@@ -673,8 +674,8 @@ namespace ehp
         }
     }
 
-    // Slot of voxel c in a tile of the Siddon back projection (no halo: the tile's own voxels,
-    // b1 fastest, then b2, then the driving axis).
+    // Slot of voxel c in a tile of the Siddon back projection with unpadded rows (no halo: the tile's own voxels,
+    // b1 fastest, then b2, then the driving axis), for the CPU checks; the kernels' rows are sid_row_slots long.
     template <int D, int A>
     EHP_HD inline int sid_slot(const TileBox& t, const TileCfg& tc, int c0, int c1, int c2)
     {
