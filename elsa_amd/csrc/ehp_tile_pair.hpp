@@ -2,6 +2,7 @@
 #pragma once
 
 #include "ehp_kernels.hpp"
+#include "ehp_tile_rules.hpp"
 
 #include <type_traits>
 
@@ -40,11 +41,6 @@ namespace ehp
         int64_t total;
         int per_xcd;
     };
-
-    inline bool two_axes(int axes)
-    {
-        return axes == 3 || axes == 5 || axes == 6;
-    }
 
     // fn(first, second) of two of three axes, as constants
     template <class Fn>

@@ -60,11 +60,30 @@ namespace ehp
         return n;
     }
 
+    inline bool two_axes(int axes)
+    {
+        return axes == 3 || axes == 5 || axes == 6;
+    }
+
+    // Whether the tiles of two driving axes run in one launch, over nvox voxels and `poses` poses. One launch waits
+    // for its slowest tiles once, which grows with the poses; but both axes' tiles then exchange their sums with the
+    // volume by atomics (add_second), about 25 ps a voxel more than reading and writing it. Joseph, us, one launch / two:
+    //   64^3    4 poses   29 / 30    48 poses   71 / 93           128^3   4 poses  125 /  74    24 poses  215 / 194
+    //   96^3    4 poses   64 / 48    12 poses   77 / 76           128^3  48 poses  335 / 332   150 poses  840 / 935
+    //   96^3   24 poses  106 / 122                                256^3  12 poses  993 / 628    48 poses 2154 / 2142
+    //   184^3  12 poses  399 / 265   72 poses 1251 / 1255         256^3 150 poses 6292 / 6523
+    // and Siddon much alike (128^3: 24 poses 218 / 212, 48 poses 362 / 372; 2D 1024^2: 12 poses 59 / 48, 24 75 / 76).
+    inline bool pair_launch(int axes, int64_t nvox, int64_t poses)
+    {
+        const int64_t small = 1 << 18, large = 1 << 21, most = 48; // 64^3: any number of poses, 128^3 and up: most
+        return two_axes(axes) && (poses >= most || poses * (large - small) >= most * (nvox - small));
+    }
+
     // Tiles of the smallest launch of a 3D back projection with these driving axes: two run in one launch, one or
     // three in a launch each
     inline int64_t least_launch_tiles(const Dims& dims, const TileCfg& tc, int axes)
     {
-        if (axes == 3 || axes == 5 || axes == 6)
+        if (two_axes(axes))
             return two_axis_tiles(dims, tc);
         int64_t least = 0;
         for (int a = 0; a < 3; ++a) {
@@ -104,7 +123,7 @@ namespace ehp
     //   112^3              4x16x16  170  4x28x28  187  4x19x19  158
     inline TileCfg joseph_tile3d(const Dims& dims, int axes, int cus)
     {
-        const bool pair = axes == 3 || axes == 5 || axes == 6;
+        const bool pair = two_axes(axes);
         const int64_t alone = 15 * (int64_t) cus / 4;
         const int64_t deep = pair ? 8 * (int64_t) cus : alone, enough = pair ? 3 * (int64_t) cus : alone;
         TileCfg tc = even_tile(dims, 8, 26);

@@ -135,3 +135,9 @@ extern "C" int voxel_tile(int det, int64_t poses)
 {
     return voxel_tile2d(det, poses, 256).LA;
 }
+
+// Whether the back projection of these driving axes runs the tiles of both in one launch
+extern "C" int one_launch(int axes, int64_t nvox, int64_t poses)
+{
+    return pair_launch(axes, nvox, poses);
+}

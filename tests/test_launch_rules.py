@@ -123,3 +123,14 @@ def test_2d_voxel_forward_tiles(lib, det, poses, width):
 def test_2d_joseph_tiles_of_a_batch(lib, problems, n, side):
     """Several tiles a compute unit before they grow."""
     assert lib.batch_tile_2d(n, ctypes.c_int64(problems * n * n), 0) == side
+
+
+@pytest.mark.parametrize("n,least", [(1, 0), (64, 0), (96, 17), (128, 48), (256, 48), (1000, 48)])
+def test_two_axes_in_one_launch(lib, n, least):
+    """From as many poses as pay for the atomics; one or three axes never."""
+    nvox = ctypes.c_int64(n ** 3)
+    for axes in (3, 5, 6):
+        assert lib.one_launch(axes, nvox, ctypes.c_int64(max(least, 1)))
+        assert least == 0 or not lib.one_launch(axes, nvox, ctypes.c_int64(least - 1))
+    for axes in (0, 1, 2, 4, 7):
+        assert not lib.one_launch(axes, nvox, ctypes.c_int64(1000))
