@@ -340,9 +340,9 @@ namespace
             if ((op->axes_present & (1 << a)) && ehp::pad_layout(dm, a, fan_axis(op, h, a), true).size >= max_elems)
                 pairs = false;
         bool planes = true;
-        const bool flat = dm.dim == 3 && ehp::flat_trajectory(op->host_geo.data(), dm.nposes);
+        const double tilt = dm.dim == 3 ? ehp::trajectory_tilt(op->host_geo.data(), dm.nposes) : 0.0;
         for (int a = 0; a < dm.dim; ++a) {
-            op->layouts[a] = ehp::pad_layout(dm, a, fan_axis(op, h, a), pairs, flat);
+            op->layouts[a] = ehp::pad_layout(dm, a, fan_axis(op, h, a), pairs, tilt);
             if ((op->axes_present & (1 << a)) && op->layouts[a].size >= max_elems)
                 planes = false;
         }

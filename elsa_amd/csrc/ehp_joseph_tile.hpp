@@ -811,9 +811,14 @@ namespace ehp
     // (m, f), (m + 1, f), (m, f + 1), (m + 1, f + 1), is 16 contiguous bytes (8 in bfloat16): one
     // load instead of two. Each voxel is stored twice (slot 0 of its own row, slot 1 of the row
     // before).
-    // Longest row (bytes) of a 3D view over which plane_span_forward takes four samples at once: flat is for
-    // trajectories whose detector rows each see one slab of the volume (flat_trajectory).
-    constexpr uint32_t kFourSampleRow = 800, kFourSampleRowFlat = 2304;
+    // Longest row (bytes) of a 3D view over which plane_span_forward takes four samples at once, by the trajectory's
+    // tilt (trajectory_tilt): up to 0.02 each detector row sees one slab of the volume.
+    constexpr uint32_t kFourSampleRowFlat = 2304;
+
+    inline uint32_t four_sample_row(double tilt)
+    {
+        return tilt <= 0.02 ? kFourSampleRowFlat : (tilt <= 0.35 ? 1312u : 800u);
+    }
 
     struct PadLayout {
         int A, m, f;
@@ -825,10 +830,10 @@ namespace ehp
         uint32_t four; // longest row of a view for four samples at once
     };
 
-    inline PadLayout pad_layout(const Dims& dims, int A, int f, bool pairs = false, bool flat = true)
+    inline PadLayout pad_layout(const Dims& dims, int A, int f, bool pairs = false, double tilt = 0.0)
     {
         PadLayout L{};
-        L.four = flat ? kFourSampleRowFlat : kFourSampleRow;
+        L.four = four_sample_row(tilt);
         L.A = A;
         L.f = f;
         L.m = 3 - A - f; // in 2D the third axis has one voxel
@@ -1337,10 +1342,10 @@ namespace ehp
         // other. ms with two / four: 256^3 / 360 poses (rows of 2080 bytes) 5.02 / 4.82, 192^3 / 270 1.64 / 1.62,
         // 384^3 / 200 (3104) 10.7 / 11.0, 512^3 / 180 (4128) 26.6 / 29.2; bfloat16 384^3 / 200 (1552) 9.05 / 8.52,
         // 512^3 / 120 (2064) 14.2 / 13.0. Where a detector row's rays cross the volume's slabs (a tilted trajectory)
-        // the caches hold less of a plane from 0.8 KB on: 90 poses, tilted by up to 46 degrees, 96^3 (800 bytes)
-        // 0.256 / 0.243, 128^3 (1056) 0.679 / 0.690, 192^3 2.19 / 2.78, 256^3 7.5 / 9.4; by up to 86 degrees 128^3
-        // 0.456 / 0.530. The rays' common middle holds most samples: pairs of samples
-        // in the masked ends as well took 4.90 at 256^3.
+        // the caches hold less of a plane: 90 poses, tilted by up to 17 degrees, 128^3 (1056 bytes) 0.371 / 0.345, 160^3
+        // (1312) 0.677 / 0.661, 192^3 (1568) 1.14 / 1.20, 224^3 1.83 / 2.20; by up to 46 degrees 96^3 (800) 0.256 / 0.243,
+        // 128^3 0.679 / 0.690, 192^3 2.19 / 2.78, 256^3 7.5 / 9.4; by up to 86 degrees 128^3 0.456 / 0.530. The rays'
+        // common middle holds most samples: pairs of samples in the masked ends as well took 4.90 at 256^3.
         if (!F64 && V.RS4 <= V.four) {
             for (; it + 3 < full1; it += 4, fs += 4.0f, poff += 4u * dp) {
                 SampleTaps T[4];

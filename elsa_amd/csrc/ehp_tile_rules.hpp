@@ -139,11 +139,13 @@ namespace ehp
         return tc;
     }
 
-    // Whether the detector's columns run along one volume axis in every pose (3D), up to 0.02: the rays of a detector
-    // row then stay in one slab of the volume over the whole trajectory.
-    inline bool flat_trajectory(const PoseGeom* poses, int n)
+    // How far the detector's columns are off one volume axis over the trajectory (3D): the largest tangent of a pose's
+    // angle to the axis nearest to it, 1e30 if that is not the same axis in all. Near 0 the rays of a detector row stay
+    // in one slab of the volume.
+    inline double trajectory_tilt(const PoseGeom* poses, int n)
     {
         int axis = -1;
+        double most = 0.0;
         for (int p = 0; p < n; ++p) {
             const float* v = poses[p].Pinv + 4; // the ray direction's change from row to row
             int k = 0;
@@ -152,11 +154,12 @@ namespace ehp
                 k = std::fabs(v[i]) > std::fabs(v[k]) ? i : k;
             for (int i = 0; i < 3; ++i)
                 off += i == k ? 0.0 : (double) v[i] * v[i];
-            if (!(std::sqrt(off) <= 0.02 * std::fabs(v[k])) || (axis >= 0 && k != axis))
-                return false;
+            if (!(std::fabs(v[k]) > 0.0f) || (axis >= 0 && k != axis))
+                return 1.0e30;
+            most = std::max(most, std::sqrt(off) / std::fabs(v[k]));
             axis = k;
         }
-        return true;
+        return most;
     }
 
     // Tile column of block id of a forward launch with tiles_u tiles across, in row bp = id / tiles_u of them. An XCD

@@ -101,13 +101,13 @@ extern "C" int wave_width(int x, int y, int z)
     return batch_wave_width(d);
 }
 
-// Whether the trajectory of n poses with the inverse projections pinv (3D, column-major 4 x 3) is flat
-extern "C" int is_flat(int n, const float* pinv)
+// The longest view row for four samples at once over n poses with the inverse projections pinv (3D, column-major 4 x 3)
+extern "C" int four_samples_up_to(int n, const float* pinv)
 {
     std::vector<PoseGeom> g(n);
     for (int p = 0; p < n; ++p)
         std::copy(pinv + 12 * p, pinv + 12 * p + 12, g[p].Pinv);
-    return flat_trajectory(g.data(), n);
+    return (int) four_sample_row(trajectory_tilt(g.data(), n));
 }
 
 // The 3D Joseph back projection's tile of an n^3 volume, as la * 1000 + width, on 256 compute units

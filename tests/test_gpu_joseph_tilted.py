@@ -1,5 +1,5 @@
-"""3D Joseph forwards over tilted trajectories, whose views take four samples at once over rows of up to 800 bytes
-and two over longer ones, against the oracle; spans that leave one to three samples over."""
+"""3D Joseph forwards over tilted trajectories, whose views take four samples at once over rows of up to 800 or 1312
+bytes and two over longer ones, against the oracle; spans that leave one to three samples over."""
 import numpy as np
 import pytest
 
@@ -9,7 +9,7 @@ from fp32_bounds import check_forward
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("vol", [(95, 6, 37), (96, 5, 9), (97, 5, 9), (9, 4, 130), (3, 110, 2)], ids=str)
+@pytest.mark.parametrize("vol", [(95, 6, 37), (96, 5, 9), (97, 5, 9), (9, 4, 130), (3, 110, 2), (160, 4, 7), (5, 3, 161)], ids=str)
 @pytest.mark.parametrize("beta", [0.3, 1.5])
 def test_forward_of_tilted_trajectories(vol, beta):
     import elsa_amd as E

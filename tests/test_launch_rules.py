@@ -79,14 +79,16 @@ def test_wavefronts_of_a_batch_of_3d_joseph_forwards(lib, vol, width):
     assert lib.wave_width(*vol) == width
 
 
-@pytest.mark.parametrize("beta,flat", [(0.0, 1), (0.015, 1), (0.03, 0), (0.8, 0), (np.pi / 2, 0)])
-def test_flat_trajectories(lib, beta, flat):
-    """A circle about y is flat, also slightly tilted; one tilted further, in turn either way, is not."""
+@pytest.mark.parametrize("beta,row", [(0.0, 2304), (0.015, 2304), (0.03, 1312), (0.3, 1312), (0.4, 800), (0.8, 800),
+                                      (np.pi / 2, 800)])
+def test_rows_for_four_samples(lib, beta, row):
+    """A circle about y takes four over long rows, also slightly tilted; one tilted further, in turn either way, does
+    not, and one whose detector columns turn from axis to axis least."""
     poses = [dict(s2c=400.0, c2d=100.0, gamma=a, beta=beta * np.sin(2.0 * a)) for a in np.linspace(0.0, 6.0, 25)]
     g = OracleBackend().setup((40, 50, 60), (70, 60), poses)
     pinv = np.ascontiguousarray(g.Pinv, np.float32)
     assert pinv.size == 25 * 12
-    assert lib.is_flat(25, pinv.ctypes.data_as(ctypes.POINTER(ctypes.c_float))) == flat
+    assert lib.four_samples_up_to(25, pinv.ctypes.data_as(ctypes.POINTER(ctypes.c_float))) == row
 
 
 @pytest.mark.parametrize("n,two,one", [(256, 8026, 8026), (192, 8024, 8024), (176, 8026, 8026), (160, 4032, 8023), (144, 4029, 4024),
