@@ -28,7 +28,7 @@ struct ehp_batch {
     std::vector<int64_t> vol_off, sino_off; // n + 1
     bool fused = false;
     int kind = KIND_JOSEPH; // of the fused passes
-    int64_t poses = 0;      // of a problem, on average over the voxels
+    double wait = 0.0;      // ehp::tile_wait of a problem, on average over the voxels
     // fused Siddon passes (device tables; the copy, segment and block tables are shared)
     ehp::SidFwdJob* d_sfjobs = nullptr;
     ehp::SidAdjJob* d_sajobs[3] = {nullptr, nullptr, nullptr};
@@ -105,10 +105,8 @@ namespace
             cus = 256;
         std::vector<ehp::JosephBatchItem> items(n);
         std::vector<double> bounds(n);
-        double rays = 0.0; // voxels times poses
         for (const ehp_op* op : b->ops)
-            rays += (double) op->dims.nvox * op->dims.nposes;
-        b->poses = (int64_t) (rays / b->vol_off.back());
+            b->wait += ehp::tile_wait(op->dims, op->axes_present) * op->dims.nvox / b->vol_off.back();
         for (int j = 0; j < n; ++j) {
             const ehp_op* op = b->ops[j];
             ehp::JosephBatchItem& it = items[j];
@@ -329,13 +327,13 @@ namespace
                 const ehp::SidAdjJob* sj[3] = {b->d_sajobs[0], b->d_sajobs[1], b->d_sajobs[2]};
                 const int* ab[3] = {b->d_ablocks[0], b->d_ablocks[1], b->d_ablocks[2]};
                 if (e == hipSuccess)
-                    e = ehp::siddon_adjoint_batch(b->dim, sj, ab, b->nablocks, b->lds, b->vol_off.back(), b->poses,
+                    e = ehp::siddon_adjoint_batch(b->dim, sj, ab, b->nablocks, b->lds, b->vol_off.back(), b->wait,
                                                   b->d_fixexp, (const float*) in, (float*) out, s);
             } else {
                 const ehp::AdjJob* aj[3] = {b->d_ajobs[0], b->d_ajobs[1], b->d_ajobs[2]};
                 const int* ab[3] = {b->d_ablocks[0], b->d_ablocks[1], b->d_ablocks[2]};
                 e = ehp::joseph_adjoint_batch(b->dim, (int) b->ops.size(), b->d_segs, b->d_sblocks, b->nsblocks,
-                                              b->d_bounds, aj, ab, b->nablocks, b->lds, b->vol_off.back(), b->poses,
+                                              b->d_bounds, aj, ab, b->nablocks, b->lds, b->vol_off.back(), b->wait,
                                               b->d_maxbits, b->d_fixexp, (const float*) in, (float*) out, s);
             }
             return e;

@@ -729,7 +729,7 @@ namespace ehp
         if (e != hipSuccess)
             return e;
         const size_t lds = joseph_tile_lds_bytes(dims, tc, batch);
-        if (pair_launch(axes_present, dims.nvox, dims.nposes)) {
+        if (pair_launch(axes_present, dims.nvox, tile_wait(dims, axes_present))) {
             with_axis_pair(axes_present, [&](auto a0, auto a1) {
                 const TileCounts c0 = axis_tiles(dims, tc, a0), c1 = axis_tiles(dims, tc, a1);
                 if ((int64_t) (c0.per_xcd + c1.per_xcd) * 8 > (int64_t) 0x7fffffff) {
@@ -876,7 +876,7 @@ namespace ehp
 
     hipError_t joseph_adjoint_batch(int dim, int nitems, const SegJob* segs, const int* sblocks, int64_t nsblocks,
                                     const double* bounds, const AdjJob* const ajobs[3], const int* const ablocks[3],
-                                    const int64_t nablocks[3], const size_t lds[3], int64_t nvol_total, int64_t poses,
+                                    const int64_t nablocks[3], const size_t lds[3], int64_t nvol_total, double wait,
                                     unsigned int* d_maxbits, int* d_fixexp, const float* sinos, float* vols,
                                     hipStream_t s)
     {
@@ -888,7 +888,7 @@ namespace ehp
         int axes = 0;
         for (int a = 0; a < dim; ++a)
             axes |= nablocks[a] > 0 ? 1 << a : 0;
-        if (dim == 3 && pair_launch(axes, nvol_total, poses)) {
+        if (dim == 3 && pair_launch(axes, nvol_total, wait)) {
             with_axis_pair(axes, [&](auto a0, auto a1) {
                 const int64_t p0 = (nablocks[a0] + 7) / 8, p1 = (nablocks[a1] + 7) / 8;
                 if ((p0 + p1) * 8 > (int64_t) 0x7fffffff) {

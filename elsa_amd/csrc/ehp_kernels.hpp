@@ -86,10 +86,10 @@ namespace ehp
     void joseph_adjoint_batch_jobs(const JosephBatchItem* items, int n, std::vector<SegJob>& segs,
                                    std::vector<int>& sblocks, std::vector<AdjJob> ajobs[3],
                                    std::vector<int> ablocks[3], size_t lds[3]);
-    // poses: of a problem, on average over the voxels
+    // wait: tile_wait of a problem, on average over the voxels
     hipError_t joseph_adjoint_batch(int dim, int nitems, const SegJob* segs, const int* sblocks, int64_t nsblocks,
                                     const double* bounds, const AdjJob* const ajobs[3], const int* const ablocks[3],
-                                    const int64_t nablocks[3], const size_t lds[3], int64_t nvol_total, int64_t poses,
+                                    const int64_t nablocks[3], const size_t lds[3], int64_t nvol_total, double wait,
                                     unsigned int* d_maxbits, int* d_fixexp, const float* sinos, float* vols,
                                     hipStream_t s);
 
@@ -135,7 +135,7 @@ namespace ehp
     void siddon_adjoint_batch_jobs(const JosephBatchItem* items, int n, std::vector<SidAdjJob> ajobs[3],
                                    std::vector<int> ablocks[3], size_t lds[3]);
     hipError_t siddon_adjoint_batch(int dim, const SidAdjJob* const ajobs[3], const int* const ablocks[3],
-                                    const int64_t nablocks[3], const size_t lds[3], int64_t nvol_total, int64_t poses,
+                                    const int64_t nablocks[3], const size_t lds[3], int64_t nvol_total, double wait,
                                     const int* d_fixexp, const float* sinos, float* vols, hipStream_t s);
 
     // What the 3D voxel kernels know of an operator: the most pixels a footprint is wide (0: the

@@ -342,7 +342,7 @@ namespace ehp
         if (e != hipSuccess)
             return e;
         const size_t lds = siddon_tile_lds_bytes(dims, tc, batch);
-        if (pair_launch(axes_present, dims.nvox, dims.nposes)) {
+        if (pair_launch(axes_present, dims.nvox, tile_wait(dims, axes_present))) {
             with_pair(dims.dim, axes_present, [&](auto d, auto a0, auto a1) {
                 constexpr int D = decltype(d)::value;
                 const TileCounts c0 = axis_tiles(dims, tc, a0), c1 = axis_tiles(dims, tc, a1);
@@ -418,7 +418,7 @@ namespace ehp
     // The tile launches of a batched back projection (the volumes already cleared and the
     // exponents d_fixexp[item] computed by fixed_point_exponent_batch).
     hipError_t siddon_adjoint_batch(int dim, const SidAdjJob* const ajobs[3], const int* const ablocks[3],
-                                    const int64_t nablocks[3], const size_t lds[3], int64_t nvol_total, int64_t poses,
+                                    const int64_t nablocks[3], const size_t lds[3], int64_t nvol_total, double wait,
                                     const int* d_fixexp, const float* sinos, float* vols, hipStream_t s)
     {
         hipError_t e = hipSuccess;
@@ -433,7 +433,7 @@ namespace ehp
         }
         if (most > (int64_t) 0x7fffffff)
             return hipErrorInvalidValue;
-        if (pair_launch(axes, nvol_total, poses)) {
+        if (pair_launch(axes, nvol_total, wait)) {
             with_pair(dim, axes, [&](auto d, auto a0, auto a1) {
                 constexpr int D = decltype(d)::value;
                 const BatchTiles<SidAdjJob> t0 = tiles(a0), t1 = tiles(a1);

@@ -65,18 +65,33 @@ namespace ehp
         return axes == 3 || axes == 5 || axes == 6;
     }
 
-    // Whether the tiles of two driving axes run in one launch, over nvox voxels and `poses` poses. One launch waits
-    // for its slowest tiles once, which grows with the poses; but both axes' tiles then exchange their sums with the
-    // volume by atomics (add_second), about 25 ps a voxel more than reading and writing it. Joseph, us, one launch / two:
-    //   64^3    4 poses   29 / 30    48 poses   71 / 93           128^3   4 poses  125 /  74    24 poses  215 / 194
-    //   96^3    4 poses   64 / 48    12 poses   77 / 76           128^3  48 poses  335 / 332   150 poses  840 / 935
-    //   96^3   24 poses  106 / 122                                256^3  12 poses  993 / 628    48 poses 2154 / 2142
-    //   184^3  12 poses  399 / 265   72 poses 1251 / 1255         256^3 150 poses 6292 / 6523
-    // and Siddon much alike (128^3: 24 poses 218 / 212, 48 poses 362 / 372; 2D 1024^2: 12 poses 59 / 48, 24 75 / 76).
-    inline bool pair_launch(int axes, int64_t nvox, int64_t poses)
+    // What the wait for the slowest tiles of a launch over these driving axes grows with: the poses, a pose's rays over
+    // a voxel's side (the steps of all its rays over the voxels), and the detector's pixels a voxel (the root of that),
+    // which set the tiles near the source apart from those far off.
+    inline double tile_wait(const Dims& dims, int axes)
     {
-        const int64_t small = 1 << 18, large = 1 << 21, most = 48; // 64^3: any number of poses, 128^3 and up: most
-        return two_axes(axes) && (poses >= most || poses * (large - small) >= most * (nvox - small));
+        int side = 0;
+        for (int a = 0; a < dims.dim; ++a)
+            side = (axes & (1 << a)) && dims.vol[a] > side ? dims.vol[a] : side;
+        const double rays = (double) dims.nrays / dims.nposes * side / dims.nvox;
+        return dims.nposes * rays * std::sqrt(rays);
+    }
+
+    // Whether the tiles of two driving axes run in one launch, over nvox voxels, whose slowest tiles are waited for by
+    // `wait` (tile_wait): one launch waits for them once; but both axes' tiles then exchange their sums with the volume
+    // by atomics (add_second), about 25 ps a voxel more than reading and writing it. Joseph, us, one launch / two, by
+    // poses; m: the magnification, the detector 1.6 m^2 rays a pose over the volume's face (fan: 2.6 rays):
+    //   64^3  fan    4    29 /  30    48   71 /  93           128^3 m1.05  48   235 /  220    72   293 /  303
+    //   96^3  fan   12    77 /  76    24  106 / 122           128^3 m2     10   251 /  259    20   420 /  467
+    //   96^3  m1.05 20    80 /  76    32   95 / 101           256^3 fan    24  1265 / 1112    48  2154 / 2142
+    //   96^3  m2    10   117 / 154    20  195 / 274           256^3 m1.05  32  1133 /  863   100  2401 / 2359
+    //   128^3 fan   24   215 / 194    48  335 / 332           256^3 m2     10  1565 / 1634    20  2960 / 3149
+    // 119 x 119 x 154, m2: 20 poses 426 / 528; 300 x 40 x 300, m1.05: 32 poses 323 / 299, 72 poses 555 / 576; and Siddon
+    // much alike (128^3 fan: 24 poses 218 / 212, 48 poses 362 / 372; 2D 1024^2: 12 poses 59 / 48, 24 poses 75 / 76).
+    inline bool pair_launch(int axes, int64_t nvox, double wait)
+    {
+        const double small = 1 << 18, large = 1 << 21, most = 150.0; // 64^3: always, from 128^3 on: most
+        return two_axes(axes) && (wait >= most || wait * (large - small) >= most * ((double) nvox - small));
     }
 
     // Tiles of the smallest launch of a 3D back projection with these driving axes: two run in one launch, one or

@@ -8,7 +8,7 @@ from backends import geom_to_descriptors
 
 pytestmark = pytest.mark.gpu
 
-# volumes of a million voxels, 5 poses: below the 20 from which one launch runs both axes' tiles
+# volumes of a million voxels, 5 poses of few rays: a launch for each axis' tiles
 CASES = {3: ((105, 90, 112), (60, 50)), 2: ((1200, 900), (700,))}
 
 

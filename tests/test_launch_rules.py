@@ -127,12 +127,12 @@ def test_2d_joseph_tiles_of_a_batch(lib, problems, n, side):
     assert lib.batch_tile_2d(n, ctypes.c_int64(problems * n * n), 0) == side
 
 
-@pytest.mark.parametrize("n,least", [(1, 0), (64, 0), (96, 17), (128, 48), (256, 48), (1000, 48)])
-def test_two_axes_in_one_launch(lib, n, least):
-    """From as many poses as pay for the atomics; one or three axes never."""
-    nvox = ctypes.c_int64(n ** 3)
+@pytest.mark.parametrize("n,det,few,many", [(64, 40, 0, 1), (96, 125, 12, 25), (96, 200, 1, 10), (128, 125, 48, 300),
+                                            (128, 208, 24, 48), (128, 320, 5, 10), (256, 335, 32, 72), (256, 640, 5, 10)])
+def test_two_axes_in_one_launch(lib, n, det, few, many):
+    """From as many poses as pay for the atomics, the fewer the larger the detector; one or three axes never."""
     for axes in (3, 5, 6):
-        assert lib.one_launch(axes, nvox, ctypes.c_int64(max(least, 1)))
-        assert least == 0 or not lib.one_launch(axes, nvox, ctypes.c_int64(least - 1))
-    for axes in (0, 1, 2, 4, 7):
-        assert not lib.one_launch(axes, nvox, ctypes.c_int64(1000))
+        assert lib.one_launch(axes, n, det, many)
+        assert few == 0 or not lib.one_launch(axes, n, det, few)
+    for axes in (1, 2, 4, 7):
+        assert not lib.one_launch(axes, n, det, 1000)
