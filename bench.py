@@ -677,8 +677,8 @@ def main():
         if a.kernels == "fast":
             fwd_name = "voxel_fwd_cols_kernel" if wl["dim"] == 3 else "voxel_fwd_tiled_kernel"
         unit, metric = "Gtaps/s", f"{a.projector} voxel projector fwd+adj footprint taps/s & %HBM roofline"
-    # A tiled 3D back projection runs one launch for the tiles of two driving axes; with one or three
-    # axes a launch each, whose durations are not timed one by one: each gets the share of the back
+    # A tiled 3D back projection of these workloads runs one launch for the tiles of two driving axes; with one or
+    # three axes a launch each, whose durations are not timed one by one: each gets the share of the back
     # projection's time that its samples have. The dominant kernel is the one with the longest launch.
     adj_launches = [(adj_name, alg_bytes, t_adj)]  # one pass, timed as a whole
     if a.kernels == "fast" and a.projector == "joseph" and wl["dim"] == 3:

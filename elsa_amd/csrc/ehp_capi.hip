@@ -710,10 +710,11 @@ namespace
 {
     // The scratch of ehp_adjoint_noalloc: the fixed-point scale of one back projection, that is
     // the per-block maxima of |y| (kAbsmaxBlocks 64-bit words) and, kScaleOffset bytes in, the
-    // exponent. Every kernel that reads a word of it writes that word first in the same call
-    // (absmax before scale, scale before the tiles), so nothing needs clearing. One copy per
-    // GPU, held until the process ends; in host code only its device address, looked up per
-    // device, is used.
+    // exponent and the counter of the blocks that have written theirs. The counter is read first
+    // and so cleared by each call; the other words are written before they are read in the same
+    // call (the maxima before the last block reduces them, the exponent before the tiles). One
+    // copy per GPU, held until the process ends; in host code only its device address, looked up
+    // per device, is used.
     constexpr size_t kScaleOffset = ehp::kAbsmaxBlocks * sizeof(unsigned long long);
     constexpr size_t kScratchBytes = kScaleOffset + 256;
     static_assert(kScaleOffset % 256 == 0, "the exponent must be 256-byte aligned");

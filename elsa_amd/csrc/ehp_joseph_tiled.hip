@@ -6,9 +6,9 @@
 // tile for all poses: it accumulates in LDS every sample of every ray whose driving axis is
 // a and whose bilinear footprint touches the tile, then adds the tile to the volume once.
 // Each voxel is owned by exactly one tile per driving axis that occurs in the trajectory. With two
-// such axes, as about any axis of rotation, one launch runs the tiles of both (joseph_adj_pair_kernel:
-// a voxel gets two sums, added by whichever workgroup comes second); otherwise one launch per axis
-// adds to the volume in plain read-modify-write. In 2D a tile takes the rays of both axes
+// such axes, as about any axis of rotation, and rays enough to pay for it (pair_launch), one launch runs the
+// tiles of both (joseph_adj_pair_kernel: a voxel gets two sums, added by whichever workgroup comes second);
+// otherwise one launch per axis adds to the volume in plain read-modify-write. In 2D a tile takes the rays of both axes
 // (adj2d_block) and one launch writes the volume.
 //
 // Accumulation: LDS float atomics are slow on this part (a ds_add_f32 wave operation costs
@@ -71,9 +71,9 @@ namespace ehp
     // ---------------------------------------------------------------------------------
     // fixed-point scale of one back projection
 
-    // Largest |y| in two stages without atomics: each block writes the maximum of its share
-    // as the bit pattern of |y| (for non-negative floats, and NaN above infinity, the integer
-    // order of the bits is the order of the values), one block reduces those.
+    // Largest |y| in two stages: each block writes the maximum of its share as the bit pattern of
+    // |y| (for non-negative floats, and NaN above infinity, the integer order of the bits is the
+    // order of the values), the block that finishes last (counts_last) reduces those.
     template <class U>
     __device__ inline U block_max_bits(U m)
     {
@@ -148,7 +148,7 @@ namespace ehp
     }
 
     // fixexp[0] = the fixed-point exponent eg for the slot bound of the operator. Each block reduces its
-    // share of x; the block that finishes last (fixexp[1] counts them and is 0 between launches)
+    // share of x; the block that finishes last (fixexp[1] counts them, wraps and so is 0 between launches)
     // reduces the blocks' maxima, so that the exponent takes one launch. A block's count releases its
     // maximum to the other XCDs, which costs more than a small block's share: at most one block a CU, of 1024
     // threads. 6.6 million FP32 values: 43 us with 1620 blocks of 256 threads and 4-byte loads, 10.7 with 256
@@ -547,8 +547,8 @@ namespace ehp
     // One launch leaves the device waiting for its last workgroups once instead of twice. Bound by the
     // LDS and VALU together (64-bit atomics, four a sample: the LDS is busy 0.97 of the time, vector
     // instructions 0.85 a cycle and CU), close to the card's power limit: after it the next kernel's clock is a few
-    // percent lower. Workgroups of 512 threads over tiles of 8 x 26 x 26 or 4 x 32 x 32 (64 VGPRs, so that
-    // 32 wavefronts a CU fit), against one launch of 256 threads per axis over 8 x 17 x 17 and 4 x 17 x 17 tiles:
+    // percent lower. Workgroups of 512 threads in 64 VGPRs over tiles of 8 x 26 x 26 (53 KB of LDS: three of them,
+    // 24 wavefronts, a CU) or 4 x 32 x 32 and less (four, 32 wavefronts), against one launch of 256 threads per axis over 8 x 17 x 17 and 4 x 17 x 17 tiles:
     // 256^3 / 360 poses 8.9 -> 8.0 ms, 192^3 / 270 3.05 -> 2.56, 128^3 / 180 0.79 -> 0.61, 96^3 / 120 0.33 -> 0.23,
     // 64^3 / 90 0.142 -> 0.081, FP64 97 x 61 x 113 / 77 0.195 -> 0.17.
     template <int A0, int A1, class ST>

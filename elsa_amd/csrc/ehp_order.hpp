@@ -11,7 +11,9 @@
 //
 // Inside a stream capture (hipGraph) the wait and the record are left out: the capture
 // orders its own nodes, and the stream that captures was ordered after the caller's stream
-// before the capture began. Replays of a captured graph are ordered by the caller.
+// before the capture began. The solvers capture an iteration on a stream of their own and enqueue
+// each replay as a call like any other (SolveOps::ordered); replays of a graph that the caller
+// captured are ordered by the caller.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -5,7 +5,7 @@
 // volume is cut into tiles long along one driving axis, one workgroup owns a tile for all
 // poses and sums in LDS every crossing of every ray (driving along that axis) that passes
 // through it, then adds the tile to the volume once; one launch for the tiles of two driving axes
-// (siddon_adj_pair_kernel), one per axis otherwise.
+// (siddon_adj_pair_kernel) where rays enough pay for it (pair_launch), one per axis otherwise.
 //
 // A ray takes the tile's planes in its own order (sid_tile_ray): its state at the first plane
 // follows from the step counts there, and each plane's segments from sorting two crossing

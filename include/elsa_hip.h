@@ -35,8 +35,9 @@
  *    and its stream first waits for the event recorded after the operator's previous call
  *    when that call went to another stream. A fused batch pass is ordered the same way with
  *    the batch and every operator in it. Calls on different operators run concurrently.
- *    Inside a stream capture (hipGraph) the capture's own order applies; replays of a
- *    captured graph are ordered by the caller.
+ *    Inside a stream capture (hipGraph) the capture's own order applies; replays of a graph
+ *    that the caller captured are ordered by the caller, those of a solver's iteration
+ *    (EHP_SOLVE_GRAPH) by the library like its other calls.
  *  - Host-only helpers (ehp_geometry_pose_*, ehp_*_lut) never touch the GPU.
  */
 #ifndef ELSA_HIP_H
