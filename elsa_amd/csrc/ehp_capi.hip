@@ -271,7 +271,7 @@ namespace
     {
         ehp::TileCfg tc;
         if (dims.dim == 2 && kind == KIND_JOSEPH)
-            return ehp::joseph_tile2d(dims.nvox, cus);
+            return ehp::joseph_tile2d(dims.vol[0], dims.vol[1], cus);
         if (dims.dim == 2)
             tc = dims.nvox >= 512 * (int64_t) cus ? ehp::TileCfg{8, 32, 1}
                                                   : (dims.nvox >= 320 * (int64_t) cus ? ehp::TileCfg{8, 16, 1}

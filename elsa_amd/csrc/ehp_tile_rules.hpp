@@ -22,10 +22,17 @@ namespace ehp
         return TileCfg{(det + nt - 1) / nt, 1, 1};
     }
 
-    // Tiles of an operator's 2D Joseph back projection over nvox voxels on a device of cus compute units
-    inline TileCfg joseph_tile2d(int64_t nvox, int cus)
+    // Tiles of an operator's 2D Joseph back projection over n0 x n1 voxels on a device of cus compute units: 32 x 32 from
+    // one a CU on, where they come out even, that is unless a CU in eight would be idle while the last run. Back
+    // projections, us, with 32 / 16 at 361 poses, magnification 1.05 (3): 512^2 (256 tiles) 109 / 123 (428 / 476),
+    // 560^2 (324) 195 / 137 (803 / 566), 481 x 673 (352) 203 / 153 (816 / 656), 680^2 (484) 201 / 207 (829 / 848), 724^2 (529)
+    // 280 / 219 (992 / 955), 800^2 (625) 315 / 241 (1250 / 1072), 1024^2 (1024) 353 / 357 (1608 / 1673).
+    inline TileCfg joseph_tile2d(int n0, int n1, int cus)
     {
-        const int t = nvox >= (int64_t) 1024 * cus ? 32 : (nvox >= (int64_t) 256 * cus ? 16 : 8);
+        const int64_t nvox = (int64_t) n0 * n1, tiles = (int64_t) ((n0 + 31) / 32) * ((n1 + 31) / 32);
+        const int64_t places = (tiles + cus - 1) / cus * cus;
+        const bool even = 8 * tiles >= 7 * places;
+        const int t = nvox >= (int64_t) 1024 * cus && even ? 32 : (nvox >= (int64_t) 256 * cus ? 16 : 8);
         return TileCfg{t, t, 1};
     }
 

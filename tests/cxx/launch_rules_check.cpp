@@ -52,8 +52,14 @@ extern "C" int refused_tiles_3d(int64_t limit)
 extern "C" int batch_tile_2d(int n, int64_t total, int set_by_caller)
 {
     const int cus = 256;
-    const TileCfg own = joseph_tile2d((int64_t) n * n, cus);
+    const TileCfg own = joseph_tile2d(n, n, cus);
     return batch_tile(own, set_by_caller != 0, joseph_batch_tile2d(total, cus)).LA;
+}
+
+// Side of the tiles of a 2D Joseph back projection over n0 x n1 voxels
+extern "C" int joseph_tile_2d(int n0, int n1)
+{
+    return joseph_tile2d(n0, n1, 256).LA;
 }
 
 // Columns of the kernel for two voxel projectors in one batch: supports, least and largest scalings, table

@@ -120,6 +120,14 @@ def test_2d_voxel_forward_tiles(lib, det, poses, width):
     assert lib.voxel_tile(det, ctypes.c_int64(poses)) == width
 
 
+@pytest.mark.parametrize("n0,n1,side", [(16, 16, 8), (256, 255, 8), (256, 256, 16), (511, 512, 16), (512, 512, 32),
+                                        (481, 673, 16), (560, 560, 16), (640, 690, 16), (680, 680, 32), (704, 704, 32),
+                                        (724, 724, 16), (800, 800, 16), (1024, 1024, 32), (30, 20000, 16)])
+def test_2d_joseph_tiles(lib, n0, n1, side):
+    """Large ones only where the compute units get them in equal numbers."""
+    assert lib.joseph_tile_2d(n0, n1) == side
+
+
 @pytest.mark.parametrize("problems,n,side", [(64, 32, 8), (16, 64, 8), (32, 64, 16), (24, 100, 16), (16, 128, 16),
                                              (32, 128, 16), (63, 128, 16), (64, 128, 32), (64, 512, 32)])
 def test_2d_joseph_tiles_of_a_batch(lib, problems, n, side):
