@@ -106,7 +106,7 @@ namespace
         std::vector<ehp::JosephBatchItem> items(n);
         std::vector<double> bounds(n);
         for (const ehp_op* op : b->ops)
-            b->wait += ehp::tile_wait(op->dims, op->axes_present) * op->dims.nvox / b->vol_off.back();
+            b->wait += op->wait * op->dims.nvox / b->vol_off.back();
         for (int j = 0; j < n; ++j) {
             const ehp_op* op = b->ops[j];
             ehp::JosephBatchItem& it = items[j];

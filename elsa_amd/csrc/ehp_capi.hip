@@ -146,6 +146,8 @@ namespace
         if (e != hipSuccess)
             return hip_fail(e, "sample count");
         op->samples = h;
+        // a ray has about 7/5 as many crossings as samples
+        op->wait = ehp::tile_wait(op->kind == KIND_SIDDON ? h / 1.4 : (double) h, op->dims);
         return EHP_OK;
     }
 } // namespace
@@ -788,19 +790,19 @@ int ehp_adjoint_noalloc(ehp_op* op, const void* d_sino, void* d_vol, void* strea
         return hip_fail(e, "adjoint launch");
     if (siddon && op->dtype == EHP_F32)
         e = ehp::siddon_adjoint_tiled<float>(op->d_geo, op->d_sidtable, dm, op->d_pose_axes, op->axes_present,
-                                             op->tile, op->batch, op->slot_bound, d_maxbits, d_fixexp,
+                                             op->tile, op->batch, op->slot_bound, op->wait, d_maxbits, d_fixexp,
                                              (const float*) d_sino, (float*) d_vol, s);
     else if (siddon)
         e = ehp::siddon_adjoint_tiled<double>(op->d_geo, op->d_sidtable, dm, op->d_pose_axes, op->axes_present,
-                                              op->tile, op->batch, op->slot_bound, d_maxbits, d_fixexp,
+                                              op->tile, op->batch, op->slot_bound, op->wait, d_maxbits, d_fixexp,
                                               (const double*) d_sino, (double*) d_vol, s);
     else if (op->dtype == EHP_F32)
         e = ehp::joseph_adjoint_tiled<float>(op->d_geo, op->d_table, dm, op->d_pose_axes, op->axes_present, op->tile,
-                                             op->batch, op->slot_bound, d_maxbits, d_fixexp, (const float*) d_sino,
+                                             op->batch, op->slot_bound, op->wait, d_maxbits, d_fixexp, (const float*) d_sino,
                                              (float*) d_vol, s);
     else
         e = ehp::joseph_adjoint_tiled<double>(op->d_geo, op->d_table, dm, op->d_pose_axes, op->axes_present,
-                                              op->tile, op->batch, op->slot_bound, d_maxbits, d_fixexp,
+                                              op->tile, op->batch, op->slot_bound, op->wait, d_maxbits, d_fixexp,
                                               (const double*) d_sino, (double*) d_vol, s);
     if (e != hipSuccess)
         return hip_fail(e, "adjoint launch");
@@ -938,7 +940,7 @@ static hipError_t launch(ehp_op* op, const void* in, void* out, hipStream_t s, b
                                                       (const ehp::bf16*) in, (ehp::bf16*) out, s);
         } else {
             e = ehp::joseph_adjoint_tiled<ehp::bf16>(op->d_geo, op->d_table, dm, op->d_pose_axes, op->axes_present,
-                                                     op->tile, op->batch, op->slot_bound, op->d_maxbits, op->d_fixexp,
+                                                     op->tile, op->batch, op->slot_bound, op->wait, op->d_maxbits, op->d_fixexp,
                                                      (const ehp::bf16*) in, op->d_acc32, s);
             if (e == hipSuccess)
                 e = ehp::launch_to_bf16(op->d_acc32, (ehp::bf16*) out, dm.nvox, s);
@@ -948,7 +950,7 @@ static hipError_t launch(ehp_op* op, const void* in, void* out, hipStream_t s, b
         float* y = (float*) out;
         if (op->kind == KIND_JOSEPH && adjoint && op->tiled)
             e = ehp::joseph_adjoint_tiled(op->d_geo, op->d_table, dm, op->d_pose_axes, op->axes_present, op->tile,
-                                          op->batch, op->slot_bound, op->d_maxbits, op->d_fixexp, x, y, s);
+                                          op->batch, op->slot_bound, op->wait, op->d_maxbits, op->d_fixexp, x, y, s);
         else if (op->kind == KIND_JOSEPH && !adjoint && op->planes)
             e = ehp::joseph_forward_planes<float>(op->d_geo, dm, op->layouts, op->d_view, op->axes_present, x, y, s);
         else if (op->kind == KIND_JOSEPH)
@@ -958,7 +960,7 @@ static hipError_t launch(ehp_op* op, const void* in, void* out, hipStream_t s, b
                                                   s);
         else if (op->kind == KIND_SIDDON && adjoint && op->tiled)
             e = ehp::siddon_adjoint_tiled(op->d_geo, op->d_sidtable, dm, op->d_pose_axes, op->axes_present, op->tile,
-                                          op->batch, op->slot_bound, op->d_maxbits, op->d_fixexp, x, y, s);
+                                          op->batch, op->slot_bound, op->wait, op->d_maxbits, op->d_fixexp, x, y, s);
         else if (op->kind == KIND_SIDDON)
             e = adjoint ? ehp::siddon_adjoint<float>(op->d_geo, dm, x, y, s) : ehp::siddon_forward<float>(op->d_geo, dm, x, y, s);
         else if (!adjoint && op->tiled)
@@ -979,7 +981,7 @@ static hipError_t launch(ehp_op* op, const void* in, void* out, hipStream_t s, b
         double* y = (double*) out;
         if (op->kind == KIND_JOSEPH && adjoint && op->tiled)
             e = ehp::joseph_adjoint_tiled<double>(op->d_geo, op->d_table, dm, op->d_pose_axes, op->axes_present,
-                                                  op->tile, op->batch, op->slot_bound, op->d_maxbits, op->d_fixexp, x,
+                                                  op->tile, op->batch, op->slot_bound, op->wait, op->d_maxbits, op->d_fixexp, x,
                                                   y, s);
         else if (op->kind == KIND_JOSEPH && !adjoint && op->planes)
             e = ehp::joseph_forward_planes<double>(op->d_geo, dm, op->layouts, op->d_view, op->axes_present, x, y, s);
@@ -990,7 +992,7 @@ static hipError_t launch(ehp_op* op, const void* in, void* out, hipStream_t s, b
                                                    y, s);
         else if (op->kind == KIND_SIDDON && adjoint && op->tiled)
             e = ehp::siddon_adjoint_tiled<double>(op->d_geo, op->d_sidtable, dm, op->d_pose_axes, op->axes_present,
-                                                  op->tile, op->batch, op->slot_bound, op->d_maxbits, op->d_fixexp, x,
+                                                  op->tile, op->batch, op->slot_bound, op->wait, op->d_maxbits, op->d_fixexp, x,
                                                   y, s);
         else if (op->kind == KIND_SIDDON)
             e = adjoint ? ehp::siddon_adjoint<double>(op->d_geo, dm, x, y, s) : ehp::siddon_forward<double>(op->d_geo, dm, x, y, s);

@@ -683,7 +683,7 @@ namespace ehp
     // FP32 either way.
     template <class ST>
     hipError_t joseph_adjoint_tiled(const PoseGeom* geo, const RayRec* table, const Dims& dims, const int* pose_axes,
-                                    int axes_present, const TileCfg& tc, int batch, double slot_bound,
+                                    int axes_present, const TileCfg& tc, int batch, double slot_bound, double wait,
                                     unsigned int* d_maxbits, int* d_fixexp, const ST* sino,
                                     typename Acc<ST>::type* vol, hipStream_t s)
     {
@@ -729,7 +729,7 @@ namespace ehp
         if (e != hipSuccess)
             return e;
         const size_t lds = joseph_tile_lds_bytes(dims, tc, batch);
-        if (pair_launch(axes_present, dims.nvox, tile_wait(dims, axes_present))) {
+        if (pair_launch(axes_present, dims.nvox, wait)) {
             with_axis_pair(axes_present, [&](auto a0, auto a1) {
                 const TileCounts c0 = axis_tiles(dims, tc, a0), c1 = axis_tiles(dims, tc, a1);
                 if ((int64_t) (c0.per_xcd + c1.per_xcd) * 8 > (int64_t) 0x7fffffff) {
@@ -768,13 +768,13 @@ namespace ehp
     }
 
     template hipError_t joseph_adjoint_tiled<float>(const PoseGeom*, const RayRec*, const Dims&, const int*, int,
-                                                    const TileCfg&, int, double, unsigned int*, int*, const float*,
+                                                    const TileCfg&, int, double, double, unsigned int*, int*, const float*,
                                                     float*, hipStream_t);
     template hipError_t joseph_adjoint_tiled<bf16>(const PoseGeom*, const RayRec*, const Dims&, const int*, int,
-                                                   const TileCfg&, int, double, unsigned int*, int*, const bf16*,
+                                                   const TileCfg&, int, double, double, unsigned int*, int*, const bf16*,
                                                    float*, hipStream_t);
     template hipError_t joseph_adjoint_tiled<double>(const PoseGeom*, const RayRec*, const Dims&, const int*, int,
-                                                     const TileCfg&, int, double, unsigned int*, int*, const double*,
+                                                     const TileCfg&, int, double, double, unsigned int*, int*, const double*,
                                                      double*, hipStream_t);
 
     // Segments of a batch's sinograms (absmax) and the tiles of every operator per driving

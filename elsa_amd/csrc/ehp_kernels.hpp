@@ -220,7 +220,7 @@ namespace ehp
     // d_maxbits: kAbsmaxBlocks 64-bit words.
     template <class ST>
     hipError_t joseph_adjoint_tiled(const PoseGeom* geo, const RayRec* table, const Dims& dims, const int* pose_axes,
-                                    int axes_present, const TileCfg& tc, int batch, double slot_bound,
+                                    int axes_present, const TileCfg& tc, int batch, double slot_bound, double wait,
                                     unsigned int* d_maxbits, int* d_fixexp, const ST* sino,
                                     typename Acc<ST>::type* vol, hipStream_t s);
     template <class T>
@@ -232,7 +232,7 @@ namespace ehp
     size_t siddon_tile_lds_bytes(const Dims& dims, const TileCfg& tc, int batch = kMaxPoseBatch);
     template <class T>
     hipError_t siddon_adjoint_tiled(const PoseGeom* geo, const SidRec* table, const Dims& dims, const int* pose_axes,
-                                    int axes_present, const TileCfg& tc, int batch, double slot_bound,
+                                    int axes_present, const TileCfg& tc, int batch, double slot_bound, double wait,
                                     unsigned int* d_maxbits, int* d_fixexp, const T* sino, T* vol, hipStream_t s);
     size_t voxel_tile_lds_bytes(const TileCfg& tc, size_t lut_bytes = sizeof(float));
     int voxel_max_lut();

@@ -32,6 +32,7 @@ struct ehp_op {
     std::vector<float> host_pix;    // the same in host memory
     bool curved_tiles = false;      // curved detectors: the coordinates allow the tiled back projections
     uint64_t samples = 0;
+    double wait = 0.0; // ehp::tile_wait of the ray-driven projectors
     // Joseph, FP32: plane-major forward and LDS-tiled back projection
     bool planes = false;
     ehp::PadLayout layouts[3]{};

@@ -331,7 +331,7 @@ namespace ehp
 
     template <class T>
     hipError_t siddon_adjoint_tiled(const PoseGeom* geo, const SidRec* table, const Dims& dims, const int* pose_axes,
-                                    int axes_present, const TileCfg& tc, int batch, double slot_bound,
+                                    int axes_present, const TileCfg& tc, int batch, double slot_bound, double wait,
                                     unsigned int* d_maxbits, int* d_fixexp, const T* sino, T* vol, hipStream_t s)
     {
         if (batch < 1 || batch > kMaxPoseBatch)
@@ -342,7 +342,7 @@ namespace ehp
         if (e != hipSuccess)
             return e;
         const size_t lds = siddon_tile_lds_bytes(dims, tc, batch);
-        if (pair_launch(axes_present, dims.nvox, tile_wait(dims, axes_present))) {
+        if (pair_launch(axes_present, dims.nvox, wait)) {
             with_pair(dims.dim, axes_present, [&](auto d, auto a0, auto a1) {
                 constexpr int D = decltype(d)::value;
                 const TileCounts c0 = axis_tiles(dims, tc, a0), c1 = axis_tiles(dims, tc, a1);
@@ -373,10 +373,10 @@ namespace ehp
     }
 
     template hipError_t siddon_adjoint_tiled<float>(const PoseGeom*, const SidRec*, const Dims&, const int*, int,
-                                                    const TileCfg&, int, double, unsigned int*, int*, const float*,
+                                                    const TileCfg&, int, double, double, unsigned int*, int*, const float*,
                                                     float*, hipStream_t);
     template hipError_t siddon_adjoint_tiled<double>(const PoseGeom*, const SidRec*, const Dims&, const int*, int,
-                                                     const TileCfg&, int, double, unsigned int*, int*,
+                                                     const TileCfg&, int, double, double, unsigned int*, int*,
                                                      const double*, double*, hipStream_t);
 
     // The tiles of every operator per driving axis (one job per operator that has rays of that

@@ -72,22 +72,18 @@ namespace ehp
         return axes == 3 || axes == 5 || axes == 6;
     }
 
-    // What the wait for the slowest tiles of a launch over these driving axes grows with: the poses, a pose's rays over
-    // a voxel's side (the steps of all its rays over the voxels), and the detector's pixels a voxel (the root of that),
-    // which set the tiles near the source apart from those far off.
-    inline double tile_wait(const Dims& dims, int axes)
+    // What the wait for the slowest of a launch's tiles grows with: the poses, the samples (Joseph) that a voxel gets from
+    // a pose, and as much again with these, as magnification sets the tiles near the source apart from those far off.
+    inline double tile_wait(double samples, const Dims& dims)
     {
-        int side = 0;
-        for (int a = 0; a < dims.dim; ++a)
-            side = (axes & (1 << a)) && dims.vol[a] > side ? dims.vol[a] : side;
-        const double rays = (double) dims.nrays / dims.nposes * side / dims.nvox;
-        return dims.nposes * rays * std::sqrt(rays);
+        const double rays = samples / ((double) dims.nvox * dims.nposes);
+        return dims.nposes * rays * rays;
     }
 
     // Whether the tiles of two driving axes run in one launch, over nvox voxels, whose slowest tiles are waited for by
     // `wait` (tile_wait): one launch waits for them once; but both axes' tiles then exchange their sums with the volume
     // by atomics (add_second), about 25 ps a voxel more than reading and writing it. Joseph, us, one launch / two, by
-    // poses; m: the magnification, the detector 1.6 m^2 rays a pose over the volume's face (fan: 2.6 rays):
+    // poses; m: the magnification, m^2 rays a voxel's face (fan: 1.7 rays):
     //   64^3  fan    4    29 /  30    48   71 /  93           128^3 m1.05  48   235 /  220    72   293 /  303
     //   96^3  fan   12    77 /  76    24  106 / 122           128^3 m2     10   251 /  259    20   420 /  467
     //   96^3  m1.05 20    80 /  76    32   95 / 101           256^3 fan    24  1265 / 1112    48  2154 / 2142
@@ -97,7 +93,7 @@ namespace ehp
     // much alike (128^3 fan: 24 poses 218 / 212, 48 poses 362 / 372; 2D 1024^2: 12 poses 59 / 48, 24 poses 75 / 76).
     inline bool pair_launch(int axes, int64_t nvox, double wait)
     {
-        const double small = 1 << 18, large = 1 << 21, most = 150.0; // 64^3: always, from 128^3 on: most
+        const double small = 1 << 18, large = 1 << 21, most = 70.0; // 64^3: always, from 128^3 on: most
         return two_axes(axes) && (wait >= most || wait * (large - small) >= most * ((double) nvox - small));
     }
 

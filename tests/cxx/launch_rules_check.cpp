@@ -142,15 +142,12 @@ extern "C" int voxel_tile(int det, int64_t poses)
     return voxel_tile2d(det, poses, 256).LA;
 }
 
-// Whether the back projection of an n^3 volume onto a det x det detector runs the tiles of these driving axes in one launch
-extern "C" int one_launch(int axes, int n, int det, int poses)
+// Whether the back projection of an n^3 volume runs the tiles of these driving axes in one launch; rays: samples that a
+// voxel gets from a pose
+extern "C" int one_launch(int axes, int n, double rays, int poses)
 {
     Dims dims{};
-    dims.dim = 3;
     dims.nposes = poses;
-    for (int i = 0; i < 3; ++i)
-        dims.vol[i] = n;
     dims.nvox = (int64_t) n * n * n;
-    dims.nrays = (int64_t) det * det * poses;
-    return pair_launch(axes, dims.nvox, tile_wait(dims, axes));
+    return pair_launch(axes, dims.nvox, tile_wait(rays * dims.nvox * poses, dims));
 }

@@ -135,12 +135,13 @@ def test_2d_joseph_tiles_of_a_batch(lib, problems, n, side):
     assert lib.batch_tile_2d(n, ctypes.c_int64(problems * n * n), 0) == side
 
 
-@pytest.mark.parametrize("n,det,few,many", [(64, 40, 0, 1), (96, 125, 12, 25), (96, 200, 1, 10), (128, 125, 48, 300),
-                                            (128, 208, 24, 48), (128, 320, 5, 10), (256, 335, 32, 72), (256, 640, 5, 10)])
-def test_two_axes_in_one_launch(lib, n, det, few, many):
-    """From as many poses as pay for the atomics, the fewer the larger the detector; one or three axes never."""
+@pytest.mark.parametrize("n,rays,few,many", [(64, 0.1, 0, 1), (96, 1.0, 20, 32), (96, 3.6, 1, 9), (128, 1.0, 48, 72),
+                                             (128, 1.5, 24, 48), (128, 3.6, 5, 9), (256, 1.0, 48, 72), (256, 8.0, 1, 2)])
+def test_two_axes_in_one_launch(lib, n, rays, few, many):
+    """From as many poses as pay for the atomics, the fewer the denser the rays; one or three axes never."""
+    rays = ctypes.c_double(rays)
     for axes in (3, 5, 6):
-        assert lib.one_launch(axes, n, det, many)
-        assert few == 0 or not lib.one_launch(axes, n, det, few)
+        assert lib.one_launch(axes, n, rays, many)
+        assert few == 0 or not lib.one_launch(axes, n, rays, few)
     for axes in (1, 2, 4, 7):
-        assert not lib.one_launch(axes, n, det, 1000)
+        assert not lib.one_launch(axes, n, rays, 1000)
