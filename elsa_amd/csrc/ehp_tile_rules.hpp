@@ -118,7 +118,9 @@ namespace ehp
     // 3D Joseph tiles: eight planes of up to 26 x 26 voxels, the widths evened over the volume (a large
     // cross-section spends less on the halo and on rays that leave sideways); while a launch of two axes has fewer
     // than eight such tiles a CU, four planes of 32 x 32, below three a CU of 24 x 24 and 16 x 16, and
-    // below one a CU two planes. A launch of one axis: either from 15/16 of four a CU, as four workgroups of
+    // below one a CU two planes. Of 32 x 32 four run on a CU at once: up to an eighth more would keep the launch
+    // waiting for a few (ms, 4x32x32 / 4x23x23: 79 x 158 x 158, 40 poses at magnification 2, 0.81 / 0.70, 18 poses over 60
+    // degrees at 3 1.28 / 1.07). A launch of one axis: either from 15/16 of four a CU, as four workgroups of
     // 512 threads run on a CU and each launch drains by itself. Back projections, us (512 threads):
     //   two axes
     //   256^3 / 360 poses  8x26x26 8015  4x32x32 7978  8x22x22 8080  8x24x24 8626  8x17x17 8873
@@ -149,7 +151,9 @@ namespace ehp
             return tc;
         for (int w = 32; w >= 16; w -= 8) {
             tc = even_tile(dims, 4, w);
-            if (least_launch_tiles(dims, tc, axes) >= enough)
+            const int64_t tiles = least_launch_tiles(dims, tc, axes);
+            const bool spill = pair && w == 32 && tiles > 4 * (int64_t) cus && 2 * tiles < 9 * (int64_t) cus;
+            if (tiles >= enough && !spill)
                 break;
         }
         if (least_launch_tiles(dims, tc, axes) < cus)

@@ -126,6 +126,18 @@ extern "C" int joseph_tile(int n, int axes)
     return t.TB == t.TC ? t.LA * 1000 + t.TB : -1;
 }
 
+// The same of n0 x n1 x n2 voxels with the driving axes 0 and 2
+extern "C" int tile_3d_box(int n0, int n1, int n2)
+{
+    Dims d{};
+    d.dim = 3;
+    d.vol[0] = n0;
+    d.vol[1] = n1;
+    d.vol[2] = n2;
+    const TileCfg t = joseph_tile3d(d, 5, 256);
+    return (t.LA * 100 + t.TB) * 100 + t.TC;
+}
+
 // Parts of the voxel gather's sums and the wavefronts that share them, as parts * 100 + waves
 extern "C" int gather_split(int dim, int64_t nvox, int poses, int width, int f64)
 {

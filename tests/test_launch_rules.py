@@ -120,6 +120,13 @@ def test_2d_voxel_forward_tiles(lib, det, poses, width):
     assert lib.voxel_tile(det, ctypes.c_int64(poses)) == width
 
 
+@pytest.mark.parametrize("n,tile", [((79, 158, 158), 42323), ((96, 184, 100), 42423), ((128, 128, 128), 43232),
+                                    ((139, 128, 121), 43232), ((147, 164, 76), 43028), ((96, 96, 96), 42424)])
+def test_3d_joseph_tiles_of_boxes(lib, n, tile):
+    """A few tiles more than run at once make them smaller."""
+    assert lib.tile_3d_box(*n) == tile
+
+
 @pytest.mark.parametrize("n0,n1,side", [(16, 16, 8), (256, 255, 8), (256, 256, 16), (511, 512, 16), (512, 512, 32),
                                         (481, 673, 16), (560, 560, 16), (640, 690, 16), (680, 680, 32), (704, 704, 32),
                                         (724, 724, 16), (800, 800, 16), (1024, 1024, 32), (30, 20000, 16)])
