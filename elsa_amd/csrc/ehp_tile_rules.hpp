@@ -1,4 +1,5 @@
-// ehp_tile_rules.hpp -- the tiles that launches take by their size, and the order of a forward's.
+// ehp_tile_rules.hpp -- the tiles and wavefronts that launches take by their size, which of them two axes share, and
+// the order of a forward's.
 #pragma once
 
 #include "ehp_joseph_tile.hpp"
