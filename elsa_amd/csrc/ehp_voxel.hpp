@@ -338,11 +338,14 @@ namespace ehp
     // device idle for on small volumes: 92 x 80 blobs, 70 poses 48.3 -> 11.9 us, 300 x 380 / 524 poses 319 -> 147,
     // 36 x 33 x 40 / 40 poses 125 -> 25. In 3D wide footprints (`width` pixels at most) fill the caches: further
     // wavefronts, at other poses, displace the detector rows that a wavefront comes back to. Up to four a SIMD past eight
-    // pixels, one and a half from sixteen on. (FP64's divisions weigh more than its loads: blobs 64^3 / 60 poses, width 13
-    // 2782 us with one, 2493 with two wavefronts.) Blobs in FP32, us, with 1 / 2 / 4 / 8 wavefronts:
-    //   width 11  64^3 / 60 poses  883  926 1032 1019   48^3 / 60  542  422  381  386   40^3 / 40  359  199  176  171
-    //   width 25  64^3 / 60       5312 7706    -    -   48^3 / 60 2704 2981 3893 3704   40^3 / 40 1587  922 1146 1270
-    //             33^3 / 50       2603 1467  886  810   24^3 / 24  920  483  341  192
+    // pixels, 2.4 past sixteen, 1.5 past 24. (FP64's divisions weigh more than its loads: blobs 64^3 / 60 poses, width 13
+    // 2782 us with one, 2493 with two wavefronts.) Blobs in FP32, us, with 1 / 2 / 4 / 8 wavefronts over 360 degrees (and,
+    // as neighbouring poses share rows, 45; columns beside the parts empty):
+    //              width 16                              width 23                              width 31
+    //   64^3 / 60   964 1121 (1551 1722)                 2437 3634 (3886 4231)                 5487 8081 (9121 9016)
+    //   56^3 / 40   525  483  598 (707 570 514)          1243 1561 1979 (1729 1458 1576)       2393 3862 4406 (3186 3581 3663)
+    //   48^3 / 60   635  474  500 (1031 647 485)         1467 1169 1636 (2318 1546 1418)       2759 2992 3911 (4180 2859 3437)
+    //   40^3 / 40   424  228  208  185 (621 366 241 213)  909  495  472  577 (1400 817 552 503) 1580  917 1165 1289
     inline int gather_waves(const Dims& dims, int width, bool f64)
     {
         const int64_t simd = 1024 * 64; // a wavefront each
@@ -350,7 +353,7 @@ namespace ehp
         if (f64 || dims.dim == 2 || width <= kVoxMaxCols)
             return parts;
         int waves = 1;
-        while (waves < parts && dims.nvox * waves < (width < 16 ? 4 * simd : 3 * simd / 2))
+        while (waves < parts && 10 * dims.nvox * waves < (width <= 16 ? 40 : (width <= 24 ? 24 : 15)) * simd)
             waves *= 2;
         return waves;
     }

@@ -102,8 +102,8 @@ def test_3d_joseph_tiles(lib, n, two, one):
 
 @pytest.mark.parametrize("dim,n,poses,width,parts,waves", [
     (3, 64, 60, 5, 2, 2), (3, 64, 60, 8, 2, 2), (3, 64, 60, 9, 2, 1), (3, 64, 60, 25, 2, 1),
-    (3, 48, 60, 5, 4, 4), (3, 48, 60, 11, 4, 4), (3, 48, 60, 16, 4, 1), (3, 40, 40, 5, 8, 8), (3, 40, 40, 15, 8, 8),
-    (3, 40, 40, 16, 8, 2), (3, 24, 24, 25, 4, 4), (3, 8, 1000, 25, 16, 16), (3, 8, 7, 5, 1, 1),
+    (3, 48, 60, 5, 4, 4), (3, 48, 60, 16, 4, 4), (3, 48, 60, 17, 4, 2), (3, 56, 40, 16, 4, 2), (3, 56, 40, 17, 4, 1),
+    (3, 40, 40, 5, 8, 8), (3, 40, 40, 16, 8, 8), (3, 40, 40, 24, 8, 4), (3, 40, 40, 25, 8, 2), (3, 24, 24, 25, 4, 4), (3, 8, 1000, 25, 16, 16), (3, 8, 7, 5, 1, 1),
     (3, 128, 500, 25, 1, 1), (2, 64, 90, 50, 16, 16), (2, 400, 360, 50, 4, 4)])
 def test_parts_of_the_voxel_gather(lib, dim, n, poses, width, parts, waves):
     """A sum's parts follow from its size alone; fewer wavefronts share them for wide footprints in 3D, whose
