@@ -146,8 +146,6 @@ namespace
         if (e != hipSuccess)
             return hip_fail(e, "sample count");
         op->samples = h;
-        // a ray has about 7/5 as many crossings as samples
-        op->wait = ehp::tile_wait(op->kind == KIND_SIDDON ? h / 1.4 : (double) h, op->dims);
         return EHP_OK;
     }
 } // namespace
@@ -403,6 +401,7 @@ namespace
         op->axes_present = 0;
         for (int v : h)
             op->axes_present |= v;
+        op->wait = ehp::tile_wait((double) op->samples, dm, op->host_geo.data(), h.data());
 
         int rc = setup_views(op, h);
         if (rc != EHP_OK)
@@ -475,6 +474,8 @@ namespace
         op->axes_present = 0;
         for (int v : h)
             op->axes_present |= v;
+        // a ray has about 7/5 as many crossings as samples
+        op->wait = ehp::tile_wait(op->samples / 1.4, dm, op->host_geo.data(), h.data());
         // the forward walks plane-major views (one element per voxel) plane by plane
         const int rc = setup_views(op, h);
         if (rc != EHP_OK)

@@ -73,25 +73,53 @@ namespace ehp
         return axes == 3 || axes == 5 || axes == 6;
     }
 
-    // What the wait for the slowest of a launch's tiles grows with: the poses, the samples (Joseph) that a voxel gets from
-    // a pose, and as much again with these, as magnification sets the tiles near the source apart from those far off.
-    inline double tile_wait(double samples, const Dims& dims)
+    // What the wait for the slowest of a launch's tiles over two driving axes grows with: the samples (Joseph) that a
+    // voxel gets, of the poses (pose_axes: their axes) that have the rarer axis, and the spread of the tiles' times, by
+    // the rays' density near the source and far off it in the plane of the axes.
+    inline double tile_wait(double samples, const Dims& dims, const PoseGeom* poses, const int* pose_axes)
     {
-        const double rays = samples / ((double) dims.nvox * dims.nposes);
-        return dims.nposes * rays * rays;
+        int axes = 0, with[3] = {0, 0, 0};
+        for (int p = 0; p < dims.nposes; ++p) {
+            axes |= pose_axes[p];
+            for (int a = 0; a < dims.dim; ++a)
+                with[a] += (pose_axes[p] >> a) & 1;
+        }
+        if (!two_axes(axes))
+            return 0.0;
+        int rarer = dims.nposes;
+        double half2 = 0.0;
+        for (int a = 0; a < dims.dim; ++a) {
+            if (!(axes & (1 << a)))
+                continue;
+            rarer = std::min(rarer, 2 * with[a]);
+            half2 += 0.25 * dims.vol[a] * dims.vol[a];
+        }
+        double spread = 0.0;
+        for (int p = 0; p < dims.nposes; ++p) {
+            double away2 = 0.0;
+            for (int a = 0; a < dims.dim; ++a) {
+                const double c = poses[p].C[a] - 0.5 * dims.vol[a];
+                away2 += c * c;
+            }
+            const double away = std::sqrt(away2), half = std::min(std::sqrt(half2), 0.75 * away);
+            const double ratio = (away + half) / (away - half);
+            spread += ratio * std::sqrt(ratio) / dims.nposes;
+        }
+        return samples / (double) dims.nvox * rarer / dims.nposes * spread;
     }
 
     // Whether the tiles of two driving axes run in one launch, over nvox voxels, whose slowest tiles are waited for by
     // `wait` (tile_wait): one launch waits for them once; but both axes' tiles then exchange their sums with the volume
     // by atomics (add_second), about 25 ps a voxel more than reading and writing it. Joseph, us, one launch / two, by
-    // poses; m: the magnification, m^2 rays a voxel's face (fan: 1.7 rays):
-    //   64^3  fan    4    29 /  30    48   71 /  93           128^3 m1.05  48   235 /  220    72   293 /  303
-    //   96^3  fan   12    77 /  76    24  106 / 122           128^3 m2     10   251 /  259    20   420 /  467
-    //   96^3  m1.05 20    80 /  76    32   95 / 101           256^3 fan    24  1265 / 1112    48  2154 / 2142
-    //   96^3  m2    10   117 / 154    20  195 / 274           256^3 m1.05  32  1133 /  863   100  2401 / 2359
-    //   128^3 fan   24   215 / 194    48  335 / 332           256^3 m2     10  1565 / 1634    20  2960 / 3149
-    // 119 x 119 x 154, m2: 20 poses 426 / 528; 300 x 40 x 300, m1.05: 32 poses 323 / 299, 72 poses 555 / 576; and Siddon
-    // much alike (128^3 fan: 24 poses 218 / 212, 48 poses 362 / 372; 2D 1024^2: 12 poses 59 / 48, 24 poses 75 / 76).
+    // poses; m: the magnification, m^2 rays a voxel's face; s: the source's distance in volume sides:
+    //   64^3  m1.3 s10     4    29 /  30    48   71 /  93     128^3 m1.05 s100  48   235 /  220    72   293 /  303
+    //   96^3  m1.3 s10    12    77 /  76    24  106 / 122     128^3 m1.05 s2    48   (90 degrees)       319 /  413
+    //   96^3  m1.05 s100  20    80 /  76    32   95 / 101     128^3 m2 s2       10   251 /  259    20   420 /  467
+    //   96^3  m2 s2       10   117 / 154    20  195 / 274     200^3 m2 s3       48   (30 degrees, 2 poses with
+    //   128^3 m1.3 s10    24   215 / 194    48  335 / 332                            the rarer axis)   4315 / 4033
+    //   256^3 m1.3 s10    24  1265 / 1112   48 2154 / 2142    256^3 m1.05 s100  32  1133 /  863   100  2401 / 2359
+    //   256^3 m2 s2       10  1565 / 1634   20 2960 / 3149
+    // and Siddon much alike (128^3 m1.3: 24 poses 218 / 212, 48 poses 362 / 372; 2D 1024^2: 12 poses 59 / 48, 24 75 / 76).
     inline bool pair_launch(int axes, int64_t nvox, double wait)
     {
         const double small = 1 << 18, large = 1 << 21, most = 70.0; // 64^3: always, from 128^3 on: most

@@ -155,11 +155,21 @@ extern "C" int voxel_tile(int det, int64_t poses)
 }
 
 // Whether the back projection of an n^3 volume runs the tiles of these driving axes in one launch; rays: samples that a
-// voxel gets from a pose
-extern "C" int one_launch(int axes, int n, double rays, int poses)
+// voxel gets from a pose; away: the source's distance in volume sides; rare: poses with the lowest of the axes
+extern "C" int one_launch(int axes, int n, double rays, int poses, double away, int rare)
 {
     Dims dims{};
+    dims.dim = 3;
+    dims.vol[0] = dims.vol[1] = dims.vol[2] = n;
     dims.nposes = poses;
     dims.nvox = (int64_t) n * n * n;
-    return pair_launch(axes, dims.nvox, tile_wait(rays * dims.nvox * poses, dims));
+    std::vector<PoseGeom> g(poses);
+    std::vector<int> of(poses, axes);
+    for (int p = 0; p < poses; ++p) {
+        for (int a = 0; a < 3; ++a)
+            g[p].C[a] = 0.5f * n + (a == 0 ? (float) away * n : 0.0f);
+        if (p >= rare)
+            of[p] = axes & (axes - 1);
+    }
+    return pair_launch(axes, dims.nvox, tile_wait(rays * dims.nvox * poses, dims, g.data(), of.data()));
 }

@@ -142,13 +142,19 @@ def test_2d_joseph_tiles_of_a_batch(lib, problems, n, side):
     assert lib.batch_tile_2d(n, ctypes.c_int64(problems * n * n), 0) == side
 
 
-@pytest.mark.parametrize("n,rays,few,many", [(64, 0.1, 0, 1), (96, 1.0, 20, 32), (96, 3.6, 1, 9), (128, 1.0, 48, 72),
-                                             (128, 1.5, 24, 48), (128, 3.6, 5, 9), (256, 1.0, 48, 72), (256, 8.0, 1, 2)])
-def test_two_axes_in_one_launch(lib, n, rays, few, many):
-    """From as many poses as pay for the atomics, the fewer the denser the rays; one or three axes never."""
-    rays = ctypes.c_double(rays)
+@pytest.mark.parametrize("n,rays,away,few,many", [
+    (64, 0.1, 100, 0, 1), (96, 1.0, 100, 20, 32), (96, 1.5, 10, 12, 24), (96, 3.6, 2, 2, 10), (128, 1.0, 100, 48, 100),
+    (128, 1.5, 10, 24, 50), (128, 3.6, 2, 5, 9), (128, 1.0, 2, 20, 48), (256, 1.0, 100, 48, 100), (256, 8.0, 3, 4, 9),
+    (256, 8.0, 0.2, 0, 1)])
+def test_two_axes_in_one_launch(lib, n, rays, away, few, many):
+    """From as many poses as pay for the atomics, fewer for denser rays and a nearer source; poses with but one of the
+    axes do not count, and one or three axes never share a launch."""
+    def one(axes, poses, rare=None):
+        return lib.one_launch(axes, n, ctypes.c_double(rays), poses, ctypes.c_double(away), poses if rare is None else rare)
+
     for axes in (3, 5, 6):
-        assert lib.one_launch(axes, n, rays, many)
-        assert few == 0 or not lib.one_launch(axes, n, rays, few)
+        assert one(axes, many) and one(axes, many, (many + 1) // 2)
+        assert few == 0 or not one(axes, few)
+        assert few == 0 or not one(axes, many, max(few // 4, 1) if few > 1 else 0)
     for axes in (1, 2, 4, 7):
-        assert not lib.one_launch(axes, n, rays, 1000)
+        assert not one(axes, 1000)
