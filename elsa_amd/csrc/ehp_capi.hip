@@ -260,14 +260,14 @@ namespace
         return tc;
     }
 
-    // axes: the driving axes that occur; cus: compute units of the device.
-    // 2D Joseph: squares, the largest of 32, 16 and 8 that give every CU a tile (large tiles spend less on their
-    // halo and on rays that only pass a corner; with fewer tiles than CUs the launch waits for its
+    // with: the poses of the driving axes that occur; cus: compute units of the device.
+    // 2D Joseph: squares, the largest of 32, 16 and 8 that give every CU a tile, and as many as the next (large tiles
+    // spend less on their halo and on rays that only pass a corner; with fewer tiles than CUs the launch waits for its
     // slowest tile): 512^2 / 360 poses 32: 109 us, 16: 123; 256^2 / 180 16: 34, 32: 59, 8: 41;
     // 128^2 / 180 8: 26, 16: 34; 64^2 / 90 8: 19, 16: 24.
     // 2D Siddon, in the same way: 500 x 420 / 500 poses 8 x 32: 177 us, 8 x 16: 230, 4 x 16: 336; 320^2 / 300
     // 92, 89, 120; 256^2 / 180 61, 54, 53.
-    ehp::TileCfg default_tile(int kind, const ehp::Dims& dims, int axes, int max_lds, int cus)
+    ehp::TileCfg default_tile(int kind, const ehp::Dims& dims, const ehp::AxisPoses& with, int max_lds, int cus)
     {
         ehp::TileCfg tc;
         if (dims.dim == 2 && kind == KIND_JOSEPH)
@@ -277,7 +277,7 @@ namespace
                                                   : (dims.nvox >= 320 * (int64_t) cus ? ehp::TileCfg{8, 16, 1}
                                                                                       : ehp::TileCfg{4, 16, 1});
         else
-            tc = kind == KIND_SIDDON ? siddon_tile3d(dims, cus) : ehp::joseph_tile3d(dims, axes, cus);
+            tc = kind == KIND_SIDDON ? siddon_tile3d(dims, cus) : ehp::joseph_tile3d(dims, with, cus);
         while (tc.LA > 1 && (int) tile_lds_bytes(kind, dims, tc) > max_lds)
             tc.LA /= 2;
         return tc;
@@ -434,7 +434,7 @@ namespace
         int max_lds = 65536;
         if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, op->device) != hipSuccess)
             max_lds = 65536;
-        op->tile = default_tile(KIND_JOSEPH, dm, op->axes_present, max_lds, device_cus(op->device));
+        op->tile = default_tile(KIND_JOSEPH, dm, ehp::axis_poses(h.data(), n), max_lds, device_cus(op->device));
         op->batch = default_pose_batch(dm);
         op->tiled = true;
         return EHP_OK;
@@ -487,7 +487,7 @@ namespace
         int max_lds = 65536;
         if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, op->device) != hipSuccess)
             max_lds = 65536;
-        op->tile = default_tile(KIND_SIDDON, dm, op->axes_present, max_lds, device_cus(op->device));
+        op->tile = default_tile(KIND_SIDDON, dm, ehp::axis_poses(h.data(), n), max_lds, device_cus(op->device));
         op->batch = default_pose_batch(dm);
         op->tiled = true;
         return EHP_OK;

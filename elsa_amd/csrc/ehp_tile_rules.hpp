@@ -73,27 +73,41 @@ namespace ehp
         return axes == 3 || axes == 5 || axes == 6;
     }
 
+    // The driving axes that occur and, of these, the poses with the rarest and the commonest
+    struct AxisPoses {
+        int axes, least, most;
+    };
+
+    inline AxisPoses axis_poses(const int* pose_axes, int n)
+    {
+        int with[3] = {0, 0, 0};
+        AxisPoses r{0, n, 0};
+        for (int p = 0; p < n; ++p) {
+            r.axes |= pose_axes[p];
+            for (int a = 0; a < 3; ++a)
+                with[a] += (pose_axes[p] >> a) & 1;
+        }
+        for (int a = 0; a < 3; ++a) {
+            if (!(r.axes & (1 << a)))
+                continue;
+            r.least = std::min(r.least, with[a]);
+            r.most = std::max(r.most, with[a]);
+        }
+        return r;
+    }
+
     // What the wait for the slowest of a launch's tiles over two driving axes grows with: the samples (Joseph) that a
     // voxel gets, of the poses (pose_axes: their axes) that have the rarer axis, and the spread of the tiles' times, by
     // the rays' density near the source and far off it in the plane of the axes.
     inline double tile_wait(double samples, const Dims& dims, const PoseGeom* poses, const int* pose_axes)
     {
-        int axes = 0, with[3] = {0, 0, 0};
-        for (int p = 0; p < dims.nposes; ++p) {
-            axes |= pose_axes[p];
-            for (int a = 0; a < dims.dim; ++a)
-                with[a] += (pose_axes[p] >> a) & 1;
-        }
-        if (!two_axes(axes))
+        const AxisPoses with = axis_poses(pose_axes, dims.nposes);
+        if (!two_axes(with.axes))
             return 0.0;
-        int rarer = dims.nposes;
+        const int rarer = std::min(dims.nposes, 2 * with.least);
         double half2 = 0.0;
-        for (int a = 0; a < dims.dim; ++a) {
-            if (!(axes & (1 << a)))
-                continue;
-            rarer = std::min(rarer, 2 * with[a]);
-            half2 += 0.25 * dims.vol[a] * dims.vol[a];
-        }
+        for (int a = 0; a < dims.dim; ++a)
+            half2 += with.axes & (1 << a) ? 0.25 * dims.vol[a] * dims.vol[a] : 0.0;
         double spread = 0.0;
         for (int p = 0; p < dims.nposes; ++p) {
             double away2 = 0.0;
@@ -149,7 +163,8 @@ namespace ehp
     // than eight such tiles a CU, four planes of 32 x 32, below three a CU of 24 x 24 and 16 x 16, and
     // below one a CU two planes. Of 32 x 32 four run on a CU at once: up to an eighth more would keep the launch
     // waiting for a few (ms, 4x32x32 / 4x23x23: 79 x 158 x 158, 40 poses at magnification 2, 0.81 / 0.70, 18 poses over 60
-    // degrees at 3 1.28 / 1.07). A launch of one axis: either from 15/16 of four a CU, as four workgroups of
+    // degrees at 3 1.28 / 1.07). Over a short arc the tiles of one axis have few samples (its poses below 0.7 of the
+    // other's) and the launch waits for the other's: twice as many, and more, of these. A launch of one axis: either from 15/16 of four a CU, as four workgroups of
     // 512 threads run on a CU and each launch drains by itself. Back projections, us (512 threads):
     //   two axes
     //   256^3 / 360 poses  8x26x26 8015  4x32x32 7978  8x22x22 8080  8x24x24 8626  8x17x17 8873
@@ -167,14 +182,21 @@ namespace ehp
     //   128^3              4x22x22 1691  4x32x32 1840  4x16x16 1641  8x16x16 1760
     //   112^3              4x16x16 1184  4x28x28 1567  4x23x23 1210  4x19x19 1096
     //   96^3               4x16x16  854  4x24x24 1054  2x24x24  826
+    //   short arcs, 48 poses: 30 degrees at magnification 2 from three volume sides, and 50 at 1.05 from a hundred
+    //   200^3              8x25x25 3953  4x29x29 3435  4x23x23 3464    8x25x25  619  4x29x29  579  4x23x23  602
+    //   160^3              4x32x32 2024  4x23x23 2100  4x16x16 1977    4x32x32  327  4x23x23  332  4x16x16  357
+    //   128^3              4x32x32 1506  4x22x22 1270  4x16x16 1125    4x32x32  212  4x22x22  216  4x16x16  201
+    //   96^3               4x24x24  734  4x16x16  616  2x16x16  499    4x24x24  133  4x16x16  116  2x16x16  127
     //   one axis, 60 poses
     //   128^3              4x22x22  234  4x32x32  236  4x16x16  214
     //   112^3              4x16x16  170  4x28x28  187  4x19x19  158
-    inline TileCfg joseph_tile3d(const Dims& dims, int axes, int cus)
+    inline TileCfg joseph_tile3d(const Dims& dims, const AxisPoses& with, int cus)
     {
-        const bool pair = two_axes(axes);
+        const int axes = with.axes;
+        const bool pair = two_axes(axes), lopsided = pair && 10 * (int64_t) with.least < 7 * (int64_t) with.most;
         const int64_t alone = 15 * (int64_t) cus / 4;
-        const int64_t deep = pair ? 8 * (int64_t) cus : alone, enough = pair ? 3 * (int64_t) cus : alone;
+        const int64_t deep = pair ? (lopsided ? 16 : 8) * (int64_t) cus : alone;
+        const int64_t enough = pair ? (lopsided ? 8 : 3) * (int64_t) cus : alone;
         TileCfg tc = even_tile(dims, 8, 26);
         if (least_launch_tiles(dims, tc, axes) >= deep)
             return tc;

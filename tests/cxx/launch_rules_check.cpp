@@ -122,19 +122,21 @@ extern "C" int joseph_tile(int n, int axes)
     Dims d{};
     d.dim = 3;
     d.vol[0] = d.vol[1] = d.vol[2] = n;
-    const TileCfg t = joseph_tile3d(d, axes, 256);
+    const TileCfg t = joseph_tile3d(d, AxisPoses{axes, 9, 9}, 256);
     return t.TB == t.TC ? t.LA * 1000 + t.TB : -1;
 }
 
-// The same of n0 x n1 x n2 voxels with the driving axes 0 and 2
-extern "C" int tile_3d_box(int n0, int n1, int n2)
+// The same of n0 x n1 x n2 voxels with the driving axes 0 and 2, the first in `rare` of 100 poses
+extern "C" int tile_3d_box(int n0, int n1, int n2, int rare)
 {
     Dims d{};
     d.dim = 3;
     d.vol[0] = n0;
     d.vol[1] = n1;
     d.vol[2] = n2;
-    const TileCfg t = joseph_tile3d(d, 5, 256);
+    std::vector<int> of(100, 4);
+    std::fill(of.begin(), of.begin() + rare, 5);
+    const TileCfg t = joseph_tile3d(d, axis_poses(of.data(), 100), 256);
     return (t.LA * 100 + t.TB) * 100 + t.TC;
 }
 

@@ -124,7 +124,14 @@ def test_2d_voxel_forward_tiles(lib, det, poses, width):
                                     ((139, 128, 121), 43232), ((147, 164, 76), 43028), ((96, 96, 96), 42424)])
 def test_3d_joseph_tiles_of_boxes(lib, n, tile):
     """A few tiles more than run at once make them smaller."""
-    assert lib.tile_3d_box(*n) == tile
+    assert lib.tile_3d_box(*n, 70) == lib.tile_3d_box(*n, 100) == tile
+
+
+@pytest.mark.parametrize("n,tile", [((200, 200, 200), 42929), ((160, 160, 160), 42323), ((128, 128, 128), 42222),
+                                    ((96, 96, 96), 41616), ((256, 256, 256), 82626), ((51, 51, 206), 41316)])
+def test_3d_joseph_tiles_of_short_arcs(lib, n, tile):
+    """Smaller where one axis has few of the poses."""
+    assert lib.tile_3d_box(*n, 69) == lib.tile_3d_box(*n, 1) == tile
 
 
 @pytest.mark.parametrize("n0,n1,side", [(16, 16, 8), (256, 255, 8), (256, 256, 16), (511, 512, 16), (512, 512, 32),
